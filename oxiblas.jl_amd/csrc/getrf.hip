@@ -26,11 +26,11 @@
 // The leaf runs as one persistent kernel over P workgroups (P co-resident,
 // P <= number of CUs) that each own a contiguous block of rows in registers;
 // per column every workgroup publishes its candidate (key, row and the whole
-// row) as a self-validating record and reads all the others until they are
-// valid (bounded wait with a timeout flag so every wave exits), so all pick
+// row) as a record of tagged words and reads all the others until they are
+// complete (bounded wait with a timeout flag so every wave exits), so all pick
 // the same winner; with P == 1 the exchange stays in LDS (panel.hip).  A
-// small kernel after each leaf applies its interchanges to its multipliers
-// and to the rest of the panel.
+// small kernel after each leaf applies its interchanges to the rest of the
+// panel.
 #include "oxi_internal.hpp"
 
 #include <vector>
@@ -322,6 +322,9 @@ __global__ __launch_bounds__(256) void apply_pairs_cm_kernel(double* __restrict_
 __global__ void zero_i64_kernel(i64* p, int n) {
     for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0;
 }
+__global__ void zero_u64_kernel(unsigned long long* p, i64 n) {
+    for (i64 i = i64(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += i64(gridDim.x) * blockDim.x) p[i] = 0;
+}
 __global__ void zero_i32_kernel(int* p, int n) {
     for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0;
 }
@@ -348,8 +351,8 @@ struct GetrfCtx {
     i64 m, n;
     i64* ipiv;
     i64* dinfo;
-    unsigned long long tag0;   // (call sequence) << 32: tags of the leaf exchange records
-    double* pub;
+    unsigned long long tag0;   // (call sequence) << 32: tags of the tournament leaf's records
+    double* tpub;
     int* pairs;
     int* flags;
     int prec;          // FP32 only: -1 FP32 trailing update, 0 BF16, 1 FP16, 2 FP8 e4m3
@@ -396,19 +399,34 @@ int swap_w(GetrfCtx<T>& g, i64 k1, i64 k2, i64 c0, i64 c1, int inverse) {
 template <typename T>
 int leaf(GetrfCtx<T>& g, i64 c0, int w) {
     const i64 mrows = g.m - c0;
-    // rows per workgroup: 256 (one per thread) up to 8192 rows (32
-    // workgroups), then 512 (two per thread: the most FP64 rows that stay in
-    // registers without spilling); FP32 rows are half the size and go to 1024
-    // per workgroup beyond 16384 rows (more than 32 workgroups of 512)
-    int kind = mrows > 8192 ? 1 : 0;
+    // rows per workgroup: up to 512 rows one workgroup holds all (two rows per
+    // thread from 257 on: 1.64 us a column against 1.77 for two workgroups
+    // that exchange; the tournament leaf exchanges once per leaf and keeps two
+    // workgroups there); then 256 (one per thread) up to 8192 rows (32
+    // workgroups; two rows per thread there: 2.22 us a column against 2.14),
+    // then 512 (at 16384 rows 2.40 us a column on 32 workgroups against 2.60
+    // on 64); FP32 rows are half the size and go to 1024 per workgroup beyond
+    // 16384 rows (more than 32 workgroups of 512)
+    const bool tournament = sizeof(T) == 4 && g.tournament;
+    int kind = mrows > 8192 || (!tournament && mrows > 256 && mrows <= 512) ? 1 : 0;
     if (sizeof(T) == 4 && mrows > 16384) kind = 2;
     const i64 R = kind == 0 ? 256 : kind == 1 ? 512 : 1024;
     const i64 P = cdiv(mrows, R);
     if (P > std::min<i64>(g.h->num_cus, OXI_LEAF_MAX_P))
         return oxi_set_error(g.h, OXI_ERR_UNSUPPORTED, "panel of %lld rows exceeds the leaf kernel capacity",
                              (long long)mrows);
-    LeafArgs a{(void*)g.Wm, g.ldw, c0, w, mrows, g.ipiv, g.dinfo, g.tag0, g.pub, int(P), g.flags, g.pc0, g.pc1};
-    if (sizeof(T) == 4 && g.tournament && kind <= 1 && P <= OXI_TP_MAX_P) return oxi_launch_lu_leaf_tp(g.h, g.s, a, kind);
+    // a leaf's number since the exchange buffer was cleared, 32 tags each; the
+    // buffer is cleared (in stream order, after the last leaf that used it)
+    // before the numbers run out, so no tag occurs twice in it
+    if (g.h->leaf_seq >= (1u << 27) - 1) {
+        hipLaunchKernelGGL(zero_u64_kernel, dim3(256), dim3(256), 0, g.s, g.h->leaf_pub, OXI_LEAF_PUB);
+        OXI_TRY(launch_check(g.h, "leaf exchange clear"));
+        g.h->leaf_seq = 0;
+    }
+    const unsigned tag = ++g.h->leaf_seq << 5;
+    LeafArgs a{(void*)g.Wm, g.ldw, c0, w, mrows, g.ipiv, g.dinfo, g.tag0, g.tpub, tag, g.h->leaf_pub, int(P),
+               g.flags, g.pc0, g.pc1};
+    if (tournament && kind <= 1 && P <= OXI_TP_MAX_P) return oxi_launch_lu_leaf_tp(g.h, g.s, a, kind);
     if (sizeof(T) == 8) OXI_TRY(oxi_launch_lu_leaf(g.h, g.s, a, kind));
     else OXI_TRY(oxi_launch_lu_leaf32(g.h, g.s, a, kind));
     return OXI_OK;
@@ -494,17 +512,13 @@ int getrf_t(oxi_handle_t h, i64 m, i64 n, T* A, i64 lda, i64* ipiv, i64 nb, i64*
     const i64 wide_until = q - (3 * q) / 8;
     auto nb_at = [&](i64 j) { return j < wide_until ? nb_wide : nb; };
 
-    // workspace: [W if rectangular][pub][pairs main][pairs side][low-precision operands]
+    // workspace: [W if rectangular][tournament records][pairs main][pairs side][low-precision operands]
     const bool square = (m == n);
     const i64 ldw = square ? lda : n;
     const size_t wbytes = square ? 0 : size_t(n) * size_t(m) * sizeof(T);
-    // leaf records: column jn < w of workgroup p < P at jn * P + p, the
-    // diagonal rows at w * P + jn (panel_kernel.hpp), P <= OXI_LEAF_MAX_P
-    const size_t pub_doubles = size_t(OXI_LEAF_W) * (size_t(OXI_LEAF_MAX_P) + 1) * OXI_PUB_STRIDE +
-                               size_t(OXI_LEAF_W) * OXI_PUB_STRIDE;
     const size_t pairs_bytes = (size_t(4 * PERM_MAX_STEPS + 4) * 4 + 255) & ~size_t(255);
     const size_t off_pub = (wbytes + 255) & ~size_t(255);
-    const size_t off_pairs = off_pub + ((pub_doubles * 8 + 255) & ~size_t(255));
+    const size_t off_pairs = off_pub + ((size_t(OXI_TP_PUB) * 8 + 255) & ~size_t(255));
     const size_t off_pairs2 = off_pairs + pairs_bytes;
     const size_t off_lowp = off_pairs2 + pairs_bytes;
     const size_t lowp_bytes = (sizeof(T) == 4 && prec >= 0) ? oxi_lowp_update_ws(prec, n, m, nb_wide) : 0;
@@ -516,7 +530,7 @@ int getrf_t(oxi_handle_t h, i64 m, i64 n, T* A, i64 lda, i64* ipiv, i64 nb, i64*
     g.h = h; g.s = s;
     g.Wm = square ? A : (T*)base; g.ldw = ldw;
     g.m = m; g.n = n; g.ipiv = ipiv; g.dinfo = h->dev_info;
-    g.pub = (double*)(base + off_pub);
+    g.tpub = (double*)(base + off_pub);
     g.pairs = (int*)(base + off_pairs);
     g.tag0 = (++h->getrf_seq) << 32;
     g.flags = h->dev_flags;

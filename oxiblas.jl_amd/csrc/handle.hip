@@ -64,7 +64,8 @@ int oxi_create(int device, oxi_handle_t* handle) {
         hipEventCreateWithFlags(&h->ev_b, hipEventDisableTiming) != hipSuccess ||
         hipMalloc(&h->dev_flags, 64 * sizeof(int)) != hipSuccess ||
         hipMalloc(&h->dev_info, 8 * sizeof(i64)) != hipSuccess ||
-        hipMalloc(&h->trsm_inv, size_t(TRSM_INV_BLOCKS) * 4096 * sizeof(double)) != hipSuccess) {
+        hipMalloc(&h->trsm_inv, size_t(TRSM_INV_BLOCKS) * 4096 * sizeof(double)) != hipSuccess ||
+        hipMalloc(&h->leaf_pub, size_t(OXI_LEAF_PUB) * 8) != hipSuccess) {
         oxi_destroy(h);
         return OXI_ERR_HIP;
     }
@@ -86,6 +87,7 @@ int oxi_create(int device, oxi_handle_t* handle) {
     }
     (void)hipMemset(h->dev_flags, 0, 64 * sizeof(int));
     (void)hipMemset(h->dev_info, 0, 8 * sizeof(i64));
+    (void)hipMemset(h->leaf_pub, 0, size_t(OXI_LEAF_PUB) * 8);
     (void)hipDeviceSynchronize();
     *handle = h;
     return OXI_OK;
@@ -104,6 +106,7 @@ int oxi_destroy(oxi_handle_t h) {
     if (h->dev_flags) (void)hipFree(h->dev_flags);
     if (h->dev_info) (void)hipFree(h->dev_info);
     if (h->trsm_inv) (void)hipFree(h->trsm_inv);
+    if (h->leaf_pub) (void)hipFree(h->leaf_pub);
     if (h->ev_a) (void)hipEventDestroy(h->ev_a);
     if (h->ev_b) (void)hipEventDestroy(h->ev_b);
     if (h->ev_c) (void)hipEventDestroy(h->ev_c);

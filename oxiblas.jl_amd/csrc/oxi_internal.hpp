@@ -49,7 +49,11 @@ struct oxi_handle_s {
     double prof_gemm_ms = 0.0, prof_gemm_flops = 0.0;
     i64 prof_gemm_launches = 0;
     int num_cus = 256;
-    unsigned long long getrf_seq = 0;   // getrf calls on this handle (tags the leaf exchange)
+    unsigned long long getrf_seq = 0;   // getrf calls on this handle (tags the tournament leaf's exchange)
+    // exchange buffer of the panel leaves (OXI_LEAF_PUB words) and the leaves
+    // run since it was last cleared: a leaf's words are tagged with its number
+    unsigned long long* leaf_pub = nullptr;
+    unsigned leaf_seq = 0;
 };
 
 int oxi_set_error(oxi_handle_t h, int code, const char* fmt, ...);
@@ -203,8 +207,12 @@ int oxi_first_zero_diag(oxi_handle_t h, hipStream_t s, const double* T, i64 ldt,
 // Panel leaf of the LU (panel.hip)
 // ---------------------------------------------------------------------------
 constexpr int OXI_LEAF_W = 32;      // maximum leaf width
-constexpr int OXI_PUB_STRIDE = 48;  // doubles per published (column, workgroup) record
-constexpr int OXI_LEAF_MAX_P = 127; // workgroups of one leaf (LDS holds P + 1 records per column)
+constexpr int OXI_PUB_STRIDE = 64;  // words per published (column, workgroup) row
+constexpr int OXI_PUB_HDR = 16;     // and of its header (a 128-byte line)
+constexpr int OXI_LEAF_MAX_P = 127; // workgroups of one leaf (LDS holds P rows for two columns)
+// words of the handle's exchange buffer: rows and headers of every column
+constexpr i64 OXI_LEAF_PUB = i64(OXI_LEAF_W) * OXI_LEAF_MAX_P * (OXI_PUB_STRIDE + OXI_PUB_HDR);
+constexpr int OXI_TP_PUB = 4096;    // doubles of the tournament leaf's records
 
 struct LeafArgs {
     void* Wm; i64 ldw;   // double* or float*
@@ -213,8 +221,10 @@ struct LeafArgs {
     i64 mrows;       // rows c0 .. c0+mrows-1 of A
     i64* ipiv;       // global pivots (1-based rows), entries c0..c0+w-1 written
     i64* info;       // device info (first zero pivot, 1-based), 0 if none
-    unsigned long long tag0;  // (getrf call sequence) << 32; column c's records carry tag0 + c
-    double* pub;     // published records [w][P][PUB_STRIDE] + diag rows [w][PUB_STRIDE]
+    unsigned long long tag0;  // tournament leaf: (getrf call sequence) << 32, the tags' base
+    double* tpub;    // tournament leaf: its records
+    unsigned tag;    // column j's words carry tag + j
+    unsigned long long* pub;  // published rows [w][P][PUB_STRIDE], then headers [w][P][PUB_HDR]
     int P;
     int* flags;      // flags[0] = 1 on barrier timeout
     i64 xlo, xhi;    // columns [xlo, xhi) of the enclosing panel: receive the leaf's interchanges

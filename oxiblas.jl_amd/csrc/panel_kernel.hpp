@@ -11,38 +11,8 @@ namespace {
 
 typedef unsigned long long u64;
 
-// Pivot key with the reference's strict '>' scan semantics: NaN in the
-// diagonal position wins (nothing compares greater), NaN elsewhere never wins.
-__device__ __forceinline__ double pivot_key(double v, bool diag) {
-    double a = __builtin_fabs(v);
-    if (a != a) return diag ? __builtin_huge_val() : -1.0;
-    return a;
-}
 __device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
 __device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-__device__ __forceinline__ bool better(double k1, long long r1, double k2, long long r2) {
-    return k1 > k2 || (k1 == k2 && r1 < r2);
-}
-
-// ---------------------------------------------------------------------------
-// Cross-workgroup exchange of one pivot column: self-validating records.
-//
-// Every workgroup publishes one record per column: its best candidate (key,
-// row) and that row's w values, plus a tag (getrf call and global column) and
-// a checksum over all other fields keyed by the tag.  Every workgroup then
-// loads all records and accepts a record only when its checksum matches what
-// the fields and the expected tag give; it reloads the others until all are
-// valid.  Nothing orders the writer's stores: a record that is still partly
-// old (an earlier column or call) fails its checksum and is simply read
-// again, so one round trip suffices once the last record has landed.  The
-// data goes through device-scope (agent) relaxed stores and loads, which are
-// coherent across XCDs without the L2 write-back / invalidate that an
-// agent-scope release / acquire pair costs.
-// ---------------------------------------------------------------------------
-constexpr int REC_N = 4 + OXI_LEAF_W;           // key, row, tag, 32 values, checksum
-constexpr int REC_CHK = REC_N - 1;
-constexpr int REC_SLOTS = OXI_LEAF_MAX_P + 1;   // records per column: P candidates + the diagonal row
-static_assert(REC_N == 36, "load9_agent reads 9 fields per lane");
 
 __device__ __forceinline__ void put_agent(double* p, double v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -52,460 +22,627 @@ __device__ __forceinline__ double get_agent(const double* p) {
 }
 __device__ __forceinline__ u64 bits(double v) { return __builtin_bit_cast(u64, v); }
 __device__ __forceinline__ double from_bits(u64 v) { return __builtin_bit_cast(double, v); }
-// Nine device-scope loads 32 bytes apart (one lane's fields of a record),
-// issued back to back and waited for once.  Relaxed atomic loads written in
-// C++ are issued one at a time, each waited for before the next.
-__device__ __forceinline__ void load9_agent(const double* p, double (&f)[9]) {
-    asm volatile(
-        "global_load_dwordx2 %0, %9, off sc1\n\t"
-        "global_load_dwordx2 %1, %9, off offset:32 sc1\n\t"
-        "global_load_dwordx2 %2, %9, off offset:64 sc1\n\t"
-        "global_load_dwordx2 %3, %9, off offset:96 sc1\n\t"
-        "global_load_dwordx2 %4, %9, off offset:128 sc1\n\t"
-        "global_load_dwordx2 %5, %9, off offset:160 sc1\n\t"
-        "global_load_dwordx2 %6, %9, off offset:192 sc1\n\t"
-        "global_load_dwordx2 %7, %9, off offset:224 sc1\n\t"
-        "global_load_dwordx2 %8, %9, off offset:256 sc1\n\t"
-        "s_waitcnt vmcnt(0)"
-        : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3]), "=&v"(f[4]), "=&v"(f[5]), "=&v"(f[6]), "=&v"(f[7]),
-          "=&v"(f[8])
-        : "v"(p)
-        : "memory");
-}
-// field f's share of the checksum (fields 0 .. REC_N-2)
+// field f's share of a record's checksum, keyed by the tag (tournament leaf)
 __device__ __forceinline__ u64 rec_term(u64 b, u64 tag, int f) {
     return (b ^ (tag * 0x9E3779B97F4A7C15ull + u64(f + 1) * 0xD1B54A32D192ED03ull)) * 0x94D049BB133111EBull;
 }
-
-// ---------------------------------------------------------------------------
-// Cross-lane helpers (DPP: data moves inside the VALU, no LDS round trip).
-// ---------------------------------------------------------------------------
-template <int CTRL, int ROWM = 0xf, int BANKM = 0xf>
-__device__ __forceinline__ u64 dpp64(u64 x) {
-    // lanes whose source is outside the row (or masked off) keep their own value
-    const int lo = __builtin_amdgcn_update_dpp(int(unsigned(x)), int(unsigned(x)), CTRL, ROWM, BANKM, false);
-    const int hi = __builtin_amdgcn_update_dpp(int(unsigned(x >> 32)), int(unsigned(x >> 32)), CTRL, ROWM, BANKM, false);
-    return (u64(unsigned(hi)) << 32) | unsigned(lo);
-}
-template <int CTRL, int ROWM = 0xf, int BANKM = 0xf>
-__device__ __forceinline__ double dppd(double x) { return from_bits(dpp64<CTRL, ROWM, BANKM>(bits(x))); }
 __device__ __forceinline__ u64 readlane64(u64 x, int l) {
     const unsigned lo = __builtin_amdgcn_readlane(unsigned(x), l), hi = __builtin_amdgcn_readlane(unsigned(x >> 32), l);
     return (u64(hi) << 32) | lo;
 }
-// maximum over the 64 lanes of a wave (all lanes active, no NaN), in every lane:
-// inclusive prefix maxima inside each row of 16, then across rows to lane 63
-__device__ __forceinline__ double wave_max(double x) {
-    x = __builtin_fmax(x, dppd<0x111>(x));         // row_shr:1
-    x = __builtin_fmax(x, dppd<0x112>(x));         // row_shr:2
-    x = __builtin_fmax(x, dppd<0x114>(x));         // row_shr:4
-    x = __builtin_fmax(x, dppd<0x118>(x));         // row_shr:8
-    x = __builtin_fmax(x, dppd<0x142, 0xa>(x));    // row_bcast:15 into rows 1, 3
-    x = __builtin_fmax(x, dppd<0x143, 0xc>(x));    // row_bcast:31 into rows 2, 3
-    return from_bits(readlane64(bits(x), 63));
-}
-// XOR over the 16 lanes of each row, in every lane of the row
-__device__ __forceinline__ u64 row_xor16(u64 h) {
-    h ^= dpp64<0x128>(h);   // row_ror:8
-    h ^= dpp64<0x124>(h);   // row_ror:4
-    h ^= dpp64<0x122>(h);   // row_ror:2
-    h ^= dpp64<0x121>(h);   // row_ror:1
-    return h;
-}
-// XOR over each quad of lanes, and a quad member's value, in every lane of the quad
-__device__ __forceinline__ u64 quad_xor(u64 h) {
-    h ^= dpp64<0xB1>(h);    // quad_perm [1,0,3,2]
-    h ^= dpp64<0x4E>(h);    // quad_perm [2,3,0,1]
-    return h;
-}
-template <int SEL>
-__device__ __forceinline__ u64 quad_bcast(u64 x) { return dpp64<SEL * 0x55>(x); }   // quad_perm [SEL x 4]
 __device__ __forceinline__ int first_lane(u64 m) { return int(__builtin_ctzll(m)); }
 
-// Publish one record by the 16 lanes of a row of a wave: lane L stores fields
-// L, L + 16 and L + 32 (the checksum is field 35 = lane 3's third) with
-// device-scope stores; the checksum is reduced across the row.  Fields: key
-// k0, row k1, the tag, then the w values row[0 .. 31] (LDS) when has, else
-// zeros.  Branch-free: every lane reads its three row values (clamped into
-// the row) and selects.
-__device__ __forceinline__ void publish16(double* rec, u64 tag, int L, const double* row, bool has, double k0,
-                                          double k1) {
-    const double r0 = row[L < 3 ? 0 : L - 3], r1 = row[L + 13], r2 = row[L < 3 ? L + 29 : OXI_LEAF_W - 1];
-    const double f0 = L == 0 ? k0 : L == 1 ? k1 : L == 2 ? from_bits(tag) : has ? r0 : 0.0;
-    const double f1 = has ? r1 : 0.0;
-    const double f2 = has ? r2 : 0.0;
-    u64 h = rec_term(bits(f0), tag, L) ^ rec_term(bits(f1), tag, L + 16);
-    if (L < 3) h ^= rec_term(bits(f2), tag, L + 32);
-    h = row_xor16(h);
-    put_agent(&rec[L], f0);
-    put_agent(&rec[L + 16], f1);
-    if (L < 4) put_agent(&rec[L + 32], L < 3 ? f2 : from_bits(h));
+// ---------------------------------------------------------------------------
+// Pivot keys.  The search compares the high words of |value| (for FP32 the
+// whole |value|) as integers, which order like the values; equal high words
+// (rare) are settled by the low word and then by the position.  Semantics of
+// the reference's strict '>' scan from the diagonal down: NaN in the diagonal
+// position wins (nothing compares greater), NaN elsewhere never wins.
+// ---------------------------------------------------------------------------
+constexpr int KEY_NONE = -2;             // no candidate
+__device__ __forceinline__ unsigned word_hi(double v) { return unsigned(bits(v) >> 32); }
+__device__ __forceinline__ unsigned word_lo(double v) { return unsigned(bits(v)); }
+__device__ __forceinline__ unsigned word_hi(float v) { return __builtin_bit_cast(unsigned, v); }
+__device__ __forceinline__ unsigned word_lo(float) { return 0u; }
+template <typename T> __device__ __forceinline__ T from_words(unsigned lo, unsigned hi);
+template <> __device__ __forceinline__ double from_words<double>(unsigned lo, unsigned hi) {
+    return from_bits((u64(hi) << 32) | lo);
+}
+template <> __device__ __forceinline__ float from_words<float>(unsigned, unsigned hi) {
+    return __builtin_bit_cast(float, hi);
+}
+template <typename T> constexpr int KEY_INF = sizeof(T) == 8 ? 0x7ff00000 : 0x7f800000;
+template <typename T>
+__device__ __forceinline__ int pivot_key(T v, bool diag) {
+    const int k = int(word_hi(v) & 0x7fffffffu);
+    return v != v ? (diag ? KEY_INF<T> : -1) : k;
+}
+template <typename T>
+__device__ __forceinline__ unsigned pivot_key_lo(T v) { return v != v ? 0u : word_lo(v); }
+// exponent all ones (infinity or NaN)
+template <typename T>
+__device__ __forceinline__ bool non_finite(T v) { return (word_hi(v) & unsigned(KEY_INF<T>)) == unsigned(KEY_INF<T>); }
+
+template <int CTRL, int ROWM = 0xf>
+__device__ __forceinline__ int dpp_imax(int x) {
+    // lanes whose source is outside the row (or masked off) keep their own
+    // value; with the maximum's identity as the old value it is one instruction
+    return max(x, __builtin_amdgcn_update_dpp(-0x7fffffff - 1, x, CTRL, ROWM, 0xf, false));
+}
+// maximum over the 64 lanes of a wave, in every lane: inclusive prefix maxima
+// inside each row of 16, then across rows to lane 63
+__device__ __forceinline__ int wave_imax(int x) {
+    x = dpp_imax<0x111>(x);         // row_shr:1
+    x = dpp_imax<0x112>(x);         // row_shr:2
+    x = dpp_imax<0x114>(x);         // row_shr:4
+    x = dpp_imax<0x118>(x);         // row_shr:8
+    x = dpp_imax<0x142, 0xa>(x);    // row_bcast:15 into rows 1, 3
+    x = dpp_imax<0x143, 0xc>(x);    // row_bcast:31 into rows 2, 3
+    return __builtin_amdgcn_readlane(x, 63);
+}
+// The lane, among those with `tie` set, whose (low word, position) wins: the
+// largest low word, then the lowest position (uniform; tie != 0).
+__device__ __forceinline__ int settle_tie(u64 tie, unsigned lo, int pos) {
+    int best = first_lane(tie);
+    unsigned blo = __builtin_amdgcn_readlane(lo, best);
+    int bpos = __builtin_amdgcn_readlane(pos, best);
+    for (tie &= tie - 1; tie; tie &= tie - 1) {
+        const int l = first_lane(tie);
+        const unsigned l_lo = __builtin_amdgcn_readlane(lo, l);
+        const int l_pos = __builtin_amdgcn_readlane(pos, l);
+        if (l_lo > blo || (l_lo == blo && l_pos < bpos)) { best = l; blo = l_lo; bpos = l_pos; }
+    }
+    return best;
+}
+template <typename T>
+__device__ __forceinline__ T readlane_t(T v, int l) {
+    if constexpr (sizeof(T) == 8) return from_bits(readlane64(bits(v), l));
+    else return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+}
+
+// x of lane N of each row of 16 lanes, in every lane of the row
+template <int N> __device__ __forceinline__ double row_bcast(double x) {
+    return __builtin_amdgcn_update_dpp(0.0, x, 0x150 + N, 0xf, 0xf, true);   // row_newbcast:N
+}
+template <int N> __device__ __forceinline__ float row_bcast(float x) {
+    return __builtin_amdgcn_update_dpp(0.0f, x, 0x150 + N, 0xf, 0xf, true);
+}
+// lane i + 1's x in lane i of each row of 16 lanes (lane 15: zero)
+__device__ __forceinline__ float row_shl1(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x101, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double row_shl1(double x) {
+    const u64 b = bits(x);
+    const unsigned lo = unsigned(__builtin_amdgcn_update_dpp(0, int(unsigned(b)), 0x101, 0xf, 0xf, true));
+    const unsigned hi = unsigned(__builtin_amdgcn_update_dpp(0, int(unsigned(b >> 32)), 0x101, 0xf, 0xf, true));
+    return from_bits((u64(hi) << 32) | lo);
+}
+// d = c - a * b with a destination of its own: the rotated update would else
+// become the two-operand form and a move per register
+__device__ __forceinline__ double nfma_to(double a, double b, double c) {
+    double d;
+    asm("v_fma_f64 %0, -%1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+    return d;
+}
+__device__ __forceinline__ float nfma_to(float a, float b, float c) {
+    float d;
+    asm("v_fma_f32 %0, -%1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+    return d;
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (N > 0) {
+        static_for<N - 1>(f);
+        f(std::integral_constant<int, N - 1>{});
+    }
 }
 
 // ---------------------------------------------------------------------------
-// The leaf kernel.  Thread t of workgroup p owns the row at position
-// p*R + s*LT + t (s < RPT) in registers.  The registers of a row rotate by
-// one per column: at column j register c holds column j + c, so the pivot
-// column is always register 0 and the rank-1 update is the same 31 FMAs at
-// every step (v[c] <- fma(-l, u[c+1], v[c+1])).  The column loop is rolled
-// and every register index is a compile-time constant.
+// Cross-workgroup exchange of one pivot column: tagged words.
+//
+// Every workgroup publishes one record per column: its best candidate row, as
+// eight-byte words { 32 data bits, 32-bit tag }, word 2c the low half of
+// value c and word 2c + 1 the high half, stored by the 64 lanes of one wave
+// in one instruction, and a header of six words in a 128-byte line of its
+// own: values 0 and 1 again and the row's position.  (Headers that share a
+// line cost up to 0.35 us an exchange at 32 workgroups: the writes of
+// different XCDs to one line follow one another.)  Everyone polls the headers
+// only; the winner's row is fetched while the multipliers and the next
+// candidates are computed.  An eight-byte store is seen whole, so a word
+// whose tag is the column's carries the column's data whatever the order in
+// which the stores land: no checksum and no fence.  Tags are unique over
+// everything that the exchange buffer has held since it was last cleared
+// (getrf.hip).  The data goes through device-scope (agent) relaxed stores and
+// loads, which are coherent across XCDs without the L2 write-back /
+// invalidate that an agent-scope release / acquire pair costs.
+// ---------------------------------------------------------------------------
+typedef unsigned uint4v __attribute__((ext_vector_type(4)));
+constexpr int NO_POS = 0x7fffffff;       // a header's position when the workgroup has no candidate
+// Three device-scope 16-byte loads (two words each), issued back to back and
+// waited for once.  Relaxed atomic loads written in C++ are issued one at a
+// time, each waited for before the next.
+__device__ __forceinline__ void load_words3(const u64* p0, const u64* p1, const u64* p2, uint4v& r0, uint4v& r1,
+                                            uint4v& r2) {
+    asm volatile(
+        "global_load_dwordx4 %0, %3, off sc1\n\t"
+        "global_load_dwordx4 %1, %4, off sc1\n\t"
+        "global_load_dwordx4 %2, %5, off sc1\n\t"
+        "s_waitcnt vmcnt(0)"
+        : "=&v"(r0), "=&v"(r1), "=&v"(r2) : "v"(p0), "v"(p1), "v"(p2) : "memory");
+}
+// The same load for one that the compiler waits for where it is used.
+__device__ __forceinline__ uint4v load_words_ahead(__amdgpu_buffer_rsrc_t r, unsigned off_bytes) {
+    return __builtin_bit_cast(uint4v, __builtin_amdgcn_raw_buffer_load_b128(r, int(off_bytes), 0, 16));   // sc1
+}
+// A workgroup barrier that orders LDS only: __syncthreads would also wait for
+// the record's stores to be acknowledged.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// ---------------------------------------------------------------------------
+// The leaf kernel.  Thread t of workgroup p holds the rows that start at
+// positions p*R + s*LT + t (s < RPT) in registers, and they stay there: an
+// interchange only changes positions (pos[s]; a row that became the pivot of
+// step j is retired to position j, pos[s] = ~j).  The registers of a row
+// rotate by one per column: at column j register c holds column j + c, so the
+// pivot column is always register 0, the rank-1 update is the same 31 FMAs at
+// every step (v[c] <- v[c+1] - l u[c+1]), and every register index is a
+// compile-time constant in a rolled loop; the multiplier enters at register 31.
+// After 32 rotations register c holds column c again, multipliers and U values
+// alike, and every row is stored once, at its final position: no store and no
+// interchange inside the column loop.  (u is zero past the row's live
+// columns, so the multipliers of earlier columns pass through the update
+// unchanged; from the first step that meets an infinity or NaN, or a zero
+// pivot, the update takes a select per value.)
 //
 // The exchange of column j+1 is overlapped with the update of column j: once
 // the multipliers of column j are known, every row computes only its next
-// column (register 1 after the update), the candidates for column j+1 are
-// chosen from those values, the candidate rows (and position j+1's row) are
-// updated on their own and published, and only then do all rows take the
-// full update while the records travel.
+// column, the candidates for column j+1 are chosen from those values, the
+// chosen row is updated on its own (one column per lane) and published, and
+// only then do all rows take the full update while the records travel.  One
+// barrier per column, for the comparison of the waves' candidates: every wave
+// reads all the headers itself and picks the winner in registers.
 //
-// Values leave the registers as they become final: the multiplier of column
-// j goes to memory at step j (at the row's position at that time), and the
-// pivot row at position j goes to memory at step j (later interchanges only
-// involve positions below j).  Interchanges of later steps are applied to
-// the stored multipliers afterwards by leaf_swaps_kernel, as getrf2 applies
-// the right half's interchanges to the left half.
+// WGS 1: one workgroup holds all the rows.  Each wave's candidate row
+// goes to LDS before that barrier, and every wave updates the winner's copy
+// itself.
+//
+// A column is a chain of dependent steps in one wave per SIMD, bound by
+// instruction and LDS latency plus one exchange between workgroups (1.1 us
+// alone for 32 of them).  Measured per FP64 column, 32 columns, launch
+// included: 1.23 us at 256 rows, 1.62 at 512 (one workgroup), 1.91 at 2048, 2.2
+// at 8192, 2.4 at 16384 rows.  Rows that move between threads at every
+// interchange, 64-bit keys, checksummed records and multipliers stored column
+// by column took 1.9, 3.4 (2048), 4.1 (8192) and 4.6 us (16384) inside an LU.
+// At 16384 rows a column's critical path is 0.1 us to the winner, 0.1 to the
+// multipliers, 0.2-0.3 to the wave's candidate, 0.2 across the barrier, 0.2 to
+// the header, then the exchange; the row's trip through LDS and the update
+// run in the exchange's shadow.
 // ---------------------------------------------------------------------------
-template <typename T, int LTT, int RPT>
+template <typename T, int LTT, int RPT, int WGS>
 __global__ __launch_bounds__(LTT) void lu_leaf_kernel(LeafArgs a) {
     constexpr int LT = LTT, NWV = LT / 64, W = OXI_LEAF_W;
-    constexpr int RPW = 16;                           // records one wave validates per pass (4 lanes each)
-    constexpr int PASS = NWV * RPW;
-    constexpr int NPASS_MAX = (REC_SLOTS + PASS - 1) / PASS;
-    constexpr unsigned SPIN_LIMIT = 1u << 22;
-    __shared__ double wkey[2][NWV];
-    __shared__ long long wrow[2][NWV];
-    // LDS copies of records keep field f at offset f + 1 of a 40-double slot,
-    // so that the row values (fields 3..34) start 16-byte aligned
-    constexpr int RS_N = 40;
-    __shared__ __align__(16) double wvals[2][NWV + 1][W];        // each wave's best row; [NWV]: position j
-    __shared__ __align__(16) double rec_sh[2][REC_SLOTS * RS_N];  // gathered records, by column parity
-    __shared__ __align__(16) double raw[NWV + 1][W];              // candidate rows before the pending update
-    __shared__ double raw_l[NWV + 1];                            // and their multipliers
-    __shared__ long long lrow_sh[2];                  // P == 1: the winner's position
-    __shared__ int lw_sh[2];                          // P == 1: the winner's wave
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int p = blockIdx.x;
-    const i64 R = i64(LT) * RPT;
+    static_assert(W == 32 && NWV == 4, "record and wave layout");
+    constexpr bool MULTI = WGS != 1;                  // WGS: 1, 64 or OXI_LEAF_MAX_P workgroups at most
+    unsigned spin_limit = 1u << 22;                   // bound of every wait
+    asm volatile("" : "+s"(spin_limit));              // not a constant: the polling loops stay rolled
+    constexpr int RS_N = W + 16 / int(sizeof(T));     // a row's LDS stride: 16-byte aligned, few bank conflicts
+    __shared__ __align__(16) T rows[2][NWV * RS_N];                // !MULTI: the waves' candidate rows, by column parity
+    __shared__ __align__(16) int4 wcand[2][NWV];                   // each wave's candidate: key, low word, position; failed
+    __shared__ __align__(16) T raw[W];                             // MULTI: the chosen row before the pending update
+    __shared__ T raw_l[2][NWV];                                    // else: the candidates' multipliers
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int p = blockIdx.x, P = a.P;
     const int w = a.w;
-    const bool global_x = a.P > 1;
-    // polling slots of the record exchange (see gather); vmask is first
-    // used after the barrier of the first select_publish
-    __shared__ u64 vmask[2][2];   // validated records of the column, by column parity
-    if (t < 4) vmask[t >> 1][t & 1] = 0;
-    const int P1 = a.P + 1;
-    const u64 full0 = P1 >= 64 ? ~0ull : (1ull << P1) - 1;
-    const u64 full1 = P1 <= 64 ? 0ull : P1 >= 128 ? ~0ull : (1ull << (P1 - 64)) - 1;
-    const int slot = wave * RPW + (lane >> 2);
-    int qs[NPASS_MAX];   // records of this lane's slot; P1 = none
-#pragma unroll
-    for (int ps = 0; ps < NPASS_MAX; ++ps) qs[ps] = min(ps * PASS + slot, P1);
+    const int R = LT * RPT;
 
     T v[RPT][W];
     T* Wm = (T*)a.Wm;
-    i64 lr[RPT];
-    T* wrow_of[RPT];   // this position's row of W (leaf column 0)
+    int pos[RPT];
 #pragma unroll
     for (int s = 0; s < RPT; ++s) {
-        lr[s] = i64(p) * R + i64(s) * LT + t;
-        const bool ok = lr[s] < a.mrows;
-        wrow_of[s] = Wm + a.c0 + (a.c0 + lr[s]) * a.ldw;
+        const int lr = p * R + s * LT + t;
+        const bool ok = lr < a.mrows;
+        pos[s] = ok ? lr : -0x40000000;               // no row: never a candidate, never stored
+        const T* row = Wm + a.c0 + (a.c0 + (ok ? lr : 0)) * a.ldw;
+        if (w == W) {   // a full leaf: wide loads (a thread without a row reads the first one)
 #pragma unroll
-        for (int c = 0; c < W; ++c) v[s][c] = (ok && c < w) ? wrow_of[s][c] : T(0);
+            for (int c = 0; c < W; ++c) v[s][c] = row[c];
+        } else {
+#pragma unroll
+            for (int c = 0; c < W; ++c) v[s][c] = c < w ? row[c] : T(0);
+        }
     }
     // a wait of an earlier leaf timed out: the factorization is already
     // reported as failed, leave at once.  The flag is read with the rows (one
     // memory round trip for both; the rows lie inside the panel either way)
     // and nothing has been stored before the test.
     const int failed = __hip_atomic_load(a.flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // the rows have arrived before the loop: otherwise the first use inside a
-    // conditional block leaves a wait on all vector memory operations (the
-    // stores of the previous column included) at the top of every column
+    // the rows have arrived before the loop (otherwise the first use inside a
+    // conditional block leaves a wait on vector memory at the top of every column)
     __builtin_amdgcn_s_waitcnt(0);
     if (failed != 0) return;
 
-    // ---- candidates of column jn and their publication.  x[s]: row s's
-    // value in column jn.  pend: the registers still await the update of
-    // column jn - 1 (multipliers lm, pivot row upp, upd false for a zero
-    // pivot); the candidate rows are then updated here, one column per lane.
-    auto select_publish = [&](int jn, const T (&x)[RPT], bool pend, const T (&lm)[RPT], const double* upp,
-                              bool upd) __attribute__((always_inline)) {
-        const int parn = jn & 1;
-        double bk = -2.0; long long br = (1ll << 62); int bs = -1;
-#pragma unroll
-        for (int s = 0; s < RPT; ++s) {
-            if (lr[s] < a.mrows && lr[s] >= jn) {
-                const double k = pivot_key(double(x[s]), lr[s] == jn);
-                if (better(k, lr[s], bk, br)) { bk = k; br = lr[s]; bs = s; }
-            }
+    // the winner of the current column, as every wave knows it
+    T d = T(0), u1 = T(0);                  // values 0 and 1 of the pivot row
+    int piv = 0;                            // its position
+    T ua = T(0), ub = T(0);                 // values lane & 15 and 16 + (lane & 15) in every row of 16 lanes
+    T uu = T(0);                            // MULTI: value lane / 2 + 1
+    unsigned row_off = 0, row_tag = 0;      // MULTI: the row's place in the exchange buffer, its tag
+    const unsigned oa = (lane & 15) * 16, ob = oa + 256, ou = min((lane >> 1) + 1, W - 1) * 16;
+    const __amdgpu_buffer_rsrc_t pub_rsrc =
+        __builtin_amdgcn_make_buffer_rsrc((void*)a.pub, 0, int(OXI_LEAF_PUB * 8), 0x00027000);
+    bool timed_out = false;                 // this wave's last wait failed
+
+    // ---- MULTI: the winner's row from the words fetched ahead; fetched again
+    // (bounded) while a word is not the column's yet
+    auto row_arrives = [&](uint4v xa, uint4v xb, uint4v xu) __attribute__((always_inline)) {
+        const unsigned tag = row_tag;
+        unsigned spins = 0;
+#pragma unroll 1
+        while (true) {
+            unsigned diff = (xa.y ^ tag) | (xa.w ^ tag) | (xb.y ^ tag) | (xb.w ^ tag) | (xu.y ^ tag) | (xu.w ^ tag);
+            asm("" : "+v"(diff));   // one compare, not six and a chain of scalar ors
+            if (__builtin_expect(__ballot(diff != 0) == 0, 1)) break;
+            if (++spins > spin_limit) { timed_out = true; break; }   // uniform per wave
+            const char* row = (const char*)a.pub + row_off;
+            load_words3((const u64*)(row + oa), (const u64*)(row + ob), (const u64*)(row + ou), xa, xb, xu);
         }
-        const double wk = wave_max(bk);
-        // rows of slot s increase with the lane, and every row of slot s is
-        // below every row of slot s + 1
-        int wl = 0, ws = -1;
-#pragma unroll
-        for (int s = RPT - 1; s >= 0; --s) {
-            const u64 m = __ballot(bk == wk && bs == s);
-            if (m) { wl = first_lane(m); ws = s; }
-        }
-        const long long wr = (long long)readlane64(u64(br), wl);
-        // the wave's candidate and position jn's row: as they are (pend false)
-        // or through raw[] and one updated column per lane
-        double (*dst)[W] = pend ? raw : wvals[parn];
-        bool diag_here = false;
-#pragma unroll
-        for (int s = 0; s < RPT; ++s) {
-            const bool cand = lane == wl && ws == s, diag = lr[s] == jn;
-            diag_here |= diag;
-            if (cand)
-#pragma unroll
-                for (int c = 0; c < W; ++c) dst[wave][c] = double(v[s][c]);
-            if (diag)
-#pragma unroll
-                for (int c = 0; c < W; ++c) dst[NWV][c] = double(v[s][c]);
-            if (pend && cand) raw_l[wave] = double(lm[s]);
-            if (pend && diag) raw_l[NWV] = double(lm[s]);
-        }
-        if (pend) {
-            diag_here = __ballot(diag_here) != 0;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // the lanes' LDS writes before the reads below
-            __builtin_amdgcn_wave_barrier();
-            if (lane < W) {
-                auto updated = [&](int slot) __attribute__((always_inline)) -> double {
-                    if (lane + 1 >= W) return 0.0;
-                    const T r = T(raw[slot][lane + 1]);
-                    return double(upd ? fma_t(-T(raw_l[slot]), T(upp[lane + 1]), r) : r);
-                };
-                if (ws >= 0) wvals[parn][wave][lane] = updated(wave);
-                if (diag_here) wvals[parn][NWV][lane] = updated(NWV);
-            }
-        }
-        if (lane == 0) { wkey[parn][wave] = wk; wrow[parn][wave] = ws >= 0 ? wr : (1ll << 62); }
-        __syncthreads();
-        double lkey = wkey[parn][0];
-        long long lrow = wrow[parn][0];
-        int lw = 0;
-#pragma unroll
-        for (int q = 1; q < NWV; ++q)
-            if (better(wkey[parn][q], wrow[parn][q], lkey, lrow)) { lkey = wkey[parn][q]; lrow = wrow[parn][q]; lw = q; }
-        if (!global_x) {
-            if (t == 0) { lrow_sh[parn] = lrow; lw_sh[parn] = lw; }
-            return;
-        }
-        const u64 tag = a.tag0 + u64(a.c0 + jn);
-        double* rec = a.pub + (size_t(jn) * a.P + p) * OXI_PUB_STRIDE;
-        double* drec = a.pub + (size_t(w) * a.P + jn) * OXI_PUB_STRIDE;
-        if (wave == 0 && lane < 16) {
-            const bool has = lrow < a.mrows;
-            publish16(rec, tag, lane, wvals[parn][lw], has, has ? lkey : -2.0,
-                      __longlong_as_double(has ? lrow : (long long)(1ll << 62)));
-        }
-        if (p == 0 && wave == NWV - 1 && lane < 16)
-            publish16(drec, tag, lane, wvals[parn][NWV], true, 0.0, 0.0);
+        ua = from_words<T>(xa.x, xa.z);
+        ub = from_words<T>(xb.x, xb.z);
+        uu = from_words<T>(xu.x, xu.z);
     };
 
-    // ---- the records of column jn into rec_sh (P > 1), then a barrier, so
-    // that no wave overwrites the buffers of column jn - 1 while another
-    // still reads them.  Returns false on timeout.
-    //
-    // Record q (q < P candidates, q == P position jn) is polled by the 4 lanes
-    // of slot q % PASS (lane sub holds fields sub, sub+4, ..., sub+32).  The
-    // waves poll on their own, without a barrier per round, and a record
-    // whose tag is not yet the column's is passed over without hashing.  A
-    // validated record goes to rec_sh and its bit to vmask (LDS); every wave
-    // stops once all bits are set.  (Polling each record from several waves
-    // at staggered times was slower: a wave cannot leave a poll in flight,
-    // so the barrier then waits for the late copies' round trips.)  vmask of
-    // the other parity is cleared after the barrier: its readers (column
-    // jn - 1) passed the barrier of select_publish before this one.
-    auto gather = [&](int jn) __attribute__((always_inline)) -> bool {
-        if (!global_x) { __syncthreads(); return true; }
+    // ---- the candidate of column jn and its publication.  x[s]: row s's
+    // value in column jn (register REG).  PEND: the registers still await the
+    // update of column jn - 1 (multipliers l, the row in xa, xb, xu); only
+    // the chosen row is then updated here.  False when a wave of the
+    // workgroup timed out.  Straight-line code but for ties: a taken branch
+    // costs about as much as ten dependent instructions.
+    auto select_publish = [&](int jn, const T (&x)[RPT], auto pend_c, const T (&l)[RPT], bool upd,
+                              uint4v xa, uint4v xb, uint4v xu) __attribute__((always_inline)) -> bool {
+        constexpr bool PEND = decltype(pend_c)::value;
+        constexpr int REG = PEND ? 1 : 0;
         const int parn = jn & 1;
-        const u64 tag = a.tag0 + u64(a.c0 + jn);
-        const double* drec = a.pub + (size_t(w) * a.P + jn) * OXI_PUB_STRIDE;
-        double* rs = rec_sh[parn];
-        u64* vm = vmask[parn];
-        const int sub = lane & 3;
-        unsigned spins = 0;
-        while (true) {
-            const u64 m0 = __hip_atomic_load(&vm[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            const u64 m1 = __hip_atomic_load(&vm[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            if (__builtin_amdgcn_readfirstlane(int(m0 == full0 && m1 == full1))) break;
+        // this lane's best row
+        int k[RPT], kb = KEY_NONE - 1, sb = 0;
+        bool tie = false;
 #pragma unroll
-            for (int ps = 0; ps < NPASS_MAX; ++ps) {
-                const int q = qs[ps];
-                const bool have = q >= P1 || (((q < 64 ? m0 >> q : m1 >> (q - 64)) & 1) != 0);
-                if (!have) {
-                    const double* src = q < a.P ? a.pub + (size_t(jn) * a.P + q) * OXI_PUB_STRIDE : drec;
-                    double fv[REC_N / 4];
-                    load9_agent(src + sub, fv);
-                    // the tag sits in quad lane 2 (field 2): a record of an
-                    // earlier column or call is passed over without hashing
-                    const u64 tg = quad_bcast<2>(bits(fv[0]));
-                    if (tg == tag) {
-                        u64 hx = 0;
+        for (int s = 0; s < RPT; ++s) {
+            k[s] = pos[s] >= 0 ? pivot_key(x[s], pos[s] == jn) : KEY_NONE;
+            tie = k[s] > kb ? false : tie || k[s] == kb;
+            sb = k[s] > kb ? s : sb;
+            kb = max(kb, k[s]);
+        }
+        const int m = wave_imax(kb);
+        u64 b = __ballot(kb == m);
+        int wl = first_lane(b);
+        const bool none = m == KEY_NONE;
+        if (__builtin_expect(!none && ((b & (b - 1)) != 0 || (RPT > 1 && (__ballot(tie) & b) != 0)), 0)) {
+            // equal high words: low word, then position
+            unsigned lob = 0;
+            int pb = NO_POS;
 #pragma unroll
-                        for (int i = 0; i < REC_N / 4; ++i) {
-                            const int f = sub + 4 * i;
-                            if (f < REC_CHK) hx ^= rec_term(bits(fv[i]), tag, f);
-                        }
-                        hx = quad_xor(hx);
-                        // the checksum sits in quad lane 3 (field 35)
-                        const u64 chk = quad_bcast<3>(bits(fv[REC_N / 4 - 1]));
-                        if (hx == chk) {
-#pragma unroll
-                            for (int i = 0; i < REC_N / 4; ++i) rs[q * RS_N + 1 + sub + 4 * i] = fv[i];
-                            if (sub == 0)
-                                __hip_atomic_fetch_or(&vm[q >> 6], 1ull << (q & 63), __ATOMIC_RELAXED,
-                                                      __HIP_MEMORY_SCOPE_WORKGROUP);
-                        }
-                    }
-                }
+            for (int s = 0; s < RPT; ++s) {
+                const unsigned lo_s = pivot_key_lo(x[s]);
+                const bool win = k[s] == m && (pb == NO_POS || lo_s > lob || (lo_s == lob && pos[s] < pb));
+                sb = win ? s : sb; lob = win ? lo_s : lob; pb = win ? pos[s] : pb;
             }
-            if (++spins > SPIN_LIMIT) break;   // uniform per wave
-            __builtin_amdgcn_s_sleep(1);
+            wl = settle_tie(b, lob, pb);
         }
-        __syncthreads();
-        const bool ok = __hip_atomic_load(&vm[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == full0 &&
-                        __hip_atomic_load(&vm[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == full1;
-        if (!ok) {   // the same in every thread: no wave writes vmask after the barrier
-            if (t == 0) __hip_atomic_store(a.flags, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return false;
+        T xs = x[0], ls = l[0], ys = REG + 1 < W ? v[0][REG + 1] : T(0);
+        int ps = pos[0];
+#pragma unroll
+        for (int s = 1; s < RPT; ++s) {
+            xs = sb == s ? x[s] : xs;
+            ls = sb == s ? l[s] : ls;
+            ps = sb == s ? pos[s] : ps;
+            if (REG + 1 < W) ys = sb == s ? v[s][REG + 1] : ys;
         }
-        if (t < 2) vmask[parn ^ 1][t] = 0;
-        return true;
+        const int pos_w = none ? NO_POS : __builtin_amdgcn_readlane(ps, wl);
+        if (lane == wl) wcand[parn][wave] = int4{m, int(pivot_key_lo(xs)), none ? NO_POS : ps, int(timed_out)};
+        const int ws = RPT > 1 ? __builtin_amdgcn_readlane(sb, wl) : 0;
+        const T lw = readlane_t(ls, wl);
+        // the chosen row from its lane's registers to LDS, eight values at a
+        // time while any of them is live (a 16-byte LDS store takes about as
+        // long for one lane as for 64)
+        auto row_out = [&](T* dst) __attribute__((always_inline)) {
+#pragma unroll
+            for (int s = 0; s < RPT; ++s)
+                if (ws == s && lane == wl) {
+                    T* o = (T*)__builtin_assume_aligned(dst, 16);
+#pragma unroll
+                    for (int g = 0; g < W; g += 8)
+                        if (g < W - jn) {
+#pragma unroll
+                            for (int c = g; c < g + 8; ++c) o[c] = REG + c < W ? v[s][REG + c] : T(0);
+                        }
+                    // keeps the slots' stores apart: merged into stores of a
+                    // chosen row they would put the rows in scratch memory
+                    asm volatile("; slot %0" ::"n"(s));
+                }
+        };
+        if constexpr (!MULTI) {
+            row_out(&rows[parn][wave * RS_N]);
+            if (lane == 0) raw_l[parn][wave] = lw;
+        }
+        lds_barrier();
+        const int4 e = wcand[parn][lane & (NWV - 1)];
+        int em = dpp_imax<0xB1>(e.x);                   // quad_perm [1,0,3,2]
+        em = dpp_imax<0x4E>(em);                        // quad_perm [2,3,0,1]
+        const u64 eb = __ballot(e.x == em) & ((1ull << NWV) - 1);
+        int ww = first_lane(eb);
+        if (__builtin_expect((eb & (eb - 1)) != 0, 0)) ww = settle_tie(eb, unsigned(e.y), e.z);
+        if constexpr (!MULTI) {
+            // every wave updates the winner's row itself: ua, ub of the new
+            // row from those of the old one, one value further
+            piv = __builtin_amdgcn_readlane(e.z, ww);
+            const T* src = &rows[parn][ww * RS_N];
+            const int i = lane & 15;
+            T na = src[i], nb = src[16 + i];
+            if (PEND && upd) {
+                const T wl_ = raw_l[parn][ww];
+                const T sa = row_shl1(ua), sb1 = row_shl1(ub), b0 = row_bcast<0>(ub);
+                na = fma_t(-wl_, i == 15 ? b0 : sa, na);
+                nb = fma_t(-wl_, i == 15 ? T(0) : sb1, nb);
+            }
+            ua = i < W - jn ? na : T(0);
+            ub = 16 + i < W - jn ? nb : T(0);
+            d = readlane_t(ua, 0);
+            u1 = readlane_t(ua, 1);
+            return true;
+        } else {
+            if (PEND) row_arrives(xa, xb, xu);
+            if (wave == ww && jn < w) {
+                // this wave holds the workgroup's candidate: the header first,
+                // from its lane's registers (value 1 is column jn + 1 updated)
+                const u64 tag = u64(a.tag + unsigned(jn)) << 32;
+                if (PEND && upd) ys = fma_t(-ls, row_bcast<2>(ua), ys);
+                const T h0 = none ? T(0) : readlane_t(xs, wl), h1 = none || jn + 1 >= W ? T(0) : readlane_t(ys, wl);
+                const unsigned hd = lane == 0 ? word_lo(h0) : lane == 1 ? word_hi(h0) : lane == 2 ? word_lo(h1)
+                                  : lane == 3 ? word_hi(h1) : unsigned(pos_w);
+                if (lane < 6)
+                    __hip_atomic_store(a.pub + size_t(w) * P * OXI_PUB_STRIDE + (size_t(jn) * P + p) * OXI_PUB_HDR + lane,
+                                       tag | hd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                // then the whole row, two lanes per column (low and high half)
+                row_out(raw);
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // the lane's LDS writes before the reads below
+                __builtin_amdgcn_wave_barrier();
+                const int c = lane >> 1;
+                T r = raw[c];
+                if (PEND && upd) r = fma_t(-lw, uu, r);
+                if (none || c >= W - jn) r = T(0);
+                const unsigned data = (lane & 1) ? word_hi(r) : word_lo(r);
+                __hip_atomic_store(a.pub + (size_t(jn) * P + p) * OXI_PUB_STRIDE + lane, tag | data, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            }
+            if (__builtin_expect(__ballot(e.w != 0) != 0, 0)) {   // a wave's wait timed out (the same in every wave)
+                if (t == 0) __hip_atomic_store(a.flags, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                return false;
+            }
+            return true;
+        }
+    };
+
+    // ---- MULTI: the headers of column jn (lane q: workgroup q), polled by
+    // every wave until all are there; the winner is found in registers
+    auto poll = [&](int jn) __attribute__((always_inline)) {
+        const unsigned tag = a.tag + unsigned(jn);
+        const u64* heads = a.pub + size_t(w) * P * OXI_PUB_STRIDE + size_t(jn) * P * OXI_PUB_HDR;
+        unsigned spins = 0;
+        auto header = [&](int q, T& v0, T& v1, int& hpos) __attribute__((always_inline)) {
+            const u64* hq = heads + q * OXI_PUB_HDR;
+            uint4v x0, x1, x2;
+#pragma unroll 1
+            while (true) {
+                load_words3(hq, hq + 2, hq + 4, x0, x1, x2);
+                unsigned diff = (x0.y ^ tag) | (x0.w ^ tag) | (x1.y ^ tag) | (x1.w ^ tag) | (x2.y ^ tag) | (x2.w ^ tag);
+                asm("" : "+v"(diff));
+                if (__builtin_expect(__ballot(diff != 0) == 0, 1)) break;
+                if (++spins > spin_limit) break;   // uniform per wave
+            }
+            v0 = from_words<T>(x0.x, x0.z);
+            v1 = from_words<T>(x1.x, x1.z);
+            hpos = int(x2.x);
+        };
+        int q = min(lane, P - 1), hp;
+        T dl, ul;
+        header(q, dl, ul, hp);
+        int key = lane < P && hp != NO_POS ? pivot_key(dl, hp == jn) : KEY_NONE;
+        if constexpr (WGS > 64) {   // two records a lane
+            const int q2 = min(lane + 64, P - 1);
+            T d2, u2;
+            int p2;
+            header(q2, d2, u2, p2);
+            const int k2 = lane + 64 < P && p2 != NO_POS ? pivot_key(d2, p2 == jn) : KEY_NONE;
+            const unsigned la = pivot_key_lo(dl), lb = pivot_key_lo(d2);
+            if (k2 > key || (k2 == key && (lb > la || (lb == la && p2 < hp)))) {
+                key = k2; hp = p2; q = q2; dl = d2; ul = u2;
+            }
+        }
+        const int m = wave_imax(key);
+        const u64 b = __ballot(key == m);
+        int gl = first_lane(b);
+        if (__builtin_expect((b & (b - 1)) != 0, 0)) gl = settle_tie(b, pivot_key_lo(dl), hp);
+        row_off = unsigned(jn * P + __builtin_amdgcn_readlane(q, gl)) * (OXI_PUB_STRIDE * 8);
+        row_tag = tag;
+        d = readlane_t(dl, gl);
+        u1 = readlane_t(ul, gl);
+        piv = __builtin_amdgcn_readlane(hp, gl);
+        if (spins > spin_limit) timed_out = true;
     };
 
     // column 0: the registers as loaded
     {
-        T x0[RPT];
+        T x0[RPT], l0[RPT];
 #pragma unroll
-        for (int s = 0; s < RPT; ++s) x0[s] = v[s][0];
-        select_publish(0, x0, false, x0, nullptr, false);
-        if (!gather(0)) return;
+        for (int s = 0; s < RPT; ++s) { x0[s] = v[s][0]; l0[s] = T(0); }
+        if (!select_publish(0, x0, std::false_type{}, l0, false, {}, {}, {})) return;
+        if constexpr (MULTI) poll(0);
     }
 
-#pragma unroll 1
-    for (int j0 = 0; j0 < w; ++j0) {
-        const int j = __builtin_amdgcn_readfirstlane(j0);
-        const int par = j & 1;
-        // ---- the winner of column j: the pivot row (up) and position j's
-        // row (dp), as doubles in LDS, in the rotated register order
-        const double* up;
-        const double* dp;
-        long long piv;
-        if (!global_x) {
-            piv = lrow_sh[par];
-            up = wvals[par][lw_sh[par]];
-            dp = wvals[par][NWV];
-        } else {
-            // the winner over the P candidates, in every wave; record q holds
-            // rows of workgroup q only, so ties go to the lowest q
-            const double* rs = rec_sh[par];
-            double k = -3.0; long long r = (1ll << 62); int wq = -1;
-            for (int q = lane; q < a.P; q += 64) {
-                const double kq = rs[q * RS_N + 1];
-                const long long rq = __double_as_longlong(rs[q * RS_N + 2]);
-                if (better(kq, rq, k, r)) { k = kq; r = rq; wq = q; }
-            }
-            const double gk = wave_max(k);
-            const u64 m0 = __ballot(k == gk && wq >= 0 && wq < 64);
-            const int gl = m0 ? first_lane(m0) : first_lane(__ballot(k == gk && wq >= 64));
-            piv = (long long)readlane64(u64(r), gl);
-            const int gq = __builtin_amdgcn_readlane(wq, gl);
-            up = (const double*)__builtin_assume_aligned(rs + gq * RS_N + 4, 16);
-            dp = (const double*)__builtin_assume_aligned(rs + a.P * RS_N + 4, 16);
-        }
+    int my_piv = 0, first_zero = -1;   // wave 0 of workgroup 0: lane j holds step j's pivot position
+    // state of column j between its record's publication and its update
+    T l[RPT], lin[RPT];   // the multiplier for the update (0: row not updated), the value entering register 31
+    T ra = T(0), rb = T(0);   // the pivot row's values
+    bool updates = false;     // column j has a pivot
+    bool odd = false;         // the update needs its selects: an infinity, a NaN or a zero pivot
 
-        // ---- interchange (the registers: columns >= j), store position j,
-        // scale, store the multipliers.  Only position piv takes a row
-        // (position j's, dp): position j's registers are not read again
-        // (candidates, multipliers and later interchanges all lie below j),
-        // its final row is the pivot row, stored from up.
-        if (p == 0 && t == 0) a.ipiv[a.c0 + j] = a.c0 + piv + 1;
-#pragma unroll
-        for (int s = 0; s < RPT; ++s) {
-            if (piv != j && lr[s] == piv) {
-#pragma unroll
-                for (int c = 0; c < W; ++c) v[s][c] = T(dp[c]);
-            }
+    // The multipliers of column j, then column j+1's values, candidate and
+    // record (past the last column nothing is published).  False on timeout.
+    auto head = [&](int j) __attribute__((always_inline)) -> bool {
+        // the winner's row starts on its way
+        uint4v xa = {}, xb = {}, xu = {};
+        if constexpr (MULTI) {
+            xa = load_words_ahead(pub_rsrc, row_off + oa);
+            xb = load_words_ahead(pub_rsrc, row_off + ob);
+            xu = load_words_ahead(pub_rsrc, row_off + ou);
         }
-        // position j now holds the pivot row, final in columns j .. w-1
-        if (p == 0 && wave == 0 && lane < w - j) Wm[a.c0 + j + (a.c0 + j) * a.ldw + lane] = T(up[lane]);
-        const T d = T(up[0]);
         const bool upd = d != T(0);
-        if (!upd && p == 0 && t == 0 && *a.info == 0) *a.info = a.c0 + j + 1;
-        T l[RPT];
+        my_piv = wave == 0 && lane == j ? piv : my_piv;
+        first_zero = !upd && first_zero < 0 ? j : first_zero;
+        updates = upd;
+        bool strange = !upd || non_finite(d);
+        T x[RPT];
 #pragma unroll
         for (int s = 0; s < RPT; ++s) {
-            l[s] = upd ? v[s][0] / d : v[s][0];   // a zero pivot leaves the column as it is
-            if (lr[s] > j && lr[s] < a.mrows) wrow_of[s][j] = l[s];
+            // interchange: positions only
+            pos[s] = pos[s] == piv ? ~j : pos[s] == j ? piv : pos[s];
+            const T qv = v[s][0] / d;
+            const bool act = pos[s] >= 0 && upd;   // a zero pivot leaves the column as it is
+            l[s] = act ? qv : T(0);
+            lin[s] = act ? qv : v[s][0];
+            x[s] = upd ? fma_t(-l[s], u1, v[s][1]) : v[s][1];
+            strange |= non_finite(l[s]);
         }
+        if constexpr (!MULTI) { ra = ua; rb = ub; }   // this column's row (select_publish makes the next one's)
+        if (!select_publish(j + 1, x, std::true_type{}, l, upd, xa, xb, xu)) return false;
+        if constexpr (MULTI) { ra = ua; rb = ub; }
+        odd = __ballot(strange || non_finite(ra) || non_finite(rb)) != 0;
+        return true;
+    };
+    if (!head(0)) return;
 
-        // ---- column j+1: its values, candidates and records first
-        const bool more = j + 1 < w;
-        if (more) {
-            T x[RPT];
-            const T u1 = T(up[1]);
+    // Per turn: the rank-1 update of column j with the rotation, while the
+    // records of column j + 1 travel, then those records and the head of
+    // column j + 1.
+    int j = 0;
+#pragma unroll 1
+    for (; j < w && !odd; ++j) {
+        static_for<W / 4>([&](auto g_c) __attribute__((always_inline)) {
+            // four broadcast values at a time (all of them ahead would not fit
+            // in the registers)
+            constexpr int G = 4 * decltype(g_c)::value;
+            T u[4];
+            static_for<4>([&](auto c_c) __attribute__((always_inline)) {
+                constexpr int C = G + decltype(c_c)::value;
+                if constexpr (C > 0) u[C - G] = C < 16 ? row_bcast<C & 15>(ra) : row_bcast<C & 15>(rb);
+            });
+            __builtin_amdgcn_sched_barrier(0);
+            static_for<4>([&](auto c_c) __attribute__((always_inline)) {
+                constexpr int C = G + decltype(c_c)::value;
+                if constexpr (C > 0) {
 #pragma unroll
-            for (int s = 0; s < RPT; ++s) x[s] = upd ? fma_t(-l[s], u1, v[s][1]) : v[s][1];
-            select_publish(j + 1, x, true, l, up, upd);
+                    for (int s = 0; s < RPT; ++s) v[s][C - 1] = nfma_to(l[s], u[C - G], v[s][C]);
+                }
+            });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+#pragma unroll
+        for (int s = 0; s < RPT; ++s) v[s][W - 1] = lin[s];
+        if (j + 1 < w) {
+            if constexpr (MULTI) poll(j + 1);
+            if (!head(j + 1)) return;
         }
-
-        // ---- the rank-1 update with the rotation, while the records travel
-        if (upd) {
-            T u[W];
-#pragma unroll
-            for (int c = 1; c < W; ++c) u[c] = T(up[c]);
+    }
+    // the same from the first odd column on, the update with a select per value
+#pragma unroll 1
+    for (; j < w; ++j) {
+        static_for<W - 1>([&](auto c_c) __attribute__((always_inline)) {
+            constexpr int C = decltype(c_c)::value + 1;
+            const T uc = C < 16 ? row_bcast<C & 15>(ra) : row_bcast<C & 15>(rb);
 #pragma unroll
             for (int s = 0; s < RPT; ++s) {
-#pragma unroll
-                for (int c = 0; c + 1 < W; ++c) v[s][c] = fma_t(-l[s], u[c + 1], v[s][c + 1]);
-                v[s][W - 1] = T(0);
+                const bool live = updates && pos[s] >= 0 && C < W - j;
+                v[s][C - 1] = live ? fma_t(-l[s], uc, v[s][C]) : v[s][C];
             }
+            if constexpr (C % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+        });
+#pragma unroll
+        for (int s = 0; s < RPT; ++s) v[s][W - 1] = lin[s];
+        if (j + 1 < w) {
+            if constexpr (MULTI) poll(j + 1);
+            if (!head(j + 1)) return;
+        }
+    }
+    // a narrower leaf completes the rotation
+#pragma unroll 1
+    for (int k = w; k < W; ++k) {
+#pragma unroll
+        for (int s = 0; s < RPT; ++s) {
+            const T x = v[s][0];
+#pragma unroll
+            for (int c = 0; c + 1 < W; ++c) v[s][c] = v[s][c + 1];
+            v[s][W - 1] = x;
+        }
+    }
+    // every workgroup has its rows in registers once the first column's
+    // records are complete: the rows go to their final positions
+#pragma unroll
+    for (int s = 0; s < RPT; ++s) {
+        if (pos[s] < -W) continue;
+        const int to = pos[s] >= 0 ? pos[s] : ~pos[s];
+        T* row = Wm + a.c0 + (a.c0 + to) * a.ldw;
+        if (w == W) {
+#pragma unroll
+            for (int c = 0; c < W; ++c) row[c] = v[s][c];
         } else {
 #pragma unroll
-            for (int s = 0; s < RPT; ++s) {
-#pragma unroll
-                for (int c = 0; c + 1 < W; ++c) v[s][c] = v[s][c + 1];
-                v[s][W - 1] = T(0);
-            }
+            for (int c = 0; c < W; ++c)
+                if (c < w) row[c] = v[s][c];
         }
-        if (more && !gather(j + 1)) return;
+    }
+    if (timed_out && lane == 0) __hip_atomic_store(a.flags, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (p == 0 && wave == 0) {
+        if (lane < w) a.ipiv[a.c0 + lane] = a.c0 + my_piv + 1;
+        if (lane == 0 && first_zero >= 0 && *a.info == 0) *a.info = a.c0 + first_zero + 1;
     }
 }
 
-// The slots of the interchanges of steps k_lo .. w-1 of a leaf at c0 (one
-// wave): lane i < n (n = w - k_lo) is step k_lo + i's own position; lane
-// n + i is the pivot position p_i of step k_lo + i when it lies below the
-// leaf's w rows and i is its first occurrence.  pos = -1 for unused lanes.
+// The slots of the interchanges of a leaf's w steps at c0 (one wave): lane
+// i < w is step i's own position; lane w + i is the pivot position p_i of step
+// i when it lies below the leaf's w rows and i is its first occurrence.
+// pos = -1 for unused lanes.
 // The interchanges are then replayed on slot ids: afterwards lane s holds
 // the slot whose original content ends at slot s.  Every lane follows its
 // own slot backwards through the transpositions (step i exchanges slot i
 // with slot sb_i, held by lane i), so the steps carry no cross-lane
 // dependence: one readlane and two selects each.
-// pi_all: lane i < w holds step i's pivot position relative to c0 (-1 beyond).
-__device__ __forceinline__ void leaf_slots(i64 pi_all, int w, int k_lo, int lane, i64& pos, int& src) {
-    const int n = w - k_lo;
-    const i64 pi_sh = (i64)__shfl((long long)pi_all, min(k_lo + lane, 63));
-    const i64 pi = lane < n ? pi_sh : -1;
+// pi: lane i < w holds step i's pivot position relative to c0 (-1 beyond).
+__device__ __forceinline__ void leaf_slots(i64 pi, int w, int lane, i64& pos, int& src) {
     // unrolled to the largest leaf without a bound test (the readlanes of
-    // different steps are independent and interleave): lanes i >= n hold
-    // pi = -1, which matches only lanes >= n, whose first is not used
+    // different steps are independent and interleave): lanes i >= w hold
+    // pi = -1, which matches only lanes >= w, whose first is not used
     int first = lane;
 #pragma unroll
     for (int i = 0; i < OXI_LEAF_W; ++i) {
         const i64 q = (i64)readlane64(u64(pi), i);
         if (i < first && q == pi) first = i;
     }
-    pos = lane < n ? k_lo + lane : -1;
-    const int src_i = lane - n;   // differs per lane: a shuffle, not readlane
-    const int src_l = (src_i >= 0 && src_i < n) ? src_i : 0;
+    pos = lane < w ? lane : -1;
+    const int src_i = lane - w;   // differs per lane: a shuffle, not readlane
+    const int src_l = (src_i >= 0 && src_i < w) ? src_i : 0;
     const i64 pos_out = (i64)__shfl((long long)pi, src_l);
     const int first_out = __shfl(first, src_l);
-    if (src_i >= 0 && src_i < n && pos_out >= w && first_out == src_i) pos = pos_out;
-    // the slot that step i exchanges with slot i (lane i < n)
-    const int sbv = lane < n ? (pi < w ? int(pi - k_lo) : n + first) : lane;
+    if (src_i >= 0 && src_i < w && pos_out >= w && first_out == src_i) pos = pos_out;
+    // the slot that step i exchanges with slot i (lane i < w)
+    const int sbv = lane < w ? (pi < w ? int(pi) : w + first) : lane;
     // the content that ends at slot `lane`: the transpositions of steps
-    // n-1 .. 0 applied to it in turn (steps i >= n exchange slot i with
+    // w-1 .. 0 applied to it in turn (steps i >= w exchange slot i with
     // itself: sbv = lane there)
     int x = lane;
 #pragma unroll
@@ -516,14 +653,10 @@ __device__ __forceinline__ void leaf_slots(i64 pi_all, int w, int k_lo, int lane
     src = x;
 }
 
-// A leaf's interchanges applied where the leaf did not apply them, blocks of
-// two waves:
-//  * its own multiplier columns c < w - 1 (one block each, the first wave):
-//    column c takes the interchanges of steps c+1 .. w-1 (the multipliers of
-//    column c were stored at the positions of step c);
-//  * the other columns of the enclosing panel, [x_lo, c0) and [c0+w, x_hi),
-//    64 per block (a lane per column): all w interchanges, half of the slots
-//    by each wave.
+// A leaf's interchanges on the other columns of the enclosing panel,
+// [x_lo, c0) and [c0+w, x_hi): blocks of two waves take 64 columns each (a
+// lane per column), half of the slots by each wave.  The leaf's own columns
+// are stored at their final positions by the leaf itself.
 // Applying a leaf's interchanges to the rest of its panel at once gives the
 // same columns as the getrf2 recursion, which applies them level by level:
 // a left subtree's multipliers are not read again once its right sibling
@@ -531,7 +664,7 @@ __device__ __forceinline__ void leaf_slots(i64 pi_all, int w, int k_lo, int lane
 // update reads them.
 template <typename T>
 __global__ __launch_bounds__(128) void leaf_swaps_kernel(T* Wm, i64 ldw, i64 c0, int w, const i64* ipiv,
-                                                         const int* flags, i64 x_lo, i64 x_hi, int first_block = 0) {
+                                                         const int* flags, i64 x_lo, i64 x_hi) {
     const int lane = threadIdx.x & 63;
     const int half = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
     // the pivots are loaded with the flag, not after its test, and without a
@@ -540,26 +673,14 @@ __global__ __launch_bounds__(128) void leaf_swaps_kernel(T* Wm, i64 ldw, i64 c0,
     const i64 pv = ipiv[c0 + (lane < w ? lane : 0)];
     if (__hip_atomic_load(flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return;
     const i64 pi_all = lane < w ? pv - 1 - c0 : -1;
-    const int b = int(blockIdx.x) + first_block;   // first_block = w - 1: the leaf's own columns are final
-    if (b < w - 1) {
-        if (half != 0) return;
-        const int c = b;
-        i64 pos; int src;
-        leaf_slots(pi_all, w, c + 1, lane, pos, src);
-        const i64 psrc = (i64)__shfl((long long)pos, src);
-        T v = T(0);
-        if (pos >= 0 && psrc != pos) v = Wm[(c0 + psrc) * ldw + c0 + c];
-        if (pos >= 0 && psrc != pos) Wm[(c0 + pos) * ldw + c0 + c] = v;
-        return;
-    }
-    const i64 fb = b - (w - 1);
+    const i64 fb = blockIdx.x;
     const i64 tl = (c0 - x_lo + 63) / 64;
     i64 x;
     bool ok;
     if (fb < tl) { x = x_lo + fb * 64 + lane; ok = x < c0; }
     else { x = c0 + w + (fb - tl) * 64 + lane; ok = x < x_hi; }
     i64 pos; int src;
-    leaf_slots(pi_all, w, 0, lane, pos, src);
+    leaf_slots(pi_all, w, lane, pos, src);
     // slot s moves when its source differs (at most 2w <= 64 slots).  Both
     // waves compute all slots; wave h moves slots 32h .. 32h+31.  All loads
     // of the block have returned before any store (a wait and a barrier) and
@@ -586,6 +707,21 @@ __global__ __launch_bounds__(128) void leaf_swaps_kernel(T* Wm, i64 ldw, i64 c0,
             const i64 to = (i64)readlane64(u64(offd), s0 + k);
             if (ok) Wm[to + x] = v[k];
         }
+}
+
+// One leaf launch.  Every workgroup asks for LEAF_LDS bytes of LDS, far more
+// than it uses, so that it gets a CU of its own: beside a workgroup of the
+// trailing update (66 KB of LDS), whose waves compete for its SIMDs, a column
+// took 3.9 us at 16384 rows instead of 2.4.  getrf keeps 32 CUs free of them.
+constexpr unsigned LEAF_LDS = 96 * 1024;
+template <typename K>
+int launch_leaf(oxi_handle_t h, hipStream_t s, const LeafArgs& a, K kernel) {
+    const hipError_t se = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LEAF_LDS);
+    if (se != hipSuccess) return oxi_set_error(h, OXI_ERR_HIP, "lu_leaf attribute: %s", hipGetErrorString(se));
+    hipLaunchKernelGGL(kernel, dim3(unsigned(a.P)), dim3(256), LEAF_LDS, s, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return oxi_set_error(h, OXI_ERR_HIP, "lu_leaf launch: %s", hipGetErrorString(e));
+    return OXI_OK;
 }
 
 }  // namespace

@@ -41,6 +41,7 @@ constexpr int TP_LEVELS = 3;             // tree levels over workgroups: 32 -> 8
 constexpr int TP_REC = 36;               // record fields: tag, count, 32 positions, spare, checksum
 constexpr unsigned TP_SPIN_LIMIT = 1u << 22;
 static_assert(OXI_TP_MAX_P <= 64, "three levels of four-way merges");
+static_assert(TP_LEVELS * OXI_TP_MAX_P * TP_REC + OXI_TP_MAX_P <= OXI_TP_PUB, "record space");
 
 __device__ __forceinline__ float tp_key(float v) {
     const float a = __builtin_fabsf(v);
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(TLT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     float* Wm = (float*)a.Wm;
     const u64 tag_base = a.tag0 + 8 * u64(a.c0);      // level l's records: tag_base + l; the flags: + 7
     const u64 tag_flag = tag_base + 7;
-    double* flg = a.pub + TP_LEVELS * OXI_TP_MAX_P * TP_REC;   // [P]
+    double* flg = a.tpub + TP_LEVELS * OXI_TP_MAX_P * TP_REC;   // [P]
     // tree levels over the workgroups: 4^levels >= P
     const int nlev = a.P <= 1 ? 0 : a.P <= 4 ? 1 : a.P <= 16 ? 2 : 3;
 
@@ -234,7 +235,7 @@ __global__ __launch_bounds__(TLT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             const int nsets = (a.P + (1 << sh) - 1) >> sh;
             const int g0 = si & ~3, g1 = min(g0 + 4, nsets);    // the group's sets
             const u64 tag = tag_base + u64(lev);
-            double* recs = a.pub + (lev - 1) * OXI_TP_MAX_P * TP_REC;
+            double* recs = a.tpub + (lev - 1) * OXI_TP_MAX_P * TP_REC;
             if ((p & ((1 << sh) - 1)) == 0) {                  // the set's leader publishes it
                 const int pos = lane >= 2 && lane < 2 + TW && lane - 2 < w ? gset[lane - 2] : INT_MAX;
                 double f = pos == INT_MAX ? -1.0 : double(pos);
@@ -399,7 +400,7 @@ int oxi_launch_lu_leaf_tp(oxi_handle_t h, hipStream_t s, const LeafArgs& a, int 
     const unsigned nblk = unsigned(cdiv(a.c0 - a.xlo, 64) + cdiv(a.xhi - a.c0 - a.w, 64));
     if (nblk > 0) {
         hipLaunchKernelGGL(leaf_swaps_kernel<float>, dim3(nblk), dim3(128), 0, s, (float*)a.Wm, a.ldw, a.c0, a.w,
-                           (const i64*)a.ipiv, (const int*)a.flags, a.xlo, a.xhi, std::max(a.w - 1, 0));
+                           (const i64*)a.ipiv, (const int*)a.flags, a.xlo, a.xhi);
         e = hipGetLastError();
         if (e != hipSuccess) return oxi_set_error(h, OXI_ERR_HIP, "leaf_swaps launch: %s", hipGetErrorString(e));
     }

@@ -1,0 +1,48 @@
+"""The panel leaf at the sizes where its work division changes: the rows of
+one workgroup (256, 512), several workgroups, two rows per thread (above 8192
+rows) and widths 1..32.  A matrix of at most 32 columns is one leaf, whose
+operations (a division, then fma(-l, u, a) in column order) are the oracle's
+(src/lapack/factorizations.jl:89-140), so factors, pivots and info are equal
+bit for bit."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 1), (33, 32), (64, 31), (255, 32), (256, 7), (257, 32), (300, 1), (511, 32), (512, 32), (513, 32),
+          (700, 23), (2048, 32), (4100, 32), (8192, 32), (8193, 32), (16500, 32)]
+
+
+def check(gpu, A):
+    F = gpu.lu(gpu.DMatrix.from_numpy(A), check=False)
+    Fo, ipo, info = O.dgetrf(A, 128)
+    np.testing.assert_array_equal(F.ipiv, ipo)
+    assert F.info == info
+    np.testing.assert_array_equal(F.factors.numpy(), Fo)
+
+
+@pytest.mark.parametrize("m,w", SHAPES)
+def test_leaf_random_and_ties(gpu, rng, m, w):
+    check(gpu, rng.standard_normal((m, w)))
+    # few distinct magnitudes: exact ties inside a thread, a wave, a
+    # workgroup and between workgroups, and columns that become zero
+    check(gpu, rng.integers(-2, 3, (m, w)).astype(np.float64))
+    # equal high words, different low words: settled by the low word
+    A = 1.0 + rng.integers(0, 1 << 20, (m, w)) * 2.0 ** -52
+    check(gpu, A * rng.choice([-1.0, 1.0], (m, w)))
+
+
+@pytest.mark.parametrize("m,w", [(40, 8), (300, 32), (700, 32), (9000, 32)])
+def test_leaf_nonfinite_and_zero_pivots(gpu, rng, m, w):
+    A = rng.standard_normal((m, w))
+    A[:, w // 2] = 0.0                      # a zero pivot in the middle
+    A[m // 2, w - 1] = np.inf
+    check(gpu, A)
+    A = rng.standard_normal((m, w))
+    A[m - 1, 1] = np.nan                    # never a pivot below the diagonal
+    check(gpu, A)
+    A = rng.standard_normal((m, w))
+    A[0, 0] = np.nan                        # wins in the diagonal position
+    check(gpu, A)
