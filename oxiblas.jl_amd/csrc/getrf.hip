@@ -396,34 +396,50 @@ int swap_w(GetrfCtx<T>& g, i64 k1, i64 k2, i64 c0, i64 c1, int inverse) {
     return launch_check(g.h, "apply_pairs_w");
 }
 
+// Rows per thread of the leaf at c0: kind 0 one (256 rows a workgroup), 1 two,
+// 2 four.  Up to 512 rows one workgroup holds all (two rows per thread from
+// 257 on: 1.6 us a column against 1.8 for two workgroups that exchange; the
+// tournament leaf exchanges once per leaf and keeps two workgroups there);
+// then one row per thread up to 8192 rows (32 workgroups; two rows per thread
+// there: 2.22 us a column against 2.14), then two (at 16384 rows 2.40 us a
+// column on 32 workgroups against 2.60 on 64); FP32 rows are half the size and
+// go to four per thread beyond 16384 rows (more than 32 workgroups of 512).
+template <typename T>
+int leaf_kind(const GetrfCtx<T>& g, i64 c0) {
+    const i64 mrows = g.m - c0;
+    if (sizeof(T) == 4 && mrows > 16384) return 2;
+    const bool tournament = sizeof(T) == 4 && g.tournament;
+    return mrows > 8192 || (!tournament && mrows > 256 && mrows <= 512) ? 1 : 0;
+}
+// Columns of the widest leaf at c0: 64 where a row of 64 fits a thread's
+// registers (one FP64 or two FP32 rows per thread), else 32.  A 64-column leaf
+// takes 133 us at 2000 rows against 123 for two of 32, which need a triangular
+// solve and a product between them (11 us and two launches).
+template <typename T>
+i64 leaf_width(const GetrfCtx<T>& g, i64 c0) {
+    if (sizeof(T) == 4 && g.tournament) return 32;
+    return leaf_kind(g, c0) * sizeof(T) <= 4 ? OXI_LEAF_W : 32;
+}
+
 template <typename T>
 int leaf(GetrfCtx<T>& g, i64 c0, int w) {
     const i64 mrows = g.m - c0;
-    // rows per workgroup: up to 512 rows one workgroup holds all (two rows per
-    // thread from 257 on: 1.64 us a column against 1.77 for two workgroups
-    // that exchange; the tournament leaf exchanges once per leaf and keeps two
-    // workgroups there); then 256 (one per thread) up to 8192 rows (32
-    // workgroups; two rows per thread there: 2.22 us a column against 2.14),
-    // then 512 (at 16384 rows 2.40 us a column on 32 workgroups against 2.60
-    // on 64); FP32 rows are half the size and go to 1024 per workgroup beyond
-    // 16384 rows (more than 32 workgroups of 512)
     const bool tournament = sizeof(T) == 4 && g.tournament;
-    int kind = mrows > 8192 || (!tournament && mrows > 256 && mrows <= 512) ? 1 : 0;
-    if (sizeof(T) == 4 && mrows > 16384) kind = 2;
+    const int kind = leaf_kind(g, c0);
     const i64 R = kind == 0 ? 256 : kind == 1 ? 512 : 1024;
     const i64 P = cdiv(mrows, R);
     if (P > std::min<i64>(g.h->num_cus, OXI_LEAF_MAX_P))
         return oxi_set_error(g.h, OXI_ERR_UNSUPPORTED, "panel of %lld rows exceeds the leaf kernel capacity",
                              (long long)mrows);
-    // a leaf's number since the exchange buffer was cleared, 32 tags each; the
+    // a leaf's number since the exchange buffer was cleared, 64 tags each; the
     // buffer is cleared (in stream order, after the last leaf that used it)
     // before the numbers run out, so no tag occurs twice in it
-    if (g.h->leaf_seq >= (1u << 27) - 1) {
+    if (g.h->leaf_seq >= (1u << 26) - 1) {
         hipLaunchKernelGGL(zero_u64_kernel, dim3(256), dim3(256), 0, g.s, g.h->leaf_pub, OXI_LEAF_PUB);
         OXI_TRY(launch_check(g.h, "leaf exchange clear"));
         g.h->leaf_seq = 0;
     }
-    const unsigned tag = ++g.h->leaf_seq << 5;
+    const unsigned tag = ++g.h->leaf_seq << 6;
     LeafArgs a{(void*)g.Wm, g.ldw, c0, w, mrows, g.ipiv, g.dinfo, g.tag0, g.tpub, tag, g.h->leaf_pub, int(P),
                g.flags, g.pc0, g.pc1};
     if (tournament && kind <= 1 && P <= OXI_TP_MAX_P) return oxi_launch_lu_leaf_tp(g.h, g.s, a, kind);
@@ -435,12 +451,12 @@ int leaf(GetrfCtx<T>& g, i64 c0, int w) {
 // getrf2 recursion on the panel A[c0:m, c0:c0+np] in W coordinates
 // (src/lapack/factorizations.jl:114-152).  Each leaf applies its
 // interchanges to all other columns of the top-level panel [g.pc0, g.pc1)
-// (leaf_swaps_kernel), which covers the recursion's "left half's
+// (other_columns, panel_kernel.hpp), which covers the recursion's "left half's
 // interchanges on the right half" and "right half's interchanges on the left
 // half" at every level.
 template <typename T>
 int panel(GetrfCtx<T>& g, i64 c0, i64 np) {
-    if (np <= OXI_LEAF_W) return leaf(g, c0, int(np));
+    if (np <= leaf_width(g, c0)) return leaf(g, c0, int(np));
     const i64 mp = g.m - c0;
     const i64 h = np / 2;
     OXI_TRY(panel(g, c0, h));
@@ -484,10 +500,14 @@ bool timed_update(i64 rows, i64 cols) {
     return sizeof(T) == 8 ? oxi_dgemm_large_tiles(rows, cols) : true;
 }
 
+// Tuned block size: the panels bound the factorization, and up to about 5000
+// columns a panel of one 64-column leaf needs no product of its own (n = 2000:
+// 4.95 ms with 64, 5.10 with 128; 4096: 10.5 and 10.6; 6000: 16.8 and 16.5;
+// 8192: 28.0, 24.7 and, with 256, 24.6).
 int choose_nb(i64 m, i64 n) {
     const i64 q = std::min(m, n);
     if (q >= 8192) return 256;
-    if (q >= 1024) return 128;
+    if (q >= 5120) return 128;
     return 64;
 }
 

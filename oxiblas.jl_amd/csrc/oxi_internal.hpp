@@ -206,10 +206,10 @@ int oxi_first_zero_diag(oxi_handle_t h, hipStream_t s, const double* T, i64 ldt,
 // ---------------------------------------------------------------------------
 // Panel leaf of the LU (panel.hip)
 // ---------------------------------------------------------------------------
-constexpr int OXI_LEAF_W = 32;      // maximum leaf width
-constexpr int OXI_PUB_STRIDE = 64;  // words per published (column, workgroup) row
+constexpr int OXI_LEAF_W = 64;      // maximum leaf width
+constexpr int OXI_PUB_STRIDE = 2 * OXI_LEAF_W;   // words per published (column, workgroup) row
 constexpr int OXI_PUB_HDR = 16;     // and of its header (a 128-byte line)
-constexpr int OXI_LEAF_MAX_P = 127; // workgroups of one leaf (LDS holds P rows for two columns)
+constexpr int OXI_LEAF_MAX_P = 127; // workgroups of one leaf
 // words of the handle's exchange buffer: rows and headers of every column
 constexpr i64 OXI_LEAF_PUB = i64(OXI_LEAF_W) * OXI_LEAF_MAX_P * (OXI_PUB_STRIDE + OXI_PUB_HDR);
 constexpr int OXI_TP_PUB = 4096;    // doubles of the tournament leaf's records
@@ -217,7 +217,7 @@ constexpr int OXI_TP_PUB = 4096;    // doubles of the tournament leaf's records
 struct LeafArgs {
     void* Wm; i64 ldw;   // double* or float*
     i64 c0;          // first column (A) of the leaf = its first diagonal row
-    int w;           // leaf width <= LEAF_W
+    int w;           // leaf width <= LEAF_W (32 where a thread holds two rows or more)
     i64 mrows;       // rows c0 .. c0+mrows-1 of A
     i64* ipiv;       // global pivots (1-based rows), entries c0..c0+w-1 written
     i64* info;       // device info (first zero pivot, 1-based), 0 if none
@@ -230,13 +230,14 @@ struct LeafArgs {
     i64 xlo, xhi;    // columns [xlo, xhi) of the enclosing panel: receive the leaf's interchanges
 };
 
-// kind 0: 256 threads x 1 row per workgroup; kind 1: 256 threads x 2 rows.
+// kind 0: 256 threads x 1 row per workgroup, leaves of up to 64 columns;
+// kind 1: 256 threads x 2 rows, up to 32 columns.
 int oxi_launch_lu_leaf(oxi_handle_t h, hipStream_t s, const LeafArgs& a, int kind);
 // FP32 leaf with tournament pivoting (panel_tp.hip), kind 0 or 1, at most
 // OXI_TP_MAX_P workgroups.
 constexpr int OXI_TP_MAX_P = 32;
 int oxi_launch_lu_leaf_tp(oxi_handle_t h, hipStream_t s, const LeafArgs& a, int kind);
-// FP32 leaf; kind 2: 256 threads x 4 rows.
+// FP32 leaf; kind 1 takes up to 64 columns too, kind 2: 256 threads x 4 rows, up to 32.
 int oxi_launch_lu_leaf32(oxi_handle_t h, hipStream_t s, const LeafArgs& a, int kind);
 
 // Bracket one trailing-update GEMM launch with profiling events (no-op when

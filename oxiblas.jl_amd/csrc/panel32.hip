@@ -5,18 +5,14 @@
 #include "panel_kernel.hpp"
 
 int oxi_launch_lu_leaf32(oxi_handle_t h, hipStream_t s, const LeafArgs& a, int kind) {
-    if (a.P == 1 && kind == 0) OXI_TRY(launch_leaf(h, s, a, lu_leaf_kernel<float, 256, 1, 1>));
-    else if (a.P == 1 && kind == 1) OXI_TRY(launch_leaf(h, s, a, lu_leaf_kernel<float, 256, 2, 1>));
-    else if (a.P <= 64 && kind == 0) OXI_TRY(launch_leaf(h, s, a, lu_leaf_kernel<float, 256, 1, 64>));
-    else if (a.P <= 64 && kind == 1) OXI_TRY(launch_leaf(h, s, a, lu_leaf_kernel<float, 256, 2, 64>));
-    else OXI_TRY(launch_leaf(h, s, a, lu_leaf_kernel<float, 256, 4, OXI_LEAF_MAX_P>));
-    // the leaf's interchanges on the rest of its panel (its own columns are final)
-    const unsigned nblk = unsigned(cdiv(a.c0 - a.xlo, 64) + cdiv(a.xhi - a.c0 - a.w, 64));
-    if (nblk > 0) {
-        hipLaunchKernelGGL(leaf_swaps_kernel<float>, dim3(nblk), dim3(128), 0, s, (float*)a.Wm, a.ldw, a.c0, a.w,
-                           (const i64*)a.ipiv, (const int*)a.flags, a.xlo, a.xhi);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return oxi_set_error(h, OXI_ERR_HIP, "leaf_swaps launch: %s", hipGetErrorString(e));
-    }
-    return OXI_OK;
+    const bool wide = a.w > 32;
+    if (a.P == 1 && kind == 0 && !wide) return launch_leaf(h, s, a, lu_leaf_kernel<float, 1, 32, 1>);
+    if (a.P == 1 && kind == 0) return launch_leaf(h, s, a, lu_leaf_kernel<float, 1, 64, 1>);
+    if (kind == 0 && !wide) return launch_leaf(h, s, a, lu_leaf_kernel<float, 1, 32, 64>);
+    if (kind == 0) return launch_leaf(h, s, a, lu_leaf_kernel<float, 1, 64, 64>);
+    if (a.P == 1 && kind == 1 && !wide) return launch_leaf(h, s, a, lu_leaf_kernel<float, 2, 32, 1>);
+    if (a.P == 1 && kind == 1) return launch_leaf(h, s, a, lu_leaf_kernel<float, 2, 64, 1>);
+    if (kind == 1 && !wide) return launch_leaf(h, s, a, lu_leaf_kernel<float, 2, 32, 64>);
+    if (kind == 1) return launch_leaf(h, s, a, lu_leaf_kernel<float, 2, 64, 64>);
+    return launch_leaf(h, s, a, lu_leaf_kernel<float, 4, 32, OXI_LEAF_MAX_P>);
 }

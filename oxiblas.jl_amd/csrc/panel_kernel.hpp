@@ -183,15 +183,100 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // ---------------------------------------------------------------------------
-// The leaf kernel.  Thread t of workgroup p holds the rows that start at
-// positions p*R + s*LT + t (s < RPT) in registers, and they stay there: an
+// A leaf's interchanges on the other columns of the enclosing panel,
+// [x_lo, c0) and [c0+w, x_hi), by the nwg workgroups of 256 threads of a grid
+// (this one: wg).  Applying a leaf's interchanges to the rest of its panel at
+// once gives the same columns as the getrf2 recursion, which applies them
+// level by level: a left subtree's multipliers are not read again once its
+// right sibling has started, and the right sibling's columns receive them
+// before any update reads them.
+//
+// pi: lane i < w holds step i's pivot position relative to c0, -1 beyond, in
+// every wave.  The interchanges move the contents of 2W slots: slot i < w is
+// position i, slot W + i the pivot position of step i when it lies below the
+// leaf's w rows and i is its first step.  Every lane follows its slots
+// backwards through the transpositions (step i exchanges slot i with slot
+// sb_i), so the steps carry no dependence between lanes: one readlane and two
+// selects per slot and step.  A wave moves 32 slots of 64 columns (a lane per
+// column): the W / 16 waves of a group of columns load everything before any
+// of them stores (a wait and a barrier).  Loads are issued without branches: a
+// slot that does not move reads position 0, a lane outside the columns reads
+// column c0 (both in bounds), and only moving slots are stored.  Lane s
+// computes its slots' row offsets once; the loops only read them back.
+// ---------------------------------------------------------------------------
+template <typename T, int W>
+__device__ __forceinline__ void other_columns(T* Wm, i64 ldw, i64 c0, int w, int pi, i64 x_lo, i64 x_hi, int wg,
+                                              int nwg) {
+    const int groups_l = int((c0 - x_lo + 63) / 64), groups = groups_l + int((x_hi - c0 - w + 63) / 64);
+    constexpr int GW = W / 16, GPW = 4 / GW;       // waves per group of columns, groups per workgroup
+    if (wg * GPW >= groups) return;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+    int first = lane;
+#pragma unroll 8
+    for (int i = 0; i < W; ++i) {
+        const int q = __builtin_amdgcn_readlane(pi, i);
+        if (i < first && q == pi) first = i;
+    }
+    const int sbv = lane >= w ? lane : pi < w ? pi : W + first;   // the slot that step `lane` exchanges with its own
+    const int outp = lane < w && pi >= w && first == lane ? pi : -1;
+    constexpr int SL = 2 * W / 64;                 // slots per lane: lane, and lane + 64
+    int x[SL], from[SL], to[SL];
+#pragma unroll
+    for (int k = 0; k < SL; ++k) x[k] = lane + 64 * k;
+#pragma unroll 8
+    for (int i = W - 1; i >= 0; --i) {
+        const int sb = __builtin_amdgcn_readlane(sbv, i);
+#pragma unroll
+        for (int k = 0; k < SL; ++k) x[k] = x[k] == i ? sb : x[k] == sb ? i : x[k];
+    }
+    u64 mv[SL], offs[SL], offd[SL];
+#pragma unroll
+    for (int k = 0; k < SL; ++k) {
+        const int slot = lane + 64 * k;
+        const int out_of = __shfl(outp, slot & (W - 1));                  // of slot W + i
+        to[k] = slot < W ? (slot < w ? slot : -1) : out_of;
+        const int pi_of = __shfl(pi, x[k] & (W - 1));                     // position of slot W + i
+        from[k] = x[k] < W ? x[k] : pi_of;
+        const bool moves = to[k] >= 0 && x[k] != slot;
+        mv[k] = __ballot(moves);
+        offs[k] = u64((c0 + (moves ? from[k] : 0)) * ldw);
+        offd[k] = u64((c0 + (moves ? to[k] : 0)) * ldw);
+    }
+    const int s0 = 32 * (wave % GW);               // this wave's slots s0 .. s0 + 31
+    const u64 moving = (SL == 2 && s0 >= 64 ? mv[SL - 1] : mv[0]) >> (s0 & 63);
+    const u64 os = SL == 2 && s0 >= 64 ? offs[SL - 1] : offs[0], od = SL == 2 && s0 >= 64 ? offd[SL - 1] : offd[0];
+#pragma unroll 1
+    for (int g0 = wg * GPW; g0 < groups; g0 += nwg * GPW) {
+        const int g = g0 + wave / GW;
+        const bool left = g < groups_l;
+        const i64 xc = left ? x_lo + i64(g) * 64 + lane : c0 + w + i64(g - groups_l) * 64 + lane;
+        const bool ok = g < groups && (left ? xc < c0 : xc < x_hi);
+        const i64 xr = ok ? xc : c0;
+        T v[32];
+#pragma unroll
+        for (int k = 0; k < 32; ++k) v[k] = Wm[i64(readlane64(os, (s0 & 63) + k)) + xr];
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 32; ++k)
+            if ((moving >> k) & 1) {
+                const i64 to_row = i64(readlane64(od, (s0 & 63) + k));
+                if (ok) Wm[to_row + xc] = v[k];
+            }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// The leaf kernel (up to W columns).  Thread t of workgroup p holds the rows
+// that start at positions p*R + s*256 + t (s < RPT) in registers, and they stay there: an
 // interchange only changes positions (pos[s]; a row that became the pivot of
 // step j is retired to position j, pos[s] = ~j).  The registers of a row
 // rotate by one per column: at column j register c holds column j + c, so the
-// pivot column is always register 0, the rank-1 update is the same 31 FMAs at
+// pivot column is always register 0, the rank-1 update is the same W - 1 FMAs at
 // every step (v[c] <- v[c+1] - l u[c+1]), and every register index is a
-// compile-time constant in a rolled loop; the multiplier enters at register 31.
-// After 32 rotations register c holds column c again, multipliers and U values
+// compile-time constant in a rolled loop; the multiplier enters at register
+// W - 1.  After W rotations register c holds column c again, multipliers and U values
 // alike, and every row is stored once, at its final position: no store and no
 // interchange inside the column loop.  (u is zero past the row's live
 // columns, so the multipliers of earlier columns pass through the update
@@ -206,9 +291,12 @@ __device__ __forceinline__ void lds_barrier() {
 // barrier per column, for the comparison of the waves' candidates: every wave
 // reads all the headers itself and picks the winner in registers.
 //
-// WGS 1: one workgroup holds all the rows.  Each wave's candidate row
-// goes to LDS before that barrier, and every wave updates the winner's copy
-// itself.
+// WGS 1: one workgroup holds all the rows; the chosen row goes to the other
+// waves through LDS.
+//
+// At the end the leaf applies its interchanges to the other columns of the
+// panel (as a kernel of its own that took 5 to 9 us a leaf: n = 2000 5.30 ->
+// 5.11 ms, 16384 84.7 -> 83.7 ms).
 //
 // A column is a chain of dependent steps in one wave per SIMD, bound by
 // instruction and LDS latency plus one exchange between workgroups (1.1 us
@@ -222,18 +310,16 @@ __device__ __forceinline__ void lds_barrier() {
 // the header, then the exchange; the row's trip through LDS and the update
 // run in the exchange's shadow.
 // ---------------------------------------------------------------------------
-template <typename T, int LTT, int RPT, int WGS>
-__global__ __launch_bounds__(LTT) void lu_leaf_kernel(LeafArgs a) {
-    constexpr int LT = LTT, NWV = LT / 64, W = OXI_LEAF_W;
-    static_assert(W == 32 && NWV == 4, "record and wave layout");
+template <typename T, int RPT, int W, int WGS>
+__global__ __launch_bounds__(256) void lu_leaf_kernel(LeafArgs a) {
+    constexpr int LT = 256, NWV = LT / 64, NB = W / 16;   // NB: values of a row per lane of its spread form
+    static_assert(W == 32 || W == 64, "record layout");
     constexpr bool MULTI = WGS != 1;                  // WGS: 1, 64 or OXI_LEAF_MAX_P workgroups at most
     unsigned spin_limit = 1u << 22;                   // bound of every wait
     asm volatile("" : "+s"(spin_limit));              // not a constant: the polling loops stay rolled
-    constexpr int RS_N = W + 16 / int(sizeof(T));     // a row's LDS stride: 16-byte aligned, few bank conflicts
-    __shared__ __align__(16) T rows[2][NWV * RS_N];                // !MULTI: the waves' candidate rows, by column parity
     __shared__ __align__(16) int4 wcand[2][NWV];                   // each wave's candidate: key, low word, position; failed
-    __shared__ __align__(16) T raw[W];                             // MULTI: the chosen row before the pending update
-    __shared__ T raw_l[2][NWV];                                    // else: the candidates' multipliers
+    __shared__ __align__(16) T raw[W];                             // the chosen row before the pending update
+    __shared__ T raw_l;                                            // !MULTI: its multiplier
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int p = blockIdx.x, P = a.P;
@@ -270,41 +356,57 @@ __global__ __launch_bounds__(LTT) void lu_leaf_kernel(LeafArgs a) {
     // the winner of the current column, as every wave knows it
     T d = T(0), u1 = T(0);                  // values 0 and 1 of the pivot row
     int piv = 0;                            // its position
-    T ua = T(0), ub = T(0);                 // values lane & 15 and 16 + (lane & 15) in every row of 16 lanes
-    T uu = T(0);                            // MULTI: value lane / 2 + 1
+    T rv[NB] = {};                          // its values 16 b + (lane & 15) in every row of 16 lanes
+    T uu = T(0);                            // MULTI: its value that the lane publishing value c needs, c + 1
     unsigned row_off = 0, row_tag = 0;      // MULTI: the row's place in the exchange buffer, its tag
-    const unsigned oa = (lane & 15) * 16, ob = oa + 256, ou = min((lane >> 1) + 1, W - 1) * 16;
+    // the lane's column of a published row: two lanes per column (low and high
+    // half) up to 32 columns, one beyond
+    const int pc = W == 32 ? lane >> 1 : lane;
+    const unsigned oa = (lane & 15) * 16, ou = min(pc + 1, W - 1) * 16;
     const __amdgpu_buffer_rsrc_t pub_rsrc =
         __builtin_amdgcn_make_buffer_rsrc((void*)a.pub, 0, int(OXI_LEAF_PUB * 8), 0x00027000);
     bool timed_out = false;                 // this wave's last wait failed
 
     // ---- MULTI: the winner's row from the words fetched ahead; fetched again
     // (bounded) while a word is not the column's yet
-    auto row_arrives = [&](uint4v xa, uint4v xb, uint4v xu) __attribute__((always_inline)) {
+    struct Ahead { uint4v b[NB], u; };
+    auto row_ahead = [&]() __attribute__((always_inline)) -> Ahead {
+        Ahead x;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) x.b[b] = load_words_ahead(pub_rsrc, row_off + oa + 256 * b);
+        x.u = load_words_ahead(pub_rsrc, row_off + ou);
+        return x;
+    };
+    auto row_arrives = [&](Ahead x) __attribute__((always_inline)) {
         const unsigned tag = row_tag;
         unsigned spins = 0;
 #pragma unroll 1
         while (true) {
-            unsigned diff = (xa.y ^ tag) | (xa.w ^ tag) | (xb.y ^ tag) | (xb.w ^ tag) | (xu.y ^ tag) | (xu.w ^ tag);
+            unsigned diff = (x.u.y ^ tag) | (x.u.w ^ tag);
+#pragma unroll
+            for (int b = 0; b < NB; ++b) diff |= (x.b[b].y ^ tag) | (x.b[b].w ^ tag);
             asm("" : "+v"(diff));   // one compare, not six and a chain of scalar ors
             if (__builtin_expect(__ballot(diff != 0) == 0, 1)) break;
             if (++spins > spin_limit) { timed_out = true; break; }   // uniform per wave
             const char* row = (const char*)a.pub + row_off;
-            load_words3((const u64*)(row + oa), (const u64*)(row + ob), (const u64*)(row + ou), xa, xb, xu);
+            load_words3((const u64*)(row + oa), (const u64*)(row + oa + 256), (const u64*)(row + ou), x.b[0], x.b[1], x.u);
+            if constexpr (NB == 4)
+                load_words3((const u64*)(row + oa + 512), (const u64*)(row + oa + 768), (const u64*)(row + ou), x.b[2], x.b[3],
+                            x.u);
         }
-        ua = from_words<T>(xa.x, xa.z);
-        ub = from_words<T>(xb.x, xb.z);
-        uu = from_words<T>(xu.x, xu.z);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) rv[b] = from_words<T>(x.b[b].x, x.b[b].z);
+        uu = from_words<T>(x.u.x, x.u.z);
     };
 
     // ---- the candidate of column jn and its publication.  x[s]: row s's
     // value in column jn (register REG).  PEND: the registers still await the
-    // update of column jn - 1 (multipliers l, the row in xa, xb, xu); only
+    // update of column jn - 1 (multipliers l, the row in ahead); only
     // the chosen row is then updated here.  False when a wave of the
     // workgroup timed out.  Straight-line code but for ties: a taken branch
     // costs about as much as ten dependent instructions.
     auto select_publish = [&](int jn, const T (&x)[RPT], auto pend_c, const T (&l)[RPT], bool upd,
-                              uint4v xa, uint4v xb, uint4v xu) __attribute__((always_inline)) -> bool {
+                              Ahead ahead) __attribute__((always_inline)) -> bool {
         constexpr bool PEND = decltype(pend_c)::value;
         constexpr int REG = PEND ? 1 : 0;
         const int parn = jn & 1;
@@ -366,10 +468,6 @@ __global__ __launch_bounds__(LTT) void lu_leaf_kernel(LeafArgs a) {
                     asm volatile("; slot %0" ::"n"(s));
                 }
         };
-        if constexpr (!MULTI) {
-            row_out(&rows[parn][wave * RS_N]);
-            if (lane == 0) raw_l[parn][wave] = lw;
-        }
         lds_barrier();
         const int4 e = wcand[parn][lane & (NWV - 1)];
         int em = dpp_imax<0xB1>(e.x);                   // quad_perm [1,0,3,2]
@@ -378,47 +476,66 @@ __global__ __launch_bounds__(LTT) void lu_leaf_kernel(LeafArgs a) {
         int ww = first_lane(eb);
         if (__builtin_expect((eb & (eb - 1)) != 0, 0)) ww = settle_tie(eb, unsigned(e.y), e.z);
         if constexpr (!MULTI) {
-            // every wave updates the winner's row itself: ua, ub of the new
-            // row from those of the old one, one value further
+            // the chosen row goes to every wave, which updates it itself: the
+            // new row's spread values from the old one's, one value further
+            // (every wave's candidate in LDS before the first barrier, and no
+            // second one, takes longer: the stores of the four waves share
+            // the LDS)
             piv = __builtin_amdgcn_readlane(e.z, ww);
-            const T* src = &rows[parn][ww * RS_N];
-            const int i = lane & 15;
-            T na = src[i], nb = src[16 + i];
-            if (PEND && upd) {
-                const T wl_ = raw_l[parn][ww];
-                const T sa = row_shl1(ua), sb1 = row_shl1(ub), b0 = row_bcast<0>(ub);
-                na = fma_t(-wl_, i == 15 ? b0 : sa, na);
-                nb = fma_t(-wl_, i == 15 ? T(0) : sb1, nb);
+            if (wave == ww) {
+                row_out(raw);
+                if (lane == 0) raw_l = lw;
             }
-            ua = i < W - jn ? na : T(0);
-            ub = 16 + i < W - jn ? nb : T(0);
-            d = readlane_t(ua, 0);
-            u1 = readlane_t(ua, 1);
+            lds_barrier();
+            const int i = lane & 15;
+            T nv[NB];
+#pragma unroll
+            for (int b = 0; b < NB; ++b) nv[b] = raw[16 * b + i];
+            if (PEND && upd) {
+                const T wl_ = raw_l;
+                T sh[NB];
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    const T next = b + 1 < NB ? row_bcast<0>(rv[b + 1 < NB ? b + 1 : 0]) : T(0);
+                    const T sl = row_shl1(rv[b]);
+                    sh[b] = i == 15 ? next : sl;
+                }
+#pragma unroll
+                for (int b = 0; b < NB; ++b) nv[b] = fma_t(-wl_, sh[b], nv[b]);
+            }
+#pragma unroll
+            for (int b = 0; b < NB; ++b) rv[b] = 16 * b + i < W - jn ? nv[b] : T(0);
+            d = readlane_t(rv[0], 0);
+            u1 = readlane_t(rv[0], 1);
             return true;
         } else {
-            if (PEND) row_arrives(xa, xb, xu);
+            if (PEND) row_arrives(ahead);
             if (wave == ww && jn < w) {
                 // this wave holds the workgroup's candidate: the header first,
                 // from its lane's registers (value 1 is column jn + 1 updated)
                 const u64 tag = u64(a.tag + unsigned(jn)) << 32;
-                if (PEND && upd) ys = fma_t(-ls, row_bcast<2>(ua), ys);
+                if (PEND && upd) ys = fma_t(-ls, row_bcast<2>(rv[0]), ys);
                 const T h0 = none ? T(0) : readlane_t(xs, wl), h1 = none || jn + 1 >= W ? T(0) : readlane_t(ys, wl);
                 const unsigned hd = lane == 0 ? word_lo(h0) : lane == 1 ? word_hi(h0) : lane == 2 ? word_lo(h1)
                                   : lane == 3 ? word_hi(h1) : unsigned(pos_w);
                 if (lane < 6)
                     __hip_atomic_store(a.pub + size_t(w) * P * OXI_PUB_STRIDE + (size_t(jn) * P + p) * OXI_PUB_HDR + lane,
                                        tag | hd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                // then the whole row, two lanes per column (low and high half)
+                // then the whole row
                 row_out(raw);
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // the lane's LDS writes before the reads below
                 __builtin_amdgcn_wave_barrier();
-                const int c = lane >> 1;
-                T r = raw[c];
+                T r = raw[pc];
                 if (PEND && upd) r = fma_t(-lw, uu, r);
-                if (none || c >= W - jn) r = T(0);
-                const unsigned data = (lane & 1) ? word_hi(r) : word_lo(r);
-                __hip_atomic_store(a.pub + (size_t(jn) * P + p) * OXI_PUB_STRIDE + lane, tag | data, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
+                if (none || pc >= W - jn) r = T(0);
+                u64* row = a.pub + (size_t(jn) * P + p) * OXI_PUB_STRIDE;
+                if constexpr (W == 32) {
+                    __hip_atomic_store(row + lane, tag | ((lane & 1) ? word_hi(r) : word_lo(r)), __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+                } else {
+                    __hip_atomic_store(row + 2 * lane, tag | word_lo(r), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(row + 2 * lane + 1, tag | word_hi(r), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
             }
             if (__builtin_expect(__ballot(e.w != 0) != 0, 0)) {   // a wave's wait timed out (the same in every wave)
                 if (t == 0) __hip_atomic_store(a.flags, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -481,14 +598,14 @@ __global__ __launch_bounds__(LTT) void lu_leaf_kernel(LeafArgs a) {
         T x0[RPT], l0[RPT];
 #pragma unroll
         for (int s = 0; s < RPT; ++s) { x0[s] = v[s][0]; l0[s] = T(0); }
-        if (!select_publish(0, x0, std::false_type{}, l0, false, {}, {}, {})) return;
+        if (!select_publish(0, x0, std::false_type{}, l0, false, {})) return;
         if constexpr (MULTI) poll(0);
     }
 
-    int my_piv = 0, first_zero = -1;   // wave 0 of workgroup 0: lane j holds step j's pivot position
+    int my_piv = -1, first_zero = -1;   // lane j holds step j's pivot position
     // state of column j between its record's publication and its update
-    T l[RPT], lin[RPT];   // the multiplier for the update (0: row not updated), the value entering register 31
-    T ra = T(0), rb = T(0);   // the pivot row's values
+    T l[RPT], lin[RPT];   // the multiplier for the update (0: row not updated), the value entering register W - 1
+    T ru[NB] = {};            // the pivot row's values
     bool updates = false;     // column j has a pivot
     bool odd = false;         // the update needs its selects: an infinity, a NaN or a zero pivot
 
@@ -496,14 +613,10 @@ __global__ __launch_bounds__(LTT) void lu_leaf_kernel(LeafArgs a) {
     // record (past the last column nothing is published).  False on timeout.
     auto head = [&](int j) __attribute__((always_inline)) -> bool {
         // the winner's row starts on its way
-        uint4v xa = {}, xb = {}, xu = {};
-        if constexpr (MULTI) {
-            xa = load_words_ahead(pub_rsrc, row_off + oa);
-            xb = load_words_ahead(pub_rsrc, row_off + ob);
-            xu = load_words_ahead(pub_rsrc, row_off + ou);
-        }
+        Ahead ahead = {};
+        if constexpr (MULTI) ahead = row_ahead();
         const bool upd = d != T(0);
-        my_piv = wave == 0 && lane == j ? piv : my_piv;
+        my_piv = lane == j ? piv : my_piv;
         first_zero = !upd && first_zero < 0 ? j : first_zero;
         updates = upd;
         bool strange = !upd || non_finite(d);
@@ -519,10 +632,16 @@ __global__ __launch_bounds__(LTT) void lu_leaf_kernel(LeafArgs a) {
             x[s] = upd ? fma_t(-l[s], u1, v[s][1]) : v[s][1];
             strange |= non_finite(l[s]);
         }
-        if constexpr (!MULTI) { ra = ua; rb = ub; }   // this column's row (select_publish makes the next one's)
-        if (!select_publish(j + 1, x, std::true_type{}, l, upd, xa, xb, xu)) return false;
-        if constexpr (MULTI) { ra = ua; rb = ub; }
-        odd = __ballot(strange || non_finite(ra) || non_finite(rb)) != 0;
+        // !MULTI: select_publish makes the next column's row
+#pragma unroll
+        for (int b = 0; b < NB; ++b) ru[b] = rv[b];
+        if (!select_publish(j + 1, x, std::true_type{}, l, upd, ahead)) return false;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            if constexpr (MULTI) ru[b] = rv[b];   // it arrived in select_publish
+            strange |= non_finite(ru[b]);
+        }
+        odd = __ballot(strange) != 0;
         return true;
     };
     if (!head(0)) return;
@@ -540,7 +659,7 @@ __global__ __launch_bounds__(LTT) void lu_leaf_kernel(LeafArgs a) {
             T u[4];
             static_for<4>([&](auto c_c) __attribute__((always_inline)) {
                 constexpr int C = G + decltype(c_c)::value;
-                if constexpr (C > 0) u[C - G] = C < 16 ? row_bcast<C & 15>(ra) : row_bcast<C & 15>(rb);
+                if constexpr (C > 0) u[C - G] = row_bcast<C & 15>(ru[C / 16]);
             });
             __builtin_amdgcn_sched_barrier(0);
             static_for<4>([&](auto c_c) __attribute__((always_inline)) {
@@ -564,7 +683,7 @@ __global__ __launch_bounds__(LTT) void lu_leaf_kernel(LeafArgs a) {
     for (; j < w; ++j) {
         static_for<W - 1>([&](auto c_c) __attribute__((always_inline)) {
             constexpr int C = decltype(c_c)::value + 1;
-            const T uc = C < 16 ? row_bcast<C & 15>(ra) : row_bcast<C & 15>(rb);
+            const T uc = row_bcast<C & 15>(ru[C / 16]);
 #pragma unroll
             for (int s = 0; s < RPT; ++s) {
                 const bool live = updates && pos[s] >= 0 && C < W - j;
@@ -611,102 +730,9 @@ __global__ __launch_bounds__(LTT) void lu_leaf_kernel(LeafArgs a) {
         if (lane < w) a.ipiv[a.c0 + lane] = a.c0 + my_piv + 1;
         if (lane == 0 && first_zero >= 0 && *a.info == 0) *a.info = a.c0 + first_zero + 1;
     }
-}
-
-// The slots of the interchanges of a leaf's w steps at c0 (one wave): lane
-// i < w is step i's own position; lane w + i is the pivot position p_i of step
-// i when it lies below the leaf's w rows and i is its first occurrence.
-// pos = -1 for unused lanes.
-// The interchanges are then replayed on slot ids: afterwards lane s holds
-// the slot whose original content ends at slot s.  Every lane follows its
-// own slot backwards through the transpositions (step i exchanges slot i
-// with slot sb_i, held by lane i), so the steps carry no cross-lane
-// dependence: one readlane and two selects each.
-// pi: lane i < w holds step i's pivot position relative to c0 (-1 beyond).
-__device__ __forceinline__ void leaf_slots(i64 pi, int w, int lane, i64& pos, int& src) {
-    // unrolled to the largest leaf without a bound test (the readlanes of
-    // different steps are independent and interleave): lanes i >= w hold
-    // pi = -1, which matches only lanes >= w, whose first is not used
-    int first = lane;
-#pragma unroll
-    for (int i = 0; i < OXI_LEAF_W; ++i) {
-        const i64 q = (i64)readlane64(u64(pi), i);
-        if (i < first && q == pi) first = i;
-    }
-    pos = lane < w ? lane : -1;
-    const int src_i = lane - w;   // differs per lane: a shuffle, not readlane
-    const int src_l = (src_i >= 0 && src_i < w) ? src_i : 0;
-    const i64 pos_out = (i64)__shfl((long long)pi, src_l);
-    const int first_out = __shfl(first, src_l);
-    if (src_i >= 0 && src_i < w && pos_out >= w && first_out == src_i) pos = pos_out;
-    // the slot that step i exchanges with slot i (lane i < w)
-    const int sbv = lane < w ? (pi < w ? int(pi) : w + first) : lane;
-    // the content that ends at slot `lane`: the transpositions of steps
-    // w-1 .. 0 applied to it in turn (steps i >= w exchange slot i with
-    // itself: sbv = lane there)
-    int x = lane;
-#pragma unroll
-    for (int i = OXI_LEAF_W - 1; i >= 0; --i) {
-        const int sb = __builtin_amdgcn_readlane(sbv, i);
-        x = x == i ? sb : x == sb ? i : x;
-    }
-    src = x;
-}
-
-// A leaf's interchanges on the other columns of the enclosing panel,
-// [x_lo, c0) and [c0+w, x_hi): blocks of two waves take 64 columns each (a
-// lane per column), half of the slots by each wave.  The leaf's own columns
-// are stored at their final positions by the leaf itself.
-// Applying a leaf's interchanges to the rest of its panel at once gives the
-// same columns as the getrf2 recursion, which applies them level by level:
-// a left subtree's multipliers are not read again once its right sibling
-// has started, and the right sibling's columns receive them before any
-// update reads them.
-template <typename T>
-__global__ __launch_bounds__(128) void leaf_swaps_kernel(T* Wm, i64 ldw, i64 c0, int w, const i64* ipiv,
-                                                         const int* flags, i64 x_lo, i64 x_hi) {
-    const int lane = threadIdx.x & 63;
-    const int half = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-    // the pivots are loaded with the flag, not after its test, and without a
-    // branch (lanes >= w read entry c0): one memory round trip for both
-    // (ipiv lies in its own allocation, always readable)
-    const i64 pv = ipiv[c0 + (lane < w ? lane : 0)];
-    if (__hip_atomic_load(flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return;
-    const i64 pi_all = lane < w ? pv - 1 - c0 : -1;
-    const i64 fb = blockIdx.x;
-    const i64 tl = (c0 - x_lo + 63) / 64;
-    i64 x;
-    bool ok;
-    if (fb < tl) { x = x_lo + fb * 64 + lane; ok = x < c0; }
-    else { x = c0 + w + (fb - tl) * 64 + lane; ok = x < x_hi; }
-    i64 pos; int src;
-    leaf_slots(pi_all, w, lane, pos, src);
-    // slot s moves when its source differs (at most 2w <= 64 slots).  Both
-    // waves compute all slots; wave h moves slots 32h .. 32h+31.  All loads
-    // of the block have returned before any store (a wait and a barrier) and
-    // are issued without branches: a slot that does not move reads its own
-    // position, a lane outside the columns reads column c0 (both in bounds),
-    // and only moving slots are stored.  Lane s computes slot s's row
-    // offsets once; the loops only read them back (two readlanes and an add
-    // per slot and access).
-    const i64 psrc = (i64)__shfl((long long)pos, src);
-    const bool moves = pos >= 0 && src != lane;
-    const u64 mv = __ballot(moves);
-    const i64 offs = (c0 + (moves ? psrc : 0)) * ldw;
-    const i64 offd = (c0 + (moves ? pos : 0)) * ldw;
-    const i64 xr = ok ? x : c0;
-    const int s0 = 32 * half;
-    T v[32];
-#pragma unroll
-    for (int k = 0; k < 32; ++k) v[k] = Wm[(i64)readlane64(u64(offs), s0 + k) + xr];
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 32; ++k)
-        if ((mv >> (s0 + k)) & 1) {
-            const i64 to = (i64)readlane64(u64(offd), s0 + k);
-            if (ok) Wm[to + x] = v[k];
-        }
+    // the interchanges on the rest of the panel: columns that no workgroup
+    // has touched
+    other_columns<T, W>(Wm, a.ldw, a.c0, w, lane < w ? my_piv : -1, a.xlo, a.xhi, p, P);
 }
 
 // One leaf launch.  Every workgroup asks for LEAF_LDS bytes of LDS, far more

@@ -35,7 +35,7 @@
 
 namespace {
 
-constexpr int TW = OXI_LEAF_W;           // 32
+constexpr int TW = 32;
 constexpr int TLT = 256, TNWV = TLT / 64;
 constexpr int TP_LEVELS = 3;             // tree levels over workgroups: 32 -> 8 -> 2 -> 1
 constexpr int TP_REC = 36;               // record fields: tag, count, 32 positions, spare, checksum
@@ -388,6 +388,16 @@ __global__ __launch_bounds__(TLT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     }
 }
 
+__global__ __launch_bounds__(256) void tp_swaps_kernel(LeafArgs a) {
+    const int lane = threadIdx.x & 63;
+    // the pivots are loaded with the flag, not after its test, and without a
+    // branch (lanes >= w read entry c0): one memory round trip for both
+    const i64 pv = a.ipiv[a.c0 + (lane < a.w ? lane : 0)];
+    if (__hip_atomic_load(a.flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return;
+    other_columns<float, TW>((float*)a.Wm, a.ldw, a.c0, a.w, lane < a.w ? int(pv - 1 - a.c0) : -1, a.xlo, a.xhi,
+                             int(blockIdx.x), int(gridDim.x));
+}
+
 }  // namespace
 
 int oxi_launch_lu_leaf_tp(oxi_handle_t h, hipStream_t s, const LeafArgs& a, int kind) {
@@ -397,12 +407,11 @@ int oxi_launch_lu_leaf_tp(oxi_handle_t h, hipStream_t s, const LeafArgs& a, int 
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return oxi_set_error(h, OXI_ERR_HIP, "lu_leaf_tp launch: %s", hipGetErrorString(e));
     // the leaf's interchanges on the rest of its panel (its own columns are final)
-    const unsigned nblk = unsigned(cdiv(a.c0 - a.xlo, 64) + cdiv(a.xhi - a.c0 - a.w, 64));
-    if (nblk > 0) {
-        hipLaunchKernelGGL(leaf_swaps_kernel<float>, dim3(nblk), dim3(128), 0, s, (float*)a.Wm, a.ldw, a.c0, a.w,
-                           (const i64*)a.ipiv, (const int*)a.flags, a.xlo, a.xhi);
+    const i64 groups = cdiv(a.c0 - a.xlo, 64) + cdiv(a.xhi - a.c0 - a.w, 64);
+    if (groups > 0) {
+        hipLaunchKernelGGL(tp_swaps_kernel, dim3(unsigned(cdiv(groups, 2))), dim3(256), 0, s, a);
         e = hipGetLastError();
-        if (e != hipSuccess) return oxi_set_error(h, OXI_ERR_HIP, "leaf_swaps launch: %s", hipGetErrorString(e));
+        if (e != hipSuccess) return oxi_set_error(h, OXI_ERR_HIP, "tp_swaps launch: %s", hipGetErrorString(e));
     }
     return OXI_OK;
 }

@@ -1,9 +1,10 @@
 """The panel leaf at the sizes where its work division changes: the rows of
-one workgroup (256, 512), several workgroups, two rows per thread (above 8192
-rows) and widths 1..32.  A matrix of at most 32 columns is one leaf, whose
-operations (a division, then fma(-l, u, a) in column order) are the oracle's
+one workgroup (256, 512), several workgroups, two rows per thread (257 to 512
+and above 8192 rows) and widths 1..64.  Up to 32 columns the leaf's operations
+(per column a division, then fma(-l, u, a)) are the oracle's
 (src/lapack/factorizations.jl:89-140), so factors, pivots and info are equal
-bit for bit."""
+bit for bit; beyond, the oracle halves the columns, and the pivots are
+LAPACK's and the reconstruction is within the LU tests' bound."""
 import numpy as np
 import pytest
 
@@ -32,6 +33,28 @@ def test_leaf_random_and_ties(gpu, rng, m, w):
     # equal high words, different low words: settled by the low word
     A = 1.0 + rng.integers(0, 1 << 20, (m, w)) * 2.0 ** -52
     check(gpu, A * rng.choice([-1.0, 1.0], (m, w)))
+
+
+@pytest.mark.parametrize("m,w", [(64, 64), (100, 33), (255, 64), (257, 64), (700, 47), (2048, 64), (8192, 63)])
+def test_wide_leaf(gpu, rng, m, w):
+    from scipy.linalg.lapack import dgetrf
+    A = rng.standard_normal((m, w))
+    F = gpu.lu(gpu.DMatrix.from_numpy(A))
+    lu, piv, info = dgetrf(A)
+    np.testing.assert_array_equal(F.ipiv, piv + 1)
+    X = F.factors.numpy()
+    L = np.tril(X, -1)
+    L[np.arange(w), np.arange(w)] = 1.0
+    R = A[F.p - 1] - L @ np.triu(X[:w])
+    assert np.linalg.norm(R) <= 30 * w * np.finfo(float).eps * np.linalg.norm(A)
+    # a zero column and a NaN row: info of the first, NaN never a pivot below
+    # the diagonal
+    A[:, w - 2] = 0.0
+    A[m - 1, w - 1] = np.nan
+    F = gpu.lu(gpu.DMatrix.from_numpy(A), check=False)
+    lu, piv, info = dgetrf(A[:, :w - 2])
+    assert F.info == w - 1
+    np.testing.assert_array_equal(F.ipiv[:w - 2], piv + 1)
 
 
 @pytest.mark.parametrize("m,w", [(40, 8), (300, 32), (700, 32), (9000, 32)])
