@@ -17,6 +17,7 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 namespace {
 
@@ -30,17 +31,6 @@ template <typename T> __device__ __forceinline__ bool pos_finite(T d);
 template <> __device__ __forceinline__ bool pos_finite(double d) { return d > 0.0 && d <= 1.7976931348623157e308; }
 template <> __device__ __forceinline__ bool pos_finite(float d) { return d > 0.0f && d <= 3.4028234663852886e38f; }
 
-// A (n x n, n <= 64, lower triangle) in place; `off` is the global index of
-// its first column; *info receives off + c + 1 at the first failing column c.
-// One wave: lane i holds row i (a[k] = A(i, k), k <= i) in registers, and
-// the column loop is unrolled, so every register index is a compile-time
-// constant and no step waits at a workgroup barrier.  Per column c: the
-// pivot from lane c (a readlane), its square root, every lane's multiplier
-// l_ic = a_ic / r into LDS, then each lane updates its row right of c
-// (a_ik = fma(-l_ic, l_kc, a_ik)) with the multipliers read back.  Elements
-// right of the diagonal take the same operations on values nobody stores.
-// A failing pivot (not finite and positive) stops the loop: the columns
-// before it are final, the rest keep their updated values.
 template <typename T>
 __device__ __forceinline__ T readlane_t(T x, int l);
 template <>
@@ -54,39 +44,131 @@ __device__ __forceinline__ float readlane_t(float x, int l) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), l));
 }
 
+// x of lane N of each row of 16 lanes, in every lane of the row
+template <int N> __device__ __forceinline__ double row_bcast(double x) {
+    return __builtin_amdgcn_update_dpp(0.0, x, 0x150 + N, 0xf, 0xf, true);   // row_newbcast:N
+}
+template <int N> __device__ __forceinline__ float row_bcast(float x) {
+    return __builtin_amdgcn_update_dpp(0.0f, x, 0x150 + N, 0xf, 0xf, true);
+}
+// d = c - a * b with a destination of its own: the rotated update would else
+// become the two-operand form and a move per register
+__device__ __forceinline__ double nfma_to(double a, double b, double c) {
+    double d;
+    asm("v_fma_f64 %0, -%1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+    return d;
+}
+__device__ __forceinline__ float nfma_to(float a, float b, float c) {
+    float d;
+    asm("v_fma_f32 %0, -%1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+    return d;
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (N > 0) {
+        static_for<N - 1>(f);
+        f(std::integral_constant<int, N - 1>{});
+    }
+}
+
+// A (n x n, n <= 64, lower triangle) in place; `off` is the global index of
+// its first column; *info receives off + c + 1 at the first failing column c.
+// One wave: lane i holds row i in registers.  The registers rotate by one per
+// column, so the loop is rolled with compile-time register indices (unrolled
+// over the columns its code is as large as the instruction cache and is
+// fetched anew by every launch).  Per column j: the pivot from lane j, its
+// square root r, every lane's multiplier l_ij = a_ij / r; the update of the
+// other columns, a_ik = fma(-l_ij, l_kj, a_ik), takes l_kj from a copy of the
+// multipliers in LDS, spread so that a DPP broadcast brings one to every lane.
+// Column j + 1 is updated first, by a readlane, and the update that column j
+// leaves to the others comes after column j + 1's square root and division.
+// Elements right of the diagonal take the same operations on values nobody
+// stores.
+// A failing pivot (not finite and positive) ends the updates: the columns
+// before it are final, the rest keep their updated values.
+// Bound by the 63 FMAs and broadcasts of a column in one wave (0.31 us a
+// column; laying the steps of the square root and the division among them
+// changed nothing): 31 us for 64 columns, launch and stores included, against
+// 41 for an unrolled form whose multipliers every lane read from LDS.
 template <typename T>
 __global__ __launch_bounds__(64) void potrf_leaf_kernel(T* __restrict__ A, i64 lda, int n, i64 off,
                                                         i64* __restrict__ info) {
-    __shared__ __align__(16) T lcol[CLEAF];   // the multipliers of the current column
+    __shared__ T lcol[2 * CLEAF];             // the multipliers of a column, zeros behind them
     if (*info != 0) return;                   // an earlier leaf failed
     const int i = threadIdx.x;
-    T a[CLEAF];
+    T v[CLEAF];
+    const T* arow = A + min(i, n - 1);
+    if (n == CLEAF) {
 #pragma unroll
-    for (int k = 0; k < CLEAF; ++k) a[k] = (i < n && k <= i) ? A[i + k * lda] : T(0);
-    bool go = true;   // uniform
+        for (int k = 0; k < CLEAF; ++k) v[k] = arow[k * lda];
+    } else {
 #pragma unroll
-    for (int c = 0; c < CLEAF; ++c) {
-        if (go && c < n) {
-            const T d = readlane_t(a[c], c);
-            if (!pos_finite(d)) {
-                if (i == 0) *info = off + c + 1;
-                go = false;
-            } else {
-                const T r = sqrt_t(d);
-                const T l = i > c ? a[c] / r : T(0);
-                a[c] = i == c ? r : i > c ? l : a[c];
-                lcol[i] = l;
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // the lanes' LDS writes before the reads below
-                __builtin_amdgcn_wave_barrier();
-#pragma unroll
-                for (int k = c + 1; k < CLEAF; ++k) a[k] = fma_t(-l, lcol[k], a[k]);
-                __builtin_amdgcn_wave_barrier();   // every read of this column before the next column's writes
-            }
-        }
+        for (int k = 0; k < CLEAF; ++k) v[k] = k < n ? arow[k * lda] : T(0);
     }
+    lcol[CLEAF + i] = T(0);
+    bool go = true;                           // uniform
+    i64 failed = 0;
+    T x = v[0];                               // column j, updated through column j - 1
+    T l = T(0), lin = T(0), u[4] = {};        // column j - 1: multipliers, final values, multipliers spread
+    // the multipliers of column j from q = x / r, and column j + 1's values
+    auto column = [&](int j, T r, T q, bool ok) __attribute__((always_inline)) {
+        failed = go && !ok ? off + j + 1 : failed;
+        go = ok;
+        l = ok && i > j ? q : T(0);
+        lin = ok ? (i == j ? r : i > j ? q : x) : x;
+        lcol[i] = l;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // the lanes' LDS writes before the reads below
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int b = 0; b < 4; ++b) u[b] = lcol[j + 16 * b + (i & 15)];
+        x = fma_t(-l, readlane_t(l, min(j + 1, CLEAF - 1)), v[1]);
+        __builtin_amdgcn_wave_barrier();      // every read before the next column's writes
+    };
+    {
+        const T d = readlane_t(x, 0), r = sqrt_t(d);
+        column(0, r, x / r, pos_finite(d));
+    }
+#pragma unroll 1
+    for (int j0 = 1; j0 < n; ++j0) {
+        const int j = __builtin_amdgcn_readfirstlane(j0);
+        const T d = readlane_t(x, j);
+        const bool ok = go && pos_finite(d);
+        const T r = sqrt_t(d);
+        const T q = x / r;
+        // column j - 1's update of the others, with the rotation: register c
+        // holds column j + c afterwards
+        static_for<CLEAF / 4>([&](auto g_c) __attribute__((always_inline)) {
+            constexpr int G = 4 * decltype(g_c)::value;
+            T b[4];
+            static_for<4>([&](auto c_c) __attribute__((always_inline)) {
+                constexpr int C = G + decltype(c_c)::value;
+                if constexpr (C > 0) b[C - G] = row_bcast<C & 15>(u[C / 16]);
+            });
+            static_for<4>([&](auto c_c) __attribute__((always_inline)) {
+                constexpr int C = G + decltype(c_c)::value;
+                if constexpr (C > 0) v[C - 1] = nfma_to(l, b[C - G], v[C]);
+            });
+        });
+        v[CLEAF - 1] = lin;
+        column(j, r, q, ok);
+    }
+    // the last column's place, then the rest of the turn
+    {
+#pragma unroll
+        for (int c = 0; c + 1 < CLEAF; ++c) v[c] = v[c + 1];
+        v[CLEAF - 1] = lin;
+    }
+#pragma unroll 1
+    for (int k = n; k < CLEAF; ++k) {
+        const T first = v[0];
+#pragma unroll
+        for (int c = 0; c + 1 < CLEAF; ++c) v[c] = v[c + 1];
+        v[CLEAF - 1] = first;
+    }
+    if (failed && i == 0) *info = failed;
 #pragma unroll
     for (int k = 0; k < CLEAF; ++k)
-        if (i < n && k <= i) A[i + k * lda] = a[k];
+        if (i < n && k <= i) A[i + k * lda] = v[k];
 }
 
 // zero the strict upper triangle (the factor's storage contract)
