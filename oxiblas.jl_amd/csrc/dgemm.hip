@@ -8,10 +8,10 @@
 // while the matrix cores consume the current one.
 //
 // Work decomposition: a 256-thread workgroup owns a tile of C, its four
-// waves split it 2 x 2.  Large products take 128 x 128 tiles on
-// v_mfma_f64_16x16x4 (dgemm_m16_kernel); products whose 128 x 128 grid would
-// leave CUs idle take 64 x 64 or 32 x 32 tiles on v_mfma_f64_4x4x4_4b
-// (dgemm_mfma_kernel).  Both instructions reach the full FP64 rate on gfx950.  The epilogue applies alpha and beta as the
+// waves split it 2 x 2.  dgemm_direct_kernel (128 x 128, 64 x 64 or 32 x 32
+// tiles on v_mfma_f64_16x16x4) takes all products but those whose operands it
+// cannot fetch in pairs; these run on dgemm_mfma_kernel (v_mfma_f64_4x4x4_4b,
+// slabs staged through registers).  The epilogue applies alpha and beta as the
 // reference's full tiles do: v = alpha*acc; C = beta == 0 ? v : fma(beta, C, v)
 // (src/blas/simd.jl:190-196); beta == 0 never reads C.
 #include "oxi_internal.hpp"
@@ -20,6 +20,7 @@
 #include <vector>
 #include <algorithm>
 #include <limits>
+#include <type_traits>
 
 namespace {
 
@@ -54,24 +55,6 @@ __device__ __forceinline__ void load_slab(double (&r)[O * BK / NT], const double
         else { kk = t % BK; o = t / BK + i * (NT / BK); }
         i64 go = o0 + o, gk = k0 + kk;
         r[i] = (go < outer && gk < K) ? (OUTER_CONTIG ? X[go + gk * ldx] : X[gk + go * ldx]) : 0.0;
-    }
-}
-
-// The same without bounds checks, for tiles that lie inside the operands
-// with K a multiple of the slab depth: no branch in the slab loop, whose
-// merge with the guarded path would otherwise leave a wait for all loads
-// between the two operands' loads.
-template <bool OUTER_CONTIG, int O, int BK>
-__device__ __forceinline__ void load_slab_inner(double (&r)[O * BK / NT], const double* __restrict__ X, i64 ldx,
-                                                i64 o0, i64 k0, int t) {
-    constexpr int LOADS = O * BK / NT;
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-        int o, kk;
-        if (OUTER_CONTIG) { o = t % O; kk = t / O + i * (NT / O); }
-        else { kk = t % BK; o = t / BK + i * (NT / BK); }
-        const i64 go = o0 + o, gk = k0 + kk;
-        r[i] = OUTER_CONTIG ? X[go + gk * ldx] : X[gk + go * ldx];
     }
 }
 
@@ -325,177 +308,266 @@ __global__ __launch_bounds__(NT) void dgemm_mfma_kernel(i64 M, i64 N, i64 K, dou
     }
 }
 
-// 128 x 128 tiles on v_mfma_f64_16x16x4: each wave owns 64 x 64 of C as 4 x 4
-// blocks of 16 x 16 (four accumulators per lane each).  One instruction does
-// four times the work of a 4x4x4_4b one for the same two LDS reads, and the
-// 16-deep slabs (66 KB of LDS, 2 x 2 slabs in flight per CU with two
-// workgroups) give each barrier twice the matrix work of a 64 x 64 tile.
-// Lane layout (measured on gfx950): A[i][k] at lane 16k + i, B[k][j] at lane
-// 16k + j, D[i][j] in accumulator i / 4 of lane 16(i % 4) + j.
+// ---------------------------------------------------------------------------
+// Slabs straight to LDS, v_mfma_f64_16x16x4: the kernel of nearly all products.
+// ---------------------------------------------------------------------------
 typedef double d4v __attribute__((ext_vector_type(4)));
-constexpr int BK16 = 16;
 
-// One tile; EDGE: the tile crosses an edge of C or K is not a multiple of
-// the slab depth (bounds-checked loads and stores).
-template <bool EDGE, bool TA, bool TB, bool BETA0, int MODE>
-__device__ __forceinline__ void m16_tile(double (*As)[BK16 * 129], double (*Bs)[BK16 * 129], double* E, i64 M, i64 N, i64 K,
-                                         double alpha, const double* __restrict__ A, i64 lda,
-                                         const double* __restrict__ B, i64 ldb, double beta, double* __restrict__ C,
-                                         i64 ldc, i64 m0, i64 n0) {
-    constexpr int BM = 128, BN = 128, LDS_A = BM + PAD, LDS_B = BN + PAD;
-    static_assert(LDS_A == 129 && LDS_B == 129, "LDS row length");
-    constexpr bool A_OC = !TA, B_OC = TB;
-    const int t = threadIdx.x;
-    const int lane = t & 63, wave = t >> 6;
-    const int wm = wave & 1, wn = wave >> 1;
+// 64 lanes x 16 bytes from base + off (per lane) to LDS at lds .. lds + 1023,
+// without registers; counted in vmcnt until the bytes are in LDS.
+__device__ __forceinline__ void load_to_lds(const char* base, unsigned off, unsigned lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds)
+                 : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
 
-    d4v acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = d4v{0.0, 0.0, 0.0, 0.0};
+// a workgroup's operand, the same in every lane, as an address in scalar registers
+__device__ __forceinline__ const char* in_sgprs(const double* p) {
+    const unsigned long long a = (unsigned long long)p;
+    const unsigned lo = __builtin_amdgcn_readfirstlane(unsigned(a)), hi = __builtin_amdgcn_readfirstlane(unsigned(a >> 32));
+    return (const char*)((unsigned long long)hi << 32 | lo);
+}
 
-    double ra[BM * BK16 / NT], rb[BN * BK16 / NT];
-    auto load = [&](i64 k0) __attribute__((always_inline)) {
-        if (EDGE) {
-            load_slab<A_OC, BM, BK16>(ra, A, lda, m0, k0, M, K, t);
-            load_slab<B_OC, BN, BK16>(rb, B, ldb, n0, k0, N, K, t);
-        } else {
-            load_slab_inner<A_OC, BM, BK16>(ra, A, lda, m0, k0, t);
-            load_slab_inner<B_OC, BN, BK16>(rb, B, ldb, n0, k0, t);
+// One operand's slab of O outer elements x BK of k in LDS.
+//   OUTER_CONTIG: rows of k, element (o, k) at k * O + (o ^ (16 * (k & 1)));
+//   else rows of o, the pair k, k + 1 in slot (k / 2) ^ f(o) of the row.
+// Either way the 32 lanes that an LDS read serves together (16 o, two k)
+// touch every bank once.  A lane fetches the pairs of its places; where the
+// contiguous direction ends inside a pair, the pair one element earlier takes
+// its place, so the last element sits one place later than its own (paired()).
+template <bool OUTER_CONTIG, int O, int BK>
+struct Slab {
+    static constexpr int LOADS = O * BK / 128;             // wave loads of a slab
+    __device__ static __forceinline__ int f(int o) {
+        return BK == 8 ? (o >> 2) & 3 : BK == 16 ? (o >> 1) & 7 : o & 15;
+    }
+    // byte offset, from the slab's first element, of what the lane fetches in
+    // load q; o_last, k_last: the last elements there are, the contiguous
+    // one's at least 1
+    __device__ static __forceinline__ unsigned source(int q, int lane, i64 ldx, i64 o_last, int k_last) {
+        const int e = q * 128 + lane * 2;                  // first of the lane's two places
+        if (OUTER_CONTIG) {
+            const int k = e / O, o = (e % O) ^ (16 * (k & 1));
+            return unsigned((min(i64(o), o_last - 1) + i64(min(k, k_last)) * ldx) * 8);
         }
+        const int o = e / BK, k = 2 * (((e % BK) / 2) ^ f(o));
+        return unsigned((i64(min(k, k_last - 1)) + min(i64(o), o_last) * ldx) * 8);
+    }
+    // place of element (o, k)
+    __device__ static __forceinline__ int at(int o, int k) {
+        if (OUTER_CONTIG) return k * O + (o ^ (16 * (k & 1)));
+        return o * BK + 2 * ((k / 2) ^ f(o)) + (k & 1);
+    }
+};
+// where element x of the contiguous direction is found when `last` is the last one there is
+__device__ __forceinline__ int paired(int x, i64 last) { return x == last && !(last & 1) ? x + 1 : x; }
+
+// A workgroup's four waves split a BM x BN tile of C 2 x 2, a wave's share as
+// 16 x 16 blocks (lane layout, measured on gfx950: A[i][k] at lane 16k + i,
+// B[k][j] at lane 16k + j, D[i][j] in accumulator i / 4 of lane 16(i % 4) + j).
+// Bound by the matrix cores once a few workgroups share a CU: a wave's 16
+// blocks of the 128 x 128 tile take 1024 cycles for each 4 of k, its LDS reads
+// about 130.  The slabs go straight to LDS (global_load_lds_dwordx4): no
+// registers hold loads in flight, so slab s + 1 is under way during the whole
+// of slab s, with no copy to LDS behind it, one barrier a slab and no rows
+// padded for the banks; what a lane fetches is permuted instead.  Rows and
+// columns of any length and 8-byte alignment take this path (pairs that start
+// at odd elements are 16-byte loads at 8-byte alignment).  8192^3: 74 TF/s,
+// against 64 with slabs staged through registers; 1500 x 1111 x 777 TN: 79 ->
+// 60 us; 1000 products of 64^3: 55 -> 17 us (5.6 TB/s).  Three and four slabs
+// deep: slower (68 TF/s for the 128 x 128 tile, 8 deep each).
+template <int BM, int BN, int BK, int OCC, bool TA, bool TB, bool BETA0, int MODE = PLAIN>
+__global__ __launch_bounds__(NT, OCC) void dgemm_direct_kernel(i64 M, i64 N, i64 K, double alpha,
+                                                               const double* __restrict__ A, i64 lda,
+                                                               const double* __restrict__ B, i64 ldb, double beta,
+                                                               double* __restrict__ C, i64 ldc, int tiles_m, int tiles_n,
+                                                               BatchArg ba = BatchArg{}) {
+    constexpr int WM = 2, WN = 2, NW = WM * WN, MI = BM / WM / 16, NJ = BN / WN / 16;
+    using SA = Slab<!TA, BM, BK>;
+    using SB = Slab<TB, BN, BK>;
+    constexpr int STAGE = (BM + BN) * BK, LA = SA::LOADS / NW, LB = SB::LOADS / NW;
+    static_assert(SA::LOADS % NW == 0 && SB::LOADS % NW == 0, "loads");
+    constexpr int EC = BN / WN > 32 ? 32 : BN / WN, LDE = BM + 1;   // epilogue: EC columns at a time
+    constexpr int SPACE = 2 * STAGE > LDE * EC ? 2 * STAGE : LDE * EC;
+    __shared__ __align__(1024) double lds[SPACE];
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wm = wave % WM, wn = wave / WM;
+    int tm, tn;
+    if ((MODE == LOWER || MODE == UPPER) && BM == BN) tri_tile_of(blockIdx.x, tiles_m, MODE == UPPER, tm, tn);
+    else tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
+    const i64 m0 = i64(tm) * BM, n0 = i64(tn) * BN;
+    if (!tile_in_triangle<MODE>(m0, n0, BM, BN)) return;
+    batch_operands<MODE>(ba, A, B, C);
+
+    // this wave's loads of a slab: LA of A's, LB of B's
+    const int nst = int((K + BK - 1) / BK), ktail = int(K - i64(nst - 1) * BK);
+    const i64 mlast = M - 1 - m0, nlast = N - 1 - n0;
+    // a single row (column) is fetched as the second of a pair
+    const char* abase = in_sgprs(TA ? A + m0 * lda : A + m0 - (mlast == 0));
+    const char* bbase = in_sgprs(TB ? B + n0 - (nlast == 0) : B + n0 * ldb);
+    const i64 astep = (TA ? i64(BK) : BK * lda) * 8, bstep = (TB ? BK * ldb : i64(BK)) * 8;
+    const unsigned lds0 = unsigned((unsigned long long)(__attribute__((address_space(3))) double*)lds);
+    const int nfull = ktail < BK ? nst - 1 : nst;          // slabs of BK
+    unsigned offa[LA], offb[LB];
+    auto offsets = [&](int klast) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < LA; ++q)
+            offa[q] = SA::source(wave * LA + q, lane, lda, TA ? mlast : max(mlast, i64(1)), TA ? max(klast, 1) : klast);
+#pragma unroll
+        for (int q = 0; q < LB; ++q)
+            offb[q] = SB::source(wave * LB + q, lane, ldb, TB ? max(nlast, i64(1)) : nlast, TB ? klast : max(klast, 1));
     };
-    const int nslab = int((K + BK16 - 1) / BK16);
-    load(0);
-    store_slab<A_OC, BM, BK16>(As[0], ra, t);
-    store_slab<B_OC, BN, BK16>(Bs[0], rb, t);
-    __syncthreads();
+    offsets(nst > 1 ? BK - 1 : ktail - 1);
+    auto issue = [&](int s) __attribute__((always_inline)) {
+        i64 back = 0;
+        if (s == nfull && nst > 1) {                       // the last ktail of k; a single one as the second of a pair
+            offsets(ktail - 1);
+            back = ktail == 1 ? 8 : 0;
+        }
+        const unsigned to = lds0 + unsigned(s & 1) * (STAGE * 8);
+        const char* a = abase + s * astep - (TA ? back : 0);
+        const char* b = bbase + s * bstep - (TB ? 0 : back);
+#pragma unroll
+        for (int q = 0; q < LA; ++q) load_to_lds(a, offa[q], to + (wave * LA + q) * 1024);
+#pragma unroll
+        for (int q = 0; q < LB; ++q) load_to_lds(b, offb[q], to + (SA::LOADS + wave * LB + q) * 1024);
+    };
 
-    const int lk = lane >> 4, li = lane & 15;
-    for (int s = 0; s < nslab; ++s) {
-        const int cur = s & 1;
-        if (s + 1 < nslab) load(i64(s + 1) * BK16);
-        const double* as = As[cur];
-        const double* bs = Bs[cur];
+    // epilogue of tiles inside C: row er of columns ec0, ec0 + CPP, .. of a
+    // piece.  The 32 x 32 tile, which runs where there are too few workgroups
+    // to cover each other's waits, loads C before the K loop (4096 x 64 x 64:
+    // 8.3 -> 7.8 us; 64 x 64 tiles: 5000 x 4936 x 64 75 -> 82 us, so not
+    // there), without branches: an element outside C reads the nearest one
+    // inside, and is not used.
+    constexpr int CPT = BM * EC / NT, CPP = NT / BM;       // columns a thread, columns a pass
+    static_assert(NT % BM == 0 && EC % 16 == 0, "epilogue");
+    constexpr bool AHEAD = !BETA0 && BM * BN < 64 * 64;
+    const int er = t % BM, ec0 = t / BM;
+    double cs[AHEAD ? BN / CPP : 1];
+    if (AHEAD) {
 #pragma unroll
-        for (int ks = 0; ks < BK16 / 4; ++ks) {
-            const int kr = ks * 4 + lk;
-            double a[4], b[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = as[kr * LDS_A + wm * 64 + i * 16 + li];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = bs[kr * LDS_B + wn * 64 + j * 16 + li];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
-        if (s + 1 < nslab) {
-            store_slab<A_OC, BM, BK16>(As[cur ^ 1], ra, t);
-            store_slab<B_OC, BN, BK16>(Bs[cur ^ 1], rb, t);
-        }
-        __syncthreads();
+        for (int k = 0; k < BN / CPP; ++k) cs[k] = C[min(n0 + ec0 + CPP * k, N - 1) * ldc + min(m0 + er, M - 1)];
     }
 
-    if (!EDGE) {
-        // Interior tile: C in two halves of 64 columns, each staged through
-        // LDS (128 x 64 doubles, row stride 129) by the two waves that hold
-        // it, then combined with C by all threads, a wave covering 64
-        // consecutive rows of one column (512 contiguous bytes) and every
-        // thread issuing its 32 loads before its first store: one memory
-        // round trip per half.
-        constexpr int LDE = 129;
-        const int er = t & 127, ec0 = t >> 7;     // row in the tile, first column (then every 2nd)
-        const int dn = diag_offset(m0, n0);
+    d4v acc[MI][NJ];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            if (wn == h) {
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < NJ; ++j) acc[i][j] = d4v{0.0, 0.0, 0.0, 0.0};
+    const int lk = lane >> 4, li = lane & 15;
+    // this lane's rows and columns in the slabs: places at k = lk where they
+    // are contiguous, else the first row or column (the others 16, 32, .. on)
+    const int ar = wm * (BM / WM) + li, bc = wn * (BN / WN) + li;
+    int pa[MI], pb[NJ];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < MI; ++i) pa[i] = SA::at(TA ? ar + i * 16 : paired(ar + i * 16, mlast), lk);
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) E[(j * 16 + li) * LDE + wm * 64 + i * 16 + lk + 4 * r] = acc[i][j][r];
+    for (int j = 0; j < NJ; ++j) pb[j] = SB::at(TB ? paired(bc + j * 16, nlast) : bc + j * 16, lk);
+    issue(0);
+    auto arrive = [&]() __attribute__((always_inline)) {
+        // slab s has arrived (this wave's loads, then everyone's)
+        wait_loads<0>();
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    };
+    auto products = [&](int s, auto tail) __attribute__((always_inline)) {
+        constexpr bool TAIL = decltype(tail)::value;
+        const double* as = lds + (s & 1) * STAGE;
+        const double* bs = as + BM * BK;
+#pragma unroll
+        for (int ks = 0; ks < BK / 4; ++ks) {
+            const int k = ks * 4 + lk;
+            const int ka = TAIL && TA ? min(paired(k, ktail - 1), BK - 1) : k;
+            const int kb = TAIL && !TB ? min(paired(k, ktail - 1), BK - 1) : k;
+            double a[MI], b[NJ];
+#pragma unroll
+            for (int i = 0; i < MI; ++i) a[i] = as[TA ? SA::at(ar, ka) + i * 16 * BK : pa[i] + ks * 4 * BM];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) b[j] = bs[TB ? pb[j] + ks * 4 * BN : SB::at(bc, kb) + j * 16 * BK];
+            if (TAIL) {   // past K: zeros
+#pragma unroll
+                for (int i = 0; i < MI; ++i) a[i] = k < ktail ? a[i] : 0.0;
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) b[j] = k < ktail ? b[j] : 0.0;
+            }
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+    };
+    for (int s = 0; s < nfull; ++s) {
+        arrive();
+        // everyone is past slab s - 1: its space takes slab s + 1
+        if (s + 1 < nst) issue(s + 1);
+        products(s, std::false_type{});
+    }
+    if (nfull < nst) {
+        arrive();
+        products(nfull, std::true_type{});
+    }
+
+    const int dn = diag_offset(m0, n0);
+    if (m0 + BM <= M && n0 + BN <= N) {
+        // C, EC columns at a time, through LDS: every wave then covers
+        // consecutive rows of a column, and every thread issues its loads of
+        // a piece before its first store
+#pragma unroll
+        for (int h = 0; h < BN / EC; ++h) {
+            constexpr int WC = BN / WN;
+            double* cc = C + (n0 + h * EC + ec0) * ldc + m0 + er;
+            double cv[CPT];
+            if (!BETA0) {
+#pragma unroll
+                for (int k = 0; k < CPT; ++k) cv[k] = AHEAD ? cs[AHEAD ? h * CPT + k : 0] : cc[i64(CPP * k) * ldc];
             }
             __syncthreads();
-            double* cc = C + (n0 + h * 64 + ec0) * ldc + m0 + er;
-            // two batches of 16 columns, the second's loads in flight while
-            // the first is stored
-            double cv[2][16];
-            auto load16 = [&](int b) __attribute__((always_inline)) {
+            if (wn == h * EC / WC) {
 #pragma unroll
-                for (int k = 0; k < 16; ++k) cv[b][k] = cc[i64(2 * (16 * b + k)) * ldc];
-            };
-            if (!BETA0) { load16(0); load16(1); }
+                for (int j = 0; j < EC / 16; ++j)
 #pragma unroll
-            for (int b = 0; b < 2; ++b)
+                    for (int i = 0; i < MI; ++i)
 #pragma unroll
-                for (int k = 0; k < 16; ++k) {
-                    const int c = 16 * b + k;
-                    const double v = alpha * E[(ec0 + 2 * c) * LDE + er];
-                    const bool in = keep_local<MODE>(er, h * 64 + ec0 + 2 * c, dn);
-                    if (BETA0) {
-                        if (in) cc[i64(2 * c) * ldc] = v;
-                    } else {
-                        // outside the triangle the element gets back the value just read
-                        cc[i64(2 * c) * ldc] = in ? __builtin_fma(beta, cv[b][k], v) : cv[b][k];
-                    }
-                }
-            if (h == 0) __syncthreads();
+                        for (int r = 0; r < 4; ++r)
+                            lds[(j * 16 + li) * LDE + wm * (BM / WM) + i * 16 + lk + 4 * r] = acc[i][h * EC % WC / 16 + j][r];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < CPT; ++k) {
+                const double v = alpha * lds[(ec0 + CPP * k) * LDE + er];
+                if (keep_local<MODE>(er, h * EC + ec0 + CPP * k, dn))
+                    cc[i64(CPP * k) * ldc] = BETA0 ? v : __builtin_fma(beta, cv[k], v);
+            }
         }
         return;
     }
-    // Edge tile: one block column at a time, its C loads (issued without
-    // branches; an element outside C reads the nearest one inside and is
-    // not stored) before its stores.
-    const int dn = diag_offset(m0, n0);
+    // edge tile: one block column at a time, its C loads (an element outside C
+    // reads the nearest one inside and is not stored) before its stores
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const i64 col = n0 + wn * 64 + j * 16 + li;
-        const i64 colc = EDGE ? min(col, N - 1) : col;
-        double cv[4][4];
+    for (int j = 0; j < NJ; ++j) {
+        const i64 col = n0 + wn * (BN / WN) + j * 16 + li, colc = min(col, N - 1);
+        double cv[MI][4];
         if (!BETA0) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < MI; ++i)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const i64 row = m0 + wm * 64 + i * 16 + lk + 4 * r;
-                    cv[i][r] = C[colc * ldc + (EDGE ? min(row, M - 1) : row)];
-                }
+                for (int r = 0; r < 4; ++r) cv[i][r] = C[colc * ldc + min(m0 + wm * (BM / WM) + i * 16 + lk + 4 * r, M - 1)];
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const i64 row = m0 + wm * 64 + i * 16 + lk + 4 * r;
+                const int rr = wm * (BM / WM) + i * 16 + lk + 4 * r;
                 const double v = alpha * acc[i][j][r];
-                if ((!EDGE || (row < M && col < N)) &&
-                    keep_local<MODE>(wm * 64 + i * 16 + lk + 4 * r, wn * 64 + j * 16 + li, dn))
-                    C[col * ldc + row] = BETA0 ? v : __builtin_fma(beta, cv[i][r], v);
+                if (m0 + rr < M && col < N && keep_local<MODE>(rr, wn * (BN / WN) + j * 16 + li, dn))
+                    C[col * ldc + m0 + rr] = BETA0 ? v : __builtin_fma(beta, cv[i][r], v);
             }
     }
-}
-
-template <bool TA, bool TB, bool BETA0, int MODE = PLAIN>
-__global__ __launch_bounds__(NT, 2) void dgemm_m16_kernel(i64 M, i64 N, i64 K, double alpha,
-                                                          const double* __restrict__ A, i64 lda,
-                                                          const double* __restrict__ B, i64 ldb, double beta,
-                                                          double* __restrict__ C, i64 ldc, int tiles_m, int tiles_n,
-                                                          BatchArg ba = BatchArg{}) {
-    // the slabs of A and B, and after the K loop the staging of C
-    __shared__ __align__(16) double lds[4 * BK16 * 129];
-    double (*As)[BK16 * 129] = (double (*)[BK16 * 129])lds;
-    double (*Bs)[BK16 * 129] = (double (*)[BK16 * 129])(lds + 2 * BK16 * 129);
-    int tm, tn;
-    if (MODE == LOWER || MODE == UPPER) tri_tile_of(blockIdx.x, tiles_m, MODE == UPPER, tm, tn);
-    else tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
-    const i64 m0 = i64(tm) * 128, n0 = i64(tn) * 128;
-    if (!tile_in_triangle<MODE>(m0, n0, 128, 128)) return;
-    batch_operands<MODE>(ba, A, B, C);
-    if (m0 + 128 <= M && n0 + 128 <= N && K % BK16 == 0)
-        m16_tile<false, TA, TB, BETA0, MODE>(As, Bs, lds, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, m0, n0);
-    else
-        m16_tile<true, TA, TB, BETA0, MODE>(As, Bs, lds, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, m0, n0);
 }
 
 __global__ void dscale_kernel(i64 m, i64 n, double beta, double* __restrict__ C, i64 ldc) {
@@ -533,108 +605,108 @@ void launch_tiles(hipStream_t s, i64 m, i64 n, i64 k, double alpha, const double
                            lda, B, ldb, beta, C, ldc, tiles_m, tiles_n, ba);
 }
 
-template <bool TA, bool TB, int MODE = PLAIN>
-void launch_m16(hipStream_t s, i64 m, i64 n, i64 k, double alpha, const double* A, i64 lda, const double* B, i64 ldb,
-                double beta, double* C, i64 ldc, unsigned batch = 1, BatchArg ba = BatchArg{}) {
-    const int tiles_m = int(cdiv(m, 128)), tiles_n = int(cdiv(n, 128));
-    const bool tri = MODE == LOWER || MODE == UPPER;   // one triangle of a square grid: only its tiles launch
+// false (nothing launched) where dgemm_direct_kernel cannot read the operands:
+// it loads pairs along their columns, at 32-bit offsets inside a tile
+template <int BM, int BN, int BK, int OCC, bool TA, bool TB, int MODE = PLAIN>
+bool launch_direct(hipStream_t s, i64 m, i64 n, i64 k, double alpha, const double* A, i64 lda, const double* B,
+                   i64 ldb, double beta, double* C, i64 ldc, unsigned batch = 1, BatchArg ba = BatchArg{}) {
+    const i64 far = std::max((TA ? BM : BK) * lda, (TB ? BK : BN) * ldb);
+    if ((TA ? k : m) < 2 || (TB ? n : k) < 2 || far > (i64(1) << 28)) return false;
+    const int tiles_m = int(cdiv(m, BM)), tiles_n = int(cdiv(n, BN));
+    // one triangle of a square grid of square tiles: only its tiles launch
+    const bool tri = (MODE == LOWER || MODE == UPPER) && BM == BN;
     dim3 grid(tri ? tiles_m * (tiles_m + 1) / 2 : tiles_m * tiles_n, batch), block(NT);
     if (beta == 0.0)
-        hipLaunchKernelGGL((dgemm_m16_kernel<TA, TB, true, MODE>), grid, block, 0, s, m, n, k, alpha, A, lda, B, ldb,
-                           beta, C, ldc, tiles_m, tiles_n, ba);
+        hipLaunchKernelGGL((dgemm_direct_kernel<BM, BN, BK, OCC, TA, TB, true, MODE>), grid, block, 0, s, m, n, k, alpha, A,
+                           lda, B, ldb, beta, C, ldc, tiles_m, tiles_n, ba);
     else
-        hipLaunchKernelGGL((dgemm_m16_kernel<TA, TB, false, MODE>), grid, block, 0, s, m, n, k, alpha, A, lda, B, ldb,
-                           beta, C, ldc, tiles_m, tiles_n, ba);
+        hipLaunchKernelGGL((dgemm_direct_kernel<BM, BN, BK, OCC, TA, TB, false, MODE>), grid, block, 0, s, m, n, k, alpha,
+                           A, lda, B, ldb, beta, C, ldc, tiles_m, tiles_n, ba);
+    return true;
 }
 
-// Tile shape of C per workgroup (measured on MI355X over the LU's products
-// and square ones, K = 32 .. 8192): 128 x 128 on the 16x16x4 instruction
-// where its grid has at least 1.75 workgroups per CU (8192^3: 64 TF/s against
-// 54 for 64 x 64; 512 x 15872 x 512, 496 tiles: 170 us against 206, but
-// 512 x 12000 x 512, 376 tiles: 191 us against 166); else 64 x 64 tiles on the 4x4x4_4b instruction (66 KB of
-// LDS, two workgroups per CU); 32 x 32 where the 64 x 64 grid has fewer than
-// about 1.5 workgroups per CU (the LU's look-ahead block, its panel updates
-// and the TRSM updates: products of 32..256 rows).  A side no longer than 32
-// takes a 32-wide tile.  OXIBLAS_DGEMM_TILE (m16, 64x64, 32x32) fixes the
-// choice (tuning); bm = bn = 16 stands for the 16x16x4 kernel.
+// Tile of C per workgroup, by what was measured over the LU's products and
+// square and long ones (us for 128 / 64 / 32):
+//  - 128 x 128, two workgroups a CU, has the fewest loads a product but waits
+//    longest for C and leaves the most CUs idle in the last pass over the
+//    grid: where K >= 192 and the grid is at least 4 workgroups a CU (4096^3:
+//    1865 / 1980 / 2326; 15872^2 x 256: 2181 / 2232 / 2697; but 7936^2 x 128:
+//    384 / 361 / 476) whose last pass of 256 is nearly full or one of many
+//    (3000^3, 576 tiles: 1134 / 931 / 1033);
+//  - 64 x 64, four a CU, where its grid has at least 1.5 workgroups a CU
+//    (1500 x 1111 x 777, 432 tiles: 115 / 60 / 61; 1000^3, 256 tiles:
+//    139 / 48 / 45);
+//  - 32 x 32 below (the LU's look-ahead block, its panel updates, the TRSM
+//    updates; 512^3: 69 / 23 / 9), and where a side is no longer than 32.
+// OXIBLAS_DGEMM_TILE (128x128 or m16, 64x64, 32x32) fixes the choice (tuning).
 constexpr int NCU = 256;
-void choose_tile(i64 m, i64 n, int& bm, int& bn, i64 batch = 1) {
+int choose_tile(i64 m, i64 n, i64 k, i64 batch = 1) {
     static int forced = -1;
     if (forced < 0) {
         forced = 0;
         if (const char* e = getenv("OXIBLAS_DGEMM_TILE")) {
             int a = 0, b = 0;
-            if (sscanf(e, "%dx%d", &a, &b) == 2 && a == b && (a == 32 || a == 64)) forced = a;
-            if (!strcmp(e, "m16")) forced = 16;
+            if (sscanf(e, "%dx%d", &a, &b) == 2 && a == b && (a == 32 || a == 64 || a == 128)) forced = a;
+            if (!strcmp(e, "m16")) forced = 128;
         }
     }
-    if (forced) { bm = bn = forced; return; }
+    if (forced) return forced;
     // a batch fills the chip with its products together
-    if (cdiv(m, 128) * cdiv(n, 128) * batch >= NCU * 7 / 4) { bm = bn = 16; return; }
-    bm = m <= 32 ? 32 : 64;
-    bn = n <= 32 ? 32 : 64;
-    if (cdiv(m, bm) * cdiv(n, bn) * batch < i64(NCU) * 3 / 2) bm = bn = 32;
+    const i64 t128 = cdiv(m, 128) * cdiv(n, 128) * batch;
+    if (k >= 192 && t128 >= 4 * NCU && (t128 >= 16 * NCU || t128 % NCU == 0 || t128 % NCU >= NCU * 3 / 4)) return 128;
+    if (m <= 32 || n <= 32 || cdiv(m, 64) * cdiv(n, 64) * batch < i64(NCU) * 3 / 2) return 32;
+    return 64;
 }
 
-// false when no kernel takes the chosen tile shape (nothing launched)
 template <bool TA, bool TB, int MODE = PLAIN>
-bool launch_variant(hipStream_t s, i64 m, i64 n, i64 k, double alpha, const double* A, i64 lda, const double* B,
+void launch_variant(hipStream_t s, i64 m, i64 n, i64 k, double alpha, const double* A, i64 lda, const double* B,
                     i64 ldb, double beta, double* C, i64 ldc, unsigned batch = 1, BatchArg ba = BatchArg{}) {
-    int bm, bn;
-    choose_tile(m, n, bm, bn, batch);
-    if (bm == 16) { launch_m16<TA, TB, MODE>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, batch, ba); return true; }
-#define OXI_TILE(X, Y)                                                                                              \
-    if (bm == X && bn == Y) {                                                                                       \
-        launch_tiles<X, Y, TA, TB, MODE>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, batch, ba);              \
-        return true;                                                                                                \
-    }
-    OXI_TILE(64, 64) OXI_TILE(32, 32) OXI_TILE(64, 32) OXI_TILE(32, 64)
-#undef OXI_TILE
-    return false;
+    const int tile = choose_tile(m, n, k, batch);
+    if (tile == 128 && launch_direct<128, 128, 16, 2, TA, TB, MODE>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, batch, ba))
+        return;
+    if (tile >= 64 && launch_direct<64, 64, 16, 4, TA, TB, MODE>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, batch, ba))
+        return;
+    if (launch_direct<32, 32, 32, 4, TA, TB, MODE>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, batch, ba)) return;
+    // a single row (column, depth) along an operand's columns, or columns a gigabyte apart
+    if (tile >= 64) launch_tiles<64, 64, TA, TB, MODE>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, batch, ba);
+    else launch_tiles<32, 32, TA, TB, MODE>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, batch, ba);
 }
 
 template <int MODE>
-bool launch_any(hipStream_t s, int ta, int tb, i64 m, i64 n, i64 k, double alpha, const double* A, i64 lda,
-                const double* B, i64 ldb, double beta, double* C, i64 ldc, unsigned batch, BatchArg ba) {
-    if (!ta && !tb) return launch_variant<false, false, MODE>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, batch, ba);
-    if (!ta && tb) return launch_variant<false, true, MODE>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, batch, ba);
-    if (ta && !tb) return launch_variant<true, false, MODE>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, batch, ba);
-    return launch_variant<true, true, MODE>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, batch, ba);
+void launch_any(hipStream_t s, int ta, int tb, i64 m, i64 n, i64 k, double alpha, const double* A, i64 lda,
+                const double* B, i64 ldb, double beta, double* C, i64 ldc, unsigned batch = 1, BatchArg ba = BatchArg{}) {
+    if (!ta && !tb) launch_variant<false, false, MODE>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, batch, ba);
+    else if (!ta) launch_variant<false, true, MODE>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, batch, ba);
+    else if (!tb) launch_variant<true, false, MODE>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, batch, ba);
+    else launch_variant<true, true, MODE>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, batch, ba);
 }
 
 }  // namespace
 
+// The in-place block products of the triangular solves: a workgroup's tile
+// has all 64 columns (rows) of its rows (columns), and it writes them only
+// after its last read of them (the epilogue follows the K loop, whose last
+// barrier all its loads have passed).  A row or column that it reads of
+// another workgroup's tile (the first of a pair at an edge) is not used.
 int oxi_dgemm_right64_inplace(hipStream_t s, i64 rows, const double* V, double* X, i64 ldx) {
-    // X[:, 0:64] <- X[:, 0:64] * V (V 64 x 64, ld 64) in place: 32 x 64 tiles,
-    // so each workgroup owns all 64 columns of its rows, and it writes them
-    // only after its last read of them (the epilogue follows the K loop)
+    // X[:, 0:64] <- X[:, 0:64] * V (V 64 x 64, ld 64)
     if (rows <= 0) return OXI_OK;
-    const int tiles_m = int(cdiv(rows, 32));
-    hipLaunchKernelGGL((dgemm_mfma_kernel<32, 64, false, false, true>), dim3(tiles_m), dim3(NT), 0, s, rows, i64(64),
-                       i64(64), 1.0, X, ldx, V, i64(64), 0.0, X, ldx, tiles_m, 1);
+    if (!launch_direct<32, 64, 32, 2, false, false>(s, rows, 64, 64, 1.0, X, ldx, V, 64, 0.0, X, ldx))
+        launch_tiles<32, 64, false, false>(s, rows, 64, 64, 1.0, X, ldx, V, 64, 0.0, X, ldx);
     return hipGetLastError() == hipSuccess ? OXI_OK : OXI_ERR_HIP;
 }
 
 int oxi_dgemm_left64_inplace(hipStream_t s, int ta, i64 ncols, const double* V, double* X, i64 ldx) {
-    // X[0:64, :] <- op(V) * X[0:64, :] (V 64 x 64, ld 64) in place: 64 x 32
-    // tiles, so each workgroup owns all 64 rows of its columns and writes
-    // them only after its last read of them (the epilogue follows the K loop)
+    // X[0:64, :] <- op(V) * X[0:64, :] (V 64 x 64, ld 64)
     if (ncols <= 0) return OXI_OK;
-    const int tiles_n = int(cdiv(ncols, 32));
-    if (ta)
-        hipLaunchKernelGGL((dgemm_mfma_kernel<64, 32, true, false, true>), dim3(tiles_n), dim3(NT), 0, s, i64(64),
-                           ncols, i64(64), 1.0, V, i64(64), X, ldx, 0.0, X, ldx, 1, tiles_n);
-    else
-        hipLaunchKernelGGL((dgemm_mfma_kernel<64, 32, false, false, true>), dim3(tiles_n), dim3(NT), 0, s, i64(64),
-                           ncols, i64(64), 1.0, V, i64(64), X, ldx, 0.0, X, ldx, 1, tiles_n);
+    const bool done = ta ? launch_direct<64, 32, 32, 2, true, false>(s, 64, ncols, 64, 1.0, V, 64, X, ldx, 0.0, X, ldx)
+                         : launch_direct<64, 32, 32, 2, false, false>(s, 64, ncols, 64, 1.0, V, 64, X, ldx, 0.0, X, ldx);
+    if (!done && ta) launch_tiles<64, 32, true, false>(s, 64, ncols, 64, 1.0, V, 64, X, ldx, 0.0, X, ldx);
+    if (!done && !ta) launch_tiles<64, 32, false, false>(s, 64, ncols, 64, 1.0, V, 64, X, ldx, 0.0, X, ldx);
     return hipGetLastError() == hipSuccess ? OXI_OK : OXI_ERR_HIP;
 }
 
-bool oxi_dgemm_large_tiles(i64 m, i64 n) {
-    int bm, bn;
-    choose_tile(m, n, bm, bn);
-    return bm == 16;
-}
+bool oxi_dgemm_large(i64 m, i64 n) { return cdiv(m, 128) * cdiv(n, 128) >= NCU * 7 / 4; }
 
 int oxi_launch_dscale(hipStream_t s, i64 m, i64 n, double beta, double* C, i64 ldc) {
     if (m <= 0 || n <= 0 || beta == 1.0) return OXI_OK;
@@ -651,12 +723,7 @@ int oxi_launch_dgemm(oxi_handle_t h, hipStream_t s, int ta, int tb, i64 m, i64 n
     if (cdiv(m, 128) * cdiv(n, 128) > (i64(1) << 31) - 1)
         return oxi_set_error(h, OXI_ERR_UNSUPPORTED, "dgemm: %lld x %lld has too many tiles", (long long)m,
                              (long long)n);
-    bool launched;
-    if (!ta && !tb) launched = launch_variant<false, false>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
-    else if (!ta && tb) launched = launch_variant<false, true>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
-    else if (ta && !tb) launched = launch_variant<true, false>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
-    else launched = launch_variant<true, true>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
-    if (!launched) return oxi_set_error(h, OXI_ERR_UNSUPPORTED, "dgemm: no kernel for the chosen tile shape");
+    launch_any<PLAIN>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return oxi_set_error(h, OXI_ERR_HIP, "dgemm launch: %s", hipGetErrorString(e));
     return OXI_OK;
@@ -678,9 +745,7 @@ int oxi_launch_dgemm_strided(oxi_handle_t h, hipStream_t s, int ta, int tb, i64 
     for (i64 z0 = 0; z0 < batch; z0 += 65535) {
         const unsigned nb = unsigned(std::min<i64>(65535, batch - z0));
         BatchArg ba{sa, sb, sc, nullptr, nullptr, nullptr};
-        if (!launch_any<STRIDED>(s, ta, tb, m, n, k, alpha, A + z0 * sa, lda, B + z0 * sb, ldb, beta, C + z0 * sc,
-                                 ldc, nb, ba))
-            return oxi_set_error(h, OXI_ERR_UNSUPPORTED, "dgemm batch: no kernel for the chosen tile shape");
+        launch_any<STRIDED>(s, ta, tb, m, n, k, alpha, A + z0 * sa, lda, B + z0 * sb, ldb, beta, C + z0 * sc, ldc, nb, ba);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return oxi_set_error(h, OXI_ERR_HIP, "dgemm batch launch: %s", hipGetErrorString(e));
     }
@@ -699,8 +764,7 @@ int oxi_launch_dgemm_ptrs(oxi_handle_t h, hipStream_t s, int ta, int tb, i64 m, 
     for (i64 z0 = 0; z0 < batch; z0 += 65535) {
         const unsigned nb = unsigned(std::min<i64>(65535, batch - z0));
         BatchArg ba{0, 0, 0, A + z0, B + z0, C + z0};
-        if (!launch_any<PTRS>(s, ta, tb, m, n, k, alpha, nullptr, lda, nullptr, ldb, beta, nullptr, ldc, nb, ba))
-            return oxi_set_error(h, OXI_ERR_UNSUPPORTED, "dgemm batch: no kernel for the chosen tile shape");
+        launch_any<PTRS>(s, ta, tb, m, n, k, alpha, nullptr, lda, nullptr, ldb, beta, nullptr, ldc, nb, ba);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return oxi_set_error(h, OXI_ERR_HIP, "dgemm batch launch: %s", hipGetErrorString(e));
     }
@@ -722,9 +786,8 @@ int oxi_launch_dsyrk(oxi_handle_t h, hipStream_t s, int upper, int trans, i64 n,
     if (cdiv(n, 32) * cdiv(n, 32) > (i64(1) << 31) - 1)
         return oxi_set_error(h, OXI_ERR_UNSUPPORTED, "syrk: n = %lld has too many tiles", (long long)n);
     const int ta = trans ? 1 : 0, tb = trans ? 0 : 1;
-    const bool ok = upper ? launch_any<UPPER>(s, ta, tb, n, n, k, alpha, A, lda, A, lda, beta, C, ldc, 1, BatchArg{})
-                          : launch_any<LOWER>(s, ta, tb, n, n, k, alpha, A, lda, A, lda, beta, C, ldc, 1, BatchArg{});
-    if (!ok) return oxi_set_error(h, OXI_ERR_UNSUPPORTED, "syrk: no kernel for the chosen tile shape");
+    if (upper) launch_any<UPPER>(s, ta, tb, n, n, k, alpha, A, lda, A, lda, beta, C, ldc);
+    else launch_any<LOWER>(s, ta, tb, n, n, k, alpha, A, lda, A, lda, beta, C, ldc);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return oxi_set_error(h, OXI_ERR_HIP, "syrk launch: %s", hipGetErrorString(e));
     return OXI_OK;

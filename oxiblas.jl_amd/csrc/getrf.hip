@@ -493,11 +493,11 @@ int trailing_rows(GetrfCtx<float>& g, i64 j0, i64 j1, i64 r0, i64 r1) {
                            g.Wm + j0 + j1 * g.ldw, g.ldw, g.Wm + r0 + j1 * g.ldw, g.ldw, g.lowp_ws, g.lowp_bytes);
 }
 
-// The trailing updates that the optional profiling times: those that run on
-// the FP64 GEMM's 128 x 128 kernel (the factorization's dominant kernel).
+// The trailing updates that the optional profiling times: those that fill the
+// chip (the bulk of the factorization's products).
 template <typename T>
 bool timed_update(i64 rows, i64 cols) {
-    return sizeof(T) == 8 ? oxi_dgemm_large_tiles(rows, cols) : true;
+    return sizeof(T) == 8 ? oxi_dgemm_large(rows, cols) : true;
 }
 
 // Tuned block size: the panels bound the factorization, and up to about 5000

@@ -107,8 +107,8 @@ int oxi_launch_dsyrk(oxi_handle_t h, hipStream_t s, int upper, int trans, i64 n,
 int oxi_potrf_device(oxi_handle_t h, hipStream_t s, i64 n, double* A, i64 lda, i64* dinfo);
 // the same in FP32 (its trailing updates write both triangles)
 int oxi_potrf_device(oxi_handle_t h, hipStream_t s, i64 n, float* A, i64 lda, i64* dinfo);
-// whether oxi_launch_dgemm runs an m x n product on its 128 x 128 (16x16x4) kernel
-bool oxi_dgemm_large_tiles(i64 m, i64 n);
+// whether an m x n product has at least 1.75 tiles of 128 x 128 a CU
+bool oxi_dgemm_large(i64 m, i64 n);
 // X[:, 0:64] <- X[:, 0:64] * V in place (V 64 x 64, column-major, ld 64)
 int oxi_dgemm_right64_inplace(hipStream_t s, i64 rows, const double* V, double* X, i64 ldx);
 // X[0:64, 0:ncols] <- op(V) X[0:64, 0:ncols] in place (V 64 x 64, ld 64; ta: V^T)

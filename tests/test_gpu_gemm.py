@@ -380,3 +380,68 @@ def test_hgemm_vs_oracle(gpu, rng, ta, tb):
     got = gpu.hgemm_(np.full((7, 5), np.nan, np.float16), A[:7] if ta == "N" else A[:, :7],
                      B[:, :5] if tb == "N" else B[:5], 1.0, 0.0, ta, tb)
     assert np.all(np.isfinite(got))                       # beta == 0 never reads C
+
+
+def _guarded(torch, x, ld, shift):
+    """Column-major copy of x with leading dimension ld, `shift` elements into
+    its buffer, NaN everywhere else."""
+    r, c = x.shape
+    buf = torch.full((shift + ld * c + 3,), float("nan"), dtype=torch.float64, device="cuda")
+    view = buf[shift:shift + ld * c]
+    view.view(c, ld)[:, :r] = x.T
+    return buf, view
+
+
+# Products at the edges of each tile (32, 64 and 128 wide, slabs of 32 and 16
+# of k) and of the pairs in which operands are fetched: odd and even lengths,
+# odd leading dimensions and 8-byte alignment, one row or column past a tile,
+# and the degenerate lengths that take the general kernel.  Integers: exact.
+EDGES = [(2, 2, 2), (3, 2, 3), (1, 5, 4), (4, 1, 3), (5, 4, 1), (33, 31, 33), (32, 65, 31), (63, 33, 64), (65, 97, 49),
+         (1217, 1281, 15), (1281, 1215, 33), (1280, 1280, 16), (4065, 3969, 193), (3968, 4096, 208), (4033, 4034, 207)]
+
+
+@pytest.mark.parametrize("mnk", EDGES)
+@pytest.mark.parametrize("ta", "NT")
+@pytest.mark.parametrize("tb", "NT")
+def test_tile_edges_exact(gpu, mnk, ta, tb):
+    import torch
+    m, n, k = mnk
+    g = torch.Generator(device="cuda").manual_seed(m * 31 + n * 7 + k)
+
+    def ints(r, c):
+        return torch.randint(-8, 9, (r, c), device="cuda", generator=g).double()
+    A = ints(m, k) if ta == "N" else ints(k, m)
+    B = ints(k, n) if tb == "N" else ints(n, k)
+    C = ints(m, n)
+    for pad, shift in ((0, 0), (1, 1), (2, 0), (3, 1)):
+        _, a = _guarded(torch, A, A.shape[0] + pad, shift)
+        _, b = _guarded(torch, B, B.shape[0] + pad, 1 - shift)
+        for beta in (0.0, -3.0):
+            cb, c = _guarded(torch, C if beta else C * float("nan"), m + pad, shift)
+            gpu.gemm_(gpu.DMatrix(c, m, n, m + pad), gpu.DMatrix(a, A.shape[0], A.shape[1], A.shape[0] + pad),
+                      gpu.DMatrix(b, B.shape[0], B.shape[1], B.shape[0] + pad), 2.0, beta, ta, tb)
+            ref = 2.0 * (op(A, ta).cpu().numpy() @ op(B, tb).cpu().numpy()) if m * n * k < 10 ** 8 else \
+                2.0 * (op(A, ta).float().contiguous() @ op(B, tb).float().contiguous()).double().cpu().numpy()
+            if beta:
+                ref = ref + beta * C.cpu().numpy()
+            cols = c.view(n, m + pad)
+            assert np.array_equal(cols[:, :m].T.cpu().numpy(), ref), (pad, shift, beta)
+            assert torch.isnan(cols[:, m:]).all() and torch.isnan(cb[:shift]).all() and torch.isnan(cb[-3:]).all()
+
+
+@pytest.mark.parametrize("n,k", [(1249, 17), (1313, 32), (4545, 193)])
+@pytest.mark.parametrize("uplo", "LU")
+@pytest.mark.parametrize("trans", "NT")
+def test_syrk_tile_edges_exact(gpu, n, k, uplo, trans):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    A = torch.randint(-8, 9, (n, k) if trans == "N" else (k, n), device="cuda", generator=g).double()
+    C = torch.randint(-8, 9, (n, n), device="cuda", generator=g).double()
+    _, a = _guarded(torch, A, A.shape[0] + 1, 1)
+    _, c = _guarded(torch, C, n + 1, 1)
+    gpu.syrk_(gpu.DMatrix(c, n, n, n + 1), gpu.DMatrix(a, A.shape[0], A.shape[1], A.shape[0] + 1), 2.0, -3.0, uplo, trans)
+    X = (A if trans == "N" else A.T).float().contiguous()
+    full = 2.0 * (X @ X.T.contiguous()).double() - 3.0 * C
+    tri = torch.tril if uplo == "L" else torch.triu
+    want = tri(full) + C - tri(C)
+    assert torch.equal(c.view(n, n + 1)[:, :n].T, want)
