@@ -2,7 +2,7 @@
 // at most 64 rows/columns solved in registers or with one wave per right-hand
 // side, and the reference's recursive halving with FP64 MFMA GEMM updates in
 // between (_trsm_blocks_left! / _trsm_blocks_right!, level3.jl:338-376).
-#include "oxi_internal.hpp"
+#include "tri_inv.hpp"
 
 #include <algorithm>
 
@@ -130,52 +130,35 @@ void launch_right_leaf(hipStream_t s, int unit, int trans, i64 rows, int n, cons
 // V = U_bb^-1 goes to inv + 4096 b, column-major (ld 64, zeros below the
 // diagonal); with strip > 0, to its place in a column-major strip of ld
 // `ldv` whose rows z*strip .. (z+1)*strip - 1 hold the strip x strip block z
-// (inv + 64 b + ((64 b) % strip) * ldv).  Thread j computes column j right-looking, with the column's
-// 64 partial sums in registers: for k = j down to 0, V[k][j] = acc_k /
-// U[k][k], then acc_i -= U[i][k] V[k][j] for every i < k.  The k steps form
-// the only dependent chain (64 divisions); the i updates of a step are
-// independent.  Lanes with k > j take no update at step k (the terms the
-// substitution V[i][j] = (delta_ij - sum_{k=i+1..j} U[i][k] V[k][j]) /
-// U[i][i] does not have), so only the order of each sum differs from it.
+// (inv + 64 b + ((64 b) % strip) * ldv).  The block, both indices reversed
+// (lower triangular), in LDS, inverted on the matrix cores (tri::invert);
+// bound by the latency of its loads and barriers: 8 us, against 27 for a
+// column a lane swept over 64 steps.
 template <bool UNIT, bool TRANS>
-__global__ __launch_bounds__(64) void trsm_inv64_kernel(const double* __restrict__ T, i64 ldt,
-                                                        double* __restrict__ inv, i64 ldv = 64, int strip = 0) {
-    __shared__ double Ut[64][65];   // Ut[c][r] = op(T)[r][c]: columns contiguous
-    __shared__ double V[64][65];
-    const int tj = threadIdx.x;
+__global__ __launch_bounds__(256) void trsm_inv64_kernel(const double* __restrict__ T, i64 ldt,
+                                                         double* __restrict__ inv, i64 ldv = 64, int strip = 0) {
+    constexpr int L = tri::LD<64>;
+    __shared__ double D[tri::SPACE<64>];   // D(i, k) = op(T)(63 - i, 63 - k)
+    const int t = threadIdx.x;
     const i64 o = i64(blockIdx.x) * 64;
-    // T's element (o + tj, o + q), the thread index along the contiguous
-    // direction, 64 loads per thread in flight; it is op(T)[tj][q], or
-    // op(T)[q][tj] when TRANS
-    double r[64];
 #pragma unroll
-    for (int q = 0; q < 64; ++q) r[q] = T[(o + tj) + (o + q) * ldt];
-#pragma unroll
-    for (int q = 0; q < 64; ++q) {
-        if (TRANS) Ut[tj][q] = r[q];   // element (row q, column tj) of op(T)
-        else Ut[q][tj] = r[q];         // element (row tj, column q)
+    for (int u = 0; u < 16; ++u) {
+        const int e = t + u * 256;
+        const int x = e % 64, y = e / 64;        // T(o + x, o + y), the thread index along its columns
+        const int i = 63 - (TRANS ? y : x), k = 63 - (TRANS ? x : y);
+        const double v = T[(o + x) + (o + y) * ldt];
+        D[k * L + i] = i == k ? (UNIT ? 1.0 : v) : i > k ? v : 0.0;
     }
     __syncthreads();
-    const int j = tj;
-    double acc[64];
-#pragma unroll
-    for (int i = 0; i < 64; ++i) acc[i] = i == j ? 1.0 : 0.0;
-#pragma unroll
-    for (int k = 63; k >= 0; --k) {
-        const double x = UNIT ? acc[k] : acc[k] / Ut[k][k];
-        V[k][j] = k > j ? 0.0 : x;
-        if (k <= j) {
-#pragma unroll
-            for (int i = 0; i < k; ++i) acc[i] = __builtin_fma(-Ut[k][i], x, acc[i]);
-        }
-    }
-    __syncthreads();
-    // column-major store, the thread index along rows
-    const i64 d = 64 * i64(blockIdx.x);
-    double* out = strip > 0 ? inv + d + (d % strip) * ldv : inv + 64 * d;
+    tri::invert<double, 64, 4, UNIT>(D, t);
+    double* out = strip > 0 ? inv + o + (o % strip) * ldv : inv + 64 * o;
     const i64 ld = strip > 0 ? ldv : 64;
-#pragma unroll 8
-    for (int c = 0; c < 64; ++c) out[tj + ld * c] = V[tj][c];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        const int e = t + u * 256;
+        const int x = e % 64, y = e / 64;
+        out[x + ld * y] = x <= y ? D[(63 - y) * L + 63 - x] : 0.0;
+    }
 }
 
 // Left side: X (n x nrhs) <- op(T)^-1 X, one wave per right-hand side, lane =
@@ -282,7 +265,7 @@ static int trsm_right_upper(oxi_handle_t h, hipStream_t s, int trans, int unit, 
 static const double* right_upper_inverses(oxi_handle_t h, hipStream_t s, int trans, int unit, i64 rows, i64 n,
                                           const double* T, i64 ldt) {
     if (rows < 1024 || n < TRL || n % TRL || n / TRL > TRSM_INV_BLOCKS || !h->trsm_inv) return nullptr;
-    const dim3 grid(unsigned(n / TRL)), block(64);
+    const dim3 grid(unsigned(n / TRL)), block(256);
     if (unit) {
         if (trans) hipLaunchKernelGGL((trsm_inv64_kernel<true, true>), grid, block, 0, s, T, ldt, h->trsm_inv);
         else hipLaunchKernelGGL((trsm_inv64_kernel<true, false>), grid, block, 0, s, T, ldt, h->trsm_inv);
@@ -309,7 +292,7 @@ static const double* left_inverses(oxi_handle_t h, hipStream_t s, int upper, int
     if (m < 2 * TRL || m % TRL || m / TRL > TRSM_INV_BLOCKS || nrhs < 16 || !h->trsm_inv) return nullptr;
     const bool lower_op = (!upper) != (trans != 0);
     const bool ktrans = lower_op ? !trans : (trans != 0);
-    const dim3 grid(unsigned(m / TRL)), block(64);
+    const dim3 grid(unsigned(m / TRL)), block(256);
     if (unit) {
         if (ktrans) hipLaunchKernelGGL((trsm_inv64_kernel<true, true>), grid, block, 0, s, A, lda, h->trsm_inv);
         else hipLaunchKernelGGL((trsm_inv64_kernel<true, false>), grid, block, 0, s, A, lda, h->trsm_inv);
@@ -352,7 +335,7 @@ static int trsm_left_blocked(oxi_handle_t h, hipStream_t s, int upper, int trans
     double* T = S + sS;
     double* X = T + sT;
     if (oxi_launch_dscale(s, m, TRB, 0.0, S, m) != OXI_OK) return oxi_set_error(h, OXI_ERR_HIP, "trsm strip clear");
-    const dim3 grid(unsigned(m / TRL)), block(64);
+    const dim3 grid(unsigned(m / TRL)), block(256);
     if (unit) {
         if (ktrans) hipLaunchKernelGGL((trsm_inv64_kernel<true, true>), grid, block, 0, s, A, lda, S, m, TRB);
         else hipLaunchKernelGGL((trsm_inv64_kernel<true, false>), grid, block, 0, s, A, lda, S, m, TRB);

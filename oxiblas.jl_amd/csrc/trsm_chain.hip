@@ -32,7 +32,7 @@
 // device-scope stores and loads; the publishing waves wait for their stores
 // to be acknowledged before `ready` moves.  Every wait is bounded: a
 // timeout sets a sticky error word, read by oxi_trsm_chain_check.
-#include "oxi_internal.hpp"
+#include "tri_inv.hpp"
 
 namespace {
 
@@ -63,74 +63,70 @@ __device__ __forceinline__ i64 block_row0(bool bwd, i64 n, int b, int rows) {
     return bwd ? n - i64(b) * CB - rows : i64(b) * CB;
 }
 
-// V_b: the inverse of diagonal block b of op(T) (T or, with TRANS, its
-// transpose), V[b][k * CB + i] = V_b(i, k) in the block's physical row
-// order, zero outside its rows.  Thread j solves
-// T_bb x = e_j by substitution (forward for the lower triangle, backward for
-// the upper one) with the block and x in LDS.
+// Per block b, in the block's physical row order: V_b, the inverse of the
+// diagonal block of op(T) (T or, with TRANS, its transpose; UPPER: op(T) is
+// upper triangular, solved backward), V[b][k * CB + i] = V_b(i, k), zero
+// outside its rows; and its couplings G_b = V_b T_{b,b-1} (b >= 1) and
+// H_b = V_b T_{b,b-2} (b >= 2), G[b][q * CB + i] over physical rows i of block
+// b and q of the earlier block (a full one).
+//
+// One workgroup per block: the block, in solve order, in LDS, inverted on the
+// matrix cores (tri::invert), then 16 columns of each coupling a wave, loaded
+// at the start.  Bound by the latency of its loads and barriers: at n = 8192
+// a triangle takes 18 us, against 50 for the inverses by substitution in LDS
+// and 35 for the couplings as two kernels on the vector units.
 template <bool UPPER, bool UNIT, bool TRANS>
-__global__ __launch_bounds__(CB) void chain_inv_kernel(const double* __restrict__ M, i64 ld, i64 n,
-                                                       double* __restrict__ V) {
-    __shared__ double Ts[CB][CB + 1];   // Ts[r][c] = T_bb(r, c)
-    __shared__ double Xs[CB][CB + 1];   // Xs[r][j]: column j of the inverse
-    const int j = threadIdx.x, b = blockIdx.x;
+__global__ __launch_bounds__(CNT) void chain_prepare_kernel(const double* __restrict__ M, i64 ld, i64 n,
+                                                            double* __restrict__ V, double* __restrict__ G,
+                                                            double* __restrict__ H) {
+    constexpr int L = tri::LD<CB>;
+    __shared__ double D[tri::SPACE<CB>];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, b = blockIdx.x;
     const int rows = int(min(i64(CB), n - i64(b) * CB));
     const i64 p0 = block_row0(UPPER, n, b, rows);
-    for (int c = 0; c < rows; ++c)
-        Ts[j][c] = j < rows ? (TRANS ? M[(p0 + c) + (p0 + j) * ld] : M[(p0 + j) + (p0 + c) * ld]) : 0.0;
-    __syncthreads();
-    for (int r = 0; r < CB; ++r) Xs[r][j] = 0.0;
-    if (j < rows) {
-        if (!UPPER) {
-            Xs[j][j] = UNIT ? 1.0 : 1.0 / Ts[j][j];
-            for (int r = j + 1; r < rows; ++r) {
-                double s = 0.0;
-                for (int m = j; m < r; ++m) s = __builtin_fma(Ts[r][m], Xs[m][j], s);
-                Xs[r][j] = UNIT ? -s : -s / Ts[r][r];
-            }
-        } else {
-            Xs[j][j] = UNIT ? 1.0 : 1.0 / Ts[j][j];
-            for (int r = j - 1; r >= 0; --r) {
-                double s = 0.0;
-                for (int m = r + 1; m <= j; ++m) s = __builtin_fma(Ts[r][m], Xs[m][j], s);
-                Xs[r][j] = UNIT ? -s : -s / Ts[r][r];
-            }
+    // physical row of logical row k in the block (and the reverse)
+    auto phys = [&](int k) __attribute__((always_inline)) { return UPPER ? rows - 1 - k : k; };
+    // D(i, k) = op(T)(i, k), the identity outside the block; the index that
+    // runs along M's columns changes fastest.  Loads without branches.
+#pragma unroll
+    for (int u = 0; u < CB * CB / CNT; ++u) {
+        const int e = t + u * CNT;
+        const int x = e % CB, y = e / CB;
+        const int i = TRANS ? y : x, k = TRANS ? x : y;
+        const int ic = phys(min(i, rows - 1)), kc = phys(min(k, rows - 1));
+        const double v = TRANS ? M[(p0 + kc) + (p0 + ic) * ld] : M[(p0 + ic) + (p0 + kc) * ld];
+        const bool in = i < rows && k < rows;
+        D[k * L + i] = i == k ? (UNIT || !in ? 1.0 : v) : in && i > k ? v : 0.0;
+    }
+    double tv[2][CB / 4];
+#pragma unroll
+    for (int d = 1; d <= 2; ++d) {
+        if (b < d) break;
+        const i64 q = block_row0(UPPER, n, b - d, CB) + w * 16 + (lane & 15);
+#pragma unroll
+        for (int s = 0; s < CB / 4; ++s) {
+            const int k = 4 * s + (lane >> 4), kc = phys(min(k, rows - 1));
+            const double v = TRANS ? M[q + (p0 + kc) * ld] : M[(p0 + kc) + q * ld];
+            tv[d - 1][s] = k < rows ? v : 0.0;
         }
     }
     __syncthreads();
+    tri::invert<double, CB, CNT / 64, UNIT>(D, t);
     double* out = V + size_t(b) * CB * CB;
-    for (int c = 0; c < CB; ++c) out[c * CB + j] = Xs[j][c];
-}
-
-// G_b = V_b T_{b,b-d} for b >= d (d = 1: G_b, d = 2: H_b): G[b][q * CB + i]
-// over physical rows i of block b and physical rows q of block b-d (a full
-// block).
-template <bool BWD, bool TRANS>
-__global__ __launch_bounds__(CNT) void chain_g_kernel(const double* __restrict__ M, i64 ld, i64 n, int d,
-                                                      const double* __restrict__ V, double* __restrict__ G) {
-    __shared__ double Tb[CB][CB + 1];   // Tb[k][q] = op(T)(row k of block b, row q of block b-d)
-    const int t = threadIdx.x, b = blockIdx.x + d;
-    const int rows = int(min(i64(CB), n - i64(b) * CB));
-    const i64 p0 = block_row0(BWD, n, b, rows), q0 = block_row0(BWD, n, b - d, CB);
-    for (int e = t; e < CB * CB; e += CNT) {
-        const int k = e % CB, q = e / CB;
-        Tb[k][q] = k < rows ? (TRANS ? M[(q0 + q) + (p0 + k) * ld] : M[(p0 + k) + (q0 + q) * ld]) : 0.0;
+#pragma unroll
+    for (int u = 0; u < CB * CB / CNT; ++u) {
+        const int e = t + u * CNT;
+        const int pi = e % CB, pk = e / CB;      // physical row and column
+        const int i = phys(min(pi, rows - 1)), k = phys(min(pk, rows - 1));
+        out[e] = pi < rows && pk < rows && i >= k ? D[k * L + i] : 0.0;
     }
-    __syncthreads();
-    const double* vb = V + size_t(b) * CB * CB;
-    const int i = t % CB, qg = t / CB;
-    constexpr int QPT = CB / (CNT / CB);
-    double acc[QPT];
 #pragma unroll
-    for (int u = 0; u < QPT; ++u) acc[u] = 0.0;
-    for (int k = 0; k < rows; ++k) {
-        const double v = vb[k * CB + i];
-#pragma unroll
-        for (int u = 0; u < QPT; ++u) acc[u] = __builtin_fma(v, Tb[k][qg * QPT + u], acc[u]);
+    for (int d = 1; d <= 2; ++d) {
+        if (b < d) break;
+        double* g = (d == 1 ? G : H) + size_t(b) * CB * CB + w * 16 * CB;
+        tri::times<double, CB>(D, tv[d - 1], lane,
+                               [&](int i, int q, double v) { g[q * CB + (i < rows ? phys(i) : i)] = v; });
     }
-    double* g = G + size_t(b) * CB * CB;
-#pragma unroll
-    for (int u = 0; u < QPT; ++u) g[(qg * QPT + u) * CB + i] = acc[u];
 }
 
 __global__ void chain_ctrl_reset(ChainCtrl* c) {
@@ -383,29 +379,14 @@ int oxi_trsm_chain_prepare(oxi_handle_t h, hipStream_t s, int tk, i64 n, const d
     double *v0 = slot_ptr(ws, n, 0), *v1 = slot_ptr(ws, n, 1), *g0 = slot_ptr(ws, n, 2), *g1 = slot_ptr(ws, n, 3);
     double *h0 = slot_ptr(ws, n, 4), *h1 = slot_ptr(ws, n, 5);
     if (tk == 0) {          // L (unit, forward), then U (backward)
-        hipLaunchKernelGGL((chain_inv_kernel<false, true, false>), dim3(nb), dim3(CB), 0, s, LU, lda, n, v0);
-        hipLaunchKernelGGL((chain_inv_kernel<true, false, false>), dim3(nb), dim3(CB), 0, s, LU, lda, n, v1);
+        hipLaunchKernelGGL((chain_prepare_kernel<false, true, false>), dim3(nb), dim3(CNT), 0, s, LU, lda, n, v0, g0, h0);
+        hipLaunchKernelGGL((chain_prepare_kernel<true, false, false>), dim3(nb), dim3(CNT), 0, s, LU, lda, n, v1, g1, h1);
     } else if (tk == 1) {   // U^T (forward), then L^T (unit, backward)
-        hipLaunchKernelGGL((chain_inv_kernel<false, false, true>), dim3(nb), dim3(CB), 0, s, LU, lda, n, v0);
-        hipLaunchKernelGGL((chain_inv_kernel<true, true, true>), dim3(nb), dim3(CB), 0, s, LU, lda, n, v1);
+        hipLaunchKernelGGL((chain_prepare_kernel<false, false, true>), dim3(nb), dim3(CNT), 0, s, LU, lda, n, v0, g0, h0);
+        hipLaunchKernelGGL((chain_prepare_kernel<true, true, true>), dim3(nb), dim3(CNT), 0, s, LU, lda, n, v1, g1, h1);
     } else {                // Cholesky: L (forward), then L^T (backward)
-        hipLaunchKernelGGL((chain_inv_kernel<false, false, false>), dim3(nb), dim3(CB), 0, s, LU, lda, n, v0);
-        hipLaunchKernelGGL((chain_inv_kernel<true, false, true>), dim3(nb), dim3(CB), 0, s, LU, lda, n, v1);
-    }
-    // the first triangle is op(T) = T except for U^T, the second T^T except for U
-    for (int d = 1; d <= 2; ++d) {
-        if (nb <= d) break;
-        double* c0 = d == 1 ? g0 : h0;
-        double* c1 = d == 1 ? g1 : h1;
-        const dim3 grid(nb - unsigned(d));
-        if (tk == 1)
-            hipLaunchKernelGGL((chain_g_kernel<false, true>), grid, dim3(CNT), 0, s, LU, lda, n, d, v0, c0);
-        else
-            hipLaunchKernelGGL((chain_g_kernel<false, false>), grid, dim3(CNT), 0, s, LU, lda, n, d, v0, c0);
-        if (tk == 0)
-            hipLaunchKernelGGL((chain_g_kernel<true, false>), grid, dim3(CNT), 0, s, LU, lda, n, d, v1, c1);
-        else
-            hipLaunchKernelGGL((chain_g_kernel<true, true>), grid, dim3(CNT), 0, s, LU, lda, n, d, v1, c1);
+        hipLaunchKernelGGL((chain_prepare_kernel<false, false, false>), dim3(nb), dim3(CNT), 0, s, LU, lda, n, v0, g0, h0);
+        hipLaunchKernelGGL((chain_prepare_kernel<true, false, true>), dim3(nb), dim3(CNT), 0, s, LU, lda, n, v1, g1, h1);
     }
     return launch_check(h, "trsm chain preparation");
 }

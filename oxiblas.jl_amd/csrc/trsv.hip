@@ -6,8 +6,7 @@
 // x of every earlier block.
 //
 // Preparation (oxi_trsv_prepare, once per factor and triangle): the inverse
-// of every RB x RB diagonal block, computed by parallel column sweeps, in the
-// arithmetic type.  A solve then does no sequential sweep: each block's x is
+// of every RB x RB diagonal block, in the arithmetic type.  A solve then does no sequential sweep: each block's x is
 // a matrix-vector product with its inverse.
 //
 // The solve (one launch per triangle): workgroups take block numbers from an
@@ -36,7 +35,7 @@
 // Solve order and memory access: `which` 0 = L (unit) forward, 1 = U backward,
 // 2 = U^T forward, 3 = L^T (unit) backward; backward solves use logical index
 // i' = n-1-i, so the same code runs both directions with coalesced access.
-#include "oxi_internal.hpp"
+#include "tri_inv.hpp"
 
 #include <cstdlib>
 
@@ -52,15 +51,6 @@ template <typename TM> struct Vec;
 template <> struct Vec<double> { typedef double type __attribute__((ext_vector_type(2))); static constexpr int N = 2; };
 template <> struct Vec<float> { typedef float type __attribute__((ext_vector_type(4))); static constexpr int N = 4; };
 
-__device__ __forceinline__ double bcast(double v, int l) {
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-    const unsigned lo = __builtin_amdgcn_readlane(unsigned(u), l);
-    const unsigned hi = __builtin_amdgcn_readlane(unsigned(u >> 32), l);
-    return __builtin_bit_cast(double, (static_cast<unsigned long long>(hi) << 32) | lo);
-}
-__device__ __forceinline__ float bcast(float v, int l) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(unsigned, v), l));
-}
 __device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
 __device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
@@ -88,110 +78,66 @@ __global__ void trsv_status_clear(TrsvCtrl* c) {
     if (threadIdx.x == 0) { c->ticket = 0; c->ready = 0; c->err = 0; c->pad = 0; }
 }
 
-// The diagonal block of block b, D[k * (RB + 1) + i] = T(i, k) in logical
-// (solve-order) indices, into LDS.
-template <typename TM, bool TRANS, bool BWD>
-__device__ __forceinline__ void load_diag(const TM* __restrict__ M, i64 ld, i64 p0, int rows, TM* D, int t) {
-    for (int e = t; e < RB * RB; e += NT) {
-        const int pr = e % RB, pc = e / RB;
-        if (pr < rows && pc < rows) {
-            const TM v = M[(p0 + pr) + (p0 + pc) * ld];
-            const int lr = BWD ? rows - 1 - pr : pr, lc = BWD ? rows - 1 - pc : pc;
-            const int i = TRANS ? lc : lr, k = TRANS ? lr : lc;
-            D[k * (RB + 1) + i] = v;
-        }
-    }
-}
-
-// Inverse of every diagonal block (logical indices, lower triangular):
+// Per block b of RB rows (logical indices, lower triangular): its inverse
 // inv[b][k * RB + i] = Dinv(i, k), zero above the diagonal and outside the
-// block.  Wave w solves T X = I for columns 16w .. 16w+15, four at a time, by
-// column sweep (lane i owns rows i and i+64; x_k broadcast by readlane).
+// block, and for b >= 1 G_b = inv_b * T_{b,b-1}, G[q * RB + i] over logical
+// rows i of block b and physical columns q of block b-1 (the order the chain
+// kernel holds x_{b-1} in), as the chain kernel's last chunk would use them.
+//
+// One workgroup per block: the block in LDS, inverted on the matrix cores
+// (tri::invert), then 16 columns of T_{b,b-1} a wave, loaded at the start.
+// Bound by the latency of its loads and barriers, and G's 144 matrix
+// instructions a wave.  A 256 x 256 factor's unit lower triangle: 38 us, against
+// 80 for an inverse swept four columns at a time by each wave and 65 for G as
+// a kernel of its own on the vector units.
 template <typename TM, typename TV, bool TRANS, bool UNIT, bool BWD>
-__global__ __launch_bounds__(NT) void trsv_dinv_kernel(const TM* __restrict__ M, i64 ld, i64 n, TV* __restrict__ inv) {
-    __shared__ TM D[RB * (RB + 1)];
-    __shared__ TV rinv[RB];
+__global__ __launch_bounds__(NT) void trsv_prepare_kernel(const TM* __restrict__ M, i64 ld, i64 n, TV* __restrict__ inv,
+                                                          TV* __restrict__ G) {
+    constexpr int L = tri::LD<RB>;
+    __shared__ TV D[tri::SPACE<RB>];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int b = blockIdx.x;
     const i64 lo = i64(b) * RB;
     const int rows = int(min(i64(RB), n - lo));
     const i64 p0 = BWD ? n - lo - rows : lo;
-    load_diag<TM, TRANS, BWD>(M, ld, p0, rows, D, t);
+    // physical row of logical row k in the block
+    auto phys = [&](int k) __attribute__((always_inline)) { return BWD ? rows - 1 - k : k; };
+    // D(i, k) = T(i, k), the identity outside the block; the index that runs
+    // along M's columns changes fastest.  Loads without branches.
+#pragma unroll 16
+    for (int u = 0; u < RB * RB / NT; ++u) {
+        const int e = t + u * NT;
+        const int x = e % RB, y = e / RB;
+        const int i = TRANS ? y : x, k = TRANS ? x : y;
+        const int ic = phys(min(i, rows - 1)), kc = phys(min(k, rows - 1));
+        const TM v = TRANS ? M[(p0 + kc) + (p0 + ic) * ld] : M[(p0 + ic) + (p0 + kc) * ld];
+        const bool in = i < rows && k < rows;
+        D[k * L + i] = i == k ? (UNIT || !in ? TV(1) : TV(v)) : in && i > k ? TV(v) : TV(0);
+    }
+    TV tv[RB / 4];
+    if (b > 0) {
+        const i64 q0 = BWD ? n - i64(b) * RB : i64(b - 1) * RB;
+        const i64 q = q0 + w * 16 + (lane & 15);
+#pragma unroll
+        for (int s = 0; s < RB / 4; ++s) {
+            const int k = 4 * s + (lane >> 4), kc = phys(min(k, rows - 1));
+            const TM v = TRANS ? M[q + (p0 + kc) * ld] : M[(p0 + kc) + q * ld];
+            tv[s] = k < rows ? TV(v) : TV(0);
+        }
+    }
     __syncthreads();
-    if (!UNIT)
-        for (int k = t; k < rows; k += NT) rinv[k] = TV(1) / TV(D[k * (RB + 1) + k]);
-    __syncthreads();
+    tri::invert<TV, RB, NT / 64, UNIT>(D, t);
     TV* out = inv + size_t(b) * RB * RB;
-    constexpr int CPW = RB / (NT / 64);   // columns per wave
-    for (int c0 = CPW * w; c0 < CPW * (w + 1); c0 += 4) {
-        TV s[4][2];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            s[r][0] = lane == c0 + r ? TV(1) : TV(0);
-            s[r][1] = lane + 64 == c0 + r ? TV(1) : TV(0);
-        }
-        for (int k = c0; k < rows; ++k) {
-            const TV d0 = TV(D[k * (RB + 1) + lane]), d1 = TV(D[k * (RB + 1) + 64 + lane]);
-            const TV rk = UNIT ? TV(1) : rinv[k];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const TV sk = k < 64 ? s[r][0] : s[r][1];
-                const TV xk = bcast(UNIT ? sk : sk * rk, k & 63);
-                if (lane > k) s[r][0] = fma_t(-d0, xk, s[r][0]);
-                if (lane + 64 > k) s[r][1] = fma_t(-d1, xk, s[r][1]);
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int c = c0 + r;
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int i = lane + 64 * h;
-                TV v = TV(0);
-                if (c < rows && i < rows) v = UNIT ? s[r][h] : s[r][h] * rinv[i];
-                out[c * RB + i] = v;
-            }
-        }
+#pragma unroll 16
+    for (int u = 0; u < RB * RB / NT; ++u) {
+        const int e = t + u * NT;
+        const int i = e % RB, k = e / RB;
+        out[e] = i >= k && i < rows ? D[k * L + i] : TV(0);
     }
-}
-
-// G_b = inv_b * T_{b,b-1} for b >= 1, G[q * RB + i] over logical rows i of
-// block b and physical columns q of block b-1 (the order the chain kernel
-// holds x_{b-1} in), as the chain kernel's last chunk would use them.  The
-// block T_{b,b-1} goes to LDS in the working type; the inverse is read from
-// memory.  Block 0 has no G.
-template <typename TM, typename TV, bool TRANS, bool BWD>
-__global__ __launch_bounds__(NT) void trsv_g_kernel(const TM* __restrict__ M, i64 ld, i64 n, const TV* __restrict__ inv,
-                                                    TV* __restrict__ G) {
-    __shared__ TV Tp[RB * (RB + 1)];   // Tp[q * (RB + 1) + pr]: physical row pr of block b, column q of block b-1
-    const int t = threadIdx.x;
-    const int b = blockIdx.x + 1;
-    const i64 lo = i64(b) * RB;
-    const int rows = int(min(i64(RB), n - lo));
-    const i64 p0 = BWD ? n - lo - rows : lo;
-    const i64 q0 = BWD ? n - i64(b) * RB : i64(b - 1) * RB;
-    for (int e = t; e < RB * RB; e += NT) {
-        const int pr = e % RB, q = e / RB;
-        TV v = TV(0);
-        if (pr < rows) v = TV(TRANS ? M[(q0 + q) + (p0 + pr) * ld] : M[(p0 + pr) + (q0 + q) * ld]);
-        Tp[q * (RB + 1) + pr] = v;
+    if (b > 0) {
+        TV* g = G + size_t(b) * RB * RB + size_t(w) * 16 * RB;
+        tri::times<TV, RB>(D, tv, lane, [&](int i, int q, TV v) { g[q * RB + i] = v; });
     }
-    __syncthreads();
-    const TV* di = inv + size_t(b) * RB * RB;
-    TV* g = G + size_t(b) * RB * RB;
-    const int i = t % RB, qg = t / RB;
-    constexpr int QPT = RB / (NT / RB);
-    TV acc[QPT];
-#pragma unroll
-    for (int k = 0; k < QPT; ++k) acc[k] = TV(0);
-    for (int j = 0; j < rows; ++j) {
-        const TV d = di[j * RB + i];
-        const int pr = BWD ? rows - 1 - j : j;
-#pragma unroll
-        for (int k = 0; k < QPT; ++k) acc[k] = fma_t(d, Tp[(qg * QPT + k) * (RB + 1) + pr], acc[k]);
-    }
-#pragma unroll
-    for (int k = 0; k < QPT; ++k) g[(qg * QPT + k) * RB + i] = acc[k];
 }
 
 // Two device-scope loads issued back to back and waited for once (relaxed
@@ -520,20 +466,11 @@ int prepare_t(oxi_handle_t h, hipStream_t s, int tk, i64 n, const TM* M, i64 ld,
     TV* g0 = slot_of<TV>(ws, n, 2);
     TV* g1 = slot_of<TV>(ws, n, 3);
     if (!tk) {
-        hipLaunchKernelGGL((trsv_dinv_kernel<TM, TV, false, true, false>), dim3(grid), dim3(NT), 0, s, M, ld, n, i0);
-        hipLaunchKernelGGL((trsv_dinv_kernel<TM, TV, false, false, true>), dim3(grid), dim3(NT), 0, s2, M, ld, n, i1);
+        hipLaunchKernelGGL((trsv_prepare_kernel<TM, TV, false, true, false>), dim3(grid), dim3(NT), 0, s, M, ld, n, i0, g0);
+        hipLaunchKernelGGL((trsv_prepare_kernel<TM, TV, false, false, true>), dim3(grid), dim3(NT), 0, s2, M, ld, n, i1, g1);
     } else {
-        hipLaunchKernelGGL((trsv_dinv_kernel<TM, TV, true, false, false>), dim3(grid), dim3(NT), 0, s, M, ld, n, i0);
-        hipLaunchKernelGGL((trsv_dinv_kernel<TM, TV, true, true, true>), dim3(grid), dim3(NT), 0, s2, M, ld, n, i1);
-    }
-    if (grid > 1) {
-        if (!tk) {
-            hipLaunchKernelGGL((trsv_g_kernel<TM, TV, false, false>), dim3(grid - 1), dim3(NT), 0, s, M, ld, n, i0, g0);
-            hipLaunchKernelGGL((trsv_g_kernel<TM, TV, false, true>), dim3(grid - 1), dim3(NT), 0, s2, M, ld, n, i1, g1);
-        } else {
-            hipLaunchKernelGGL((trsv_g_kernel<TM, TV, true, false>), dim3(grid - 1), dim3(NT), 0, s, M, ld, n, i0, g0);
-            hipLaunchKernelGGL((trsv_g_kernel<TM, TV, true, true>), dim3(grid - 1), dim3(NT), 0, s2, M, ld, n, i1, g1);
-        }
+        hipLaunchKernelGGL((trsv_prepare_kernel<TM, TV, true, false, false>), dim3(grid), dim3(NT), 0, s, M, ld, n, i0, g0);
+        hipLaunchKernelGGL((trsv_prepare_kernel<TM, TV, true, true, true>), dim3(grid), dim3(NT), 0, s2, M, ld, n, i1, g1);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return oxi_set_error(h, OXI_ERR_HIP, "trsv prepare launch: %s", hipGetErrorString(e));

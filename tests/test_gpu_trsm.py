@@ -70,3 +70,30 @@ def test_trsm_singular_reported_before_write(gpu, rng):
         gpu.trsm_(B, T, 1.0, "L", "U", "N", False)
     assert e.value.info == 8
     assert np.array_equal(B, B0)
+
+
+# Solves through the inverted diagonal blocks (128 rows for one right-hand
+# side, 64 for several) at the edges of the blocks and of their 16-wide tiles.
+# Backward error of LU or Cholesky plus two triangular solves: at most a small
+# multiple of n eps (|A| |x| + |b|), 4 for each of the factorization and the
+# solves, of well-conditioned blocks.
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 144, 255, 257, 385])
+@pytest.mark.parametrize("nrhs", [1, 3, 40])
+def test_block_inverse_solves(gpu, rng, n, nrhs):
+    A = rng.standard_normal((n, n)) + 2.0 * np.sqrt(n) * np.eye(n)
+    B = np.asfortranarray(rng.standard_normal((n, nrhs)))
+    S = A @ A.T + n * np.eye(n)
+
+    def residual(M, X, eps):
+        r = np.linalg.norm(M @ X - B)
+        assert r <= 8 * max(n, 8) * eps * (np.linalg.norm(M) * np.linalg.norm(X) + np.linalg.norm(B)), r
+    F = gpu.lu(np.asfortranarray(A))
+    for t in "NT":
+        residual(A if t == "N" else A.T, F.solve(B, t), EPS)
+        residual(A if t == "N" else A.T, F.solve(B, t), EPS)      # the second solve runs on a kept plan
+    residual(S, gpu.cholesky(np.asfortranarray(S)).solve(B), EPS)
+    F32 = gpu.lu_lowp(np.asfortranarray(A.astype(np.float32)), "float32")
+    for t in "NT":
+        X = F32.solve(np.asfortranarray(B.astype(np.float32)), t)
+        X = X.numpy() if hasattr(X, "numpy") else X
+        residual((A if t == "N" else A.T).astype(np.float32).astype(float), X.astype(float), np.finfo(np.float32).eps)
