@@ -684,25 +684,15 @@ void launch_any(hipStream_t s, int ta, int tb, i64 m, i64 n, i64 k, double alpha
 }  // namespace
 
 // The in-place block products of the triangular solves: a workgroup's tile
-// has all 64 columns (rows) of its rows (columns), and it writes them only
-// after its last read of them (the epilogue follows the K loop, whose last
-// barrier all its loads have passed).  A row or column that it reads of
-// another workgroup's tile (the first of a pair at an edge) is not used.
+// has all 64 columns of its rows, and it writes them only after its last read
+// of them (the epilogue follows the K loop, whose last barrier all its loads
+// have passed).  A row that it reads of another workgroup's tile (the first of
+// a pair at an edge) is not used.
 int oxi_dgemm_right64_inplace(hipStream_t s, i64 rows, const double* V, double* X, i64 ldx) {
     // X[:, 0:64] <- X[:, 0:64] * V (V 64 x 64, ld 64)
     if (rows <= 0) return OXI_OK;
     if (!launch_direct<32, 64, 32, 2, false, false>(s, rows, 64, 64, 1.0, X, ldx, V, 64, 0.0, X, ldx))
         launch_tiles<32, 64, false, false>(s, rows, 64, 64, 1.0, X, ldx, V, 64, 0.0, X, ldx);
-    return hipGetLastError() == hipSuccess ? OXI_OK : OXI_ERR_HIP;
-}
-
-int oxi_dgemm_left64_inplace(hipStream_t s, int ta, i64 ncols, const double* V, double* X, i64 ldx) {
-    // X[0:64, :] <- op(V) * X[0:64, :] (V 64 x 64, ld 64)
-    if (ncols <= 0) return OXI_OK;
-    const bool done = ta ? launch_direct<64, 32, 32, 2, true, false>(s, 64, ncols, 64, 1.0, V, 64, X, ldx, 0.0, X, ldx)
-                         : launch_direct<64, 32, 32, 2, false, false>(s, 64, ncols, 64, 1.0, V, 64, X, ldx, 0.0, X, ldx);
-    if (!done && ta) launch_tiles<64, 32, true, false>(s, 64, ncols, 64, 1.0, V, 64, X, ldx, 0.0, X, ldx);
-    if (!done && !ta) launch_tiles<64, 32, false, false>(s, 64, ncols, 64, 1.0, V, 64, X, ldx, 0.0, X, ldx);
     return hipGetLastError() == hipSuccess ? OXI_OK : OXI_ERR_HIP;
 }
 

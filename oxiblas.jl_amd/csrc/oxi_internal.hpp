@@ -111,9 +111,8 @@ int oxi_potrf_device(oxi_handle_t h, hipStream_t s, i64 n, float* A, i64 lda, i6
 bool oxi_dgemm_large(i64 m, i64 n);
 // X[:, 0:64] <- X[:, 0:64] * V in place (V 64 x 64, column-major, ld 64)
 int oxi_dgemm_right64_inplace(hipStream_t s, i64 rows, const double* V, double* X, i64 ldx);
-// X[0:64, 0:ncols] <- op(V) X[0:64, 0:ncols] in place (V 64 x 64, ld 64; ta: V^T)
-int oxi_dgemm_left64_inplace(hipStream_t s, int ta, i64 ncols, const double* V, double* X, i64 ldx);
-// Left-side triangular solve, host-recursive with GEMM updates.
+// Triangular solves, host-recursive with GEMM updates; the right-side one is for
+// factorizations (it shares no scratch memory between streams below 1024 rows).
 int oxi_dtrsm_left(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit, i64 m, i64 nrhs,
                    const double* A, i64 lda, double* B, i64 ldb);
 int oxi_dtrsm_right(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit, i64 m, i64 n,

@@ -11,6 +11,7 @@ __device__ __forceinline__ double fma_t(double a, double b, double c) { return _
 __device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
 constexpr int TRL = 64;
+constexpr int SB = 256;   // rows of a block of the blocked solves
 
 // Right side: X (rows x n) <- X * op(T)^-1, n <= 64.  Element order matches
 // the reference's right leaf (src/blas/level3.jl:319-333):
@@ -126,38 +127,166 @@ void launch_right_leaf(hipStream_t s, int unit, int trans, i64 rows, int n, cons
     }
 }
 
-// Inverses of the 64 x 64 diagonal blocks of an upper op(T): block b's
-// V = U_bb^-1 goes to inv + 4096 b, column-major (ld 64, zeros below the
-// diagonal); with strip > 0, to its place in a column-major strip of ld
-// `ldv` whose rows z*strip .. (z+1)*strip - 1 hold the strip x strip block z
-// (inv + 64 b + ((64 b) % strip) * ldv).  The block, both indices reversed
-// (lower triangular), in LDS, inverted on the matrix cores (tri::invert);
-// bound by the latency of its loads and barriers: 8 us, against 27 for a
-// column a lane swept over 64 steps.
-template <bool UNIT, bool TRANS>
-__global__ __launch_bounds__(256) void trsm_inv64_kernel(const double* __restrict__ T, i64 ldt,
+// Inverses of the 64 x 64 diagonal blocks of a triangle M of n rows, M(i, k) =
+// T(i, k) (TRANS: T(k, i)), UPPER or lower: block b's goes to inv + 4096 b,
+// column-major (ld 64, zeros in the other triangle, the identity beyond n);
+// with strip > 0, to its place in a column-major strip of ld `ldv` whose rows
+// z*strip .. (z+1)*strip - 1 hold the strip x strip block z (inv + 64 b +
+// ((64 b) % strip) * ldv); CLEAN: to inv + 8192 b, and the block itself,
+// completed in the same way, 4096 elements behind it.  The block in
+// LDS (UPPER: both indices reversed, so that it is lower triangular), inverted
+// on the matrix cores (tri::invert); bound by the latency of its loads and
+// barriers: 8 us, against 27 for a column a lane swept over 64 steps.
+template <bool UNIT, bool TRANS, bool UPPER, bool CLEAN>
+__global__ __launch_bounds__(256) void trsm_inv64_kernel(const double* __restrict__ T, i64 ldt, i64 n,
                                                          double* __restrict__ inv, i64 ldv = 64, int strip = 0) {
     constexpr int L = tri::LD<64>;
-    __shared__ double D[tri::SPACE<64>];   // D(i, k) = op(T)(63 - i, 63 - k)
+    __shared__ double D[tri::SPACE<64>];   // D(i, k) = M(i, k), or M(63 - i, 63 - k)
     const int t = threadIdx.x;
     const i64 o = i64(blockIdx.x) * 64;
+    double* out = strip > 0 ? inv + o + (o % strip) * ldv : inv + 64 * (CLEAN ? 2 : 1) * o;
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
         const int e = t + u * 256;
         const int x = e % 64, y = e / 64;        // T(o + x, o + y), the thread index along its columns
-        const int i = 63 - (TRANS ? y : x), k = 63 - (TRANS ? x : y);
-        const double v = T[(o + x) + (o + y) * ldt];
-        D[k * L + i] = i == k ? (UNIT ? 1.0 : v) : i > k ? v : 0.0;
+        const int r = TRANS ? y : x, c = TRANS ? x : y, i = UPPER ? 63 - r : r, k = UPPER ? 63 - c : c;
+        const double v = T[min(o + x, n - 1) + min(o + y, n - 1) * ldt];
+        const bool in = o + x < n && o + y < n;
+        D[k * L + i] = i == k ? (UNIT || !in ? 1.0 : v) : in && i > k ? v : 0.0;
     }
     __syncthreads();
+    auto store = [&](double* to) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const int e = t + u * 256, r = e % 64, c = e / 64, i = UPPER ? 63 - r : r, k = UPPER ? 63 - c : c;
+            to[r + c * ldv] = i >= k ? D[k * L + i] : 0.0;
+        }
+    };
+    if (CLEAN) {
+        store(out + 4096);
+        __syncthreads();
+    }
     tri::invert<double, 64, 4, UNIT>(D, t);
-    double* out = strip > 0 ? inv + o + (o % strip) * ldv : inv + 64 * o;
-    const i64 ld = strip > 0 ? ldv : 64;
+    store(out);
+}
+
+// One block of up to SB = 256 rows of a triangular solve M x = b in place, M
+// lower (BWD: upper) triangular, M(i, k) = T(i, k) (TM: T(k, i)); LEFT: right-
+// hand sides are columns of B, element (i, j) at B[i + j * ldb], else rows, at
+// B[j + i * ldb] (X op(T) = B is op(T)^T X^T = B^T).  V: for each of the block's
+// 64-row diagonal blocks, M_pp^-1 and M_pp (trsm_inv64_kernel).  FULL: rows is
+// SB (no masks; a load behind one is waited for at once).
+//
+// A workgroup owns 16 right-hand sides and goes through the 64-row blocks in
+// solve order: r = b_p - sum M_pq x_q over the blocks before, x = M_pp^-1 r, and
+// one refinement x += M_pp^-1 (r - M_pp x), so that x is no further off than by
+// substitution; a wave has 16 of the 64 rows, x in LDS, the operands of M and
+// V straight from memory, the next product's loaded while one runs.  256 rows cost one launch and no scratch memory.  Bound by the
+// 18 products a wave has one after the other (16 matrix instructions of 64
+// cycles each, 9 us) and the 16 turns through LDS and a barrier: 22 us.
+template <bool LEFT, bool TM, bool BWD, bool FULL>
+__global__ __launch_bounds__(256, 1) void trsm_block_kernel(const double* __restrict__ T, i64 ldt,
+                                                            const double* __restrict__ V, double* __restrict__ B,
+                                                            i64 ldb, int nrows, i64 nrhs) {
+    typedef tri::Mfma<double> Mf;
+    constexpr int C = 16, LX = C + 1;
+    __shared__ double xs[SB * LX], rs[64 * LX];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, lk = lane >> 4, li = lane & 15;
+    const int rows = FULL ? SB : nrows, nsb = (rows + 63) / 64;
+    const i64 j0 = i64(blockIdx.x) * C;
+    const int nc = int(min(i64(C), nrhs - j0));
+    // this lane's operands of M_pq, and of M_pp^-1 (at 0) or M_pp (at 4096) of block p
+    auto load_m = [&](int p, int q, double (&a)[16]) __attribute__((always_inline)) {
+        const int i = p * 64 + w * 16 + li, ic = FULL ? i : min(i, rows - 1);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int k = q * 64 + 4 * e + lk, kc = FULL ? k : min(k, rows - 1);
+            const double m = TM ? T[kc + i64(ic) * ldt] : T[ic + i64(kc) * ldt];
+            a[e] = FULL || (i < rows && k < rows) ? m : 0.0;
+        }
+    };
+    auto load_v = [&](int p, int off, double (&a)[16]) __attribute__((always_inline)) {
+        const double* vp = V + p * 8192 + off + w * 16 + li + 64 * lk;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) a[e] = vp[256 * e];
+    };
+    auto product = [&](const double (&a)[16], const double* x, Mf::acc c) __attribute__((always_inline)) {
+        double y[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) y[e] = x[(4 * e + lk) * LX + li];
+        __builtin_amdgcn_sched_barrier(0);   // all of x on its way before the first product
+#pragma unroll
+        for (int e = 0; e < 16; ++e) c = Mf::mul(a[e], y[e], c);
+        return c;
+    };
+    auto copy = [&](const double (&from)[16], double (&to)[16]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) to[e] = from[e];
+    };
+    // barrier of the LDS traffic alone: loads stay in flight
+    auto barrier_lds = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    };
+    const int j = LEFT ? 0 : t % C, i0 = LEFT ? t : t / C;   // this thread's elements of B: rows i0 + 16 u, or column u
+    auto element = [&](int u) __attribute__((always_inline)) {
+        return LEFT ? min(i0, rows - 1) + (j0 + min(u, nc - 1)) * ldb : j0 + min(j, nc - 1) + min(i0 + 16 * u, rows - 1) * ldb;
+    };
+    double b[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) b[u] = B[element(u)];
+    double cur[16], nxt[16];
+    load_v(BWD ? nsb - 1 : 0, 0, cur);
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
-        const int e = t + u * 256;
-        const int x = e % 64, y = e / 64;
-        out[x + ld * y] = x <= y ? D[(63 - y) * L + 63 - x] : 0.0;
+        const int i = LEFT ? i0 : i0 + 16 * u;
+        xs[i * LX + (LEFT ? u : j)] = FULL || i < rows ? b[u] : 0.0;
+    }
+    __syncthreads();
+    const int own = (w * 16 + lk) * LX + li;                 // this lane's element of a block's rows, + 4 LX r
+    // Rolled (unrolled, the code of the 18 products took longer to fetch than
+    // to run: 25 us), the operands of the next product in flight
+#pragma unroll 1
+    for (int s = 0; s < nsb; ++s) {
+        const int p = BWD ? nsb - 1 - s : s;
+        double* xp = xs + p * 64 * LX;
+        const Mf::acc zero = {0, 0, 0, 0};
+        Mf::acc r = zero;
+#pragma unroll 1
+        for (int u = 0; u < s; ++u) {
+            const int q = BWD ? nsb - 1 - u : u;
+            if (u + 1 < s) load_m(p, BWD ? q - 1 : q + 1, nxt);
+            else load_v(p, 0, nxt);
+            r = product(cur, xs + q * 64 * LX, r);
+            copy(nxt, cur);
+        }
+        load_v(p, 4096, nxt);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            r[k] = xp[own + 4 * LX * k] - r[k];
+            rs[own + 4 * LX * k] = r[k];
+        }
+        barrier_lds();
+        Mf::acc x = product(cur, rs, zero);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) xp[own + 4 * LX * k] = x[k];
+        barrier_lds();
+        const Mf::acc m = product(nxt, xp, zero);
+        if (s + 1 < nsb) load_m(BWD ? p - 1 : p + 1, BWD ? nsb - 1 : 0, nxt);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) rs[own + 4 * LX * k] = r[k] - m[k];
+        barrier_lds();
+        x = product(cur, rs, x);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) xp[own + 4 * LX * k] = x[k];
+        copy(nxt, cur);
+        barrier_lds();
+    }
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        const int i = LEFT ? i0 : i0 + 16 * u, c = LEFT ? u : j;
+        if ((FULL || i < rows) && c < nc) B[element(u)] = xs[i * LX + c];
     }
 }
 
@@ -258,6 +387,19 @@ static int trsm_right_upper(oxi_handle_t h, hipStream_t s, int trans, int unit, 
                             inv ? inv + (hh / TRL) * 4096 : nullptr);
 }
 
+template <bool UPPER, bool CLEAN>
+static void launch_inv64(hipStream_t s, int trans, int unit, i64 n, const double* T, i64 ldt, double* inv, i64 ldv = 64,
+                         int strip = 0) {
+    const dim3 grid(unsigned(cdiv(n, TRL))), block(256);
+    if (unit) {
+        if (trans) hipLaunchKernelGGL((trsm_inv64_kernel<true, true, UPPER, CLEAN>), grid, block, 0, s, T, ldt, n, inv, ldv, strip);
+        else hipLaunchKernelGGL((trsm_inv64_kernel<true, false, UPPER, CLEAN>), grid, block, 0, s, T, ldt, n, inv, ldv, strip);
+    } else {
+        if (trans) hipLaunchKernelGGL((trsm_inv64_kernel<false, true, UPPER, CLEAN>), grid, block, 0, s, T, ldt, n, inv, ldv, strip);
+        else hipLaunchKernelGGL((trsm_inv64_kernel<false, false, UPPER, CLEAN>), grid, block, 0, s, T, ldt, n, inv, ldv, strip);
+    }
+}
+
 // Tall right-side solves (FP64, rows >= 1024, n a multiple of 64): the
 // diagonal blocks' inverses first, then the recursion with in-place products
 // for the leaves (a leaf's column sweep is a chain of 64 dependent steps per
@@ -265,14 +407,7 @@ static int trsm_right_upper(oxi_handle_t h, hipStream_t s, int trans, int unit, 
 static const double* right_upper_inverses(oxi_handle_t h, hipStream_t s, int trans, int unit, i64 rows, i64 n,
                                           const double* T, i64 ldt) {
     if (rows < 1024 || n < TRL || n % TRL || n / TRL > TRSM_INV_BLOCKS || !h->trsm_inv) return nullptr;
-    const dim3 grid(unsigned(n / TRL)), block(256);
-    if (unit) {
-        if (trans) hipLaunchKernelGGL((trsm_inv64_kernel<true, true>), grid, block, 0, s, T, ldt, h->trsm_inv);
-        else hipLaunchKernelGGL((trsm_inv64_kernel<true, false>), grid, block, 0, s, T, ldt, h->trsm_inv);
-    } else {
-        if (trans) hipLaunchKernelGGL((trsm_inv64_kernel<false, true>), grid, block, 0, s, T, ldt, h->trsm_inv);
-        else hipLaunchKernelGGL((trsm_inv64_kernel<false, false>), grid, block, 0, s, T, ldt, h->trsm_inv);
-    }
+    launch_inv64<true, false>(s, trans, unit, n, T, ldt, h->trsm_inv);
     return hipGetLastError() == hipSuccess ? h->trsm_inv : nullptr;
 }
 
@@ -281,26 +416,65 @@ template <typename TY>
 static int trsm_right_lower(oxi_handle_t h, hipStream_t s, int trans, int unit, i64 rows, i64 n, const TY* T,
                             i64 ldt, TY* X, i64 ldx);
 
-// Left solves with many right-hand sides (FP64, m a multiple of 64 and at
-// most 64 * TRSM_INV_BLOCKS rows): the inverses of op(A)'s 64 x 64 diagonal
-// blocks first, so that every leaf of the recursion is one in-place product
-// on the matrix cores instead of a column sweep per right-hand side.  For an
-// upper op(A) the kernel gives V_b = op(A)_bb^-1; for a lower op(A) it gives
-// V_b = (op(A)_bb^T)^-1 and the leaf multiplies by V_b^T.
-static const double* left_inverses(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit, i64 m, i64 nrhs,
-                                   const double* A, i64 lda) {
-    if (m < 2 * TRL || m % TRL || m / TRL > TRSM_INV_BLOCKS || nrhs < 16 || !h->trsm_inv) return nullptr;
-    const bool lower_op = (!upper) != (trans != 0);
-    const bool ktrans = lower_op ? !trans : (trans != 0);
-    const dim3 grid(unsigned(m / TRL)), block(256);
-    if (unit) {
-        if (ktrans) hipLaunchKernelGGL((trsm_inv64_kernel<true, true>), grid, block, 0, s, A, lda, h->trsm_inv);
-        else hipLaunchKernelGGL((trsm_inv64_kernel<true, false>), grid, block, 0, s, A, lda, h->trsm_inv);
-    } else {
-        if (ktrans) hipLaunchKernelGGL((trsm_inv64_kernel<false, true>), grid, block, 0, s, A, lda, h->trsm_inv);
-        else hipLaunchKernelGGL((trsm_inv64_kernel<false, false>), grid, block, 0, s, A, lda, h->trsm_inv);
+// Solves with FP64 triangles of n >= 128 rows, `other` (>= 16) right-hand
+// sides (columns of B on the left side, rows on the right), in place: by
+// halves down to blocks of SB rows, which are one launch of trsm_block_kernel
+// each, the updates one product each.  (Right-looking over the blocks took the
+// same time, but rounds an element once per block before it instead of once
+// per level: error against 64 bits 3.4e-16 instead of 2.8e-16 at 2048 x 2048.)
+// 2048 x 2048: 437 us by a recursion down to in-place products with 64 x 64
+// inverses, 393 so; 2001 x 1999, whose 64-row leaves were column sweeps: 897
+// and 395.  Bound by the chain of blocks and the smaller updates.
+static int trsm_blocked(oxi_handle_t h, hipStream_t s, bool left, int upper, int trans, int unit, i64 n, i64 other,
+                        const double* A, i64 lda, double* B, i64 ldb) {
+    const bool lower_op = (!upper) != (trans != 0);   // op(A) lower?
+    const bool ascending = left == lower_op;
+    // M of the block kernel: op(A) on the left side, op(A)^T on the right
+    const bool mt = left == (trans != 0), bwd = !ascending;
+    // rows (left) or columns (right) of B from i on
+    auto at = [&](i64 i) { return left ? B + i : B + i * ldb; };
+    const i64 most = i64(TRSM_INV_BLOCKS) / 2 * TRL;  // rows whose blocks and inverses fit the handle's buffer
+    i64 inv0 = -1;                                    // first row of those in it
+    auto block = [&](i64 b0, i64 nb) -> int {
+        const dim3 grid(unsigned(cdiv(other, 16))), bl(256);
+        const double* Ab = A + b0 * (lda + 1);
+        const double* Vb = h->trsm_inv + (b0 - inv0) / TRL * 8192;
+#define OXI_BLOCK(L, M, W)                                                                                           \
+    if (left == L && mt == M && bwd == W) {                                                                          \
+        if (nb == SB) hipLaunchKernelGGL((trsm_block_kernel<L, M, W, true>), grid, bl, 0, s, Ab, lda, Vb, at(b0), ldb, int(nb), other); \
+        else hipLaunchKernelGGL((trsm_block_kernel<L, M, W, false>), grid, bl, 0, s, Ab, lda, Vb, at(b0), ldb, int(nb), other); \
     }
-    return hipGetLastError() == hipSuccess ? h->trsm_inv : nullptr;
+        OXI_BLOCK(true, false, false) OXI_BLOCK(true, false, true) OXI_BLOCK(true, true, false) OXI_BLOCK(true, true, true)
+        OXI_BLOCK(false, false, false) OXI_BLOCK(false, false, true) OXI_BLOCK(false, true, false) OXI_BLOCK(false, true, true)
+#undef OXI_BLOCK
+        return launch_check(h, "trsm block");
+    };
+    // rows [i, i + ni) of B -= op(A)[i.., k..] X, X rows [k, k + nk) (columns on the right side)
+    auto update = [&](i64 i, i64 ni, i64 k, i64 nk) -> int {
+        const i64 r = left ? i : k, c = left ? k : i;   // op(A) from element (r, c) on
+        const double* Ar = trans ? A + c + r * lda : A + r + c * lda;
+        if (left) return oxi_launch_dgemm(h, s, trans ? 1 : 0, 0, ni, other, nk, -1.0, Ar, lda, at(k), ldb, 1.0, at(i), ldb);
+        return oxi_launch_dgemm(h, s, 0, trans ? 1 : 0, other, ni, nk, -1.0, at(k), ldb, Ar, lda, 1.0, at(i), ldb);
+    };
+    auto solve = [&](auto& self, i64 i, i64 ni) -> int {
+        const bool fill = inv0 < 0 && ni <= most;
+        if (fill) {
+            inv0 = i;
+            if (bwd) launch_inv64<true, true>(s, mt, unit, ni, A + i * (lda + 1), lda, h->trsm_inv);
+            else launch_inv64<false, true>(s, mt, unit, ni, A + i * (lda + 1), lda, h->trsm_inv);
+        }
+        if (ni <= SB) {
+            OXI_TRY(block(i, ni));
+        } else {
+            const i64 hh = cdiv(ni / 2, SB) * SB, i1 = i + hh, n1 = ni - hh;
+            OXI_TRY(ascending ? self(self, i, hh) : self(self, i1, n1));
+            OXI_TRY(ascending ? update(i1, n1, i, hh) : update(i, hh, i1, n1));
+            OXI_TRY(ascending ? self(self, i1, n1) : self(self, i, hh));
+        }
+        if (fill) inv0 = -1;
+        return OXI_OK;
+    };
+    return solve(solve, 0, n);
 }
 
 // Left solves with a moderate number of right-hand sides on large triangles
@@ -312,15 +486,16 @@ static const double* left_inverses(oxi_handle_t h, hipStream_t s, int upper, int
 // inverse, then B_rest -= op(A)[rest, b] X_b, whose rows spread over the
 // chip.  The TRB x TRB inverses come from the 64 x 64 ones by doubling: for
 // U = [U11 U12; 0 U22], U^-1 = [V11, -V11 U12 V22; 0, V22], two batched
-// products per doubling and position.  As in the 64 x 64 leaves, each
-// block's solve is a product with its inverse rather than a substitution.
+// products per doubling and position.  (trsm_block_kernel's 22 us a block
+// are hidden only by updates of more right-hand sides: 4096 x 100 486 us so
+// and 610 with it, 8192 x 128 901 and 1008, 4096 x 512 587 and 615.)
 constexpr int TRB = 256, TRB_MAX_RHS = 512;
 
-static bool left_blocked_applies(i64 m, i64 nrhs) {
+static bool left_strip_applies(i64 m, i64 nrhs) {
     return m >= 2 * TRB && m % TRB == 0 && nrhs >= 16 && nrhs <= TRB_MAX_RHS;
 }
 
-static int trsm_left_blocked(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit, i64 m, i64 nrhs,
+static int trsm_left_strip(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit, i64 m, i64 nrhs,
                              const double* A, i64 lda, double* B, i64 ldb) {
     const bool lower_op = (!upper) != (trans != 0);   // op(A) lower?
     // the upper matrix U' whose inverse the kernels build: U' = op(A) for an
@@ -335,14 +510,7 @@ static int trsm_left_blocked(oxi_handle_t h, hipStream_t s, int upper, int trans
     double* T = S + sS;
     double* X = T + sT;
     if (oxi_launch_dscale(s, m, TRB, 0.0, S, m) != OXI_OK) return oxi_set_error(h, OXI_ERR_HIP, "trsm strip clear");
-    const dim3 grid(unsigned(m / TRL)), block(256);
-    if (unit) {
-        if (ktrans) hipLaunchKernelGGL((trsm_inv64_kernel<true, true>), grid, block, 0, s, A, lda, S, m, TRB);
-        else hipLaunchKernelGGL((trsm_inv64_kernel<true, false>), grid, block, 0, s, A, lda, S, m, TRB);
-    } else {
-        if (ktrans) hipLaunchKernelGGL((trsm_inv64_kernel<false, true>), grid, block, 0, s, A, lda, S, m, TRB);
-        else hipLaunchKernelGGL((trsm_inv64_kernel<false, false>), grid, block, 0, s, A, lda, S, m, TRB);
-    }
+    launch_inv64<true, false>(s, ktrans, unit, m, A, lda, S, m, int(TRB));
     OXI_TRY(launch_check(h, "trsm block inverses"));
     const i64 nz = m / TRB;
     for (i64 w = TRL; w < TRB; w *= 2) {
@@ -386,16 +554,9 @@ static int trsm_left_blocked(oxi_handle_t h, hipStream_t s, int upper, int trans
 
 template <typename TY>
 static int trsm_left_t(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit, i64 m, i64 nrhs, const TY* A,
-                       i64 lda, TY* B, i64 ldb, const double* inv = nullptr) {
+                       i64 lda, TY* B, i64 ldb) {
     if (m <= 0 || nrhs <= 0) return OXI_OK;
     const bool lower_op = (!upper) != (trans != 0);  // op(A) lower?
-    if constexpr (sizeof(TY) == 8) {
-        if (inv && m == TRL) {
-            if (oxi_dgemm_left64_inplace(s, lower_op ? 1 : 0, nrhs, inv, (double*)B, ldb) != OXI_OK)
-                return oxi_set_error(h, OXI_ERR_HIP, "trsm in-place block product launch failed");
-            return OXI_OK;
-        }
-    }
     if (m <= TRL) {
         dim3 grid(unsigned(cdiv(nrhs, 4)));
         if (lower_op) {
@@ -412,19 +573,18 @@ static int trsm_left_t(oxi_handle_t h, hipStream_t s, int upper, int trans, int 
     // op(A) = [A11 A12; A21 A22] in op coordinates; op(A)[i][j] = trans ? A[j][i] : A[i][j]
     const TY* A11 = A;
     const TY* A22 = A + hh + hh * lda;
-    const double* inv2 = inv ? inv + (hh / TRL) * 4096 : nullptr;   // the blocks of A22
     if (lower_op) {
-        OXI_TRY(trsm_left_t(h, s, upper, trans, unit, hh, nrhs, A11, lda, B, ldb, inv));
+        OXI_TRY(trsm_left_t(h, s, upper, trans, unit, hh, nrhs, A11, lda, B, ldb));
         // B2 -= op(A)[hh:, :hh] * B1 ; op(A)[hh][0] = trans ? A[0][hh] : A[hh][0]
         const TY* A21 = trans ? A + hh * lda : A + hh;
         OXI_TRY(gemm_t<TY>(h, s, trans, 0, m - hh, nrhs, hh, TY(-1), A21, lda, B, ldb, TY(1), B + hh, ldb));
-        return trsm_left_t(h, s, upper, trans, unit, m - hh, nrhs, A22, lda, B + hh, ldb, inv2);
+        return trsm_left_t(h, s, upper, trans, unit, m - hh, nrhs, A22, lda, B + hh, ldb);
     }
-    OXI_TRY(trsm_left_t(h, s, upper, trans, unit, m - hh, nrhs, A22, lda, B + hh, ldb, inv2));
+    OXI_TRY(trsm_left_t(h, s, upper, trans, unit, m - hh, nrhs, A22, lda, B + hh, ldb));
     // B1 -= op(A)[:hh, hh:] * B2 ; op(A)[0][hh] = trans ? A[hh][0] : A[0][hh]
     const TY* A12 = trans ? A + hh : A + hh * lda;
     OXI_TRY(gemm_t<TY>(h, s, trans, 0, hh, nrhs, m - hh, TY(-1), A12, lda, B + hh, ldb, TY(1), B, ldb));
-    return trsm_left_t(h, s, upper, trans, unit, hh, nrhs, A11, lda, B, ldb, inv);
+    return trsm_left_t(h, s, upper, trans, unit, hh, nrhs, A11, lda, B, ldb);
 }
 
 // Right-side solve with op(T) lower: X <- X * op(T)^-1.  op(T) = [L11 0; L21 L22]:
@@ -458,14 +618,16 @@ static int trsm_right_t(oxi_handle_t h, hipStream_t s, int upper, int trans, int
 }
 
 
+// From 128 rows and 16 right-hand sides: below, the sweeps' launches are as few.
+static bool blocked_applies(oxi_handle_t h, i64 n, i64 other) { return n >= 2 * TRL && other >= 16 && h->trsm_inv; }
+
 int oxi_dtrsm_left(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit, i64 m, i64 nrhs, const double* A,
                    i64 lda, double* B, i64 ldb) {
-    static const bool blocked = !getenv("OXIBLAS_TRSM_RECURSIVE");   // tuning: the recursion throughout
-    if (blocked && left_blocked_applies(m, nrhs))
-        return trsm_left_blocked(h, s, upper, trans, unit, m, nrhs, A, lda, B, ldb);
-    const double* inv = left_inverses(h, s, upper, trans, unit, m, nrhs, A, lda);
-    return trsm_left_t<double>(h, s, upper, trans, unit, m, nrhs, A, lda, B, ldb, inv);
+    if (left_strip_applies(m, nrhs)) return trsm_left_strip(h, s, upper, trans, unit, m, nrhs, A, lda, B, ldb);
+    if (blocked_applies(h, m, nrhs)) return trsm_blocked(h, s, true, upper, trans, unit, m, nrhs, A, lda, B, ldb);
+    return trsm_left_t<double>(h, s, upper, trans, unit, m, nrhs, A, lda, B, ldb);
 }
+// Inside a factorization (rows of B below its panel), on either of its streams.
 int oxi_dtrsm_right(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit, i64 m, i64 n, const double* A,
                     i64 lda, double* B, i64 ldb) {
     return trsm_right_t<double>(h, s, upper, trans, unit, m, n, A, lda, B, ldb);
@@ -532,6 +694,7 @@ extern "C" int oxi_dtrsm(oxi_handle_t h, char side, char uplo, char trans, char 
     }
     if (alpha != 1.0) OXI_TRY(oxi_launch_dscale(s, m, n, alpha, B, ldb));
     if (left) return oxi_dtrsm_left(h, s, upper, tk, unit, m, n, A, lda, B, ldb);
+    if (blocked_applies(h, n, m)) return trsm_blocked(h, s, false, upper, tk, unit, n, m, A, lda, B, ldb);
     return oxi_dtrsm_right(h, s, upper, tk, unit, m, n, A, lda, B, ldb);
 }
 

@@ -97,3 +97,40 @@ def test_block_inverse_solves(gpu, rng, n, nrhs):
         X = F32.solve(np.asfortranarray(B.astype(np.float32)), t)
         X = X.numpy() if hasattr(X, "numpy") else X
         residual((A if t == "N" else A.T).astype(np.float32).astype(float), X.astype(float), np.finfo(np.float32).eps)
+
+
+# Blocks of 256 rows, full ones and a last one of fewer, on either side, against
+# op(A) X = B (X op(A) = B): a backward error of at most 8 n eps, blocks well
+# conditioned; 8400 rows are more than the buffer of block inverses holds.
+@pytest.mark.parametrize("side,uplo,trans,diag", list(itertools.product("LR", "UL", "NT", "NU")))
+@pytest.mark.parametrize("n,other", [(129, 16), (191, 40), (512, 16), (513, 33), (600, 17), (640, 300), (1023, 129)])
+def test_trsm_blocked_edges(gpu, side, uplo, trans, diag, n, other):
+    _blocked(gpu, side, uplo, trans, diag, n, other)
+
+
+@pytest.mark.parametrize("side", "LR")
+@pytest.mark.parametrize("uplo", "LU")
+def test_trsm_blocked_large(gpu, side, uplo):
+    _blocked(gpu, side, uplo, "N", "N", 8400, 24)
+
+
+def _blocked(gpu, side, uplo, trans, diag, n, other):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n + other)
+    ld = n + 3
+    A = torch.randn(n, ld, dtype=torch.float64, device="cuda", generator=g) / n      # A[c][r]; the other triangle is noise
+    A[:, :n].diagonal().copy_(1.0 + torch.rand(n, dtype=torch.float64, device="cuda", generator=g))
+    m, k = (n, other) if side == "L" else (other, n)
+    B = torch.randn(k, m + 1, dtype=torch.float64, device="cuda", generator=g)
+    B0 = B.clone()
+    gpu.trsm_(gpu.DMatrix(B.view(-1), m, k, m + 1), gpu.DMatrix(A.view(-1), n, n, ld), side=side, uplo=uplo, trans=trans,
+              unit=diag == "U")
+    T = A[:, :n].T
+    T = torch.tril(T) if uplo == "L" else torch.triu(T)
+    if diag == "U":
+        T = T - torch.diag(T.diagonal()) + torch.eye(n, dtype=torch.float64, device="cuda")
+    T = (T.T if trans == "T" else T).contiguous()
+    X, R = B[:, :m].T.contiguous(), B0[:, :m].T
+    r = (T @ X if side == "L" else X @ T) - R
+    assert r.norm() <= 8 * n * EPS * (T.norm() * X.norm() + R.norm())
+    assert torch.equal(B[:, m], B0[:, m])
