@@ -21,35 +21,42 @@
 // had published.)  (Inverting the diagonal blocks changes the rounding
 // of a substitution, not the result beyond it; the solve is deterministic.)
 //
-// The solve: a workgroup per block and group of CR = 32 right-hand sides
+// The solve: a workgroup per block and group of CR = 16 right-hand sides
 // (the groups are independent chains, one `ready` counter each).
 // Workgroups take their (block, group) from an atomic ticket, so a
 // workgroup only ever waits on workgroups that are already running.  Each
-// of its four waves owns 16 rows of the block and both 16-column tiles of
-// the group: every product is 2 x 16 v_mfma_f64_16x16x4 per wave.  The
-// operands: the factor's blocks straight from memory (coalesced along the
-// rows), X of earlier blocks staged in LDS.  X goes between workgroups with
-// device-scope stores and loads; the publishing waves wait for their stores
-// to be acknowledged before `ready` moves.  Every wait is bounded: a
-// timeout sets a sticky error word, read by oxi_trsm_chain_check.
+// of its four waves owns 16 rows of the block: every product is 16
+// v_mfma_f64_16x16x4 per wave.  The operands: the factor's blocks straight
+// from memory, a block ahead of the X they wait for, X of earlier blocks
+// staged in LDS.  X goes between workgroups with device-scope stores and
+// loads; the publishing waves wait for their stores to be acknowledged before
+// `ready` moves.  Every wait is bounded: a timeout sets a sticky error word,
+// read by oxi_trsm_chain_check.
+//
+// Bound, at n = 8192 with 64 right-hand sides, by the factor's traffic while
+// many blocks sum (each chain reads it; 5 TB/s in the first half) and by the
+// hand-over of 128 blocks; 370 us a triangle.  Groups of 32: 455 (twice the
+// matrix work on the chain); without the block loaded ahead and the pairs of
+// k, transposed: 536.  X handed over as tagged words instead of by the counter:
+// 357, and 4 % slower with one right-hand side; groups of 32 with that: spills.
 #include "tri_inv.hpp"
 
 namespace {
 
 constexpr int CB = 64;       // rows per block
-constexpr int CR = 32;       // right-hand sides per workgroup
+constexpr int CR = 16;       // right-hand sides per workgroup
+constexpr int CT = CR / 16, XPT = CB * CR / 256;   // 16-column tiles; X elements per thread of a staged block
 constexpr int CNT = 256;     // threads per workgroup
-constexpr int XBC = 1;       // published blocks of X applied per round
 constexpr int CHAINS = OXI_CHAIN_MAX_RHS / CR;
 constexpr unsigned CSPIN_LIMIT = 1u << 20;
-static_assert(CNT == 4 * 64 && CB == 4 * 16 && CR == 2 * 16, "four waves of 16 rows, two 16-column tiles");
-static_assert(CB * CR == 8 * CNT, "eight X elements per thread per staged block");
+static_assert(CNT == 4 * 64 && CB == 4 * 16 && CR % 16 == 0, "four waves of 16 rows");
 
 // Control words: the ticket and the chains' counters (per launch), and the
 // error word, sticky across the launches of one solve.
 struct ChainCtrl { unsigned ticket, err, ready[CHAINS]; };
 
 typedef double d4v __attribute__((ext_vector_type(4)));
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));   // 16 bytes at any element
 
 __device__ __forceinline__ d4v mfma16(double a, double b, d4v c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
@@ -157,16 +164,16 @@ __device__ __forceinline__ double load_sc1(__amdgpu_buffer_rsrc_t r, unsigned of
 // Thread t's eight elements of an X block (rows q0 + t % CB, columns
 // t / CB + 4r of the group, clamped into the group's ncol columns): loads
 // only; the caller writes them to LDS.
-__device__ __forceinline__ void load_x(__amdgpu_buffer_rsrc_t r, i64 ldb, i64 q0, int ncol, int t, double (&v)[8]) {
+__device__ __forceinline__ void load_x(__amdgpu_buffer_rsrc_t r, i64 ldb, i64 q0, int ncol, int t, double (&v)[XPT]) {
     const int q = t % CB, jq = t / CB;
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
+    for (int u = 0; u < XPT; ++u)
         v[u] = load_sc1(r, unsigned((q0 + q + i64(min(jq + 4 * u, ncol - 1)) * ldb) * 8));
 }
-__device__ __forceinline__ void store_x(double (*xs)[CR + 1], int ncol, int t, const double (&v)[8]) {
+__device__ __forceinline__ void store_x(double (*xs)[CR + 1], int ncol, int t, const double (&v)[XPT]) {
     const int q = t % CB, jq = t / CB;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) xs[q][jq + 4 * u] = jq + 4 * u < ncol ? v[u] : 0.0;
+    for (int u = 0; u < XPT; ++u) xs[q][jq + 4 * u] = jq + 4 * u < ncol ? v[u] : 0.0;
 }
 
 // Wait until the chain's counter exceeds `need` (thread 0 polls, the block
@@ -203,7 +210,7 @@ __global__ __launch_bounds__(CNT, 2) void trsm_chain_kernel(const double* __rest
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     if (t == 0) s_tk = int(atomicAdd(&ctrl->ticket, 1u));
     __syncthreads();
-    const int b = s_tk / nchains, h = s_tk % nchains;
+    const int tk = __builtin_amdgcn_readfirstlane(s_tk), b = tk / nchains, h = tk % nchains;
     const int j0 = h * CR, ncol = min(CR, nrhs - j0);
     const int rows = int(min(i64(CB), n - i64(b) * CB));
     const i64 p0 = block_row0(BWD, n, b, rows);
@@ -211,17 +218,16 @@ __global__ __launch_bounds__(CNT, 2) void trsm_chain_kernel(const double* __rest
     // accumulator r of lane 16a + j holds D[4r + a][j]
     const int fi = lane & 15, fk = lane >> 4;
     const int ra = wave * 16 + fi;               // this lane's A-operand row in the block
-    const bool ra_ok = ra < rows;
-    d4v acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};   // sum over chunks, per column tile
-    d4v xb[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};    // X_b
+    d4v acc[CT] = {};                            // sum over chunks, per column tile
+    d4v xb[CT] = {};                             // X_b
     const __amdgpu_buffer_rsrc_t xr = x_rsrc(B, ldb, j0);
     // everything the block needs besides X of other blocks, loaded first so
     // that no memory round trip is left between the last published block
     // and this block's own X: its rows of B, and its operands of V_b, H_b
     // and G_b (read-only here)
-    double bb[2][4], av[16], ah[16], ag[16];
+    double bb[CT][4], av[16], ah[16], ag[16];
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct)
+    for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int row = wave * 16 + 4 * r + fk, col = ct * 16 + fi;
@@ -239,54 +245,52 @@ __global__ __launch_bounds__(CNT, 2) void trsm_chain_kernel(const double* __rest
         }
     }
 
-    // 1. sum over the blocks c < b - 2 as they are published, up to XBC
-    // published blocks per round, their X and factor blocks loaded together
-    // (more than one per round measured no faster: the workgroups keep up)
+    // 1. sum over the blocks c < b - 2 as they are published, one a round; the
+    // factor's block of the next round is loaded during this one's products
+    // (it does not wait for X).  TRANS: the factor is contiguous along k, so a
+    // lane takes pairs of k (16-byte loads, 64 contiguous bytes a column and
+    // instruction instead of 32), and the products their k in that order.
     int avail = 0;
     const int cend = b - 2;
-    for (int c = 0; c < cend;) {
+    const i64 prow = p0 + min(ra, rows - 1);
+    auto kof = [&](int s) __attribute__((always_inline)) { return TRANS ? 8 * (s / 2) + 2 * fk + s % 2 : 4 * s + fk; };
+    auto load_block = [&](int c, double (&a)[16]) __attribute__((always_inline)) {
+        const i64 q0 = block_row0(BWD, n, c, CB);
+        if (TRANS) {
+#pragma unroll
+            for (int s = 0; s < 16; s += 2) {
+                const d2u v = *(const d2u*)(M + q0 + kof(s) + prow * ld);
+                a[s] = v[0];
+                a[s + 1] = v[1];
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < 16; ++s) a[s] = M[prow + (q0 + kof(s)) * ld];
+        }
+    };
+    double ak[16];
+    if (cend > 0) load_block(0, ak);
+    for (int c = 0; c < cend; ++c) {
         if (c >= avail) {
             avail = wait_ready(ctrl, h, c, t, &s_ready);
             if (avail < 0) return;
         }
-        const int nbat = min(min(avail, cend) - c, XBC);
-        double ak[XBC][16];
-        {
-            double v[XBC][8];
-#pragma unroll
-            for (int k = 0; k < XBC; ++k) {
-                if (k < nbat) {
-                    const i64 q0 = block_row0(BWD, n, c + k, CB);
-                    load_x(xr, ldb, q0, ncol, t, v[k]);
-#pragma unroll
-                    for (int s = 0; s < 16; ++s)
-                        ak[k][s] = !ra_ok ? 0.0
-                                          : TRANS ? M[(q0 + 4 * s + fk) + (p0 + ra) * ld]
-                                                  : M[(p0 + ra) + (q0 + 4 * s + fk) * ld];
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < XBC; ++k)
-                if (k < nbat) store_x(xs[k], ncol, t, v[k]);
-        }
+        double v[XPT], an[16];
+        load_x(xr, ldb, block_row0(BWD, n, c, CB), ncol, t, v);
+        load_block(min(c + 1, cend - 1), an);
+        store_x(xs[0], ncol, t, v);
         __syncthreads();
 #pragma unroll
-        for (int k = 0; k < XBC; ++k) {
-            if (k < nbat) {
+        for (int s = 0; s < 16; ++s)
 #pragma unroll
-                for (int s = 0; s < 16; ++s) {
-                    acc[0] = mfma16(ak[k][s], xs[k][4 * s + fk][fi], acc[0]);
-                    acc[1] = mfma16(ak[k][s], xs[k][4 * s + fk][16 + fi], acc[1]);
-                }
-            }
-        }
+            for (int ct = 0; ct < CT; ++ct) acc[ct] = mfma16(ak[s], xs[0][kof(s)][16 * ct + fi], acc[ct]);
         __syncthreads();   // xs is refilled next
-        c += nbat;
+#pragma unroll
+        for (int s = 0; s < 16; ++s) ak[s] = an[s];
     }
-
     // 2. rs = B_b - sum, then X_b = V_b rs
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct)
+    for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int row = wave * 16 + 4 * r + fk, col = ct * 16 + fi;
@@ -295,8 +299,7 @@ __global__ __launch_bounds__(CNT, 2) void trsm_chain_kernel(const double* __rest
     __syncthreads();
 #pragma unroll
     for (int s = 0; s < 16; ++s) {
-        xb[0] = mfma16(av[s], rs[4 * s + fk][fi], xb[0]);
-        xb[1] = mfma16(av[s], rs[4 * s + fk][16 + fi], xb[1]);
+        for (int ct = 0; ct < CT; ++ct) xb[ct] = mfma16(av[s], rs[4 * s + fk][16 * ct + fi], xb[ct]);
     }
 
     // 3. X_b -= H_b X_{b-2}, then X_b -= G_b X_{b-1}: the products that
@@ -308,15 +311,14 @@ __global__ __launch_bounds__(CNT, 2) void trsm_chain_kernel(const double* __rest
             if (avail < 0) return;
         }
         {
-            double v[8];
+            double v[XPT];
             load_x(xr, ldb, block_row0(BWD, n, b - 2, CB), ncol, t, v);
             store_x(xs[0], ncol, t, v);
         }
         __syncthreads();
 #pragma unroll
         for (int s = 0; s < 16; ++s) {
-            xb[0] = mfma16(ah[s], xs[0][4 * s + fk][fi], xb[0]);
-            xb[1] = mfma16(ah[s], xs[0][4 * s + fk][16 + fi], xb[1]);
+            for (int ct = 0; ct < CT; ++ct) xb[ct] = mfma16(ah[s], xs[0][4 * s + fk][16 * ct + fi], xb[ct]);
         }
     }
     if (b > 0) {
@@ -327,21 +329,20 @@ __global__ __launch_bounds__(CNT, 2) void trsm_chain_kernel(const double* __rest
             __syncthreads();   // every wave has finished the V_b product: xs[1] is free
         }
         {
-            double v[8];
+            double v[XPT];
             load_x(xr, ldb, block_row0(BWD, n, b - 1, CB), ncol, t, v);
             store_x(xs[1], ncol, t, v);
         }
         __syncthreads();
 #pragma unroll
         for (int s = 0; s < 16; ++s) {
-            xb[0] = mfma16(ag[s], xs[1][4 * s + fk][fi], xb[0]);
-            xb[1] = mfma16(ag[s], xs[1][4 * s + fk][16 + fi], xb[1]);
+            for (int ct = 0; ct < CT; ++ct) xb[ct] = mfma16(ag[s], xs[1][4 * s + fk][16 * ct + fi], xb[ct]);
         }
     }
 
     // 4. X_b to B, acknowledged, then the chain's counter
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct)
+    for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int row = wave * 16 + 4 * r + fk, col = ct * 16 + fi;
