@@ -13,7 +13,7 @@
 // column in a device word and stops; later leaves see the word and do
 // nothing, so the first failing column is the one reported (the reference's
 // PosDefException(j) / info).
-#include "oxi_internal.hpp"
+#include "tri_inv.hpp"
 
 #include <algorithm>
 #include <cstdlib>
@@ -23,8 +23,6 @@ namespace {
 
 constexpr int CLEAF = 64;
 
-__device__ __forceinline__ double sqrt_t(double v) { return __builtin_sqrt(v); }
-__device__ __forceinline__ float sqrt_t(float v) { return __builtin_sqrtf(v); }
 __device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
 __device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 template <typename T> __device__ __forceinline__ bool pos_finite(T d);
@@ -71,104 +69,139 @@ __device__ __forceinline__ void static_for(F&& f) {
     }
 }
 
+// r = sqrt(d) and q = x / r, d the same in every lane.  In FP64, where nothing
+// can overflow or lose bits on the way, the reciprocal that the square root's
+// Newton steps carry along also serves the division, whose result its residual
+// corrects: 14 dependent operations instead of the two library sequences' 40.
+__device__ __forceinline__ void sqrt_div(double d, double x, double& r, double& q) {
+    const double y = __builtin_amdgcn_rsq(d);
+    double g = d * y, h = 0.5 * y;
+    const double e = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, e, g);
+    h = __builtin_fma(h, e, h);
+    g = __builtin_fma(__builtin_fma(-g, g, d), h, g);
+    r = __builtin_fma(__builtin_fma(-g, g, d), h, g);
+    double z = 2.0 * h;
+    z = __builtin_fma(z, __builtin_fma(-r, z, 1.0), z);
+    const double t = x * z;
+    q = __builtin_fma(__builtin_fma(-t, r, x), z, t);
+    if (!(d > 0x1p-500 && d < 0x1p500)) {
+        r = __builtin_sqrt(d);
+        q = x / r;
+    }
+}
+__device__ __forceinline__ void sqrt_div(float d, float x, float& r, float& q) {
+    r = __builtin_sqrtf(d);
+    q = x / r;
+}
+
 // A (n x n, n <= 64, lower triangle) in place; `off` is the global index of
 // its first column; *info receives off + c + 1 at the first failing column c.
-// One wave: lane i holds row i in registers.  The registers rotate by one per
-// column, so the loop is rolled with compile-time register indices (unrolled
-// over the columns its code is as large as the instruction cache and is
-// fetched anew by every launch).  Per column j: the pivot from lane j, its
-// square root r, every lane's multiplier l_ij = a_ij / r; the update of the
-// other columns, a_ik = fma(-l_ij, l_kj, a_ik), takes l_kj from a copy of the
-// multipliers in LDS, spread so that a DPP broadcast brings one to every lane.
-// Column j + 1 is updated first, by a readlane, and the update that column j
-// leaves to the others comes after column j + 1's square root and division.
-// Elements right of the diagonal take the same operations on values nobody
-// stores.
+// One wave, panels of 16 columns: lane i holds row i of the panel in
+// registers, the block is in LDS, and the columns right of the panel take its
+// rank-16 update on the matrix cores, 16 x 16 blocks of the lower triangle.
+// In a panel the registers rotate by one per column, so the loop is rolled
+// with compile-time register indices (unrolled, its code is fetched anew by
+// every launch and takes longer than it runs).  Per column j: the pivot from
+// lane j, its square root r, every lane's multiplier l_ij = a_ij / r; the
+// update of the panel's other columns, a_ik = fma(-l_ij, l_kj, a_ik), takes
+// l_kj from the multipliers in LDS, spread so that a DPP broadcast brings one
+// to every lane.  Column j + 1 is updated first, by a readlane, and the update
+// that column j leaves to the others comes beside column j + 1's square root
+// and division.  Elements right of the diagonal take the same operations on
+// values nobody stores.
 // A failing pivot (not finite and positive) ends the updates: the columns
 // before it are final, the rest keep their updated values.
-// Bound by the 63 FMAs and broadcasts of a column in one wave (0.31 us a
-// column; laying the steps of the square root and the division among them
-// changed nothing): 31 us for 64 columns, launch and stores included, against
-// 41 for an unrolled form whose multipliers every lane read from LDS.
+// Bound by the chain of pivot, square root, division and next column: 24.7 us
+// for 64 columns, launch, loads and stores included, against 31 without panels
+// (63 FMAs and broadcasts a column in one wave) and 41 for that unrolled; with
+// the library's square root and division and readlanes for the multipliers 42.
 template <typename T>
 __global__ __launch_bounds__(64) void potrf_leaf_kernel(T* __restrict__ A, i64 lda, int n, i64 off,
                                                         i64* __restrict__ info) {
-    __shared__ T lcol[2 * CLEAF];             // the multipliers of a column, zeros behind them
+    typedef tri::Mfma<T> Mf;
+    constexpr int W = 16, L = CLEAF + 1;
+    __shared__ T S[CLEAF * L + W];              // S[k * L + i]: element (i, k); a done column: its multipliers
     if (*info != 0) return;                   // an earlier leaf failed
-    const int i = threadIdx.x;
-    T v[CLEAF];
-    const T* arow = A + min(i, n - 1);
-    if (n == CLEAF) {
+    const int i = threadIdx.x, lk = i >> 4, li = i & 15;
+    {
+        T a[CLEAF];
+        const int ic = min(i, n - 1);
+        const T* col = A;
 #pragma unroll
-        for (int k = 0; k < CLEAF; ++k) v[k] = arow[k * lda];
-    } else {
+        for (int k = 0; k < CLEAF; ++k) {
+            a[k] = col[ic];
+            col += k + 1 < n ? lda : 0;
+        }
 #pragma unroll
-        for (int k = 0; k < CLEAF; ++k) v[k] = k < n ? arow[k * lda] : T(0);
+        for (int k = 0; k < CLEAF; ++k) S[k * L + i] = a[k];
     }
-    lcol[CLEAF + i] = T(0);
+    if (n < CLEAF) {                          // beyond n the identity: pivots that pass and change nothing
+#pragma unroll 1
+        for (int k = 0; k < CLEAF; ++k)
+            if (i >= n || k >= n) S[k * L + i] = i == k ? T(1) : T(0);
+    }
+    __syncthreads();
     bool go = true;                           // uniform
     i64 failed = 0;
-    T x = v[0];                               // column j, updated through column j - 1
-    T l = T(0), lin = T(0), u[4] = {};        // column j - 1: multipliers, final values, multipliers spread
-    // the multipliers of column j from q = x / r, and column j + 1's values
-    auto column = [&](int j, T r, T q, bool ok) __attribute__((always_inline)) {
-        failed = go && !ok ? off + j + 1 : failed;
-        go = ok;
-        l = ok && i > j ? q : T(0);
-        lin = ok ? (i == j ? r : i > j ? q : x) : x;
-        lcol[i] = l;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // the lanes' LDS writes before the reads below
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int b = 0; b < 4; ++b) u[b] = lcol[j + 16 * b + (i & 15)];
-        x = fma_t(-l, readlane_t(l, min(j + 1, CLEAF - 1)), v[1]);
-        __builtin_amdgcn_wave_barrier();      // every read before the next column's writes
-    };
-    {
-        const T d = readlane_t(x, 0), r = sqrt_t(d);
-        column(0, r, x / r, pos_finite(d));
-    }
 #pragma unroll 1
-    for (int j0 = 1; j0 < n; ++j0) {
-        const int j = __builtin_amdgcn_readfirstlane(j0);
-        const T d = readlane_t(x, j);
-        const bool ok = go && pos_finite(d);
-        const T r = sqrt_t(d);
-        const T q = x / r;
-        // column j - 1's update of the others, with the rotation: register c
-        // holds column j + c afterwards
-        static_for<CLEAF / 4>([&](auto g_c) __attribute__((always_inline)) {
-            constexpr int G = 4 * decltype(g_c)::value;
-            T b[4];
-            static_for<4>([&](auto c_c) __attribute__((always_inline)) {
-                constexpr int C = G + decltype(c_c)::value;
-                if constexpr (C > 0) b[C - G] = row_bcast<C & 15>(u[C / 16]);
-            });
-            static_for<4>([&](auto c_c) __attribute__((always_inline)) {
-                constexpr int C = G + decltype(c_c)::value;
-                if constexpr (C > 0) v[C - 1] = nfma_to(l, b[C - G], v[C]);
-            });
-        });
-        v[CLEAF - 1] = lin;
-        column(j, r, q, ok);
-    }
-    // the last column's place, then the rest of the turn
-    {
+    for (int p = 0; p < n; p += W) {
+        T v[W + 1];                           // before column j: register c holds column j - 1 + c
+        v[0] = T(0);
 #pragma unroll
-        for (int c = 0; c + 1 < CLEAF; ++c) v[c] = v[c + 1];
-        v[CLEAF - 1] = lin;
-    }
+        for (int c = 0; c < W; ++c) v[c + 1] = S[(p + c) * L + i];
+        T x = v[1];                           // column j, updated through column j - 1
+        T l = T(0), u = T(0);                 // column j - 1's multipliers; those of rows j - 1 + (lane % 16)
 #pragma unroll 1
-    for (int k = n; k < CLEAF; ++k) {
-        const T first = v[0];
+        for (int j0 = p; j0 < p + W; ++j0) {
+            const int j = __builtin_amdgcn_readfirstlane(j0);
+            const T d = readlane_t(x, j);
+            const bool ok = go && pos_finite(d);
+            T r, q;
+            // column j - 1's update of the others, with the rotation: register
+            // c holds column j + c afterwards (those past the panel hold
+            // nothing; at column p the multipliers are zero)
+            static_for<W>([&](auto c_c) __attribute__((always_inline)) {
+                constexpr int C = decltype(c_c)::value + 1;
+                v[C - 1] = nfma_to(l, row_bcast<(C < W ? C : W - 1)>(u), v[C]);
+            });
+            sqrt_div(d, x, r, q);
+            failed = go && !ok ? off + j + 1 : failed;
+            go = ok;
+            l = ok && i > j ? q : T(0);
+            S[j * L + i] = l;
+            if (i < n && i >= j) A[i + j * lda] = !ok ? x : i == j ? r : q;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // the lanes' LDS writes before the read below
+            __builtin_amdgcn_wave_barrier();
+            u = S[j * L + j + li];
+            x = fma_t(-l, readlane_t(l, min(j + 1, CLEAF - 1)), v[1]);
+        }
+        __syncthreads();
+#pragma unroll 1
+        for (int tj = p + W; tj < n; tj += W) {
+            // block column tj: rows tj, tj + 16, .. together (rows from 64 on repeat the last)
+            typename Mf::acc c[CLEAF / W - 1];
+            T b[W / 4];
 #pragma unroll
-        for (int c = 0; c + 1 < CLEAF; ++c) v[c] = v[c + 1];
-        v[CLEAF - 1] = first;
+            for (int k = 0; k < W / 4; ++k) b[k] = S[(p + 4 * k + lk) * L + tj + li];
+#pragma unroll
+            for (int u = 0; u < CLEAF / W - 1; ++u) {
+                const int ti = min(tj + u * W, CLEAF - W);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) c[u][k] = S[(tj + li) * L + ti + Mf::row(lk, k)];
+#pragma unroll
+                for (int k = 0; k < W / 4; ++k) c[u] = Mf::mul(-S[(p + 4 * k + lk) * L + ti + li], b[k], c[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < CLEAF / W - 1; ++u)
+                if (tj + u * W < CLEAF) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) S[(tj + li) * L + tj + u * W + Mf::row(lk, k)] = c[u][k];
+                }
+        }
+        __syncthreads();
     }
     if (failed && i == 0) *info = failed;
-#pragma unroll
-    for (int k = 0; k < CLEAF; ++k)
-        if (i < n && k <= i) A[i + k * lda] = v[k];
 }
 
 // zero the strict upper triangle (the factor's storage contract)

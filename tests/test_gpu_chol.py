@@ -122,3 +122,40 @@ def test_cholesky_n8192(gpu):
     berr = torch.linalg.matrix_norm(R).item() / (torch.linalg.matrix_norm(A).item() *
                                                  torch.linalg.matrix_norm(Xt).item() * n * EPS)
     assert berr <= 30, berr
+
+
+# The leaf of 64 columns at the edges of its panels of 16, where its square
+# roots and divisions take their short form and (2^+-600) where they may not.
+# Componentwise error of a Cholesky factor: |L L^T - A| <= gamma_{n+1} |L| |L^T|,
+# 4 more for the square root and division.
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 31, 33, 48, 49, 63, 64, 65, 127])
+@pytest.mark.parametrize("e", [0, -600, 600])
+def test_potrf_leaf_edges(gpu, rng, n, e):
+    A = spd(rng, n) * 2.0 ** e
+    Au = A.copy(); Au[np.triu_indices(n, 1)] = np.nan
+    L = gpu.cholesky_factor(gpu.DMatrix.from_numpy(Au)).factors.numpy()
+    L, A = np.tril(L) * 2.0 ** (-e // 2), A * 2.0 ** -e
+    assert (np.abs(L @ L.T - A) <= (n + 5) * EPS * (np.abs(L) @ np.abs(L.T))).all()
+    d = np.exp(rng.uniform(-20, 20, n)) * 2.0 ** e
+    D = gpu.cholesky_factor(gpu.DMatrix.from_numpy(np.diag(d))).factors.numpy()
+    np.testing.assert_allclose(np.diag(D), np.sqrt(d), rtol=EPS, atol=0)
+    if n > 16 and e == 0:
+        b = rng.standard_normal(n)
+        x = gpu.mixed_solve(A, b, factorization="cholesky").x
+        x = x.numpy().ravel() if hasattr(x, "numpy") else np.ravel(x)
+        assert np.linalg.norm(A @ x - b) <= 1e-12 * (np.linalg.norm(A) * np.linalg.norm(x))
+
+
+@pytest.mark.parametrize("j", [0, 1, 14, 15, 16, 17, 31, 40, 62, 63])
+@pytest.mark.parametrize("bad", [-1.0, 0.0, np.nan, np.inf])
+def test_potrf_leaf_failing_column(gpu, rng, j, bad):
+    A = spd(rng, 64)
+    good = gpu.cholesky_factor(gpu.DMatrix.from_numpy(A)).factors.numpy()
+    if np.isfinite(bad):
+        A[j, j] = bad - (good[j, :j] ** 2).sum() * 0.5       # below what the columns before take off
+    else:
+        A[j, j] = bad
+    F = gpu.cholesky(gpu.DMatrix.from_numpy(A), check=False)
+    assert F.info == j + 1
+    got = F.factors.numpy()
+    assert np.array_equal(got[:, :j][np.tril_indices(64, 0, j)], good[:, :j][np.tril_indices(64, 0, j)])
