@@ -305,6 +305,77 @@ __global__ __launch_bounds__(256) void apply_pairs_w_kernel(T* __restrict__ Wm, 
         for (int q = q0; q < np; q += qs) Wm[c + (i64(pl[2 * q]) + roff) * ldw] = buf[q * PAIR_ROWS + r];
 }
 
+// The look-ahead block of a 64-column panel at column k1 in one launch: its
+// interchanges and U12 = L11^-1 A12 for the columns [c0, c1) of A (rows of W).
+// A wave takes one of them: it replays the 64 interchanges on indices (lane s:
+// where position k1 + s, and the row that step s reaches past the panel, take
+// their values from), fetches both, and solves with the unit triangle by a
+// column sweep, lane q = column q, in the operations and order of the TRSM's.
+// Every step p_s >= s (0-based, from k1), as LU pivots are.
+// Bound by three memory round trips and 64 dependent steps, twice; it stands on
+// the chain between two panels: 9.6 us for 64 columns in FP64, against 17 for
+// the pair list, its application and the TRSM, and two launches more (LU solve
+// n = 2000: 5.21 -> 5.01 ms).  The triangle goes through LDS: fetched by every
+// wave, a column a lane, 11.6 us.
+__device__ __forceinline__ double lane_of(double v, int l) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = __builtin_amdgcn_readlane(unsigned(u), l), hi = __builtin_amdgcn_readlane(unsigned(u >> 32), l);
+    return __builtin_bit_cast(double, (static_cast<unsigned long long>(hi) << 32) | lo);
+}
+__device__ __forceinline__ float lane_of(float v, int l) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(unsigned, v), l));
+}
+__device__ __forceinline__ double nfma(double a, double b, double c) { return __builtin_fma(-a, b, c); }
+__device__ __forceinline__ float nfma(float a, float b, float c) { return __builtin_fmaf(-a, b, c); }
+
+constexpr int SW = 64;
+template <typename T>
+__global__ __launch_bounds__(256) void swap_solve_kernel(T* __restrict__ Wm, i64 ldw, i64 k1,
+                                                         const i64* __restrict__ ipiv, i64 c0, i64 c1) {
+    __shared__ T U[SW * (SW + 1)];                    // U[q * (SW + 1) + s] = L11^T(s, q)
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const bool mine = c0 + i64(blockIdx.x) * 4 + w < c1;
+    const i64 c = mine ? c0 + i64(blockIdx.x) * 4 + w : c0;
+    const int p = int(ipiv[k1 + lane] - 1 - k1);
+    T d[SW / 4];                                      // columns w, w + 4, .. of the triangle
+#pragma unroll
+    for (int i = 0; i < SW / 4; ++i) d[i] = Wm[k1 + lane + (k1 + w + 4 * i) * ldw];
+    int first = lane;                                 // the first step that reaches the same row
+#pragma unroll 8
+    for (int s = SW - 1; s >= 0; --s) first = __builtin_amdgcn_readlane(p, s) == p ? s : first;
+    int xi = lane, ei = p;                            // sources of position k1 + lane, and of row k1 + p (lane = first)
+#pragma unroll 4
+    for (int s = 0; s < SW; ++s) {
+        const int ps = __builtin_amdgcn_readlane(p, s), a = __builtin_amdgcn_readlane(xi, s);
+        int b;
+        if (ps < SW) {
+            b = __builtin_amdgcn_readlane(xi, ps);
+            xi = lane == ps ? a : xi;
+        } else {
+            const int f = __builtin_amdgcn_readlane(first, s);
+            b = __builtin_amdgcn_readlane(ei, f);
+            ei = lane == f ? a : ei;
+        }
+        xi = lane == s ? b : xi;
+    }
+    T x = Wm[c + (k1 + xi) * ldw];
+    const T y = Wm[c + (k1 + ei) * ldw];
+#pragma unroll
+    for (int i = 0; i < SW / 4; ++i) U[(w + 4 * i) * (SW + 1) + lane] = d[i];
+    __syncthreads();
+    T u[SW];
+#pragma unroll
+    for (int s = 0; s < SW; ++s) u[s] = U[lane * (SW + 1) + s];
+#pragma unroll
+    for (int s = 0; s < SW; ++s) {
+        const T xs = lane_of(x, s);
+        if (lane > s) x = nfma(xs, u[s], x);
+    }
+    if (!mine) return;
+    Wm[c + (k1 + lane) * ldw] = x;
+    if (p >= SW && first == lane) Wm[c + (k1 + p) * ldw] = y;
+}
+
 // Column-major (LAPACK) form: rows of A (n x ncols, lda) permuted by pairs.
 __global__ __launch_bounds__(256) void apply_pairs_cm_kernel(double* __restrict__ A, i64 lda, i64 ncols,
                                                              const int* __restrict__ pairs, i64 roff) {
@@ -394,6 +465,22 @@ int swap_w(GetrfCtx<T>& g, i64 k1, i64 k2, i64 c0, i64 c1, int inverse) {
     hipLaunchKernelGGL(apply_pairs_w_kernel<T>, dim3(unsigned(cdiv(c1 - c0, PAIR_ROWS))), dim3(256), shm, g.s, g.Wm,
                        g.ldw, c0, c1, g.pairs, i64(0));
     return launch_check(g.h, "apply_pairs_w");
+}
+
+// The interchanges of the panel [j0, j1) and U12 on the next panel's columns
+// [c0, c1): one launch for a 64-column panel and a block of up to two (each
+// workgroup of four columns replays the interchanges: with more of them the
+// pair list and the TRSM's products are cheaper); else the interchanges, then
+// the TRSM.
+template <typename T>
+int swap_solve(GetrfCtx<T>& g, i64 j0, i64 j1, i64 c0, i64 c1) {
+    if (j1 - j0 == SW && c1 - c0 <= 2 * SW) {
+        hipLaunchKernelGGL(swap_solve_kernel<T>, dim3(unsigned(cdiv(c1 - c0, 4))), dim3(256), 0, g.s, g.Wm, g.ldw, j0, g.ipiv,
+                           c0, c1);
+        return launch_check(g.h, "swap_solve");
+    }
+    OXI_TRY(swap_w(g, j0, j1 - 1, c0, c1, 0));
+    return trsm_ru(g.h, g.s, c1 - c0, j1 - j0, g.Wm + j0 + j0 * g.ldw, g.ldw, g.Wm + c0 + j0 * g.ldw, g.ldw);
 }
 
 // Rows per thread of the leaf at c0: kind 0 one (256 rows a workgroup), 1 two,
@@ -676,8 +763,7 @@ int getrf_t(oxi_handle_t h, i64 m, i64 n, T* A, i64 lda, i64* ipiv, i64 nb, i64*
                 // waits for the main stream's update of [j1, j2) of the
                 // previous step, or the transpose)
                 OXI_HIP(h, hipStreamWaitEvent(h->side, h->ev_a, 0));
-                OXI_TRY(swap_w(gs, j0, j1 - 1, j1, j2, 0));
-                OXI_TRY(trsm_ru(h, gs.s, j2 - j1, jb, g.Wm + j0 + j0 * ldw, ldw, g.Wm + j1 + j0 * ldw, ldw));
+                OXI_TRY(swap_solve(gs, j0, j1, j1, j2));
                 hipEvent_t pe = nullptr;
                 if (timed_update<T>(j2 - j1, m - j1)) OXI_TRY(oxi_prof_begin(h, gs.s, &pe));
                 OXI_TRY(trailing_rows(gs, j0, j1, j1, j2));

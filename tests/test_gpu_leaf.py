@@ -69,3 +69,31 @@ def test_leaf_nonfinite_and_zero_pivots(gpu, rng, m, w):
     A = rng.standard_normal((m, w))
     A[0, 0] = np.nan                        # wins in the diagonal position
     check(gpu, A)
+
+
+# Interchanges of 64-column panels on the next panel's columns, where the same
+# row is reached again and again (a cyclic shift: step s takes the last row every
+# time) or rows move about inside the panel and out of it (random permutations,
+# with a lower part of the factor that the solve has to apply): exact.
+@pytest.mark.parametrize("n", [65, 127, 128, 129, 192, 200, 257, 320, 450])
+@pytest.mark.parametrize("kind", ["shift", "back", "random", "scaled"])
+def test_interchanges_of_panels_exact(gpu, rng, n, kind):
+    if kind == "shift":
+        A = np.roll(np.eye(n), 1, axis=1)
+    elif kind == "back":
+        A = np.roll(np.eye(n), -1, axis=1)
+    else:
+        # P^T L U with entries that every operation leaves exact
+        L = np.tril((rng.integers(-1, 2, (n, n)) * (rng.random((n, n)) < 2.0 / n)).astype(float) * 0.5, -1) + np.eye(n)
+        if kind == "random":
+            L = np.eye(n)
+        A = (L @ np.diag(2.0 ** rng.integers(-2, 3, n)))[rng.permutation(n)]
+    for lowp in (False, True):
+        M = np.asfortranarray(A.astype(np.float32) if lowp else A)
+        F = gpu.lu_lowp(M, "float32", blocksize=64) if lowp else gpu.lu(M, blocksize=64)
+        LU = F.factors.numpy().astype(float)
+        perm = np.arange(n)
+        for i, q in enumerate(F.ipiv_dev.cpu().numpy().astype(int) - 1):
+            assert q >= i
+            perm[[i, q]] = perm[[q, i]]
+        assert np.array_equal((np.tril(LU, -1) + np.eye(n)) @ np.triu(LU), A[perm]), lowp
