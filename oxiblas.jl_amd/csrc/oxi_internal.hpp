@@ -117,6 +117,10 @@ int oxi_dtrsm_left(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit
                    const double* A, i64 lda, double* B, i64 ldb);
 int oxi_dtrsm_right(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit, i64 m, i64 n,
                     const double* A, i64 lda, double* B, i64 ldb);
+// The same where no other stream solves at the same time (it takes the handle's
+// buffer of block inverses).
+int oxi_dtrsm_right_alone(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit, i64 m, i64 n,
+                          const double* A, i64 lda, double* B, i64 ldb);
 int oxi_strsm_left(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit, i64 m, i64 nrhs,
                    const float* A, i64 lda, float* B, i64 ldb);
 int oxi_strsm_right(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit, i64 m, i64 n,

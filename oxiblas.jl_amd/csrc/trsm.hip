@@ -632,6 +632,11 @@ int oxi_dtrsm_right(oxi_handle_t h, hipStream_t s, int upper, int trans, int uni
                     i64 lda, double* B, i64 ldb) {
     return trsm_right_t<double>(h, s, upper, trans, unit, m, n, A, lda, B, ldb);
 }
+int oxi_dtrsm_right_alone(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit, i64 m, i64 n, const double* A,
+                          i64 lda, double* B, i64 ldb) {
+    if (blocked_applies(h, n, m)) return trsm_blocked(h, s, false, upper, trans, unit, n, m, A, lda, B, ldb);
+    return oxi_dtrsm_right(h, s, upper, trans, unit, m, n, A, lda, B, ldb);
+}
 int oxi_strsm_left(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit, i64 m, i64 nrhs, const float* A,
                    i64 lda, float* B, i64 ldb) {
     return trsm_left_t<float>(h, s, upper, trans, unit, m, nrhs, A, lda, B, ldb);
@@ -694,7 +699,6 @@ extern "C" int oxi_dtrsm(oxi_handle_t h, char side, char uplo, char trans, char 
     }
     if (alpha != 1.0) OXI_TRY(oxi_launch_dscale(s, m, n, alpha, B, ldb));
     if (left) return oxi_dtrsm_left(h, s, upper, tk, unit, m, n, A, lda, B, ldb);
-    if (blocked_applies(h, n, m)) return trsm_blocked(h, s, false, upper, tk, unit, n, m, A, lda, B, ldb);
-    return oxi_dtrsm_right(h, s, upper, tk, unit, m, n, A, lda, B, ldb);
+    return oxi_dtrsm_right_alone(h, s, upper, tk, unit, m, n, A, lda, B, ldb);
 }
 
