@@ -205,12 +205,11 @@ def cpu_baseline(n=8192, reps=3, n_openblas=16384):
 
 def trailing_shapes(n=16384):
     """(M, N, K) in the factorization's transposed coordinates of the trailing
-    updates that run on the 128 x 128 kernel, in issue order: getrf's tuned
+    updates that getrf's profiling times, in issue order: getrf's tuned
     block-size schedule (512 while more than 3/8 of the columns remain, then
     256), its three updates per panel [j0, j1) (the next panel's columns
     [j1, j2) on the side stream, then [j2, j3) and [j3, n) on the main
-    stream) and the GEMM's tile rule (128 x 128 tiles when that grid has at
-    least 448 workgroups)."""
+    stream), those of at least 448 tiles of 128 x 128."""
     cdiv = lambda a, b: (a + b - 1) // b
     wide_until = n - (3 * n) // 8
     nb_at = lambda j: 512 if j < wide_until else 256
@@ -228,8 +227,14 @@ def trailing_shapes(n=16384):
     return out
 
 
+def on_large_tiles(M, N, K):
+    """Whether the FP64 GEMM takes its 128 x 128 tiles (choose_tile, dgemm.hip)."""
+    t = ((M + 127) // 128) * ((N + 127) // 128)
+    return K >= 192 and t >= 1024 and (t >= 4096 or t % 256 == 0 or t % 256 >= 192)
+
+
 def traffic_summary(fetch_csv, write_csv, copy_fetch_csv, copy_write_csv, out_json):
-    """HBM bytes per dgemm_m16_kernel launch of the n = 16384 factorization
+    """HBM bytes per launch of the 128 x 128 dgemm_direct_kernel in the n = 16384 factorization
     from a FETCH_SIZE run and a WRITE_SIZE run of
     'bench.py --steps 1 --warmup 0 --no-cpu --no-extra --no-mixed', each
     scaled by what the same counter reads for a 1 GiB device copy
@@ -239,18 +244,18 @@ def traffic_summary(fetch_csv, write_csv, copy_fetch_csv, copy_write_csv, out_js
     def rows(path, counter, name):
         return [float(r["Counter_Value"]) for r in csv.DictReader(open(path))
                 if r["Counter_Name"] == counter and name in r["Kernel_Name"]]
-    f = rows(fetch_csv, "FETCH_SIZE", "dgemm_m16_kernel<false, false, false, 0>")
-    w = rows(write_csv, "WRITE_SIZE", "dgemm_m16_kernel<false, false, false, 0>")
+    f = rows(fetch_csv, "FETCH_SIZE", "dgemm_direct_kernel<128, 128, 16, 2, false, false, false, 0>")
+    w = rows(write_csv, "WRITE_SIZE", "dgemm_direct_kernel<128, 128, 16, 2, false, false, false, 0>")
     cf = rows(copy_fetch_csv, "FETCH_SIZE", "copyBuffer")
     cw = rows(copy_write_csv, "WRITE_SIZE", "copyBuffer")
     kf = (1 << 20) / (sum(cf) / len(cf))          # KiB per KiB the counter reports
     kw = (1 << 20) / (sum(cw) / len(cw))
-    shapes = trailing_shapes()
+    shapes = [x for x in trailing_shapes() if on_large_tiles(*x)]
     reps = len(f) // len(shapes)
     assert reps >= 1 and len(f) == reps * len(shapes) and len(w) == len(f), (len(f), len(w), len(shapes))
     alg = [8 * (M * K + K * N + 2 * M * N) for (M, N, K) in shapes] * reps
     meas = [(a * kf + b * kw) * 1024 for a, b in zip(f, w)]
-    out = {"kernel": "dgemm_m16_kernel: getrf trailing updates on 128x128 tiles, n=16384, tuned block sizes",
+    out = {"kernel": "dgemm_direct_kernel: getrf trailing updates on 128x128 tiles, n=16384, tuned block sizes",
            "hbm_bytes_per_launch": round(sum(meas) / len(meas)),
            "algorithmic_bytes_per_launch": round(sum(alg) / len(alg)),
            "fetch_scale": round(kf, 4), "write_scale": round(kw, 4),
@@ -326,7 +331,7 @@ def main():
     ap.add_argument("--kappa", type=float, default=1e6)
     ap.add_argument("--traffic-summary", nargs=5, metavar=("FETCH_CSV", "WRITE_CSV", "COPY_FETCH_CSV",
                                                            "COPY_WRITE_CSV", "OUT_JSON"),
-                    help="write the HBM traffic per dgemm_m16_kernel launch from counter runs and exit")
+                    help="write the HBM traffic per launch of the 128x128 GEMM kernel from counter runs and exit")
     ap.add_argument("--part", choices=("cholesky", "getrs64", "trsv", "mixed32", "mixed32tp", "lowp", "gemm", "lowp_gemm"),
                     default=None,
                     help="only run one extra part a few times (for rocprofv3 summaries of its kernels) and exit")
@@ -389,9 +394,9 @@ def main():
     berr = torch.linalg.norm(r).item() / (torch.linalg.matrix_norm(At).item() * torch.linalg.norm(xt).item() * n * eps)
     del F, x
 
-    # roofline of the dominant kernel: the trailing-update GEMM inside getrf on
-    # its 128 x 128 tiles (dgemm_m16_kernel), events around each of those
-    # launches on the stream it runs on
+    # roofline of the dominant kernel: the trailing-update GEMM inside getrf
+    # (dgemm_direct_kernel), events around each of the launches of at least 448
+    # tiles of 128 x 128 on the stream it runs on
     h = ox.handle()
     h._L.oxi_profile_enable(h.ptr, 1)
     F, x = step()
@@ -401,7 +406,7 @@ def main():
     h._L.oxi_profile_enable(h.ptr, 0)
     del F, x
     gemm_tflops = fl.value / (ms.value * 1e-3) / 1e12 if ms.value > 0 else 0.0
-    log(f"trailing GEMM (dgemm_m16_kernel): {nl.value} launches, {ms.value:.2f} ms, {gemm_tflops:.1f} TFLOP/s")
+    log(f"trailing GEMM (dgemm_direct_kernel): {nl.value} launches, {ms.value:.2f} ms, {gemm_tflops:.1f} TFLOP/s")
 
     extra = {}
     if not args.no_extra:
@@ -516,7 +521,7 @@ def main():
         "pct_fp64_peak": round(100.0 * value / (PEAK_FP64_TFLOPS * 1e3), 2),
         "roofline": {"bound": "mfma", "achieved": round(gemm_tflops, 3), "peak": PEAK_FP64_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(gemm_tflops / PEAK_FP64_TFLOPS, 4), "traffic": None,
-                     "kernel": "dgemm_m16_kernel: getrf trailing updates on 128x128 tiles (all such launches of one step)",
+                     "kernel": "dgemm_direct_kernel: getrf trailing updates of 448 or more 128x128 tiles (all such launches of one step)",
                      "launches": int(nl.value)},
         "cpu_baseline": cpu,
         "cpu_openblas": cpu_ob,
@@ -529,7 +534,7 @@ def main():
         t = json.load(open(tf))
         out["roofline"]["traffic"] = t["hbm_bytes_per_launch"]
         out["roofline"]["traffic_algorithmic"] = t["algorithmic_bytes_per_launch"]
-        out["roofline"]["traffic_launches"] = f"{t['launches_measured']} dgemm_m16_kernel launches"
+        out["roofline"]["traffic_launches"] = f"{t['launches_measured']} launches on 128x128 tiles"
     if mixed:
         at = [v for v in mixed.values() if v["kappa"] == args.kappa and v["converged"]]
         best = max(at, key=lambda v: v["speedup_vs_fp64_lu_solve"]) if at else None

@@ -6,9 +6,10 @@
 // The recursion is the reference's (LAPACK potrf2): L11 first, then
 // L21 = A21 L11^-T (right-side TRSM), A22 -= L21 L21^T (the lower-triangle
 // SYRK on the matrix cores: only tiles that touch the lower triangle run),
-// then L22.  Leaves of at most 64 columns are factored right-looking by one
-// workgroup with the block in LDS, with the reference leaf's operations in its
-// order: d = sqrt(a_cc), l_ic = a_ic / d, a_ij = fma(-l_ic, l_jc, a_ij).
+// then L22.  Leaves of at most 64 columns are factored by one wave with the
+// block in LDS, right-looking in panels of 16 columns with the reference leaf's
+// operations: d = sqrt(a_cc), l_ic = a_ic / d, a_ij = fma(-l_ic, l_jc, a_ij); the
+// columns right of a panel take its 16 products at once.
 // A leaf that meets a non-positive or non-finite pivot records its global
 // column in a device word and stops; later leaves see the word and do
 // nothing, so the first failing column is the one reported (the reference's

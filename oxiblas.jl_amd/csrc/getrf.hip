@@ -13,7 +13,7 @@
 //
 // Algorithm (the reference's, in W's coordinates):
 //   for each panel of nb columns:
-//     getrf2 recursion on the panel (halving, leaves of <= 32 columns)
+//     getrf2 recursion on the panel (halving, leaves of <= 64 columns)
 //     interchanges applied to the columns left and right of the panel
 //     U12 <- L11^-1 A12           (right-side solve with L11^T in W)
 //     A22 <- A22 - L21*U12        (FP64 MFMA GEMM)
@@ -28,9 +28,8 @@
 // per column every workgroup publishes its candidate (key, row and the whole
 // row) as a record of tagged words and reads all the others until they are
 // complete (bounded wait with a timeout flag so every wave exits), so all pick
-// the same winner; with P == 1 the exchange stays in LDS (panel.hip).  A
-// small kernel after each leaf applies its interchanges to the rest of the
-// panel.
+// the same winner; with P == 1 the exchange stays in LDS (panel.hip).  At its
+// end it applies its interchanges to the rest of the panel.
 #include "oxi_internal.hpp"
 
 #include <vector>

@@ -1,5 +1,5 @@
 // Panel leaf of the blocked LU: column-by-column elimination of an m x w
-// block (w <= 32) held in registers across P co-resident workgroups.
+// block (w <= 64) held in registers across P co-resident workgroups.
 //
 // Restates the leaf of _lu_panel! (src/lapack/factorizations.jl:116-140) with
 // the pivot choice of _lu_pivot (:89-107): the pivot is the first row of

@@ -1,7 +1,8 @@
-// Triangular solves (trsm!, src/blas/level3.jl:309-544) on gfx950: leaves of
-// at most 64 rows/columns solved in registers or with one wave per right-hand
-// side, and the reference's recursive halving with FP64 MFMA GEMM updates in
-// between (_trsm_blocks_left! / _trsm_blocks_right!, level3.jl:338-376).
+// Triangular solves (trsm!, src/blas/level3.jl:309-544) on gfx950: the
+// reference's recursive halving (_trsm_blocks_left! / _trsm_blocks_right!,
+// level3.jl:338-376) with FP64 MFMA GEMM updates, down to blocks of 256 rows in
+// one launch (trsm_block_kernel), or to leaves of at most 64 rows solved in
+// registers, one wave per right-hand side.
 #include "tri_inv.hpp"
 
 #include <algorithm>
