@@ -497,14 +497,17 @@ int leaf_kind(const GetrfCtx<T>& g, i64 c0) {
     const bool tournament = sizeof(T) == 4 && g.tournament;
     return mrows > 8192 || (!tournament && mrows > 256 && mrows <= 512) ? 1 : 0;
 }
-// Columns of the widest leaf at c0: 64 where a row of 64 fits a thread's
-// registers (one FP64 or two FP32 rows per thread), else 32.  A 64-column leaf
-// takes 133 us at 2000 rows against 123 for two of 32, which need a triangular
-// solve and a product between them (11 us and two launches).
+// Columns of the widest leaf at c0: 64 in FP64 where a row of 64 fits a thread's
+// registers (one row per thread), else 32.  A 64-column leaf takes 133 us at
+// 2000 rows against 123 for two of 32, which need a triangular solve and a
+// product between them (11 us and two launches).  Not in FP32: there the 32
+// columns' products are summed before they meet the next 32, in a 64-column
+// leaf they round one by one, and the factor's error shows in the mixed solve
+// (4096 shifted: the FP32 solve's error 2.6e-7 with leaves of 32 and panels of
+// 128, 3.2e-7 with 64 and 64; 10.6 ms a factor against 9.2).
 template <typename T>
 i64 leaf_width(const GetrfCtx<T>& g, i64 c0) {
-    if (sizeof(T) == 4 && g.tournament) return 32;
-    return leaf_kind(g, c0) * sizeof(T) <= 4 ? OXI_LEAF_W : 32;
+    return sizeof(T) == 8 && leaf_kind(g, c0) == 0 ? OXI_LEAF_W : 32;
 }
 
 template <typename T>
@@ -587,13 +590,14 @@ bool timed_update(i64 rows, i64 cols) {
 }
 
 // Tuned block size: the panels bound the factorization, and up to about 5000
-// columns a panel of one 64-column leaf needs no product of its own (n = 2000:
-// 4.95 ms with 64, 5.10 with 128; 4096: 10.5 and 10.6; 6000: 16.8 and 16.5;
-// 8192: 28.0, 24.7 and, with 256, 24.6).
-int choose_nb(i64 m, i64 n) {
+// columns a panel of one 64-column leaf (FP64) needs no product of its own (n =
+// 2000: 4.95 ms with 64, 5.10 with 128; 4096: 10.5 and 10.6; 6000: 16.8 and
+// 16.5; 8192: 28.0, 24.7 and, with 256, 24.6).  FP32 keeps 128 from 1024 on: an
+// element rounds once per panel.
+int choose_nb(i64 m, i64 n, bool fp32) {
     const i64 q = std::min(m, n);
     if (q >= 8192) return 256;
-    if (q >= 5120) return 128;
+    if (q >= (fp32 ? 1024 : 5120)) return 128;
     return 64;
 }
 
@@ -606,7 +610,7 @@ int getrf_t(oxi_handle_t h, i64 m, i64 n, T* A, i64 lda, i64* ipiv, i64 nb, i64*
     hipStream_t s = h->stream;
     const i64 q = std::min(m, n);
     const bool tuned = nb == 0;
-    if (nb == 0) nb = choose_nb(m, n);
+    if (nb == 0) nb = choose_nb(m, n, sizeof(T) == 4);
     if (nb > PERM_MAX_STEPS) nb = PERM_MAX_STEPS;
     // Tuned block size on large matrices: 512-wide panels while more than 3/8
     // of the columns remain (the trailing update bounds those steps and runs
