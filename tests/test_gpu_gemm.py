@@ -386,7 +386,7 @@ def _guarded(torch, x, ld, shift):
     """Column-major copy of x with leading dimension ld, `shift` elements into
     its buffer, NaN everywhere else."""
     r, c = x.shape
-    buf = torch.full((shift + ld * c + 3,), float("nan"), dtype=torch.float64, device="cuda")
+    buf = torch.full((shift + ld * c + 3,), float("nan"), dtype=x.dtype, device="cuda")
     view = buf[shift:shift + ld * c]
     view.view(c, ld)[:, :r] = x.T
     return buf, view
@@ -426,6 +426,41 @@ def test_tile_edges_exact(gpu, mnk, ta, tb):
                 ref = ref + beta * C.cpu().numpy()
             cols = c.view(n, m + pad)
             assert np.array_equal(cols[:, :m].T.cpu().numpy(), ref), (pad, shift, beta)
+            assert torch.isnan(cols[:, m:]).all() and torch.isnan(cb[:shift]).all() and torch.isnan(cb[-3:]).all()
+
+
+# The same for FP32, whose operands are fetched in fours and whose slabs have 32
+# of k: every remainder of four, one row or column past a tile, 4-byte
+# alignment, and the lengths below four that take the general kernel.
+EDGES32 = [(2, 4, 5), (3, 5, 3), (4, 4, 4), (5, 6, 7), (6, 7, 1), (33, 35, 34), (34, 66, 31), (65, 97, 67),
+           (1217, 1282, 35), (1283, 1215, 32), (1280, 1280, 64), (2689, 2690, 97), (2688, 2691, 98), (2688, 2816, 96)]
+
+
+@pytest.mark.parametrize("mnk", EDGES32)
+@pytest.mark.parametrize("ta", "NT")
+@pytest.mark.parametrize("tb", "NT")
+def test_sgemm_tile_edges_exact(gpu, mnk, ta, tb):
+    import torch
+    m, n, k = mnk
+    g = torch.Generator(device="cuda").manual_seed(m * 31 + n * 7 + k)
+
+    def ints(r, c):
+        return torch.randint(-8, 9, (r, c), device="cuda", generator=g).float()
+    A = ints(m, k) if ta == "N" else ints(k, m)
+    B = ints(k, n) if tb == "N" else ints(n, k)
+    C = ints(m, n)
+    # sums of at most 98 products of 64: whole numbers below 2^24, exact in FP32
+    base = 2.0 * (op(A, ta).double().cpu().numpy() @ op(B, tb).double().cpu().numpy())
+    for pad, shift in ((0, 0), (1, 1), (3, 2), (4, 0)):
+        _, a = _guarded(torch, A, A.shape[0] + pad, shift)
+        _, b = _guarded(torch, B, B.shape[0] + pad, 3 - shift)
+        for beta in (0.0, -3.0):
+            cb, c = _guarded(torch, C if beta else C * float("nan"), m + pad, shift)
+            gpu.sgemm_(gpu.DMatrix(c, m, n, m + pad), gpu.DMatrix(a, A.shape[0], A.shape[1], A.shape[0] + pad),
+                       gpu.DMatrix(b, B.shape[0], B.shape[1], B.shape[0] + pad), 2.0, beta, ta, tb)
+            ref = base + beta * C.double().cpu().numpy() if beta else base
+            cols = c.view(n, m + pad)
+            assert np.array_equal(cols[:, :m].T.double().cpu().numpy(), ref), (pad, shift, beta)
             assert torch.isnan(cols[:, m:]).all() and torch.isnan(cb[:shift]).all() and torch.isnan(cb[-3:]).all()
 
 
