@@ -240,7 +240,7 @@ int oxi_launch_lu_leaf(oxi_handle_t h, hipStream_t s, const LeafArgs& a, int kin
 // OXI_TP_MAX_P workgroups.
 constexpr int OXI_TP_MAX_P = 32;
 int oxi_launch_lu_leaf_tp(oxi_handle_t h, hipStream_t s, const LeafArgs& a, int kind);
-// FP32 leaf; kind 1 takes up to 64 columns too, kind 2: 256 threads x 4 rows, up to 32.
+// FP32 leaf, up to 32 columns; kind 2: 256 threads x 4 rows.
 int oxi_launch_lu_leaf32(oxi_handle_t h, hipStream_t s, const LeafArgs& a, int kind);
 
 // Bracket one trailing-update GEMM launch with profiling events (no-op when

@@ -21,9 +21,9 @@
 // Rows never move between threads: an interchange changes the positions that
 // the threads hold, and every row, multipliers included, is stored once at
 // its final position, which gives the same rows as swapping whole rows at
-// each step.  A second, small kernel applies the leaf's interchanges to the
-// other columns of the enclosing panel (the sibling swaps of the getrf2
-// recursion, done once per leaf).
+// each step.  At its end the leaf applies its interchanges to the other
+// columns of the enclosing panel (the sibling swaps of the getrf2 recursion,
+// done once per leaf).
 #include "panel_kernel.hpp"
 
 int oxi_launch_lu_leaf(oxi_handle_t h, hipStream_t s, const LeafArgs& a, int kind) {
