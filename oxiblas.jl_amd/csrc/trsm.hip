@@ -13,6 +13,13 @@ __device__ __forceinline__ float fma_t(float a, float b, float c) { return __bui
 
 constexpr int TRL = 64;
 constexpr int SB = 256;   // rows of a block of the blocked solves
+// A 64-row diagonal block M is solved through its inverse V only while the row
+// sums of |V| |M| stay below this (and are numbers).  Up to there one refinement leaves
+// a backward error no larger than substitution's (emulated for random, row- and
+// column-scaled triangles and the blocks of LU factors, sums of 1 to 10^10: at
+// most 3.2e-16 componentwise, 4.8e-16 by substitution, 6e-15 without the
+// refinement); far beyond, 64 eps times the sum passes 1 and it need not contract.
+constexpr double MAX_COND = 0x1p40;
 
 // Right side: X (rows x n) <- X * op(T)^-1, n <= 64.  Element order matches
 // the reference's right leaf (src/blas/level3.jl:319-333):
@@ -134,7 +141,8 @@ void launch_right_leaf(hipStream_t s, int unit, int trans, i64 rows, int n, cons
 // with strip > 0, to its place in a column-major strip of ld `ldv` whose rows
 // z*strip .. (z+1)*strip - 1 hold the strip x strip block z (inv + 64 b +
 // ((64 b) % strip) * ldv); CLEAN: to inv + 8192 b, and the block itself,
-// completed in the same way, 4096 elements behind it.  The block in
+// completed in the same way, 4096 elements behind it, where an inverse that
+// trsm_block_kernel must not use is NaN throughout.  The block in
 // LDS (UPPER: both indices reversed, so that it is lower triangular), inverted
 // on the matrix cores (tri::invert); bound by the latency of its loads and
 // barriers: 8 us, against 27 for a column a lane swept over 64 steps.
@@ -143,6 +151,8 @@ __global__ __launch_bounds__(256) void trsm_inv64_kernel(const double* __restric
                                                          double* __restrict__ inv, i64 ldv = 64, int strip = 0) {
     constexpr int L = tri::LD<64>;
     __shared__ double D[tri::SPACE<64>];   // D(i, k) = M(i, k), or M(63 - i, 63 - k)
+    __shared__ double part[CLEAN ? 256 : 1], sums[CLEAN ? 64 : 1];   // of each row of |D|
+    __shared__ int avoid;
     const int t = threadIdx.x;
     const i64 o = i64(blockIdx.x) * 64;
     double* out = strip > 0 ? inv + o + (o % strip) * ldv : inv + 64 * (CLEAN ? 2 : 1) * o;
@@ -156,19 +166,43 @@ __global__ __launch_bounds__(256) void trsm_inv64_kernel(const double* __restric
         D[k * L + i] = i == k ? (UNIT || !in ? 1.0 : v) : in && i > k ? v : 0.0;
     }
     __syncthreads();
-    auto store = [&](double* to) __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const int e = t + u * 256, r = e % 64, c = e / 64, i = UPPER ? 63 - r : r, k = UPPER ? 63 - c : c;
-            to[r + c * ldv] = i >= k ? D[k * L + i] : 0.0;
-        }
+    // this thread's elements of the result: row r, columns t / 64 + 4 u
+    const int r = t % 64, i = UPPER ? 63 - r : r;
+    auto column = [&](int u) __attribute__((always_inline)) { return t / 64 + 4 * u; };
+    auto lower = [&](int u) __attribute__((always_inline)) {
+        const int k = UPPER ? 63 - column(u) : column(u);
+        return i >= k ? D[k * L + i] : 0.0;
     };
     if (CLEAN) {
-        store(out + 4096);
+        double sum = 0.0;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const double v = lower(u);
+            out[4096 + r + column(u) * 64] = v;
+            sum += __builtin_fabs(v);
+        }
+        part[t / 64 * 64 + i] = sum;
+        if (t == 0) avoid = 0;
         __syncthreads();
+        if (t < 64) sums[t] = (part[t] + part[t + 64]) + (part[t + 128] + part[t + 192]);
     }
     tri::invert<double, 64, 4, UNIT>(D, t);
-    store(out);
+    double v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = lower(u);
+    if (CLEAN) {
+        // row i of |D^-1| |D| e, a quarter of its columns
+        double c = 0.0;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) c += __builtin_fabs(v[u]) * sums[UPPER ? 63 - column(u) : column(u)];
+        if (!(c < MAX_COND)) avoid = 1;
+        __syncthreads();
+        if (avoid)
+#pragma unroll
+            for (int u = 0; u < 16; ++u) v[u] = __builtin_nan("");
+    }
+#pragma unroll
+    for (int u = 0; u < 16; ++u) out[r + column(u) * ldv] = v[u];
 }
 
 // One block of up to SB = 256 rows of a triangular solve M x = b in place, M
@@ -182,7 +216,14 @@ __global__ __launch_bounds__(256) void trsm_inv64_kernel(const double* __restric
 // solve order: r = b_p - sum M_pq x_q over the blocks before, x = M_pp^-1 r, and
 // one refinement x += M_pp^-1 (r - M_pp x), so that x is no further off than by
 // substitution; a wave has 16 of the 64 rows, x in LDS, the operands of M and
-// V straight from memory, the next product's loaded while one runs.  256 rows cost one launch and no scratch memory.  Bound by the
+// V straight from memory, the next product's loaded while one runs.  The
+// products take their k in solve order (the diagonal's large term last).
+// Where an element of x is not finite, the right-hand sides are solved again
+// with the 64-row blocks by substitution: the products multiply the zeros of
+// the other triangle too, so an infinity of r reaches the rows before it, an
+// inverse may overflow where x does not, and an inverse not to be used is NaN
+// (trsm_inv64_kernel).
+// 256 rows cost one launch.  Bound by the
 // 18 products a wave has one after the other (16 matrix instructions of 64
 // cycles each, 9 us) and the 16 turns through LDS and a barrier: 22 us.
 template <bool LEFT, bool TM, bool BWD, bool FULL>
@@ -192,6 +233,7 @@ __global__ __launch_bounds__(256, 1) void trsm_block_kernel(const double* __rest
     typedef tri::Mfma<double> Mf;
     constexpr int C = 16, LX = C + 1;
     __shared__ double xs[SB * LX], rs[64 * LX];
+    __shared__ int again;                          // an element of x is not finite
     const int t = threadIdx.x, lane = t & 63, w = t >> 6, lk = lane >> 4, li = lane & 15;
     const int rows = FULL ? SB : nrows, nsb = (rows + 63) / 64;
     const i64 j0 = i64(blockIdx.x) * C;
@@ -217,7 +259,7 @@ __global__ __launch_bounds__(256, 1) void trsm_block_kernel(const double* __rest
         for (int e = 0; e < 16; ++e) y[e] = x[(4 * e + lk) * LX + li];
         __builtin_amdgcn_sched_barrier(0);   // all of x on its way before the first product
 #pragma unroll
-        for (int e = 0; e < 16; ++e) c = Mf::mul(a[e], y[e], c);
+        for (int e = 0; e < 16; ++e) c = Mf::mul(a[BWD ? 15 - e : e], y[BWD ? 15 - e : e], c);
         return c;
     };
     auto copy = [&](const double (&from)[16], double (&to)[16]) __attribute__((always_inline)) {
@@ -239,20 +281,24 @@ __global__ __launch_bounds__(256, 1) void trsm_block_kernel(const double* __rest
     for (int u = 0; u < 16; ++u) b[u] = B[element(u)];
     double cur[16], nxt[16];
     load_v(BWD ? nsb - 1 : 0, 0, cur);
+    auto b_to_x = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-        const int i = LEFT ? i0 : i0 + 16 * u;
-        xs[i * LX + (LEFT ? u : j)] = FULL || i < rows ? b[u] : 0.0;
-    }
+        for (int u = 0; u < 16; ++u) {
+            const int i = LEFT ? i0 : i0 + 16 * u;
+            xs[i * LX + (LEFT ? u : j)] = FULL || i < rows ? b[u] : 0.0;
+        }
+    };
+    b_to_x();
+    if (t == 0) again = 0;
     __syncthreads();
     const int own = (w * 16 + lk) * LX + li;                 // this lane's element of a block's rows, + 4 LX r
+    const Mf::acc zero = {0, 0, 0, 0};
     // Rolled (unrolled, the code of the 18 products took longer to fetch than
     // to run: 25 us), the operands of the next product in flight
 #pragma unroll 1
     for (int s = 0; s < nsb; ++s) {
         const int p = BWD ? nsb - 1 - s : s;
         double* xp = xs + p * 64 * LX;
-        const Mf::acc zero = {0, 0, 0, 0};
         Mf::acc r = zero;
 #pragma unroll 1
         for (int u = 0; u < s; ++u) {
@@ -278,16 +324,76 @@ __global__ __launch_bounds__(256, 1) void trsm_block_kernel(const double* __rest
 #pragma unroll
         for (int k = 0; k < 4; ++k) rs[own + 4 * LX * k] = r[k] - m[k];
         barrier_lds();
-        x = product(cur, rs, x);
+        const Mf::acc d = product(cur, rs, zero);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) xp[own + 4 * LX * k] = x[k];
+        for (int k = 0; k < 4; ++k) xp[own + 4 * LX * k] = x[k] + d[k];
         copy(nxt, cur);
         barrier_lds();
+    }
+    bool finite = true;
+    double xo[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        const int i = LEFT ? i0 : i0 + 16 * u;
+        xo[u] = xs[i * LX + (LEFT ? u : j)];
+        finite = finite && (__builtin_isfinite(xo[u]) || !(FULL || i < rows));
+    }
+    if (!finite) again = 1;
+    __syncthreads();
+    if (__builtin_expect(again, 0)) {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) b[u] = B[element(u)];
+        b_to_x();
+        __syncthreads();
+#pragma unroll 1
+        for (int s = 0; s < nsb; ++s) {
+            const int p = BWD ? nsb - 1 - s : s;
+            double* xp = xs + p * 64 * LX;
+            Mf::acc r = zero;
+#pragma unroll 1
+            for (int u = 0; u < s; ++u) {
+                const int q = BWD ? nsb - 1 - u : u;
+                load_m(p, q, cur);
+                r = product(cur, xs + q * 64 * LX, r);
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) xp[own + 4 * LX * k] -= r[k];
+            __syncthreads();
+            // a lane per row, a wave for four right-hand sides
+            const double* mp = V + p * 8192 + 4096 + lane;
+            double y[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) y[c] = xp[lane * LX + 4 * w + c];
+#pragma unroll 1
+            for (int g = 0; g < 64; g += 8) {
+                double m[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) m[u] = mp[64 * (BWD ? 63 - g - u : g + u)];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int k = BWD ? 63 - g - u : g + u;
+                    double yk = rlane(y[3], k);              // lane c: of right-hand side c
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) yk = lane == c ? rlane(y[c], k) : yk;
+                    yk /= rlane(m[u], k);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        const double v = rlane(yk, c);
+                        y[c] = lane == k ? v : (BWD ? lane < k : lane > k) ? fma_t(-m[u], v, y[c]) : y[c];
+                    }
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < 4; ++c) xp[lane * LX + 4 * w + c] = y[c];
+            __syncthreads();
+        }
+#pragma unroll
+        for (int u = 0; u < 16; ++u) xo[u] = xs[(LEFT ? i0 : i0 + 16 * u) * LX + (LEFT ? u : j)];
     }
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
         const int i = LEFT ? i0 : i0 + 16 * u, c = LEFT ? u : j;
-        if ((FULL || i < rows) && c < nc) B[element(u)] = xs[i * LX + c];
+        if ((FULL || i < rows) && c < nc) B[element(u)] = xo[u];
     }
 }
 

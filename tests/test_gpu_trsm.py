@@ -134,3 +134,84 @@ def _blocked(gpu, side, uplo, trans, diag, n, other):
     r = (T @ X if side == "L" else X @ T) - R
     assert r.norm() <= 8 * n * EPS * (T.norm() * X.norm() + R.norm())
     assert torch.equal(B[:, m], B0[:, m])
+
+
+# What a substitution leaves finite stays finite.  An infinity (NaN) in B reaches
+# the rows solved after it and no others, in its own right-hand side alone; a
+# triangle whose block inverses overflow (2^17 below a unit diagonal), or where a
+# reciprocal of the diagonal does, still gives what the substitution gives.
+VARIANTS = list(itertools.product("LR", "UL", "NT", "NU"))
+
+
+def oracle_trsm(B, T, side, uplo, trans, diag):
+    Xo = B.copy(order="F")
+    with np.errstate(all="ignore"):
+        assert O.dtrsm(Xo, T, 1.0, side, uplo, trans, diag == "U") == 0
+    return Xo
+
+
+@pytest.mark.parametrize("side,uplo,trans,diag", VARIANTS)
+@pytest.mark.parametrize("n,other", [(129, 16), (130, 33), (513, 20)])
+def test_trsm_nonfinite_right_hand_sides(gpu, rng, side, uplo, trans, diag, n, other):
+    T = tri(rng, n, uplo, diag == "U")
+    m, k = (n, other) if side == "L" else (other, n)
+    B = np.asfortranarray(rng.standard_normal((m, k)))
+    Bs = B if side == "L" else B.T                  # right-hand sides as columns, in place
+    Bs[100, 3] = np.inf
+    Bs[20, 7] = np.nan
+    Bs[n - 1, 15] = -np.inf
+    Xo = oracle_trsm(B, T, side, uplo, trans, diag)
+    X = gpu.trsm_(B.copy(order="F"), T, 1.0, side, uplo, trans, diag == "U")
+    fin = np.isfinite(Xo)
+    assert 0 < (~fin).sum() < 3 * n
+    np.testing.assert_array_equal(np.isfinite(X), fin)
+    assert np.abs(X[fin] - Xo[fin]).max() <= 1e-12 * np.abs(Xo[fin]).max() * n
+
+
+@pytest.mark.parametrize("side,uplo,trans,diag", VARIANTS)
+@pytest.mark.parametrize("n,other", [(129, 16), (256, 17), (513, 40)])
+def test_trsm_inverses_out_of_range(gpu, rng, side, uplo, trans, diag, n, other):
+    m, k = (n, other) if side == "L" else (other, n)
+    off = 1 if uplo == "U" else -1
+
+    def exact(T, X):
+        op = T.T if trans == "T" else T
+        B = np.asfortranarray(op @ X if side == "L" else X @ op)      # sums of two numbers: exact
+        np.testing.assert_array_equal(gpu.trsm_(B, np.asfortranarray(T), 1.0, side, uplo, trans, diag == "U"), X)
+    exact(np.eye(n) + 2.0 ** 17 * np.eye(n, k=off), np.ones((m, k)))
+    if diag == "N":                                  # 2^-1070: its reciprocal is infinite
+        T = np.eye(n) + np.eye(n, k=off)
+        T[77, 77] = 2.0 ** -1070
+        X = rng.integers(-4, 5, (m, k)).astype(float)
+        if side == "L":
+            X[76:79:2] = 0.0
+        else:
+            X[:, 76:79:2] = 0.0
+        T[77, 77 + off] = T[77 - off, 77] = 0.0
+        exact(T, X)
+
+
+@pytest.mark.parametrize("side,uplo,trans,diag", VARIANTS)
+def test_trsm_graded_triangles(gpu, rng, side, uplo, trans, diag):
+    """Columns (rows) falling by 10^-27 and more over a block: the componentwise
+    backward error of a substitution, at most (n + 2) unit roundoffs."""
+    n, other = 200, 24
+    for grade in (-0.5, 0.5):
+        for by_rows in (False, True):
+            T = rng.standard_normal((n, n)) / 8 + np.diag(1.0 + rng.random(n))
+            g = 10.0 ** (grade * np.arange(n))
+            T = np.asfortranarray(g[:, None] * T if by_rows else T * g)
+            T = np.triu(T) if uplo == "U" else np.tril(T)
+            if diag == "U":
+                T = np.asfortranarray(T / (T.diagonal()[:, None] if by_rows else T.diagonal()[None, :]))
+            m, k = (n, other) if side == "L" else (other, n)
+            B = np.asfortranarray(rng.standard_normal((m, k)))
+            X = gpu.trsm_(B.copy(order="F"), np.asfortranarray(T), 1.0, side, uplo, trans, diag == "U")
+            op = (T.T if trans == "T" else T).astype(np.longdouble)
+            if side == "R":
+                op, X, B = op.T, X.T, B.T
+            fin = np.isfinite(X).all(axis=0) & (np.abs(X) < 1e280).all(axis=0)
+            X, B = X[:, fin].astype(np.longdouble), B[:, fin]
+            assert fin.any()
+            R = np.abs(op @ X - B)
+            assert (R <= (n + 2) * (EPS / 2) * (np.abs(op) @ np.abs(X) + np.abs(B))).all()
