@@ -1,5 +1,6 @@
 // Inverse of a triangular block in LDS on the matrix cores, shared by the
-// preparations of the triangular solves (trsv.hip, trsm_chain.hip, trsm.hip).
+// preparations of the triangular solves (trsv.hip, trsm_chain.hip, trsm.hip),
+// and by substitution for blocks whose inverse is not finite.
 #pragma once
 #include "oxi_internal.hpp"
 
@@ -101,6 +102,32 @@ __device__ __forceinline__ void invert(T* D, int t) {
         }
         __syncthreads();
     }
+}
+
+// The same by substitution, a thread (t < N) per column, for the rare block
+// whose inverse holds an infinity or NaN (N^2 / 2 dependent loads).  Such an
+// element of D at (i, k) then reaches rows i on of the columns up to k and
+// nothing else; the products above, which multiply the zeros of a tile too,
+// carry it to all rows and columns of its 16 x 16 tile.  Column t goes through
+// tmp (N columns of memory, leading dimension ld, this workgroup's alone).
+template <typename T, int N, bool UNIT>
+__device__ __forceinline__ void invert_by_substitution(T* D, int t, T* tmp, i64 ld) {
+    constexpr int L = LD<N>;
+    T* x = tmp + t * ld;
+    if (t < N) {
+#pragma unroll 1
+        for (int i = t; i < N; ++i) {
+            T s = i == t ? T(1) : T(0);
+#pragma unroll 1
+            for (int k = t; k < i; ++k) s = nfma(D[k * L + i], x[k], s);
+            x[i] = UNIT ? s : s / D[i * L + i];
+        }
+    }
+    __syncthreads();
+    if (t < N)
+#pragma unroll 1
+        for (int i = 0; i < N; ++i) D[t * L + i] = i < t ? T(0) : x[i];
+    __syncthreads();
 }
 
 // G (rows i of the block, 16 columns q of this wave, value(i, q) given to

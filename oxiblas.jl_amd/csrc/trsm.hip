@@ -152,19 +152,23 @@ __global__ __launch_bounds__(256) void trsm_inv64_kernel(const double* __restric
     constexpr int L = tri::LD<64>;
     __shared__ double D[tri::SPACE<64>];   // D(i, k) = M(i, k), or M(63 - i, 63 - k)
     __shared__ double part[CLEAN ? 256 : 1], sums[CLEAN ? 64 : 1];   // of each row of |D|
-    __shared__ int avoid;
+    __shared__ int avoid;                                            // the inverse as it is
     const int t = threadIdx.x;
     const i64 o = i64(blockIdx.x) * 64;
     double* out = strip > 0 ? inv + o + (o % strip) * ldv : inv + 64 * (CLEAN ? 2 : 1) * o;
+    auto load = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-        const int e = t + u * 256;
-        const int x = e % 64, y = e / 64;        // T(o + x, o + y), the thread index along its columns
-        const int r = TRANS ? y : x, c = TRANS ? x : y, i = UPPER ? 63 - r : r, k = UPPER ? 63 - c : c;
-        const double v = T[min(o + x, n - 1) + min(o + y, n - 1) * ldt];
-        const bool in = o + x < n && o + y < n;
-        D[k * L + i] = i == k ? (UNIT || !in ? 1.0 : v) : in && i > k ? v : 0.0;
-    }
+        for (int u = 0; u < 16; ++u) {
+            const int e = t + u * 256;
+            const int x = e % 64, y = e / 64;        // T(o + x, o + y), the thread index along its columns
+            const int r = TRANS ? y : x, c = TRANS ? x : y, i = UPPER ? 63 - r : r, k = UPPER ? 63 - c : c;
+            const double v = T[min(o + x, n - 1) + min(o + y, n - 1) * ldt];
+            const bool in = o + x < n && o + y < n;
+            D[k * L + i] = i == k ? (UNIT || !in ? 1.0 : v) : in && i > k ? v : 0.0;
+        }
+    };
+    load();
+    if (t == 0) avoid = 0;
     __syncthreads();
     // this thread's elements of the result: row r, columns t / 64 + 4 u
     const int r = t % 64, i = UPPER ? 63 - r : r;
@@ -182,7 +186,6 @@ __global__ __launch_bounds__(256) void trsm_inv64_kernel(const double* __restric
             sum += __builtin_fabs(v);
         }
         part[t / 64 * 64 + i] = sum;
-        if (t == 0) avoid = 0;
         __syncthreads();
         if (t < 64) sums[t] = (part[t] + part[t + 64]) + (part[t + 128] + part[t + 192]);
     }
@@ -200,6 +203,20 @@ __global__ __launch_bounds__(256) void trsm_inv64_kernel(const double* __restric
         if (avoid)
 #pragma unroll
             for (int u = 0; u < 16; ++u) v[u] = __builtin_nan("");
+    } else {
+        bool finite = true;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) finite = finite && __builtin_isfinite(v[u]);
+        if (!finite) avoid = 1;
+        __syncthreads();
+        if (__builtin_expect(avoid, 0)) {
+            load();
+            __syncthreads();
+            tri::invert_by_substitution<double, 64, UNIT>(D, t, out, ldv);
+#pragma unroll
+            for (int u = 0; u < 16; ++u) v[u] = lower(u);
+            __syncthreads();   // out has been read
+        }
     }
 #pragma unroll
     for (int u = 0; u < 16; ++u) out[r + column(u) * ldv] = v[u];

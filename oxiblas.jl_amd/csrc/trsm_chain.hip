@@ -88,6 +88,7 @@ __global__ __launch_bounds__(CNT) void chain_prepare_kernel(const double* __rest
                                                             double* __restrict__ H) {
     constexpr int L = tri::LD<CB>;
     __shared__ double D[tri::SPACE<CB>];
+    __shared__ int odd;                       // the inverse is not finite
     const int t = threadIdx.x, lane = t & 63, w = t >> 6, b = blockIdx.x;
     const int rows = int(min(i64(CB), n - i64(b) * CB));
     const i64 p0 = block_row0(UPPER, n, b, rows);
@@ -95,16 +96,20 @@ __global__ __launch_bounds__(CNT) void chain_prepare_kernel(const double* __rest
     auto phys = [&](int k) __attribute__((always_inline)) { return UPPER ? rows - 1 - k : k; };
     // D(i, k) = op(T)(i, k), the identity outside the block; the index that
     // runs along M's columns changes fastest.  Loads without branches.
+    auto load = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < CB * CB / CNT; ++u) {
-        const int e = t + u * CNT;
-        const int x = e % CB, y = e / CB;
-        const int i = TRANS ? y : x, k = TRANS ? x : y;
-        const int ic = phys(min(i, rows - 1)), kc = phys(min(k, rows - 1));
-        const double v = TRANS ? M[(p0 + kc) + (p0 + ic) * ld] : M[(p0 + ic) + (p0 + kc) * ld];
-        const bool in = i < rows && k < rows;
-        D[k * L + i] = i == k ? (UNIT || !in ? 1.0 : v) : in && i > k ? v : 0.0;
-    }
+        for (int u = 0; u < CB * CB / CNT; ++u) {
+            const int e = t + u * CNT;
+            const int x = e % CB, y = e / CB;
+            const int i = TRANS ? y : x, k = TRANS ? x : y;
+            const int ic = phys(min(i, rows - 1)), kc = phys(min(k, rows - 1));
+            const double v = TRANS ? M[(p0 + kc) + (p0 + ic) * ld] : M[(p0 + ic) + (p0 + kc) * ld];
+            const bool in = i < rows && k < rows;
+            D[k * L + i] = i == k ? (UNIT || !in ? 1.0 : v) : in && i > k ? v : 0.0;
+        }
+    };
+    load();
+    if (t == 0) odd = 0;
     double tv[2][CB / 4];
 #pragma unroll
     for (int d = 1; d <= 2; ++d) {
@@ -120,12 +125,27 @@ __global__ __launch_bounds__(CNT) void chain_prepare_kernel(const double* __rest
     __syncthreads();
     tri::invert<double, CB, CNT / 64, UNIT>(D, t);
     double* out = V + size_t(b) * CB * CB;
+    // true where an element is not finite
+    auto store = [&]() __attribute__((always_inline)) {
+        bool bad = false;
 #pragma unroll
-    for (int u = 0; u < CB * CB / CNT; ++u) {
-        const int e = t + u * CNT;
-        const int pi = e % CB, pk = e / CB;      // physical row and column
-        const int i = phys(min(pi, rows - 1)), k = phys(min(pk, rows - 1));
-        out[e] = pi < rows && pk < rows && i >= k ? D[k * L + i] : 0.0;
+        for (int u = 0; u < CB * CB / CNT; ++u) {
+            const int e = t + u * CNT;
+            const int pi = e % CB, pk = e / CB;      // physical row and column
+            const int i = phys(min(pi, rows - 1)), k = phys(min(pk, rows - 1));
+            const double v = pi < rows && pk < rows && i >= k ? D[k * L + i] : 0.0;
+            bad = bad || !__builtin_isfinite(v);
+            out[e] = v;
+        }
+        return bad;
+    };
+    if (store()) odd = 1;
+    __syncthreads();
+    if (__builtin_expect(odd, 0)) {
+        load();
+        __syncthreads();
+        tri::invert_by_substitution<double, CB, UNIT>(D, t, out, CB);
+        store();
     }
 #pragma unroll
     for (int d = 1; d <= 2; ++d) {

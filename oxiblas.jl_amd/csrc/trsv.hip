@@ -95,6 +95,7 @@ __global__ __launch_bounds__(NT) void trsv_prepare_kernel(const TM* __restrict__
                                                           TV* __restrict__ G) {
     constexpr int L = tri::LD<RB>;
     __shared__ TV D[tri::SPACE<RB>];
+    __shared__ int odd;                       // the inverse is not finite
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int b = blockIdx.x;
     const i64 lo = i64(b) * RB;
@@ -104,16 +105,20 @@ __global__ __launch_bounds__(NT) void trsv_prepare_kernel(const TM* __restrict__
     auto phys = [&](int k) __attribute__((always_inline)) { return BWD ? rows - 1 - k : k; };
     // D(i, k) = T(i, k), the identity outside the block; the index that runs
     // along M's columns changes fastest.  Loads without branches.
+    auto load = [&]() __attribute__((always_inline)) {
 #pragma unroll 16
-    for (int u = 0; u < RB * RB / NT; ++u) {
-        const int e = t + u * NT;
-        const int x = e % RB, y = e / RB;
-        const int i = TRANS ? y : x, k = TRANS ? x : y;
-        const int ic = phys(min(i, rows - 1)), kc = phys(min(k, rows - 1));
-        const TM v = TRANS ? M[(p0 + kc) + (p0 + ic) * ld] : M[(p0 + ic) + (p0 + kc) * ld];
-        const bool in = i < rows && k < rows;
-        D[k * L + i] = i == k ? (UNIT || !in ? TV(1) : TV(v)) : in && i > k ? TV(v) : TV(0);
-    }
+        for (int u = 0; u < RB * RB / NT; ++u) {
+            const int e = t + u * NT;
+            const int x = e % RB, y = e / RB;
+            const int i = TRANS ? y : x, k = TRANS ? x : y;
+            const int ic = phys(min(i, rows - 1)), kc = phys(min(k, rows - 1));
+            const TM v = TRANS ? M[(p0 + kc) + (p0 + ic) * ld] : M[(p0 + ic) + (p0 + kc) * ld];
+            const bool in = i < rows && k < rows;
+            D[k * L + i] = i == k ? (UNIT || !in ? TV(1) : TV(v)) : in && i > k ? TV(v) : TV(0);
+        }
+    };
+    load();
+    if (t == 0) odd = 0;
     TV tv[RB / 4];
     if (b > 0) {
         const i64 q0 = BWD ? n - i64(b) * RB : i64(b - 1) * RB;
@@ -128,11 +133,26 @@ __global__ __launch_bounds__(NT) void trsv_prepare_kernel(const TM* __restrict__
     __syncthreads();
     tri::invert<TV, RB, NT / 64, UNIT>(D, t);
     TV* out = inv + size_t(b) * RB * RB;
+    // true where an element is not finite
+    auto store = [&]() __attribute__((always_inline)) {
+        bool bad = false;
 #pragma unroll 16
-    for (int u = 0; u < RB * RB / NT; ++u) {
-        const int e = t + u * NT;
-        const int i = e % RB, k = e / RB;
-        out[e] = i >= k && i < rows ? D[k * L + i] : TV(0);
+        for (int u = 0; u < RB * RB / NT; ++u) {
+            const int e = t + u * NT;
+            const int i = e % RB, k = e / RB;
+            const TV v = i >= k && i < rows ? D[k * L + i] : TV(0);
+            bad = bad || !__builtin_isfinite(v);
+            out[e] = v;
+        }
+        return bad;
+    };
+    if (store()) odd = 1;
+    __syncthreads();
+    if (__builtin_expect(odd, 0)) {
+        load();
+        __syncthreads();
+        tri::invert_by_substitution<TV, RB, UNIT>(D, t, out, RB);
+        store();
     }
     if (b > 0) {
         TV* g = G + size_t(b) * RB * RB + size_t(w) * 16 * RB;

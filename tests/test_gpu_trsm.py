@@ -215,3 +215,47 @@ def test_trsm_graded_triangles(gpu, rng, side, uplo, trans, diag):
             assert fin.any()
             R = np.abs(op @ X - B)
             assert (R <= (n + 2) * (EPS / 2) * (np.abs(op) @ np.abs(X) + np.abs(B))).all()
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+@pytest.mark.parametrize("n,i,k", [(100, 50, 53), (200, 100, 103), (200, 150, 163), (385, 300, 301)])
+@pytest.mark.parametrize("nrhs", [1, 8])
+@pytest.mark.parametrize("lowp", [False, True])
+def test_solve_with_nonfinite_factor(gpu, rng, value, n, i, k, nrhs, lowp):
+    """U(i, k) not finite, inside a diagonal block that the solves invert: rows
+    i + 1 on of x do not depend on it and are what substitution gives, rows up
+    to i are not finite.  (L is the identity.)"""
+    A = np.triu(rng.standard_normal((n, n)) / n) + np.diag(1.0 + rng.random(n))
+    A = np.asfortranarray(A.astype(np.float32) if lowp else A)
+    F = gpu.lu_lowp(A, "float32") if lowp else gpu.lu(A)
+    F.factors.buf[F.factors.offset + i + k * F.factors.ld] = value
+    B = np.asfortranarray(rng.standard_normal((n, nrhs)).astype(A.dtype))
+    X = F.solve(B)
+    X = X.numpy() if hasattr(X, "numpy") else X
+    assert not np.isfinite(X[:i + 1]).any()
+    assert np.isfinite(X[i + 1:]).all()
+    R = A[i + 1:, i + 1:].astype(float) @ X[i + 1:].astype(float) - B[i + 1:]
+    eps = np.finfo(A.dtype).eps
+    assert np.linalg.norm(R) <= 8 * n * eps * (np.linalg.norm(A) * np.linalg.norm(X[i + 1:]) + np.linalg.norm(B))
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+@pytest.mark.parametrize("side,uplo,trans", list(itertools.product("LR", "UL", "NT")))
+@pytest.mark.parametrize("n,other", [(200, 24), (512, 24), (512, 700)])
+def test_trsm_nonfinite_triangle(gpu, rng, value, side, uplo, trans, n, other):
+    """An element of the triangle that is not finite, inside a 16 x 16 tile of a
+    diagonal block: what is solved before its row is finite and right."""
+    T = tri(rng, n, uplo, False)
+    lo, hi = 101, 107
+    T0 = T.copy()
+    T[(lo, hi) if uplo == "U" else (hi, lo)] = value
+    m, k = (n, other) if side == "L" else (other, n)
+    B = np.asfortranarray(rng.standard_normal((m, k)))
+    X = gpu.trsm_(B.copy(order="F"), T, 1.0, side, uplo, trans)
+    Xo = oracle_trsm(B, T0, side, uplo, trans, "N")
+    if side == "R":
+        X, Xo = X.T, Xo.T
+    up = (uplo == "U") ^ (trans == "T") ^ (side == "R")       # solved from the last row (column) up
+    first, rest = (slice(lo + 1, None), slice(None, lo + 1)) if up else (slice(None, hi), slice(hi, None))
+    assert not np.isfinite(X[rest]).any() and np.isfinite(X[first]).all()
+    assert np.abs(X[first] - Xo[first]).max() <= 1e-12 * np.abs(Xo[first]).max() * n
