@@ -144,8 +144,11 @@ __global__ __launch_bounds__(256) void transpose_square_kernel(T* __restrict__ A
 constexpr int PERM_MAX_STEPS = 512;
 constexpr int HASH = 2048;
 
+// failed (may be null): a word that is set when a panel's wait has timed out; its
+// pivots were not written then, and the list is empty.
 __global__ __launch_bounds__(256) void perm_pairs_kernel(const i64* __restrict__ ipiv, i64 poff, i64 k1, int cnt,
-                                                         int inverse, int* __restrict__ pairs /*[2*2*cnt+1]*/) {
+                                                         int inverse, const int* __restrict__ failed,
+                                                         int* __restrict__ pairs /*[2*2*cnt+1]*/) {
     __shared__ int pv[PERM_MAX_STEPS];     // 0-based pivot row of each step
     __shared__ int prv[PERM_MAX_STEPS];    // prev(t)
     __shared__ int sm[PERM_MAX_STEPS];     // same(s)
@@ -153,12 +156,17 @@ __global__ __launch_bounds__(256) void perm_pairs_kernel(const i64* __restrict__
     __shared__ int islast[PERM_MAX_STEPS];
     __shared__ int slot_row[2 * PERM_MAX_STEPS], slot_src[2 * PERM_MAX_STEPS];
     __shared__ int hkey[HASH], hval[HASH];
-    __shared__ int np, ordered, unresolved;
+    __shared__ int np, ordered, unresolved, stop;
     const int t = threadIdx.x, nt = blockDim.x;
     const int K1 = int(k1);
-    if (t == 0) { np = 0; ordered = 1; unresolved = 0; }
+    // one thread reads the word: a leaf of the next panel may set it meanwhile
+    if (t == 0) { np = 0; ordered = 1; unresolved = 0; stop = failed ? *failed : 0; }
     for (int i = t; i < cnt; i += nt) pv[i] = int(ipiv[k1 + i] - 1 - poff);
     __syncthreads();
+    if (stop) {
+        if (t == 0) pairs[0] = 0;
+        return;
+    }
     for (int i = t; i < cnt; i += nt) {
         if (pv[i] < K1 + i) ordered = 0;
         prv[i] = -1; islast[i] = 1;
@@ -315,7 +323,8 @@ __global__ __launch_bounds__(256) void apply_pairs_w_kernel(T* __restrict__ Wm, 
 // the chain between two panels: 9.6 us for 64 columns in FP64, against 17 for
 // the pair list, its application and the TRSM, and two launches more (LU solve
 // n = 2000: 5.21 -> 5.01 ms).  The triangle goes through LDS: fetched by every
-// wave, a column a lane, 11.6 us.
+// wave, a column a lane, 11.6 us.  Nothing is touched when a leaf's wait has timed
+// out (failed), whose pivots were not written.
 __device__ __forceinline__ double lane_of(double v, int l) {
     const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
     const unsigned lo = __builtin_amdgcn_readlane(unsigned(u), l), hi = __builtin_amdgcn_readlane(unsigned(u >> 32), l);
@@ -330,15 +339,18 @@ __device__ __forceinline__ float nfma(float a, float b, float c) { return __buil
 constexpr int SW = 64;
 template <typename T>
 __global__ __launch_bounds__(256) void swap_solve_kernel(T* __restrict__ Wm, i64 ldw, i64 k1,
-                                                         const i64* __restrict__ ipiv, i64 c0, i64 c1) {
+                                                         const i64* __restrict__ ipiv, i64 c0, i64 c1,
+                                                         const int* __restrict__ failed) {
     __shared__ T U[SW * (SW + 1)];                    // U[q * (SW + 1) + s] = L11^T(s, q)
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const bool mine = c0 + i64(blockIdx.x) * 4 + w < c1;
     const i64 c = mine ? c0 + i64(blockIdx.x) * 4 + w : c0;
+    const int stop = *failed;
     const int p = int(ipiv[k1 + lane] - 1 - k1);
     T d[SW / 4];                                      // columns w, w + 4, .. of the triangle
 #pragma unroll
     for (int i = 0; i < SW / 4; ++i) d[i] = Wm[k1 + lane + (k1 + w + 4 * i) * ldw];
+    if (stop) return;                                 // the same in every wave: no leaf is running
     int first = lane;                                 // the first step that reaches the same row
 #pragma unroll 8
     for (int s = SW - 1; s >= 0; --s) first = __builtin_amdgcn_readlane(p, s) == p ? s : first;
@@ -458,7 +470,8 @@ int swap_w(GetrfCtx<T>& g, i64 k1, i64 k2, i64 c0, i64 c1, int inverse) {
     if (k2 < k1 || c1 <= c0) return OXI_OK;
     const int cnt = int(k2 - k1 + 1);
     if (cnt > PERM_MAX_STEPS) return oxi_set_error(g.h, OXI_ERR_UNSUPPORTED, "laswp block of %d steps", cnt);
-    hipLaunchKernelGGL(perm_pairs_kernel, dim3(1), dim3(256), 0, g.s, g.ipiv, i64(0), k1, cnt, inverse, g.pairs);
+    hipLaunchKernelGGL(perm_pairs_kernel, dim3(1), dim3(256), 0, g.s, g.ipiv, i64(0), k1, cnt, inverse, g.flags,
+                       g.pairs);
     OXI_TRY(launch_check(g.h, "perm_pairs"));
     const size_t shm = size_t(2 * cnt) * (PAIR_ROWS * sizeof(T) + 2 * sizeof(int));
     hipLaunchKernelGGL(apply_pairs_w_kernel<T>, dim3(unsigned(cdiv(c1 - c0, PAIR_ROWS))), dim3(256), shm, g.s, g.Wm,
@@ -475,7 +488,7 @@ template <typename T>
 int swap_solve(GetrfCtx<T>& g, i64 j0, i64 j1, i64 c0, i64 c1) {
     if (j1 - j0 == SW && c1 - c0 <= 2 * SW) {
         hipLaunchKernelGGL(swap_solve_kernel<T>, dim3(unsigned(cdiv(c1 - c0, 4))), dim3(256), 0, g.s, g.Wm, g.ldw, j0, g.ipiv,
-                           c0, c1);
+                           c0, c1, g.flags);
         return launch_check(g.h, "swap_solve");
     }
     OXI_TRY(swap_w(g, j0, j1 - 1, c0, c1, 0));
@@ -523,14 +536,14 @@ int leaf(GetrfCtx<T>& g, i64 c0, int w) {
     // a leaf's number since the exchange buffer was cleared, 64 tags each; the
     // buffer is cleared (in stream order, after the last leaf that used it)
     // before the numbers run out, so no tag occurs twice in it
-    if (g.h->leaf_seq >= (1u << 26) - 1) {
+    if (g.h->leaf_seq >= g.h->leaf_tags) {
         hipLaunchKernelGGL(zero_u64_kernel, dim3(256), dim3(256), 0, g.s, g.h->leaf_pub, OXI_LEAF_PUB);
         OXI_TRY(launch_check(g.h, "leaf exchange clear"));
         g.h->leaf_seq = 0;
     }
     const unsigned tag = ++g.h->leaf_seq << 6;
     LeafArgs a{(void*)g.Wm, g.ldw, c0, w, mrows, g.ipiv, g.dinfo, g.tag0, g.tpub, tag, g.h->leaf_pub, int(P),
-               g.flags, g.pc0, g.pc1};
+               g.flags, g.pc0, g.pc1, g.h->leaf_spins};
     if (tournament && kind <= 1 && P <= OXI_TP_MAX_P) return oxi_launch_lu_leaf_tp(g.h, g.s, a, kind);
     if (sizeof(T) == 8) OXI_TRY(oxi_launch_lu_leaf(g.h, g.s, a, kind));
     else OXI_TRY(oxi_launch_lu_leaf32(g.h, g.s, a, kind));
@@ -1019,7 +1032,7 @@ extern "C" int oxi_dlaswp_noalloc(oxi_handle_t h, int64_t ncols, double* A, int6
         const i64 b = inverse ? nblocks - 1 - bi : bi;
         const i64 s1 = (k1 - 1) + b * PERM_MAX_STEPS;
         const int cnt = int(std::min<i64>(PERM_MAX_STEPS, (k2 - 1) - s1 + 1));
-        hipLaunchKernelGGL(perm_pairs_kernel, dim3(1), dim3(256), 0, s, ipiv, i64(0), s1, cnt, inverse, sp);
+        hipLaunchKernelGGL(perm_pairs_kernel, dim3(1), dim3(256), 0, s, ipiv, i64(0), s1, cnt, inverse, (const int*)nullptr, sp);
         const size_t shm = size_t(2 * cnt) * sizeof(double);
         hipLaunchKernelGGL(apply_pairs_cm_kernel, dim3(unsigned(ncols)), dim3(256), shm, s, A, lda, ncols, sp, i64(0));
         OXI_TRY(launch_check(h, "laswp"));
@@ -1061,7 +1074,7 @@ extern "C" int oxi_dlaswp(oxi_handle_t h, int64_t ncols, double* A, int64_t lda,
         const i64 b = inverse ? nblocks - 1 - bi : bi;
         const i64 s1 = (k1 - 1) + b * PERM_MAX_STEPS;
         const int cnt = int(std::min<i64>(PERM_MAX_STEPS, (k2 - 1) - s1 + 1));
-        hipLaunchKernelGGL(perm_pairs_kernel, dim3(1), dim3(256), 0, s, ipiv, i64(0), s1, cnt, inverse, pairs);
+        hipLaunchKernelGGL(perm_pairs_kernel, dim3(1), dim3(256), 0, s, ipiv, i64(0), s1, cnt, inverse, (const int*)nullptr, pairs);
         const size_t shm = size_t(2 * cnt) * sizeof(double);
         hipLaunchKernelGGL(apply_pairs_cm_kernel, dim3(unsigned(ncols)), dim3(256), shm, s, A, lda, ncols, pairs, i64(0));
         OXI_TRY(launch_check(h, "laswp"));

@@ -2,6 +2,7 @@
 #include "oxi_internal.hpp"
 
 #include <hip/hip_ext.h>
+#include <algorithm>
 #include <cstdlib>
 
 #include <cstdarg>
@@ -85,6 +86,8 @@ int oxi_create(int device, oxi_handle_t* handle) {
             return OXI_ERR_HIP;
         }
     }
+    if (const char* e = getenv("OXIBLAS_LEAF_TAGS")) h->leaf_tags = std::clamp(unsigned(atoi(e)), 1u, h->leaf_tags);
+    if (const char* e = getenv("OXIBLAS_LEAF_SPINS")) h->leaf_spins = std::min(unsigned(atoi(e)), h->leaf_spins);
     (void)hipMemset(h->dev_flags, 0, 64 * sizeof(int));
     (void)hipMemset(h->dev_info, 0, 8 * sizeof(i64));
     (void)hipMemset(h->leaf_pub, 0, size_t(OXI_LEAF_PUB) * 8);

@@ -54,6 +54,9 @@ struct oxi_handle_s {
     // run since it was last cleared: a leaf's words are tagged with its number
     unsigned long long* leaf_pub = nullptr;
     unsigned leaf_seq = 0;
+    // leaves between two clears (64 tags each) and the polls that a leaf's wait
+    // is bounded by; OXIBLAS_LEAF_TAGS and OXIBLAS_LEAF_SPINS lower them (tests)
+    unsigned leaf_tags = (1u << 26) - 1, leaf_spins = 1u << 22;
 };
 
 int oxi_set_error(oxi_handle_t h, int code, const char* fmt, ...);
@@ -231,6 +234,7 @@ struct LeafArgs {
     int P;
     int* flags;      // flags[0] = 1 on barrier timeout
     i64 xlo, xhi;    // columns [xlo, xhi) of the enclosing panel: receive the leaf's interchanges
+    unsigned spins;  // bound of every wait, in polls
 };
 
 // kind 0: 256 threads x 1 row per workgroup, leaves of up to 64 columns;

@@ -315,8 +315,7 @@ __global__ __launch_bounds__(256) void lu_leaf_kernel(LeafArgs a) {
     constexpr int LT = 256, NWV = LT / 64, NB = W / 16;   // NB: values of a row per lane of its spread form
     static_assert(W == 32 || W == 64, "record layout");
     constexpr bool MULTI = WGS != 1;                  // WGS: 1, 64 or OXI_LEAF_MAX_P workgroups at most
-    unsigned spin_limit = 1u << 22;                   // bound of every wait
-    asm volatile("" : "+s"(spin_limit));              // not a constant: the polling loops stay rolled
+    const unsigned spin_limit = a.spins;              // bound of every wait
     __shared__ __align__(16) int4 wcand[2][NWV];                   // each wave's candidate: key, low word, position; failed
     __shared__ __align__(16) T raw[W];                             // the chosen row before the pending update
     __shared__ T raw_l;                                            // !MULTI: its multiplier
@@ -590,7 +589,10 @@ __global__ __launch_bounds__(256) void lu_leaf_kernel(LeafArgs a) {
         d = readlane_t(dl, gl);
         u1 = readlane_t(ul, gl);
         piv = __builtin_amdgcn_readlane(hp, gl);
-        if (spins > spin_limit) timed_out = true;
+        if (spins > spin_limit) {   // what came is not this column's: keep positions in range until the leaf ends
+            timed_out = true;
+            piv = jn;
+        }
     };
 
     // column 0: the registers as loaded

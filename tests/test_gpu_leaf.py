@@ -97,3 +97,68 @@ def test_interchanges_of_panels_exact(gpu, rng, n, kind):
             assert q >= i
             perm[[i, q]] = perm[[q, i]]
         assert np.array_equal((np.tril(LU, -1) + np.eye(n)) @ np.triu(LU), A[perm]), lowp
+
+
+@pytest.fixture
+def own_handle(gpu, monkeypatch):
+    """A handle of its own, made under the given environment, in place of the
+    device's while the test runs."""
+    from oxiblas_mi355x import _lib
+    made = []
+
+    def make(**env):
+        for k, v in env.items():
+            monkeypatch.setenv(k, v)
+        h = gpu.Handle(0)
+        made.append(h)
+        monkeypatch.setitem(_lib._handles, 0, h)
+        return h
+    yield make
+    import torch
+    torch.cuda.synchronize()
+    for h in made:
+        h.close()
+
+
+@pytest.mark.parametrize("n,nb", [(600, 0), (700, 64), (1500, 0), (2600, 128)])
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+def test_wait_that_gives_up(gpu, rng, own_handle, n, nb, dtype):
+    """Leaves whose waits give up at once: the call reports it, pivots that were
+    never written are not followed (they name rows far outside), and nothing
+    around the matrix changes; one-workgroup factorizations still work."""
+    import ctypes as C
+    import torch
+    h = own_handle(OXIBLAS_LEAF_SPINS="0")
+    dt = torch.float64 if dtype == "f64" else torch.float32
+    pad, ld = 4096, n + 5
+    buf = torch.randn(2 * pad + ld * n, dtype=dt, device="cuda", generator=torch.Generator(device="cuda").manual_seed(n))
+    before = buf.clone()
+    ipiv = torch.full((n,), 1 << 40, dtype=torch.int64, device="cuda")
+    info = C.c_int64(0)
+    A = buf.data_ptr() + pad * buf.element_size()
+    h.bind_stream(torch.cuda.current_stream().cuda_stream)
+    if dtype == "f64":
+        rc = h._L.oxi_dgetrf(h.ptr, n, n, A, ld, ipiv.data_ptr(), nb, C.byref(info))
+    else:
+        rc = h._L.oxi_sgetrf_lowp(h.ptr, 3, n, n, A, ld, ipiv.data_ptr(), nb, C.byref(info))
+    assert rc == 5                                       # OXI_ERR_TIMEOUT
+    outside = torch.ones(buf.numel(), dtype=torch.bool, device="cuda")
+    outside[pad:pad + ld * n].view(n, ld)[:, :n] = False
+    assert torch.equal(buf[outside], before[outside])
+    check(gpu, rng.standard_normal((300, 32)))
+
+
+@pytest.mark.parametrize("n", [513, 1000])
+def test_exchange_buffer_cleared_between_leaves(gpu, rng, own_handle, n):
+    """The exchange buffer cleared after every second leaf, where the tags start
+    again: the same factors as without."""
+    A = rng.standard_normal((n, n))
+    F = gpu.lu(gpu.DMatrix.from_numpy(A))
+    F32 = gpu.lu_lowp(A.astype(np.float32), "float32")
+    own_handle(OXIBLAS_LEAF_TAGS="2")
+    for _ in range(2):
+        G = gpu.lu(gpu.DMatrix.from_numpy(A))
+        np.testing.assert_array_equal(F.ipiv, G.ipiv)
+        np.testing.assert_array_equal(F.factors.numpy(), G.factors.numpy())
+        G = gpu.lu_lowp(A.astype(np.float32), "float32")
+        np.testing.assert_array_equal(F32.factors.numpy(), G.factors.numpy())
