@@ -13,7 +13,7 @@
 //
 // Algorithm (the reference's, in W's coordinates):
 //   for each panel of nb columns:
-//     getrf2 recursion on the panel (halving, leaves of <= 64 columns)
+//     getrf2 recursion on the panel (halving, leaves of <= 32 columns)
 //     interchanges applied to the columns left and right of the panel
 //     U12 <- L11^-1 A12           (right-side solve with L11^T in W)
 //     A22 <- A22 - L21*U12        (FP64 MFMA GEMM)
@@ -321,8 +321,8 @@ __global__ __launch_bounds__(256) void apply_pairs_w_kernel(T* __restrict__ Wm, 
 // Every step p_s >= s (0-based, from k1), as LU pivots are.
 // Bound by three memory round trips and 64 dependent steps, twice; it stands on
 // the chain between two panels: 9.6 us for 64 columns in FP64, against 17 for
-// the pair list, its application and the TRSM, and two launches more (LU solve
-// n = 2000: 5.21 -> 5.01 ms).  The triangle goes through LDS: fetched by every
+// the pair list, its application and the TRSM, and two launches more (LU of
+// n = 256: 599 -> 552 us, 1000: 2430 -> 2310 us).  The triangle goes through LDS: fetched by every
 // wave, a column a lane, 11.6 us.  Nothing is touched when a leaf's wait has timed
 // out (failed), whose pivots were not written.
 __device__ __forceinline__ double lane_of(double v, int l) {
@@ -510,19 +510,6 @@ int leaf_kind(const GetrfCtx<T>& g, i64 c0) {
     const bool tournament = sizeof(T) == 4 && g.tournament;
     return mrows > 8192 || (!tournament && mrows > 256 && mrows <= 512) ? 1 : 0;
 }
-// Columns of the widest leaf at c0: 64 in FP64 where a row of 64 fits a thread's
-// registers (one row per thread), else 32.  A 64-column leaf takes 133 us at
-// 2000 rows against 123 for two of 32, which need a triangular solve and a
-// product between them (11 us and two launches).  Not in FP32: there the 32
-// columns' products are summed before they meet the next 32, in a 64-column
-// leaf they round one by one, and the factor's error shows in the mixed solve
-// (4096 shifted: the FP32 solve's error 2.6e-7 with leaves of 32 and panels of
-// 128, 3.2e-7 with 64 and 64; 10.6 ms a factor against 9.2).
-template <typename T>
-i64 leaf_width(const GetrfCtx<T>& g, i64 c0) {
-    return sizeof(T) == 8 && leaf_kind(g, c0) == 0 ? OXI_LEAF_W : 32;
-}
-
 template <typename T>
 int leaf(GetrfCtx<T>& g, i64 c0, int w) {
     const i64 mrows = g.m - c0;
@@ -533,7 +520,7 @@ int leaf(GetrfCtx<T>& g, i64 c0, int w) {
     if (P > std::min<i64>(g.h->num_cus, OXI_LEAF_MAX_P))
         return oxi_set_error(g.h, OXI_ERR_UNSUPPORTED, "panel of %lld rows exceeds the leaf kernel capacity",
                              (long long)mrows);
-    // a leaf's number since the exchange buffer was cleared, 64 tags each; the
+    // a leaf's number since the exchange buffer was cleared, 32 tags each; the
     // buffer is cleared (in stream order, after the last leaf that used it)
     // before the numbers run out, so no tag occurs twice in it
     if (g.h->leaf_seq >= g.h->leaf_tags) {
@@ -541,7 +528,7 @@ int leaf(GetrfCtx<T>& g, i64 c0, int w) {
         OXI_TRY(launch_check(g.h, "leaf exchange clear"));
         g.h->leaf_seq = 0;
     }
-    const unsigned tag = ++g.h->leaf_seq << 6;
+    const unsigned tag = ++g.h->leaf_seq << 5;
     LeafArgs a{(void*)g.Wm, g.ldw, c0, w, mrows, g.ipiv, g.dinfo, g.tag0, g.tpub, tag, g.h->leaf_pub, int(P),
                g.flags, g.pc0, g.pc1, g.h->leaf_spins};
     if (tournament && kind <= 1 && P <= OXI_TP_MAX_P) return oxi_launch_lu_leaf_tp(g.h, g.s, a, kind);
@@ -558,7 +545,7 @@ int leaf(GetrfCtx<T>& g, i64 c0, int w) {
 // half" at every level.
 template <typename T>
 int panel(GetrfCtx<T>& g, i64 c0, i64 np) {
-    if (np <= leaf_width(g, c0)) return leaf(g, c0, int(np));
+    if (np <= OXI_LEAF_W) return leaf(g, c0, int(np));
     const i64 mp = g.m - c0;
     const i64 h = np / 2;
     OXI_TRY(panel(g, c0, h));
@@ -602,15 +589,16 @@ bool timed_update(i64 rows, i64 cols) {
     return sizeof(T) == 8 ? oxi_dgemm_large(rows, cols) : true;
 }
 
-// Tuned block size: the panels bound the factorization, and up to about 5000
-// columns a panel of one 64-column leaf (FP64) needs no product of its own (n =
-// 2000: 4.95 ms with 64, 5.10 with 128; 4096: 10.5 and 10.6; 6000: 16.8 and
-// 16.5; 8192: 28.0, 24.7 and, with 256, 24.6).  FP32 keeps 128 from 1024 on: an
-// element rounds once per panel.
-int choose_nb(i64 m, i64 n, bool fp32) {
+// Tuned block size.  Narrower leaves' products are summed before they meet an
+// element, which so rounds once per leaf and panel: leaves of 64 columns, and
+// panels of 64 from 1024 to 5120 columns, take 5.02 ms at n = 2000 against 5.32, but
+// the error of x grows (systems shifted by 2 sqrt(n), against extended
+// precision: 256 columns 3.3e-16 -> 4.2e-16, 2000 4.0e-16 -> 4.7e-16, 4096
+// 5.2e-16 -> 6.1e-16; FP32 likewise).
+int choose_nb(i64 m, i64 n) {
     const i64 q = std::min(m, n);
     if (q >= 8192) return 256;
-    if (q >= (fp32 ? 1024 : 5120)) return 128;
+    if (q >= 1024) return 128;
     return 64;
 }
 
@@ -623,7 +611,7 @@ int getrf_t(oxi_handle_t h, i64 m, i64 n, T* A, i64 lda, i64* ipiv, i64 nb, i64*
     hipStream_t s = h->stream;
     const i64 q = std::min(m, n);
     const bool tuned = nb == 0;
-    if (nb == 0) nb = choose_nb(m, n, sizeof(T) == 4);
+    if (nb == 0) nb = choose_nb(m, n);
     if (nb > PERM_MAX_STEPS) nb = PERM_MAX_STEPS;
     // Tuned block size on large matrices: 512-wide panels while more than 3/8
     // of the columns remain (the trailing update bounds those steps and runs

@@ -54,9 +54,9 @@ struct oxi_handle_s {
     // run since it was last cleared: a leaf's words are tagged with its number
     unsigned long long* leaf_pub = nullptr;
     unsigned leaf_seq = 0;
-    // leaves between two clears (64 tags each) and the polls that a leaf's wait
+    // leaves between two clears (32 tags each) and the polls that a leaf's wait
     // is bounded by; OXIBLAS_LEAF_TAGS and OXIBLAS_LEAF_SPINS lower them (tests)
-    unsigned leaf_tags = (1u << 26) - 1, leaf_spins = 1u << 22;
+    unsigned leaf_tags = (1u << 27) - 1, leaf_spins = 1u << 22;
 };
 
 int oxi_set_error(oxi_handle_t h, int code, const char* fmt, ...);
@@ -212,7 +212,7 @@ int oxi_first_zero_diag(oxi_handle_t h, hipStream_t s, const double* T, i64 ldt,
 // ---------------------------------------------------------------------------
 // Panel leaf of the LU (panel.hip)
 // ---------------------------------------------------------------------------
-constexpr int OXI_LEAF_W = 64;      // maximum leaf width
+constexpr int OXI_LEAF_W = 32;      // maximum leaf width
 constexpr int OXI_PUB_STRIDE = 2 * OXI_LEAF_W;   // words per published (column, workgroup) row
 constexpr int OXI_PUB_HDR = 16;     // and of its header (a 128-byte line)
 constexpr int OXI_LEAF_MAX_P = 127; // workgroups of one leaf
@@ -223,7 +223,7 @@ constexpr int OXI_TP_PUB = 4096;    // doubles of the tournament leaf's records
 struct LeafArgs {
     void* Wm; i64 ldw;   // double* or float*
     i64 c0;          // first column (A) of the leaf = its first diagonal row
-    int w;           // leaf width <= LEAF_W (32 where a thread holds two rows or more)
+    int w;           // leaf width <= LEAF_W
     i64 mrows;       // rows c0 .. c0+mrows-1 of A
     i64* ipiv;       // global pivots (1-based rows), entries c0..c0+w-1 written
     i64* info;       // device info (first zero pivot, 1-based), 0 if none
@@ -237,14 +237,13 @@ struct LeafArgs {
     unsigned spins;  // bound of every wait, in polls
 };
 
-// kind 0: 256 threads x 1 row per workgroup, leaves of up to 64 columns;
-// kind 1: 256 threads x 2 rows, up to 32 columns.
+// kind 0: 256 threads x 1 row per workgroup; kind 1: 256 threads x 2 rows.
 int oxi_launch_lu_leaf(oxi_handle_t h, hipStream_t s, const LeafArgs& a, int kind);
 // FP32 leaf with tournament pivoting (panel_tp.hip), kind 0 or 1, at most
 // OXI_TP_MAX_P workgroups.
 constexpr int OXI_TP_MAX_P = 32;
 int oxi_launch_lu_leaf_tp(oxi_handle_t h, hipStream_t s, const LeafArgs& a, int kind);
-// FP32 leaf, up to 32 columns; kind 2: 256 threads x 4 rows.
+// FP32 leaf; kind 2: 256 threads x 4 rows.
 int oxi_launch_lu_leaf32(oxi_handle_t h, hipStream_t s, const LeafArgs& a, int kind);
 
 // Bracket one trailing-update GEMM launch with profiling events (no-op when

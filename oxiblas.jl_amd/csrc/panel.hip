@@ -1,5 +1,5 @@
 // Panel leaf of the blocked LU: column-by-column elimination of an m x w
-// block (w <= 64) held in registers across P co-resident workgroups.
+// block (w <= 32) held in registers across P co-resident workgroups.
 //
 // Restates the leaf of _lu_panel! (src/lapack/factorizations.jl:116-140) with
 // the pivot choice of _lu_pivot (:89-107): the pivot is the first row of
@@ -27,12 +27,9 @@
 #include "panel_kernel.hpp"
 
 int oxi_launch_lu_leaf(oxi_handle_t h, hipStream_t s, const LeafArgs& a, int kind) {
-    const bool wide = a.w > 32;
-    if (a.P == 1 && kind == 0 && !wide) return launch_leaf(h, s, a, lu_leaf_kernel<double, 1, 32, 1>);
-    if (a.P == 1 && kind == 0) return launch_leaf(h, s, a, lu_leaf_kernel<double, 1, 64, 1>);
-    if (kind == 0 && !wide) return launch_leaf(h, s, a, lu_leaf_kernel<double, 1, 32, 64>);
-    if (kind == 0) return launch_leaf(h, s, a, lu_leaf_kernel<double, 1, 64, 64>);
-    if (a.P == 1) return launch_leaf(h, s, a, lu_leaf_kernel<double, 2, 32, 1>);
-    if (a.P <= 64) return launch_leaf(h, s, a, lu_leaf_kernel<double, 2, 32, 64>);
-    return launch_leaf(h, s, a, lu_leaf_kernel<double, 2, 32, OXI_LEAF_MAX_P>);
+    if (a.P == 1 && kind == 0) return launch_leaf(h, s, a, lu_leaf_kernel<double, 1, 1>);
+    if (kind == 0) return launch_leaf(h, s, a, lu_leaf_kernel<double, 1, 64>);
+    if (a.P == 1) return launch_leaf(h, s, a, lu_leaf_kernel<double, 2, 1>);
+    if (a.P <= 64) return launch_leaf(h, s, a, lu_leaf_kernel<double, 2, 64>);
+    return launch_leaf(h, s, a, lu_leaf_kernel<double, 2, OXI_LEAF_MAX_P>);
 }

@@ -5,9 +5,9 @@
 #include "panel_kernel.hpp"
 
 int oxi_launch_lu_leaf32(oxi_handle_t h, hipStream_t s, const LeafArgs& a, int kind) {
-    if (a.P == 1 && kind == 0) return launch_leaf(h, s, a, lu_leaf_kernel<float, 1, 32, 1>);
-    if (kind == 0) return launch_leaf(h, s, a, lu_leaf_kernel<float, 1, 32, 64>);
-    if (a.P == 1 && kind == 1) return launch_leaf(h, s, a, lu_leaf_kernel<float, 2, 32, 1>);
-    if (kind == 1) return launch_leaf(h, s, a, lu_leaf_kernel<float, 2, 32, 64>);
-    return launch_leaf(h, s, a, lu_leaf_kernel<float, 4, 32, OXI_LEAF_MAX_P>);
+    if (a.P == 1 && kind == 0) return launch_leaf(h, s, a, lu_leaf_kernel<float, 1, 1>);
+    if (kind == 0) return launch_leaf(h, s, a, lu_leaf_kernel<float, 1, 64>);
+    if (a.P == 1 && kind == 1) return launch_leaf(h, s, a, lu_leaf_kernel<float, 2, 1>);
+    if (kind == 1) return launch_leaf(h, s, a, lu_leaf_kernel<float, 2, 64>);
+    return launch_leaf(h, s, a, lu_leaf_kernel<float, 4, OXI_LEAF_MAX_P>);
 }

@@ -198,17 +198,19 @@ __device__ __forceinline__ void lds_barrier() {
 // backwards through the transpositions (step i exchanges slot i with slot
 // sb_i), so the steps carry no dependence between lanes: one readlane and two
 // selects per slot and step.  A wave moves 32 slots of 64 columns (a lane per
-// column): the W / 16 waves of a group of columns load everything before any
+// column): the two waves of a group of columns load everything before any
 // of them stores (a wait and a barrier).  Loads are issued without branches: a
 // slot that does not move reads position 0, a lane outside the columns reads
 // column c0 (both in bounds), and only moving slots are stored.  Lane s
 // computes its slots' row offsets once; the loops only read them back.
 // ---------------------------------------------------------------------------
-template <typename T, int W>
+template <typename T>
 __device__ __forceinline__ void other_columns(T* Wm, i64 ldw, i64 c0, int w, int pi, i64 x_lo, i64 x_hi, int wg,
                                               int nwg) {
+    constexpr int W = OXI_LEAF_W;
     const int groups_l = int((c0 - x_lo + 63) / 64), groups = groups_l + int((x_hi - c0 - w + 63) / 64);
-    constexpr int GW = W / 16, GPW = 4 / GW;       // waves per group of columns, groups per workgroup
+    static_assert(2 * W == 64, "a slot per lane");
+    constexpr int GW = 2, GPW = 2;                 // waves per group of columns, groups per workgroup
     if (wg * GPW >= groups) return;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
@@ -220,32 +222,18 @@ __device__ __forceinline__ void other_columns(T* Wm, i64 ldw, i64 c0, int w, int
     }
     const int sbv = lane >= w ? lane : pi < w ? pi : W + first;   // the slot that step `lane` exchanges with its own
     const int outp = lane < w && pi >= w && first == lane ? pi : -1;
-    constexpr int SL = 2 * W / 64;                 // slots per lane: lane, and lane + 64
-    int x[SL], from[SL], to[SL];
-#pragma unroll
-    for (int k = 0; k < SL; ++k) x[k] = lane + 64 * k;
+    int x = lane;
 #pragma unroll 8
     for (int i = W - 1; i >= 0; --i) {
         const int sb = __builtin_amdgcn_readlane(sbv, i);
-#pragma unroll
-        for (int k = 0; k < SL; ++k) x[k] = x[k] == i ? sb : x[k] == sb ? i : x[k];
+        x = x == i ? sb : x == sb ? i : x;
     }
-    u64 mv[SL], offs[SL], offd[SL];
-#pragma unroll
-    for (int k = 0; k < SL; ++k) {
-        const int slot = lane + 64 * k;
-        const int out_of = __shfl(outp, slot & (W - 1));                  // of slot W + i
-        to[k] = slot < W ? (slot < w ? slot : -1) : out_of;
-        const int pi_of = __shfl(pi, x[k] & (W - 1));                     // position of slot W + i
-        from[k] = x[k] < W ? x[k] : pi_of;
-        const bool moves = to[k] >= 0 && x[k] != slot;
-        mv[k] = __ballot(moves);
-        offs[k] = u64((c0 + (moves ? from[k] : 0)) * ldw);
-        offd[k] = u64((c0 + (moves ? to[k] : 0)) * ldw);
-    }
+    const int out_of = __shfl(outp, lane & (W - 1)), pi_of = __shfl(pi, x & (W - 1));   // of slots W + i
+    const int to = lane >= W ? out_of : lane < w ? lane : -1, from = x < W ? x : pi_of;
+    const bool moves = to >= 0 && x != lane;
+    const u64 os = u64((c0 + (moves ? from : 0)) * ldw), od = u64((c0 + (moves ? to : 0)) * ldw);
     const int s0 = 32 * (wave % GW);               // this wave's slots s0 .. s0 + 31
-    const u64 moving = (SL == 2 && s0 >= 64 ? mv[SL - 1] : mv[0]) >> (s0 & 63);
-    const u64 os = SL == 2 && s0 >= 64 ? offs[SL - 1] : offs[0], od = SL == 2 && s0 >= 64 ? offd[SL - 1] : offd[0];
+    const u64 moving = __ballot(moves) >> s0;
 #pragma unroll 1
     for (int g0 = wg * GPW; g0 < groups; g0 += nwg * GPW) {
         const int g = g0 + wave / GW;
@@ -255,20 +243,20 @@ __device__ __forceinline__ void other_columns(T* Wm, i64 ldw, i64 c0, int w, int
         const i64 xr = ok ? xc : c0;
         T v[32];
 #pragma unroll
-        for (int k = 0; k < 32; ++k) v[k] = Wm[i64(readlane64(os, (s0 & 63) + k)) + xr];
+        for (int k = 0; k < 32; ++k) v[k] = Wm[i64(readlane64(os, s0 + k)) + xr];
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < 32; ++k)
             if ((moving >> k) & 1) {
-                const i64 to_row = i64(readlane64(od, (s0 & 63) + k));
+                const i64 to_row = i64(readlane64(od, s0 + k));
                 if (ok) Wm[to_row + xc] = v[k];
             }
     }
 }
 
 // ---------------------------------------------------------------------------
-// The leaf kernel (up to W columns).  Thread t of workgroup p holds the rows
+// The leaf kernel (up to W = 32 columns).  Thread t of workgroup p holds the rows
 // that start at positions p*R + s*256 + t (s < RPT) in registers, and they stay there: an
 // interchange only changes positions (pos[s]; a row that became the pivot of
 // step j is retired to position j, pos[s] = ~j).  The registers of a row
@@ -310,10 +298,10 @@ __device__ __forceinline__ void other_columns(T* Wm, i64 ldw, i64 c0, int w, int
 // the header, then the exchange; the row's trip through LDS and the update
 // run in the exchange's shadow.
 // ---------------------------------------------------------------------------
-template <typename T, int RPT, int W, int WGS>
+template <typename T, int RPT, int WGS>
 __global__ __launch_bounds__(256) void lu_leaf_kernel(LeafArgs a) {
-    constexpr int LT = 256, NWV = LT / 64, NB = W / 16;   // NB: values of a row per lane of its spread form
-    static_assert(W == 32 || W == 64, "record layout");
+    constexpr int W = OXI_LEAF_W, LT = 256, NWV = LT / 64, NB = W / 16;   // NB: values of a row per lane of its spread form
+    static_assert(W == 32, "record layout");
     constexpr bool MULTI = WGS != 1;                  // WGS: 1, 64 or OXI_LEAF_MAX_P workgroups at most
     const unsigned spin_limit = a.spins;              // bound of every wait
     __shared__ __align__(16) int4 wcand[2][NWV];                   // each wave's candidate: key, low word, position; failed
@@ -358,9 +346,8 @@ __global__ __launch_bounds__(256) void lu_leaf_kernel(LeafArgs a) {
     T rv[NB] = {};                          // its values 16 b + (lane & 15) in every row of 16 lanes
     T uu = T(0);                            // MULTI: its value that the lane publishing value c needs, c + 1
     unsigned row_off = 0, row_tag = 0;      // MULTI: the row's place in the exchange buffer, its tag
-    // the lane's column of a published row: two lanes per column (low and high
-    // half) up to 32 columns, one beyond
-    const int pc = W == 32 ? lane >> 1 : lane;
+    // the lane's column of a published row: two lanes per column (low and high half)
+    const int pc = lane >> 1;
     const unsigned oa = (lane & 15) * 16, ou = min(pc + 1, W - 1) * 16;
     const __amdgpu_buffer_rsrc_t pub_rsrc =
         __builtin_amdgcn_make_buffer_rsrc((void*)a.pub, 0, int(OXI_LEAF_PUB * 8), 0x00027000);
@@ -389,9 +376,6 @@ __global__ __launch_bounds__(256) void lu_leaf_kernel(LeafArgs a) {
             if (++spins > spin_limit) { timed_out = true; break; }   // uniform per wave
             const char* row = (const char*)a.pub + row_off;
             load_words3((const u64*)(row + oa), (const u64*)(row + oa + 256), (const u64*)(row + ou), x.b[0], x.b[1], x.u);
-            if constexpr (NB == 4)
-                load_words3((const u64*)(row + oa + 512), (const u64*)(row + oa + 768), (const u64*)(row + ou), x.b[2], x.b[3],
-                            x.u);
         }
 #pragma unroll
         for (int b = 0; b < NB; ++b) rv[b] = from_words<T>(x.b[b].x, x.b[b].z);
@@ -528,13 +512,8 @@ __global__ __launch_bounds__(256) void lu_leaf_kernel(LeafArgs a) {
                 if (PEND && upd) r = fma_t(-lw, uu, r);
                 if (none || pc >= W - jn) r = T(0);
                 u64* row = a.pub + (size_t(jn) * P + p) * OXI_PUB_STRIDE;
-                if constexpr (W == 32) {
-                    __hip_atomic_store(row + lane, tag | ((lane & 1) ? word_hi(r) : word_lo(r)), __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-                } else {
-                    __hip_atomic_store(row + 2 * lane, tag | word_lo(r), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    __hip_atomic_store(row + 2 * lane + 1, tag | word_hi(r), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
+                __hip_atomic_store(row + lane, tag | ((lane & 1) ? word_hi(r) : word_lo(r)), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
             }
             if (__builtin_expect(__ballot(e.w != 0) != 0, 0)) {   // a wave's wait timed out (the same in every wave)
                 if (t == 0) __hip_atomic_store(a.flags, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -734,7 +713,7 @@ __global__ __launch_bounds__(256) void lu_leaf_kernel(LeafArgs a) {
     }
     // the interchanges on the rest of the panel: columns that no workgroup
     // has touched
-    other_columns<T, W>(Wm, a.ldw, a.c0, w, lane < w ? my_piv : -1, a.xlo, a.xhi, p, P);
+    other_columns(Wm, a.ldw, a.c0, w, lane < w ? my_piv : -1, a.xlo, a.xhi, p, P);
 }
 
 // One leaf launch.  Every workgroup asks for LEAF_LDS bytes of LDS, far more

@@ -35,7 +35,7 @@
 
 namespace {
 
-constexpr int TW = 32;
+constexpr int TW = OXI_LEAF_W;           // 32
 constexpr int TLT = 256, TNWV = TLT / 64;
 constexpr int TP_LEVELS = 3;             // tree levels over workgroups: 32 -> 8 -> 2 -> 1
 constexpr int TP_REC = 36;               // record fields: tag, count, 32 positions, spare, checksum
@@ -394,7 +394,7 @@ __global__ __launch_bounds__(256) void tp_swaps_kernel(LeafArgs a) {
     // branch (lanes >= w read entry c0): one memory round trip for both
     const i64 pv = a.ipiv[a.c0 + (lane < a.w ? lane : 0)];
     if (__hip_atomic_load(a.flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return;
-    other_columns<float, TW>((float*)a.Wm, a.ldw, a.c0, a.w, lane < a.w ? int(pv - 1 - a.c0) : -1, a.xlo, a.xhi,
+    other_columns((float*)a.Wm, a.ldw, a.c0, a.w, lane < a.w ? int(pv - 1 - a.c0) : -1, a.xlo, a.xhi,
                              int(blockIdx.x), int(gridDim.x));
 }
 

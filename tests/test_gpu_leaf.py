@@ -162,3 +162,20 @@ def test_exchange_buffer_cleared_between_leaves(gpu, rng, own_handle, n):
         np.testing.assert_array_equal(F.factors.numpy(), G.factors.numpy())
         G = gpu.lu_lowp(A.astype(np.float32), "float32")
         np.testing.assert_array_equal(F32.factors.numpy(), G.factors.numpy())
+
+
+@pytest.mark.parametrize("lowp", [False, True])
+@pytest.mark.parametrize("n,width", [(64, 32), (150, 32), (700, 32), (513, 64), (1023, 64), (1100, 128), (2000, 128),
+                                     (4500, 128)])
+def test_products_summed_before_an_element_rounds(gpu, n, width, lowp):
+    """`width` products that together make 1 against an element of 2^53 (2^24):
+    subtracted as one sum the element is one less, one by one, or in two halves,
+    it stays.  Leaves have 32 columns, panels 64, and 128 from 1024 columns on."""
+    big = 2.0 ** 24 if lowp else 2.0 ** 53
+    A = np.zeros((n, n), dtype=np.float32 if lowp else np.float64)
+    i = np.arange(n)
+    A[i, i] = np.where(i < width, 4.0, big)
+    A[width:, :width] = 4.0 / width                  # multipliers 1 / width
+    A[:width, width:] = 1.0
+    F = gpu.lu_lowp(A, "float32") if lowp else gpu.lu(gpu.DMatrix.from_numpy(A))
+    assert F.factors.numpy()[width, width] == big - 1.0
