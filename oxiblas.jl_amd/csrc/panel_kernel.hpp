@@ -716,16 +716,21 @@ __global__ __launch_bounds__(256) void lu_leaf_kernel(LeafArgs a) {
     other_columns(Wm, a.ldw, a.c0, w, lane < w ? my_piv : -1, a.xlo, a.xhi, p, P);
 }
 
-// One leaf launch.  Every workgroup asks for LEAF_LDS bytes of LDS, far more
-// than it uses, so that it gets a CU of its own: beside a workgroup of the
-// trailing update (66 KB of LDS), whose waves compete for its SIMDs, a column
-// took 3.9 us at 16384 rows instead of 2.4.  getrf keeps 32 CUs free of them.
+// One leaf launch.  Up to as many workgroups as getrf keeps CUs free of the
+// trailing update ask for LEAF_LDS bytes of LDS each, far more than they use, so
+// that each gets one of those CUs to itself: beside a workgroup of the update
+// (66 KB of LDS), whose waves compete for its SIMDs, a column took 3.9 us at 16384
+// rows instead of 2.4.  More workgroups than that (above 16384 FP64 rows, 32768
+// FP32 rows) have to share CUs with the update, which the LDS would not let
+// them: the last would wait until both tiles of some CU end at once, and the
+// rest for them (n = 20000 132 ms with it, 124 without, 24576 230 and 206,
+// 33000 525 and 469; 17000 84.5 and 84.8).
 constexpr unsigned LEAF_LDS = 96 * 1024;
 template <typename K>
 int launch_leaf(oxi_handle_t h, hipStream_t s, const LeafArgs& a, K kernel) {
     const hipError_t se = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LEAF_LDS);
     if (se != hipSuccess) return oxi_set_error(h, OXI_ERR_HIP, "lu_leaf attribute: %s", hipGetErrorString(se));
-    hipLaunchKernelGGL(kernel, dim3(unsigned(a.P)), dim3(256), LEAF_LDS, s, a);
+    hipLaunchKernelGGL(kernel, dim3(unsigned(a.P)), dim3(256), a.P <= h->panel_cus ? LEAF_LDS : 0, s, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return oxi_set_error(h, OXI_ERR_HIP, "lu_leaf launch: %s", hipGetErrorString(e));
     return OXI_OK;

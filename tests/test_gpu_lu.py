@@ -401,3 +401,19 @@ def test_pivots_equal_lapack_n16384(gpu):
         anorm = torch.linalg.matrix_norm(At).item()
         berr = torch.linalg.matrix_norm(R).item() / (anorm * torch.linalg.matrix_norm(Xt).item() * n * EPS)
         assert berr <= 30, (trans, berr)
+
+
+def test_square_of_more_rows_than_free_cus_take(gpu):
+    """17000 rows: 34 leaf workgroups beside the trailing update, two more than
+    the CUs kept free of it.  Backward error of the factorization and two solves,
+    at most 8 n eps."""
+    import torch
+    n = 17000
+    g = torch.Generator(device="cuda").manual_seed(n)
+    At = torch.randn(n, n, dtype=torch.float64, device="cuda", generator=g)      # columns of A
+    b = torch.randn(n, dtype=torch.float64, device="cuda", generator=g)
+    F = gpu.lu(gpu.DMatrix(At.view(-1), n, n))
+    x = F.solve(gpu.DMatrix(b.clone(), n, 1)).buf
+    r = At.T @ x - b
+    assert r.norm() <= 8 * n * np.finfo(float).eps * (At.norm() * x.norm() + b.norm())
+    assert F.info == 0 and torch.equal(F.ipiv_dev.clamp(1, n), F.ipiv_dev)
