@@ -654,8 +654,10 @@ int choose_tile(i64 m, i64 n, i64 k, i64 batch = 1) {
     // a batch fills the chip with its products together
     const i64 t128 = cdiv(m, 128) * cdiv(n, 128) * batch;
     if (k >= 192 && t128 >= 4 * NCU && (t128 >= 16 * NCU || t128 % NCU == 0 || t128 % NCU >= NCU * 3 / 4)) return 128;
-    if (m <= 32 || n <= 32 || cdiv(m, 64) * cdiv(n, 64) * batch < i64(NCU) * 3 / 2) return 32;
-    return 64;
+    // (no more tiles than a launch takes: tall and narrow ones with over 2^29 rows)
+    const i64 t64 = cdiv(m, 64) * cdiv(n, 64);
+    if ((m <= 32 || n <= 32 || t64 * batch < i64(NCU) * 3 / 2) && cdiv(m, 32) * cdiv(n, 32) < OXI_MAX_WG) return 32;
+    return t64 < OXI_MAX_WG ? 64 : 128;
 }
 
 template <bool TA, bool TB, int MODE = PLAIN>
@@ -710,9 +712,13 @@ int oxi_launch_dgemm(oxi_handle_t h, hipStream_t s, int ta, int tb, i64 m, i64 n
                      const double* A, i64 lda, const double* B, i64 ldb, double beta, double* C, i64 ldc) {
     if (m <= 0 || n <= 0) return OXI_OK;
     if (alpha == 0.0 || k <= 0) return oxi_launch_dscale(s, m, n, beta, C, ldc);
-    if (cdiv(m, 128) * cdiv(n, 128) > (i64(1) << 31) - 1)
-        return oxi_set_error(h, OXI_ERR_UNSUPPORTED, "dgemm: %lld x %lld has too many tiles", (long long)m,
-                             (long long)n);
+    if (cdiv(m, 64) * cdiv(n, 64) >= OXI_MAX_WG) {
+        // more tiles than a launch takes: the longer side in two
+        const i64 hm = m >= n ? cdiv(m / 2, 128) * 128 : 0, hn = m >= n ? 0 : cdiv(n / 2, 128) * 128;
+        OXI_TRY(oxi_launch_dgemm(h, s, ta, tb, hm ? hm : m, hn ? hn : n, k, alpha, A, lda, B, ldb, beta, C, ldc));
+        return oxi_launch_dgemm(h, s, ta, tb, m - hm, n - hn, k, alpha, A + (ta ? hm * lda : hm), lda,
+                                B + (tb ? hn : hn * ldb), ldb, beta, C + hm + hn * ldc, ldc);
+    }
     launch_any<PLAIN>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return oxi_set_error(h, OXI_ERR_HIP, "dgemm launch: %s", hipGetErrorString(e));
@@ -729,7 +735,7 @@ int oxi_launch_dgemm_strided(oxi_handle_t h, hipStream_t s, int ta, int tb, i64 
         for (i64 z = 0; z < batch; ++z) OXI_TRY(oxi_launch_dscale(s, m, n, beta, C + z * sc, ldc));
         return OXI_OK;
     }
-    if (cdiv(m, 32) * cdiv(n, 32) > (i64(1) << 31) - 1)
+    if (cdiv(m, 128) * cdiv(n, 128) >= OXI_MAX_WG)
         return oxi_set_error(h, OXI_ERR_UNSUPPORTED, "dgemm batch: %lld x %lld has too many tiles", (long long)m,
                              (long long)n);
     for (i64 z0 = 0; z0 < batch; z0 += 65535) {
@@ -748,7 +754,7 @@ int oxi_launch_dgemm_ptrs(oxi_handle_t h, hipStream_t s, int ta, int tb, i64 m, 
                           const double* const* A, i64 lda, const double* const* B, i64 ldb, double beta,
                           double* const* C, i64 ldc, i64 batch) {
     if (m <= 0 || n <= 0 || batch <= 0) return OXI_OK;
-    if (cdiv(m, 32) * cdiv(n, 32) > (i64(1) << 31) - 1)
+    if (cdiv(m, 128) * cdiv(n, 128) >= OXI_MAX_WG)
         return oxi_set_error(h, OXI_ERR_UNSUPPORTED, "dgemm batch: %lld x %lld has too many tiles", (long long)m,
                              (long long)n);
     for (i64 z0 = 0; z0 < batch; z0 += 65535) {
@@ -773,7 +779,7 @@ int oxi_launch_dsyrk(oxi_handle_t h, hipStream_t s, int upper, int trans, i64 n,
         hipLaunchKernelGGL(dscale_tri_kernel, dim3(blocks), dim3(256), 0, s, n, beta, C, ldc, upper);
         return hipGetLastError() == hipSuccess ? OXI_OK : oxi_set_error(h, OXI_ERR_HIP, "syrk scale launch");
     }
-    if (cdiv(n, 32) * cdiv(n, 32) > (i64(1) << 31) - 1)
+    if (cdiv(n, 128) * cdiv(n, 128) >= OXI_MAX_WG)
         return oxi_set_error(h, OXI_ERR_UNSUPPORTED, "syrk: n = %lld has too many tiles", (long long)n);
     const int ta = trans ? 1 : 0, tb = trans ? 0 : 1;
     if (upper) launch_any<UPPER>(s, ta, tb, n, n, k, alpha, A, lda, A, lda, beta, C, ldc);

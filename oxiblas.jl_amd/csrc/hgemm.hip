@@ -278,7 +278,7 @@ extern "C" int oxi_hgemm(oxi_handle_t h, char transA, char transB, int64_t m, in
     if (!A) return -8;
     if (!B) return -10;
     const i64 Kp = cdiv(k, HBK) * HBK;
-    if (cdiv(m, 64) * cdiv(n, 64) > (i64(1) << 31) - 1 || cdiv(Kp, 64) > 65535)
+    if (cdiv(m, 128) * cdiv(n, 128) >= OXI_MAX_WG || std::max(cdiv(m, 64), cdiv(n, 64)) >= OXI_MAX_WG || cdiv(Kp, 64) > 65535)
         return oxi_set_error(h, OXI_ERR_UNSUPPORTED, "hgemm: %lld x %lld x %lld is too large", (long long)m, (long long)n,
                              (long long)k);
     // read in place: k contiguous, aligned, no padding, apart from C

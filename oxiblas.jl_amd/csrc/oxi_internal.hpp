@@ -59,6 +59,10 @@ struct oxi_handle_s {
     unsigned leaf_tags = (1u << 27) - 1, leaf_spins = 1u << 22;
 };
 
+// Workgroups of 256 threads in one launch: a grid dimension takes fewer than
+// 2^32 threads.
+constexpr i64 OXI_MAX_WG = i64(1) << 24;
+
 int oxi_set_error(oxi_handle_t h, int code, const char* fmt, ...);
 
 #define OXI_HIP(h, expr)                                                                 \

@@ -440,6 +440,12 @@ int oxi_launch_sgemm(oxi_handle_t h, hipStream_t s, int ta, int tb, i64 m, i64 n
         if (beta == 1.0f) return OXI_OK;
         const int blocks = int(std::min<i64>(cdiv(m * n, 256), 4096));
         hipLaunchKernelGGL(sscale_kernel, dim3(blocks), dim3(256), 0, s, m, n, beta, C, ldc);
+    } else if (cdiv(m, 64) * cdiv(n, 64) >= OXI_MAX_WG) {
+        // more tiles than a launch takes: the longer side in two
+        const i64 hm = m >= n ? cdiv(m / 2, 128) * 128 : 0, hn = m >= n ? 0 : cdiv(n / 2, 128) * 128;
+        OXI_TRY(oxi_launch_sgemm(h, s, ta, tb, hm ? hm : m, hn ? hn : n, k, alpha, A, lda, B, ldb, beta, C, ldc));
+        return oxi_launch_sgemm(h, s, ta, tb, m - hm, n - hn, k, alpha, A + (ta ? hm * lda : hm), lda,
+                                B + (tb ? hn : hn * ldb), ldb, beta, C + hm + hn * ldc, ldc);
     } else if (!ta && !tb) launch_variant<false, false>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
     else if (!ta && tb) launch_variant<false, true>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
     else if (ta && !tb) launch_variant<true, false>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);

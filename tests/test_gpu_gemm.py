@@ -480,3 +480,46 @@ def test_syrk_tile_edges_exact(gpu, n, k, uplo, trans):
     tri = torch.tril if uplo == "L" else torch.triu
     want = tri(full) + C - tri(C)
     assert torch.equal(c.view(n, n + 1)[:, :n].T, want)
+
+
+# More tiles than one launch takes (2^24 workgroups of 256 threads): tall and
+# narrow, wide and low, and with operands that are not read in pairs; small
+# integers, exact.
+@pytest.mark.parametrize("dtype,m,n,k", [("f64", 2 ** 29 + 40, 2, 2), ("f64", 2, 2 ** 29 + 40, 2), ("f64", 2 ** 30 + 70, 1, 1),
+                                         ("f32", 2 ** 30 + 70, 1, 1)])
+def test_more_tiles_than_a_launch_takes(gpu, dtype, m, n, k):
+    import torch
+    dt = torch.float64 if dtype == "f64" else torch.float32
+    g = torch.Generator(device="cuda").manual_seed(7)
+    A = torch.randint(-8, 9, (k, m), generator=g, device="cuda", dtype=torch.int8).to(dt)      # columns
+    B = torch.randint(-8, 9, (n, k), generator=g, device="cuda", dtype=torch.int8).to(dt)
+    C = torch.ones((n, m), dtype=dt, device="cuda")
+    D = gpu.DMatrix
+    (gpu.gemm_ if dtype == "f64" else gpu.sgemm_)(D(C.view(-1), m, n), D(A.view(-1), m, k), D(B.view(-1), k, n), 1.0, 2.0)
+    for j in range(n) if n < m else ():
+        assert torch.equal(C[j], sum(A[p] * B[j, p] for p in range(k)) + 2.0), j
+    for i in range(m) if m < n else ():
+        assert torch.equal(C[:, i], sum(A[p, i] * B[:, p] for p in range(k)) + 2.0), i
+
+
+# Columns too far apart for the 32-bit offsets inside a tile.
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+@pytest.mark.parametrize("which", "AB")
+@pytest.mark.parametrize("trans", "NT")
+def test_columns_far_apart(gpu, dtype, which, trans):
+    import torch
+    dt = torch.float64 if dtype == "f64" else torch.float32
+    g = torch.Generator(device="cuda").manual_seed(5)
+    far, (m, n, k) = (1 << 23) + 5, (37, 35, 5) if which == "A" else (35, 37, 5)
+    ta, tb = (trans, "N") if which == "A" else ("N", trans)
+
+    def mat(r, c, ld):
+        buf = torch.full((ld * (c - 1) + r,), float("nan"), dtype=dt, device="cuda")
+        v = buf.as_strided((c, r), (ld, 1))
+        v.copy_(torch.randint(-8, 9, (c, r), generator=g, device="cuda", dtype=torch.int8).to(dt))
+        return gpu.DMatrix(buf, r, c, ld), v.T.cpu().double().numpy()
+    A, a = mat(*((m, k) if ta == "N" else (k, m)), far if which == "A" else (m if ta == "N" else k))
+    B, b = mat(*((k, n) if tb == "N" else (n, k)), far if which == "B" else (k if tb == "N" else n))
+    C, c = mat(m, n, m)
+    (gpu.gemm_ if dtype == "f64" else gpu.sgemm_)(C, A, B, 2.0, -1.0, ta, tb)
+    np.testing.assert_array_equal(C.numpy(), 2.0 * (op(a, ta) @ op(b, tb)) - c)
