@@ -255,12 +255,14 @@ __global__ __launch_bounds__(256, 1) void trsm_block_kernel(const double* __rest
     const int rows = FULL ? SB : nrows, nsb = (rows + 63) / 64;
     const i64 j0 = i64(blockIdx.x) * C;
     const int nc = int(min(i64(C), nrhs - j0));
+    // the k of a product, four at a time, in solve order
+    auto in_order = [](int e) __attribute__((always_inline)) { return BWD ? 15 - e : e; };
     // this lane's operands of M_pq, and of M_pp^-1 (at 0) or M_pp (at 4096) of block p
     auto load_m = [&](int p, int q, double (&a)[16]) __attribute__((always_inline)) {
         const int i = p * 64 + w * 16 + li, ic = FULL ? i : min(i, rows - 1);
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-            const int k = q * 64 + 4 * e + lk, kc = FULL ? k : min(k, rows - 1);
+            const int k = q * 64 + 4 * in_order(e) + lk, kc = FULL ? k : min(k, rows - 1);
             const double m = TM ? T[kc + i64(ic) * ldt] : T[ic + i64(kc) * ldt];
             a[e] = FULL || (i < rows && k < rows) ? m : 0.0;
         }
@@ -268,15 +270,15 @@ __global__ __launch_bounds__(256, 1) void trsm_block_kernel(const double* __rest
     auto load_v = [&](int p, int off, double (&a)[16]) __attribute__((always_inline)) {
         const double* vp = V + p * 8192 + off + w * 16 + li + 64 * lk;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) a[e] = vp[256 * e];
+        for (int e = 0; e < 16; ++e) a[e] = vp[256 * in_order(e)];
     };
     auto product = [&](const double (&a)[16], const double* x, Mf::acc c) __attribute__((always_inline)) {
         double y[16];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) y[e] = x[(4 * e + lk) * LX + li];
+        for (int e = 0; e < 16; ++e) y[e] = x[(4 * in_order(e) + lk) * LX + li];
         __builtin_amdgcn_sched_barrier(0);   // all of x on its way before the first product
 #pragma unroll
-        for (int e = 0; e < 16; ++e) c = Mf::mul(a[BWD ? 15 - e : e], y[BWD ? 15 - e : e], c);
+        for (int e = 0; e < 16; ++e) c = Mf::mul(a[e], y[e], c);
         return c;
     };
     auto copy = [&](const double (&from)[16], double (&to)[16]) __attribute__((always_inline)) {
