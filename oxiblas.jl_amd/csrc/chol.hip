@@ -355,7 +355,9 @@ int potrf_any(oxi_handle_t h, hipStream_t s, i64 n, T* A, i64 lda, i64* dinfo) {
 int oxi_potrf_device(oxi_handle_t h, hipStream_t s, i64 n, double* A, i64 lda, i64* dinfo) {
     hipLaunchKernelGGL(set_i64_kernel, dim3(1), dim3(64), 0, s, dinfo, i64(0));
     OXI_TRY(launch_check(h, "potrf info"));
-    return potrf_any<double>(h, s, n, A, lda, dinfo);
+    OXI_TRY(oxi_inv_acquire(h, s));
+    OXI_TRY(potrf_any<double>(h, s, n, A, lda, dinfo));
+    return oxi_inv_release(h, s);
 }
 int oxi_potrf_device(oxi_handle_t h, hipStream_t s, i64 n, float* A, i64 lda, i64* dinfo) {
     hipLaunchKernelGGL(set_i64_kernel, dim3(1), dim3(64), 0, s, dinfo, i64(0));

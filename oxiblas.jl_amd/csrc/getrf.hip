@@ -658,6 +658,7 @@ int getrf_t(oxi_handle_t h, i64 m, i64 n, T* A, i64 lda, i64* ipiv, i64 nb, i64*
                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         attr_set = true;
     }
+    if (sizeof(T) == 8) OXI_TRY(oxi_inv_acquire(h, s));   // tall solves with L11; the call ends synchronised
     hipLaunchKernelGGL(zero_i64_kernel, dim3(1), dim3(64), 0, s, g.dinfo, 1);
     hipLaunchKernelGGL(zero_i32_kernel, dim3(1), dim3(64), 0, s, g.flags, 1);
     OXI_TRY(launch_check(h, "zero"));

@@ -29,6 +29,11 @@ struct oxi_handle_s {
     // inverses of 64 x 64 diagonal blocks for tall right-side triangular
     // solves (trsm.hip), TRSM_INV_BLOCKS blocks of 64 x 64 doubles
     double* trsm_inv = nullptr;
+    // the stream of its last use and, once the handle has been used on more than
+    // one stream, an event behind it (oxi_inv_acquire)
+    hipStream_t inv_stream = nullptr;
+    hipEvent_t inv_ev = nullptr;
+    bool inv_used = false, inv_streams = false;
     int panel_cus = 0;
     hipEvent_t ev_a = nullptr, ev_b = nullptr, ev_c = nullptr;
     void* ws = nullptr;                 // device workspace (kernels' scratch)
@@ -118,6 +123,12 @@ int oxi_potrf_device(oxi_handle_t h, hipStream_t s, i64 n, float* A, i64 lda, i6
 bool oxi_dgemm_large(i64 m, i64 n);
 // X[:, 0:64] <- X[:, 0:64] * V in place (V 64 x 64, column-major, ld 64)
 int oxi_dgemm_right64_inplace(hipStream_t s, i64 rows, const double* V, double* X, i64 ldx);
+// The handle's buffer of block inverses, for work on `s` from here to the release:
+// a call on another stream than the last one waits for that one's use.  Nothing
+// is recorded or waited for while `s` is being captured (a graph's replays are
+// the caller's to order).
+int oxi_inv_acquire(oxi_handle_t h, hipStream_t s);
+int oxi_inv_release(oxi_handle_t h, hipStream_t s);
 // Triangular solves, host-recursive with GEMM updates; the right-side one is for
 // factorizations (it shares no scratch memory between streams below 1024 rows).
 int oxi_dtrsm_left(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit, i64 m, i64 nrhs,
@@ -125,7 +136,7 @@ int oxi_dtrsm_left(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit
 int oxi_dtrsm_right(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit, i64 m, i64 n,
                     const double* A, i64 lda, double* B, i64 ldb);
 // The same where no other stream solves at the same time (it takes the handle's
-// buffer of block inverses).
+// buffer of block inverses, which the caller has acquired).
 int oxi_dtrsm_right_alone(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit, i64 m, i64 n,
                           const double* A, i64 lda, double* B, i64 ldb);
 int oxi_strsm_left(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit, i64 m, i64 nrhs,

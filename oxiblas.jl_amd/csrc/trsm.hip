@@ -750,7 +750,11 @@ static bool blocked_applies(oxi_handle_t h, i64 n, i64 other) { return n >= 2 * 
 int oxi_dtrsm_left(oxi_handle_t h, hipStream_t s, int upper, int trans, int unit, i64 m, i64 nrhs, const double* A,
                    i64 lda, double* B, i64 ldb) {
     if (left_strip_applies(m, nrhs)) return trsm_left_strip(h, s, upper, trans, unit, m, nrhs, A, lda, B, ldb);
-    if (blocked_applies(h, m, nrhs)) return trsm_blocked(h, s, true, upper, trans, unit, m, nrhs, A, lda, B, ldb);
+    if (blocked_applies(h, m, nrhs)) {
+        OXI_TRY(oxi_inv_acquire(h, s));
+        OXI_TRY(trsm_blocked(h, s, true, upper, trans, unit, m, nrhs, A, lda, B, ldb));
+        return oxi_inv_release(h, s);
+    }
     return trsm_left_t<double>(h, s, upper, trans, unit, m, nrhs, A, lda, B, ldb);
 }
 // Inside a factorization (rows of B below its panel), on either of its streams.
@@ -825,6 +829,8 @@ extern "C" int oxi_dtrsm(oxi_handle_t h, char side, char uplo, char trans, char 
     }
     if (alpha != 1.0) OXI_TRY(oxi_launch_dscale(s, m, n, alpha, B, ldb));
     if (left) return oxi_dtrsm_left(h, s, upper, tk, unit, m, n, A, lda, B, ldb);
-    return oxi_dtrsm_right_alone(h, s, upper, tk, unit, m, n, A, lda, B, ldb);
+    OXI_TRY(oxi_inv_acquire(h, s));
+    OXI_TRY(oxi_dtrsm_right_alone(h, s, upper, tk, unit, m, n, A, lda, B, ldb));
+    return oxi_inv_release(h, s);
 }
 

@@ -259,3 +259,36 @@ def test_trsm_nonfinite_triangle(gpu, rng, value, side, uplo, trans, n, other):
     first, rest = (slice(lo + 1, None), slice(None, lo + 1)) if up else (slice(None, hi), slice(hi, None))
     assert not np.isfinite(X[rest]).any() and np.isfinite(X[first]).all()
     assert np.abs(X[first] - Xo[first]).max() <= 1e-12 * np.abs(Xo[first]).max() * n
+
+
+@pytest.mark.parametrize("side", "LR")
+def test_solves_on_two_streams(gpu, side):
+    """Calls of one handle on two streams, the second enqueued while the first
+    runs: each gives what it gives alone.  Then a factorization on the second."""
+    import torch
+
+    def make(n, other, seed):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        A = torch.randn(n, n, dtype=torch.float64, device="cuda", generator=g) / n
+        B = torch.randn(other * n, dtype=torch.float64, device="cuda", generator=g)
+        return gpu.DMatrix(A.view(-1), n, n), gpu.DMatrix(B, *((n, other) if side == "L" else (other, n)))
+
+    def solve(A, B, uplo):
+        return gpu.trsm_(B, A, 1.0, side, uplo, "N", True).buf       # a unit diagonal: no synchronisation
+    A1, B1 = make(4001, 3000, 1)
+    A2, B2 = make(1500, 300, 2)
+    S = A2.copy()
+    S.strided().copy_(S.strided() @ S.strided().T + torch.eye(1500, dtype=torch.float64, device="cuda"))
+    want1, want2 = solve(A1, B1.copy(), "L"), solve(A2, B2.copy(), "U")
+    wantC = gpu.cholesky(S).factors.buf
+    torch.cuda.synchronize()
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    for chol in (False, True):
+        X1, X2 = B1.copy(), B2.copy()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s1):
+            got1 = solve(A1, X1, "L")
+        with torch.cuda.stream(s2):
+            got2 = gpu.cholesky(S).factors.buf if chol else solve(A2, X2, "U")
+        torch.cuda.synchronize()
+        assert torch.equal(got1, want1) and torch.equal(got2, wantC if chol else want2)
