@@ -71,9 +71,11 @@ __device__ __forceinline__ void static_for(F&& f) {
 }
 
 // r = sqrt(d) and q = x / r, d the same in every lane.  In FP64, where nothing
-// can overflow or lose bits on the way, the reciprocal that the square root's
-// Newton steps carry along also serves the division, whose result its residual
-// corrects: 14 dependent operations instead of the two library sequences' 40.
+// can overflow or lose bits on the way, by Goldschmidt's iteration from the
+// hardware's estimate of 1 / sqrt(d): g -> sqrt(d) and h -> 1 / (2 sqrt(d))
+// together, then a residual correction of each; 2 h also serves the division,
+// whose result its residual corrects: 14 dependent operations instead of the
+// two library sequences' 40.
 __device__ __forceinline__ void sqrt_div(double d, double x, double& r, double& q) {
     const double y = __builtin_amdgcn_rsq(d);
     double g = d * y, h = 0.5 * y;

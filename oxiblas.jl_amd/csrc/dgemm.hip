@@ -119,8 +119,8 @@ __device__ __forceinline__ void tri_tile_of(int bid, int T, bool upper, int& tm,
 // blockIdx.y of a batch whose operands sit at fixed strides.  PTRS: product
 // blockIdx.y of a batch given by device arrays of operand pointers.  LOWER /
 // UPPER: one product of which only the lower (row >= column) or upper
-// triangle of C is computed and written (syrk!/herk!): tiles outside the
-// triangle leave at once, tiles across the diagonal mask their stores.
+// triangle of C is computed and written (syrk!/herk!): square tiles, of which
+// only the triangle's are launched; those across the diagonal mask their stores.
 enum GemmMode { PLAIN = 0, STRIDED = 1, PTRS = 2, LOWER = 3, UPPER = 4 };
 struct BatchArg {
     i64 sa, sb, sc;                    // STRIDED: element strides between the products' operands
@@ -138,13 +138,6 @@ __device__ __forceinline__ void batch_operands(const BatchArg& ba, const double*
         const int z = blockIdx.y;
         A = ba.pa[z]; B = ba.pb[z]; C = ba.pc[z];
     }
-}
-// false when the BM x BN tile at (m0, n0) has no element in the triangle
-template <int MODE>
-__device__ __forceinline__ bool tile_in_triangle(i64 m0, i64 n0, int BM, int BN) {
-    if (MODE == LOWER) return m0 + BM - 1 >= n0;
-    if (MODE == UPPER) return n0 + BN - 1 >= m0;
-    return true;
 }
 template <int MODE>
 __device__ __forceinline__ bool keep(i64 row, i64 col) {
@@ -181,10 +174,11 @@ __global__ __launch_bounds__(NT) void dgemm_mfma_kernel(i64 M, i64 N, i64 K, dou
     const int lane = t & 63, wave = t >> 6;
     const int wm = wave & 1, wn = wave >> 1;
     int tm, tn;
-    if ((MODE == LOWER || MODE == UPPER) && BM == BN) tri_tile_of(blockIdx.x, tiles_m, MODE == UPPER, tm, tn);
+    constexpr bool TRI = MODE == LOWER || MODE == UPPER;
+    static_assert(!TRI || BM == BN, "square tiles");
+    if (TRI) tri_tile_of(blockIdx.x, tiles_m, MODE == UPPER, tm, tn);
     else tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
     const i64 m0 = i64(tm) * BM, n0 = i64(tn) * BN;
-    if (!tile_in_triangle<MODE>(m0, n0, BM, BN)) return;
     batch_operands<MODE>(ba, A, B, C);
 
     // op(A) rows contiguous when A is 'N'; op(B) columns contiguous when B is 'T'
@@ -212,18 +206,17 @@ __global__ __launch_bounds__(NT) void dgemm_mfma_kernel(i64 M, i64 N, i64 K, dou
     const int kq = lane >> 4, grp = (lane >> 2) & 3, li = lane & 3;
     const int erow = wm * (BM / 2) + 4 * (grp & 1) + kq;
     const int ecol = wn * (BN / 2) + 4 * (grp >> 1) + li;
-    // Tiles inside C (tiles up to 64 x 64) combine with C in a staged layout:
+    // Tiles inside C combine with C in a staged layout:
     // thread t owns row sr = t % BM of columns sc0 + SCS*k, a wave covering
     // BM consecutive rows of a column.  Those C values are loaded before the
     // K loop, so that they travel while the matrix cores run, and without
     // branches (an element outside C reads the nearest one inside; edge tiles
     // do not use them): a load behind a bounds branch is waited for at once.
-    constexpr bool STAGED = BM * BN <= 64 * 64;
-    constexpr int CPT = STAGED ? BM * BN / NT : 1, SCS = NT / BM;
+    constexpr int CPT = BM * BN / NT, SCS = NT / BM;
     const int sr = t % BM, sc0 = t / BM;
     const bool inner = m0 + BM <= M && n0 + BN <= N;
     double cs[CPT];
-    if (STAGED && !BETA0) {
+    if (!BETA0) {
 #pragma unroll
         for (int k = 0; k < CPT; ++k)
             cs[k] = C[min(n0 + sc0 + SCS * k, N - 1) * ldc + min(m0 + sr, M - 1)];
@@ -263,11 +256,11 @@ __global__ __launch_bounds__(NT) void dgemm_mfma_kernel(i64 M, i64 N, i64 K, dou
         __syncthreads();
     }
 
-    if (STAGED && inner) {
+    if (inner) {
         // the accumulators through LDS (the A slabs' space, free after the
         // last barrier: 2 * BK * (BM + 1) >= BN * (BM + 1) doubles), then
         // one coalesced pass over C
-        static_assert(!STAGED || 2 * BK >= BN, "staging space");
+        static_assert(2 * BK >= BN, "staging space");
         double* E = &As[0][0];
 #pragma unroll
         for (int p = 0; p < QN; ++p)
@@ -397,10 +390,11 @@ __global__ __launch_bounds__(NT, OCC) void dgemm_direct_kernel(i64 M, i64 N, i64
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = wave % WM, wn = wave / WM;
     int tm, tn;
-    if ((MODE == LOWER || MODE == UPPER) && BM == BN) tri_tile_of(blockIdx.x, tiles_m, MODE == UPPER, tm, tn);
+    constexpr bool TRI = MODE == LOWER || MODE == UPPER;
+    static_assert(!TRI || BM == BN, "square tiles");
+    if (TRI) tri_tile_of(blockIdx.x, tiles_m, MODE == UPPER, tm, tn);
     else tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
     const i64 m0 = i64(tm) * BM, n0 = i64(tn) * BN;
-    if (!tile_in_triangle<MODE>(m0, n0, BM, BN)) return;
     batch_operands<MODE>(ba, A, B, C);
 
     // this wave's loads of a slab: LA of A's, LB of B's
@@ -594,8 +588,7 @@ template <int BM, int BN, bool TA, bool TB, int MODE = PLAIN>
 void launch_tiles(hipStream_t s, i64 m, i64 n, i64 k, double alpha, const double* A, i64 lda, const double* B,
                   i64 ldb, double beta, double* C, i64 ldc, unsigned batch = 1, BatchArg ba = BatchArg{}) {
     const int tiles_m = int(cdiv(m, BM)), tiles_n = int(cdiv(n, BN));
-    // one triangle of a square grid of square tiles: only its tiles launch
-    const bool tri = (MODE == LOWER || MODE == UPPER) && BM == BN;
+    const bool tri = MODE == LOWER || MODE == UPPER;
     dim3 grid(tri ? tiles_m * (tiles_m + 1) / 2 : tiles_m * tiles_n, batch), block(NT);
     if (beta == 0.0)
         hipLaunchKernelGGL((dgemm_mfma_kernel<BM, BN, TA, TB, true, MODE>), grid, block, 0, s, m, n, k, alpha, A, lda,
@@ -613,8 +606,7 @@ bool launch_direct(hipStream_t s, i64 m, i64 n, i64 k, double alpha, const doubl
     const i64 far = std::max((TA ? BM : BK) * lda, (TB ? BK : BN) * ldb);
     if ((TA ? k : m) < 2 || (TB ? n : k) < 2 || far > (i64(1) << 28)) return false;
     const int tiles_m = int(cdiv(m, BM)), tiles_n = int(cdiv(n, BN));
-    // one triangle of a square grid of square tiles: only its tiles launch
-    const bool tri = (MODE == LOWER || MODE == UPPER) && BM == BN;
+    const bool tri = MODE == LOWER || MODE == UPPER;
     dim3 grid(tri ? tiles_m * (tiles_m + 1) / 2 : tiles_m * tiles_n, batch), block(NT);
     if (beta == 0.0)
         hipLaunchKernelGGL((dgemm_direct_kernel<BM, BN, BK, OCC, TA, TB, true, MODE>), grid, block, 0, s, m, n, k, alpha, A,
@@ -669,7 +661,7 @@ void launch_variant(hipStream_t s, i64 m, i64 n, i64 k, double alpha, const doub
     if (tile >= 64 && launch_direct<64, 64, 16, 4, TA, TB, MODE>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, batch, ba))
         return;
     if (launch_direct<32, 32, 32, 4, TA, TB, MODE>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, batch, ba)) return;
-    // a single row (column, depth) along an operand's columns, or columns a gigabyte apart
+    // a single row (column, depth) along an operand's columns, or columns at least 64 MiB apart
     if (tile >= 64) launch_tiles<64, 64, TA, TB, MODE>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, batch, ba);
     else launch_tiles<32, 32, TA, TB, MODE>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, batch, ba);
 }

@@ -426,7 +426,7 @@ void launch_variant(hipStream_t s, i64 m, i64 n, i64 k, float alpha, const float
     if (tile == 128 && launch_direct<128, 128, 2, TA, TB>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc)) return;
     if (tile >= 64 && launch_direct<64, 64, 4, TA, TB>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc)) return;
     if (launch_direct<32, 32, 4, TA, TB>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc)) return;
-    // fewer than four along an operand's columns, or columns a gigabyte apart
+    // fewer than four along an operand's columns, or columns at least 32 MiB apart
     if (t64 >= NCU * 3 / 2) return launch_tiles<64, 64, TA, TB>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
     return launch_tiles<32, 32, TA, TB>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
 }
