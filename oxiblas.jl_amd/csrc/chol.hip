@@ -312,8 +312,7 @@ int potrf_blocked(oxi_handle_t h, hipStream_t s_caller, i64 n, T* A, i64 lda, i6
     }
     // 512-column blocks over the first half of large matrices (rank-512
     // SYRKs run faster while the trailing matrix is large), POTRF_NB after.
-    // Measured at n = 16384: 256 throughout 43.7 ms, 384 throughout 42.5,
-    // 512 throughout 42.7, this schedule 41.6-41.9 (512 then 384: 41.7-42.3).
+    // n = 16384: 33.5 ms, 256 throughout 36.5, 512 throughout 33.6.
     const i64 nb_wide = n >= 8192 ? 2 * POTRF_NB : POTRF_NB;
     auto nb_at = [&](i64 j) { return std::min<i64>(2 * j < n ? nb_wide : POTRF_NB, n - j); };
     OXI_TRY(panel_factor<T>(h, ms, nb_at(0), n, A, lda, 0, dinfo));
@@ -342,9 +341,8 @@ int potrf_blocked(oxi_handle_t h, hipStream_t s_caller, i64 n, T* A, i64 lda, i6
     return OXI_OK;
 }
 
-// The blocked form from 1024 columns (n = 16384: 53.0 ms against 55.3 ms for
-// the recursion, both with the 256-thread leaf and the triangle-only SYRK
-// grid); OXIBLAS_POTRF_RECURSIVE selects the recursion throughout (tuning).
+// The blocked form from 1024 columns (n = 16384: 33.5 ms against 40.5 ms for
+// the recursion); OXIBLAS_POTRF_RECURSIVE selects the recursion throughout (tuning).
 template <typename T>
 int potrf_any(oxi_handle_t h, hipStream_t s, i64 n, T* A, i64 lda, i64* dinfo) {
     static const bool recursive = getenv("OXIBLAS_POTRF_RECURSIVE") != nullptr;

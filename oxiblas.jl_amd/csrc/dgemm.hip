@@ -370,7 +370,8 @@ __device__ __forceinline__ int paired(int x, i64 last) { return x == last && !(l
 // columns of any length and 8-byte alignment take this path (pairs that start
 // at odd elements are 16-byte loads at 8-byte alignment).  8192^3: 74 TF/s,
 // against 64 with slabs staged through registers; 1500 x 1111 x 777 TN: 79 ->
-// 60 us; 1000 products of 64^3: 55 -> 17 us (5.6 TB/s).  Three and four slabs
+// 55.7 us; 1000 products of 64^3: 61 -> 19.6 us (5.0 TB/s; 16.4 where the caches
+// still hold the inputs).  Three and four slabs
 // deep: slower (68 TF/s for the 128 x 128 tile, 8 deep each).
 template <int BM, int BN, int BK, int OCC, bool TA, bool TB, bool BETA0, int MODE = PLAIN>
 __global__ __launch_bounds__(NT, OCC) void dgemm_direct_kernel(i64 M, i64 N, i64 K, double alpha,
@@ -618,18 +619,19 @@ bool launch_direct(hipStream_t s, i64 m, i64 n, i64 k, double alpha, const doubl
 }
 
 // Tile of C per workgroup, by what was measured over the LU's products and
-// square and long ones (us for 128 / 64 / 32):
+// square and long ones (us a call for 128 / 64 / 32; calls under 8 us are bound by
+// their launch):
 //  - 128 x 128, two workgroups a CU, has the fewest loads a product but waits
 //    longest for C and leaves the most CUs idle in the last pass over the
 //    grid: where K >= 192 and the grid is at least 4 workgroups a CU (4096^3:
-//    1865 / 1980 / 2326; 15872^2 x 256: 2181 / 2232 / 2697; but 7936^2 x 128:
-//    384 / 361 / 476) whose last pass of 256 is nearly full or one of many
-//    (3000^3, 576 tiles: 1134 / 931 / 1033);
+//    1866 / 1968 / 2186; 15872^2 x 256: 2201 / 2241 / 2592; but 7936^2 x 128:
+//    348 / 322 / 430) whose last pass of 256 is nearly full or one of many
+//    (3000^3, 576 tiles: 1071 / 825 / 897);
 //  - 64 x 64, four a CU, where its grid has at least 1.5 workgroups a CU
-//    (1500 x 1111 x 777, 432 tiles: 115 / 60 / 61; 1000^3, 256 tiles:
-//    139 / 48 / 45);
+//    (1500 x 1111 x 777, 432 tiles: 114 / 55.7 / 58; 1000^3, 256 tiles:
+//    136 / 43 / 39.7);
 //  - 32 x 32 below (the LU's look-ahead block, its panel updates, the TRSM
-//    updates; 512^3: 69 / 23 / 9), and where a side is no longer than 32.
+//    updates; 512^3: 70 / 23 / 9), and where a side is no longer than 32.
 // OXIBLAS_DGEMM_TILE (128x128 or m16, 64x64, 32x32) fixes the choice (tuning).
 constexpr int NCU = 256;
 int choose_tile(i64 m, i64 n, i64 k, i64 batch = 1) {

@@ -615,10 +615,8 @@ int getrf_t(oxi_handle_t h, i64 m, i64 n, T* A, i64 lda, i64* ipiv, i64 nb, i64*
     if (nb > PERM_MAX_STEPS) nb = PERM_MAX_STEPS;
     // Tuned block size on large matrices: 512-wide panels while more than 3/8
     // of the columns remain (the trailing update bounds those steps and runs
-    // faster with K = 512), 256 after (the panel bounds them).  Measured on
-    // MI355X at n = 16384: 256 throughout 136 ms, 512 throughout 134 ms.
-    // Wider early panels lose: 768 or 1024 (over 3/8 to 5/8 of the columns)
-    // 117-123 ms against 115 ms for this schedule.
+    // faster with K = 512), 256 after (the panel bounds them).  lu of n = 16384:
+    // 78.7 ms, 256 throughout 81.5, 512 throughout 79.3, 128 throughout 90.2.
     const i64 nb_wide = (tuned && q >= 12288) ? std::min<i64>(2 * nb, PERM_MAX_STEPS) : nb;
     const i64 wide_until = q - (3 * q) / 8;
     auto nb_at = [&](i64 j) { return j < wide_until ? nb_wide : nb; };

@@ -60,11 +60,11 @@ __device__ __forceinline__ void wait_loads() {
 // of row r sits in slot c ^ ((r / 4) % 4), and the 16 lanes that read chunk c
 // of 16 rows touch every bank once.
 // Bound by the matrix cores (1024 cycles of products per 768 of LDS reads a
-// slab and CU for the 256 x 256 tile).  Measured (kernel alone): 4096^3 136 us
-// = 1010 TF/s, 8192^3 1033 TF/s with its packing pass; before, packing both
-// operands, clearing and updating an FP32 C, and a conversion pass around a
-// register-staged 128 x 128 kernel took 269 us at 4096^3 (now 170, of which
-// the transposing pack of A is 12).
+// slab and CU for the 256 x 256 tile).  Measured: 4096^3 131 us = 1050 TF/s with
+// nothing to pack (A transposed), 140 us with A packed, 8192^3 1063 us = 1034 TF/s
+// with its packing pass; before, packing both operands, clearing and updating
+// an FP32 C, and a conversion pass around a register-staged 128 x 128 kernel took
+// 271 us at 4096^3.
 // vec: C 8-byte aligned with ldc a multiple of 4.
 template <int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN) void hgemm_kernel(i64 M, i64 N, i64 K, float aw, float bw, int beta0,
@@ -317,11 +317,11 @@ extern "C" int oxi_hgemm(oxi_handle_t h, char transA, char transB, int64_t m, in
                            s, m, n, Kp, aw, bw, beta0, Ak, ldka, Bk, ldkb, C, ldc, tm, tn, vec);                      \
     } while (0)
     // Rounds over the chip (one 256 x 256 tile a CU, two 128 x 128): a round of
-    // the large tile takes 1.56 times one of the other (K = 4096: 136 and
-    // 87 us), so it is taken where it needs that many fewer rounds (5000^3
-    // 343 us against 411, 4096^3 170 against 213; but 2500^3 99 against 71).
+    // the large tile takes 1.56 times one of the other (K = 4096: 131 and
+    // 84 us), so it is taken where it needs that many fewer rounds (5000^3
+    // 333 us against 393, 4096^3 140 against 177; but 2500^3 96 against 69).
     // Products of fewer than 192 128 x 128 tiles take 64 x 64 ones (1000^3:
-    // 21 us against 30; 512 x 512 x 8192: 54 against 94).
+    // 18.5 us against 27; 512 x 512 x 8192: 54 against 95).
     const i64 t256 = cdiv(m, 256) * cdiv(n, 256), t128 = cdiv(m, 128) * cdiv(n, 128);
     if (t128 < 192) OXI_HGEMM(64, 64, 2, 2);
     else if (156 * cdiv(t256, 256) <= 100 * cdiv(t128, 512)) OXI_HGEMM(256, 256, 2, 4);
