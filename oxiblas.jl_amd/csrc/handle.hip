@@ -45,7 +45,8 @@ int oxi_workspace3(oxi_handle_t h, size_t bytes, void** out) { return grow(h, h-
 
 static bool capturing(hipStream_t s) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) (void)hipGetLastError();
+    return st != hipStreamCaptureStatusNone;
 }
 // An event behind every use costs a short solve 4 us (128 x 16: 43 -> 49 us with the
 // rest of the call), so none is recorded while all uses are on one stream; the

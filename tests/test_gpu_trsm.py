@@ -292,3 +292,29 @@ def test_solves_on_two_streams(gpu, side):
             got2 = gpu.cholesky(S).factors.buf if chol else solve(A2, X2, "U")
         torch.cuda.synchronize()
         assert torch.equal(got1, want1) and torch.equal(got2, wantC if chol else want2)
+
+
+@pytest.mark.parametrize("n,other", [(200, 100), (600, 40)])
+def test_captured_solve(gpu, n, other):
+    """A solve with a unit diagonal neither synchronises nor allocates: captured
+    into a graph, each replay gives what the call gives, with calls between."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n)
+    A = gpu.DMatrix(torch.randn(n * n, dtype=torch.float64, device="cuda", generator=g) / n, n, n)
+    B = torch.randn(n * other, dtype=torch.float64, device="cuda", generator=g)
+    X = gpu.DMatrix(B.clone(), n, other)
+
+    def solve(M):
+        return gpu.trsm_(M, A, 1.0, "L", "L", "N", True).buf
+    want = solve(gpu.DMatrix(B.clone(), n, other)).clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        solve(X)
+    for _ in range(3):
+        X.buf.copy_(B)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(X.buf, want)
+        assert torch.equal(solve(gpu.DMatrix(B.clone(), n, other)), want)
+        torch.cuda.synchronize()
